@@ -320,6 +320,8 @@ int hipml_attn_init(int device)
     if (rc == 0)
         rc = proj_init();
     if (rc == 0)
+        rc = gemm_init();
+    if (rc == 0)
         rc = yardstick_init();
     if (before != device)
         (void)hipSetDevice(before);

@@ -24,34 +24,9 @@
 //   meet in LDS in a fixed order (no atomics: the result does not depend on timing).
 // gemv_q8_tile_kernel (further down): the same stream for 3 to 128 rows, activations as full A tiles.
 
-#include "common.h"
+#include "q8_weights.h"
 
 namespace hipml {
-
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-typedef float float4v __attribute__((ext_vector_type(4)));
-typedef uint32_t uint4v __attribute__((ext_vector_type(4)));
-typedef uint32_t uint2a4 __attribute__((ext_vector_type(2), aligned(4)));
-typedef uint32_t uint3a4 __attribute__((ext_vector_type(3), aligned(4)));
-
-constexpr int kQ8Block = 34;
-
-
-// 8 int8 (two dwords) -> 8 f16 holding the same integers, exactly.
-__device__ __forceinline__ half8 int8x8_to_f16(uint32_t w0, uint32_t w1)
-{
-    const uint32_t x0 = w0 ^ 0x80808080u, x1 = w1 ^ 0x80808080u;
-    const uint32_t hi = 0x64646464u;
-    uint4v r;
-    r[0] = __builtin_amdgcn_perm(hi, x0, 0x04010400u);
-    r[1] = __builtin_amdgcn_perm(hi, x0, 0x04030402u);
-    r[2] = __builtin_amdgcn_perm(hi, x1, 0x04010400u);
-    r[3] = __builtin_amdgcn_perm(hi, x1, 0x04030402u);
-    half8 h = __builtin_bit_cast(half8, r);
-    const half8 off = {1152, 1152, 1152, 1152, 1152, 1152, 1152, 1152};
-    return h - off;
-}
 
 // 8 f32 -> hi and lo f16 halves with hi + lo = x to ~22 bits.
 __device__ __forceinline__ void split_hi_lo(const float4v &a, const float4v &b, half8 &hi, half8 &lo)
@@ -1268,312 +1243,6 @@ int launch_gemv_q8_rows(hipStream_t st, const uint8_t *w, const float *x, float 
 }
 
 
-// ---- gemm_q8_f16_kernel: many activation rows (a prefill chunk) ---------------------------------
-//
-// y[t][row] for a 128 (tokens) x 128 (weight rows) tile per workgroup, MFMA-bound:
-// v_mfma_f32_32x32x16_f16 with A = x (f32 -> f16, round to nearest), B = W dequantized to f16 (d*q, one
-// rounding: the precision class of the reference's f16-operand prefill kernels and of this library's
-// chunk attention), fp32 accumulation.  Four consumer waves, each a 64 x 64 piece (2 x 2 MFMA tiles),
-// and eight producer waves that fetch and stage.  A k step is 64 values = one 68-byte pair of blocks per
-// weight row; both operand tiles are staged as [128 rows][64 f16] with a 144-byte row pitch (128-bit
-// reads and writes of 16 consecutive rows then touch every bank once), double buffered, one barrier
-// per step.  A fetch record is refilled as soon as it has been staged.  (One set of four waves doing
-// both, interleaved by hand MFMA by MFMA, took 1,600 cycles per step with a single workgroup on the
-// CU: every wait left its SIMD idle.)
-// Weight fetch uses the lane order of the row kernel above (quad = the four quarters of a pair of
-// blocks, dword-aligned loads).
-// X16: the activations arrive as f16 (written by gate_f16_kernel below).  With f32 activations a
-// step moves 32 KB of them through the CU's 64-byte-per-cycle vector memory path -- more cycles
-// than the step's MFMAs take (measured: 700 of a step's 2,200 cycles are spent issuing loads) -- and
-// every one of the m/128 workgroups of a token tile repeats that; f16 halves it and drops the
-// conversion.
-
-
-typedef float float16v __attribute__((ext_vector_type(16)));
-typedef _Float16 half4v __attribute__((ext_vector_type(4)));
-
-constexpr int kGemmT = 128, kGemmM = 128;
-constexpr int kGemmUnits = 1;                     // 64-value units (pairs of blocks) per step
-constexpr int kGemmK = 64 * kGemmUnits;           // values per step
-constexpr int kGemmPitch = kGemmK * 2 + 16;       // 144: an odd number of 16-byte groups
-constexpr int kGemmTile = 128 * kGemmPitch;       // one operand tile
-constexpr int kGemmBuf = 2 * kGemmTile;           // x tile + w tile
-constexpr int kGemmLds = 2 * kGemmBuf;            // double buffered: 73,728 bytes
-constexpr int kGemmWaves = 8;                     // producer waves
-constexpr int kGemmCWaves = 4;                    // consumer waves
-
-// What one producer thread fetches for one step: per unit WN weight (row, quarter) pairs, and XN
-// 16-byte pieces of the activation tile.
-template <int WN, int XN>
-struct GemmFetch {
-    uint3a4 e[kGemmUnits][WN];   // even-block quarter (+ scales in quad lanes 0 and 3)
-    uint2a4 o[kGemmUnits][WN];   // odd-block quarter
-    float4v x[XN];               // f32: 4 activations; f16: 8
-};
-
-// 8 exact integer f16 times the block scale (f16): the product has at most 19 significant bits and
-// is rounded once, as f16(d * q) is.
-__device__ __forceinline__ half8 dequant8(uint32_t w0, uint32_t w1, _Float16 d)
-{
-    const half8 q = int8x8_to_f16(w0, w1);
-    const half8 dv = {d, d, d, d, d, d, d, d};
-    return q * dv;
-}
-
-// kGemmCWaves consumer waves first, then NW producer waves: 4 + 8.  Consumers own 64 x 64 pieces
-// (2 x 2 MFMA tiles: every operand read feeds two MFMAs, 64 KB of LDS reads per step instead of the
-// 96 KB of eight 32 x 64 pieces), producers one weight (row, quarter) pair and two activation pieces
-// per thread and step.  LDS serves a wave at about 34 B/clk for 128-bit reads and 16-20 B/clk for
-// 128-bit writes whatever the others do, up to well over 128 B/clk in all (measured), so eight
-// producer waves stage a tile in less time than four.  Measured at 5120 x 6144, 672 tokens, gate
-// pass included: 4 + 4 waves 77.3, 8 + 8 waves 76.5, 4 + 8 waves 71.6 us.
-template <bool X16, int NW>
-__global__ void __launch_bounds__(64 * (NW + kGemmCWaves)) gemm_q8_f16_kernel(const uint8_t *__restrict__ w,
-                                                              const void *__restrict__ xv,
-                                                              float *__restrict__ y, int m, int k, int tokens)
-{
-    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-    constexpr int NT = 64 * NW; // producer threads
-    constexpr int NC = kGemmCWaves;
-    constexpr int KU = kGemmUnits;
-    const bool producer = threadIdx.x >= 64 * NC;
-    const int tid = producer ? threadIdx.x - 64 * NC : threadIdx.x;
-    const int wave = tid >> 6, lane = tid & 63; // within the role
-    const int m0 = blockIdx.x * kGemmM, t0 = blockIdx.y * kGemmT;
-    const int nunits = k >> 6;
-    const int nsteps = (nunits + KU - 1) / KU;   // the last step may hold fewer units: zero weights
-    const size_t row_bytes = (size_t)(k >> 5) * kQ8Block;
-    constexpr int WN = 512 / NT;                 // weight (row, quarter) pairs per producer thread and unit
-    constexpr int WROWS = NT / 4;                // rows covered by one such pair of the workgroup
-    constexpr int XELT = X16 ? 2 : 4;            // bytes per activation
-    constexpr int XV = 16 / XELT;                // activations per 16-byte piece
-    constexpr int XPR = kGemmK / XV;             // pieces per tile row
-    constexpr int XN = 128 * XPR / NT;           // pieces per producer thread
-    constexpr int XROWS = NT / XPR;              // rows covered by one piece of the workgroup
-
-    // fetch roles
-    const int fr = tid >> 2, fg = tid & 3; // weight rows fr + WROWS h, k quarter fg of each block
-    const uint8_t *wp[WN];
-#pragma unroll
-    for (int h = 0; h < WN; h++) {
-        const int row = m0 + fr + WROWS * h < m ? m0 + fr + WROWS * h : m - 1;
-        wp[h] = w + (size_t)row * row_bytes + fg * 8;
-    }
-    // activations: 16 bytes per load, XPR consecutive lanes cover a tile row
-    const int xr = tid / XPR, xc = tid % XPR;
-    const uint8_t *xp[XN];
-#pragma unroll
-    for (int i = 0; i < XN; i++) {
-        const int t = t0 + xr + XROWS * i < tokens ? t0 + xr + XROWS * i : tokens - 1;
-        xp[i] = static_cast<const uint8_t *>(xv) + ((size_t)t * k) * XELT;
-    }
-    typedef GemmFetch<WN, XN> Fetch;
-    auto fetch = [&](Fetch &f, int s) {
-        const int sc = s < nsteps ? s : nsteps - 1;
-#pragma unroll
-        for (int u = 0; u < KU; u++) {
-            const int g = sc * KU + u < nunits ? sc * KU + u : nunits - 1;
-#pragma unroll
-            for (int h = 0; h < WN; h++) {
-                const uint8_t *unit = wp[h] + (size_t)g * (2 * kQ8Block);
-                f.e[u][h] = *reinterpret_cast<const uint3a4 *>(unit);
-                f.o[u][h] = *reinterpret_cast<const uint2a4 *>(unit + 36);
-            }
-        }
-        // a piece past the end of the row (second unit of a short last step) repeats the row's last
-        // piece: it meets zero weights
-        int kx = sc * kGemmK + xc * XV;
-        if (KU > 1)
-            kx = kx + XV <= k ? kx : k - XV;
-#pragma unroll
-        for (int i = 0; i < XN; i++)
-            f.x[i] = *reinterpret_cast<const float4v *>(xp[i] + (size_t)kx * XELT);
-    };
-    auto stage = [&](const Fetch &f, uint8_t *buf, int s) {
-        uint8_t *xt = buf, *wt = buf + kGemmTile;
-#pragma unroll
-        for (int i = 0; i < XN; i++) {
-            if (X16) {
-                *reinterpret_cast<float4v *>(xt + (xr + XROWS * i) * kGemmPitch + xc * 16) = f.x[i];
-            } else {
-                // round to nearest even (v_cvt_pk_f16_f32): truncation would bias every product the same way
-                const half4v v = __builtin_convertvector(f.x[i], half4v);
-                *reinterpret_cast<half4v *>(xt + (xr + XROWS * i) * kGemmPitch + xc * 8) = v;
-            }
-        }
-#pragma unroll
-        for (int u = 0; u < KU; u++) {
-            const bool live = KU == 1 || s * KU + u < nunits;
-#pragma unroll
-            for (int h = 0; h < WN; h++) {
-                const uint3a4 e = f.e[u][h];
-                const uint32_t s0 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)e[0], 0x00, 0xf, 0xf, true);
-                const uint32_t s1 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)e[2], 0xFF, 0xf, 0xf, true);
-                const _Float16 d0 = __builtin_bit_cast(_Float16, (uint16_t)(live ? s0 & 0xffffu : 0u));
-                const _Float16 d1 = __builtin_bit_cast(_Float16, (uint16_t)(live ? s1 >> 16 : 0u));
-                const half8 v0 = dequant8(__builtin_amdgcn_alignbit(e[1], e[0], 16),
-                                          __builtin_amdgcn_alignbit(e[2], e[1], 16), d0);
-                const half8 v1 = dequant8(f.o[u][h][0], f.o[u][h][1], d1);
-                uint8_t *dst = wt + (fr + WROWS * h) * kGemmPitch + u * 128 + fg * 16;
-                *reinterpret_cast<half8 *>(dst) = v0;        // k = fg*8 .. of the even block
-                *reinterpret_cast<half8 *>(dst + 64) = v1;   // k = 32 + fg*8 .. (the odd block)
-            }
-        }
-    };
-
-    // MFMA roles: consumer wave (wt, wm) owns AT 32-token tiles from token wt * 32 AT and weight rows
-    // wm*64..: 64 x 64 per wave with four consumers, 32 x 64 with eight
-    constexpr int AT = 8 / NC;
-    const int wt_ = wave >> 1, wm_ = wave & 1;
-    const int ln = lane & 31, lh = lane >> 5;
-    float16v acc[AT][2];
-#pragma unroll
-    for (int a = 0; a < AT; a++)
-#pragma unroll
-        for (int b = 0; b < 2; b++)
-#pragma unroll
-            for (int i = 0; i < 16; i++)
-                acc[a][b][i] = 0.0f;
-    // All operands of a step are named first and the scheduling groups below pin the order: the reads
-    // of the first 16 values of k, then one MFMA and one read in turn, so that a read's LDS latency
-    // is covered by MFMAs (left to itself the compiler read, waited, multiplied: 840 cycles per step
-    // for 512 of MFMA).
-    auto multiply = [&](const uint8_t *buf) {
-        const uint8_t *xa = buf + (wt_ * 32 * AT + ln) * kGemmPitch + lh * 16;
-        const uint8_t *wb = buf + kGemmTile + (wm_ * 64 + ln) * kGemmPitch + lh * 16;
-        half8 A[4 * KU][AT], B[4 * KU][2];
-#pragma unroll
-        for (int kk = 0; kk < 4 * KU; kk++) {
-#pragma unroll
-            for (int a = 0; a < AT; a++)
-                A[kk][a] = *reinterpret_cast<const half8 *>(xa + a * 32 * kGemmPitch + kk * 32);
-#pragma unroll
-            for (int b = 0; b < 2; b++)
-                B[kk][b] = *reinterpret_cast<const half8 *>(wb + b * 32 * kGemmPitch + kk * 32);
-        }
-#pragma unroll
-        for (int kk = 0; kk < 4 * KU; kk++)
-#pragma unroll
-            for (int a = 0; a < AT; a++)
-#pragma unroll
-                for (int b = 0; b < 2; b++)
-                    acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[kk][a], B[kk][b], acc[a][b], 0, 0, 0);
-        constexpr int per = AT + 2;             // reads per 16 values of k
-        constexpr int reads = 4 * KU * per, mfmas = 4 * KU * AT * 2;
-        __builtin_amdgcn_sched_group_barrier(0x100, per, 0);
-#pragma unroll
-        for (int i = 0; i < reads - per; i++) {
-            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-            __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-        }
-        __builtin_amdgcn_sched_group_barrier(0x008, mfmas - (reads - per), 0);
-    };
-
-    // The second half of the waves produce (fetch, dequantize, write the next step's tiles), the first
-    // half consume (operand reads and MFMAs of the current step); one barrier per step hands a buffer
-    // over.  A SIMD holds waves of both kinds, and a VALU wave and an MFMA wave of one SIMD issue side
-    // by side.  (Two units per step, half as many barriers, measured slower: 76.5 against 72.8 us at
-    // 672 tokens.)
-    if (producer) {
-        // Four fetch records in rotation: a record is refilled as soon as it has been staged and is
-        // staged again four steps later, so its loads have three steps to arrive (with two records the
-        // producers spent 860 cycles of a 1,400-cycle step waiting for them).  Four steps per turn keep
-        // the records in the same registers; a fetch past the last step repeats it.
-        Fetch r0, r1, r2, r3;
-        fetch(r0, 0);
-        fetch(r1, 1);
-        fetch(r2, 2);
-        fetch(r3, 3);
-        stage(r0, lds, 0);
-        fetch(r0, 4);
-        __syncthreads();
-        int s = 0;
-        for (; s + 4 <= nsteps; s += 4) {
-            stage(r1, lds + kGemmBuf, s + 1); // step s + 1, while step s is multiplied
-            fetch(r1, s + 5);
-            __syncthreads();
-            stage(r2, lds, s + 2);
-            fetch(r2, s + 6);
-            __syncthreads();
-            stage(r3, lds + kGemmBuf, s + 3);
-            fetch(r3, s + 7);
-            __syncthreads();
-            stage(r0, lds, s + 4);            // step s + 4
-            fetch(r0, s + 8);
-            __syncthreads();
-        }
-        // the last one to three steps: their records are already on the way
-        const int rest = nsteps - s;
-        if (rest >= 1) {
-            if (rest >= 2)
-                stage(r1, lds + kGemmBuf, s + 1);
-            __syncthreads();
-        }
-        if (rest >= 2) {
-            if (rest >= 3)
-                stage(r2, lds, s + 2);
-            __syncthreads();
-        }
-        if (rest >= 3)
-            __syncthreads();
-        return;
-    }
-    __syncthreads();
-    for (int s = 0; s + 2 <= nsteps; s += 2) {
-        multiply(lds);
-        __syncthreads();
-        multiply(lds + kGemmBuf);
-        __syncthreads();
-    }
-    if (nsteps & 1) {
-        multiply(lds);
-        __syncthreads();
-    }
-
-    // C tile: lane holds column ln (weight row), rows (i/4)*8 + lh*4 + i%4 (tokens)
-#pragma unroll
-    for (int a = 0; a < AT; a++)
-#pragma unroll
-        for (int b = 0; b < 2; b++) {
-            const int row = m0 + wm_ * 64 + b * 32 + ln;
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const int t = t0 + wt_ * 32 * AT + a * 32 + (i >> 2) * 8 + lh * 4 + (i & 3);
-                if (t < tokens && row < m)
-                    y[(size_t)t * m + row] = acc[a][b][i];
-            }
-        }
-}
-
-// x16[i] = f16(x[i] * sigmoid(gate[i])) (gate may be null: plain conversion), 8 values per thread.
-// The gate is the expression every gating kernel of this library uses, the rounding the one the
-// f32-activation GEMM applies when it stages x: the two routes give the same bits.
-__global__ void __launch_bounds__(256) gate_f16_kernel(const float4v *__restrict__ x,
-                                                      const float4v *__restrict__ gate,
-                                                      half8 *__restrict__ x16, size_t n8)
-{
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n8)
-        return;
-    float4v a = x[2 * i], b = x[2 * i + 1];
-    if (gate != nullptr) {
-        const float4v ga = gate[2 * i], gb = gate[2 * i + 1];
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            a[j] = gated(a[j], ga[j]);
-            b[j] = gated(b[j], gb[j]);
-        }
-    }
-    const half4v ha = __builtin_convertvector(a, half4v), hb = __builtin_convertvector(b, half4v);
-    half8 h;
-#pragma unroll
-    for (int j = 0; j < 4; j++) {
-        h[j] = ha[j];
-        h[4 + j] = hb[j];
-    }
-    x16[i] = h;
-}
-
 template <int WAVES, int TILES, int CH>
 static hipError_t raise_gemv_lds()
 {
@@ -1590,13 +1259,7 @@ static hipError_t raise_gemv_lds()
 
 int proj_init()
 {
-    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_q8_f16_kernel<false, kGemmWaves>),
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, kGemmLds);
-    if (e == hipSuccess)
-        e = hipFuncSetAttribute(reinterpret_cast<const void *>(&gemm_q8_f16_kernel<true, kGemmWaves>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, kGemmLds);
-    if (e == hipSuccess)
-        e = raise_gemv_lds<8, 1, 6>();
+    hipError_t e = raise_gemv_lds<8, 1, 6>();
     auto raise = [&](const void *f) {
         if (e == hipSuccess)
             e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 << 10);
@@ -1626,31 +1289,6 @@ int proj_init()
     if (e != hipSuccess)
         return fail((int)e, "hipFuncSetAttribute(projection LDS) failed: %d (%s)", (int)e, hipGetErrorString(e));
     return 0;
-}
-
-// x16 != nullptr: gate (optional) and convert into x16 first, then the GEMM over f16 activations;
-// x == nullptr: x16 already holds them.
-int launch_gemm_q8_f16(hipStream_t st, const uint8_t *w, const float *x, const float *gate, float *y, int m,
-                       int k, int tokens, void *x16)
-{
-    const dim3 grid((unsigned)((m + kGemmM - 1) / kGemmM), (unsigned)((tokens + kGemmT - 1) / kGemmT), 1);
-    if (x16 == nullptr) {
-        HIPML_LAUNCH((gemm_q8_f16_kernel<false, kGemmWaves>), grid, dim3(64 * (kGemmWaves + kGemmCWaves), 1, 1), kGemmLds,
-                           st, w, x, y, m, k, tokens);
-        return launched("gemm_q8_0_f16");
-    }
-    if (x != nullptr) {
-        const size_t n8 = (size_t)tokens * k / 8;
-        HIPML_LAUNCH(gate_f16_kernel, dim3((unsigned)((n8 + 255) / 256), 1, 1), dim3(256, 1, 1), 0, st,
-                           reinterpret_cast<const float4v *>(x), reinterpret_cast<const float4v *>(gate),
-                           static_cast<half8 *>(x16), n8);
-        int rc = launched("gate_f16");
-        if (rc)
-            return rc;
-    }
-    HIPML_LAUNCH((gemm_q8_f16_kernel<true, kGemmWaves>), grid, dim3(64 * (kGemmWaves + kGemmCWaves), 1, 1), kGemmLds, st, w,
-                       x16, y, m, k, tokens);
-    return launched("gemm_q8_0_f16");
 }
 
 } // namespace hipml

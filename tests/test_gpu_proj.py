@@ -312,3 +312,27 @@ def test_qkv_projection_shapes(m, k):
     assert ok
     ok, _, _ = report(f"chunk {m}x{k} t=3", want, run_gemm(w, x, m, k, 3), *F16_LARGE)
     assert ok
+
+
+@pytest.mark.parametrize("m,k,t", [(33, 256, 33), (1029, 512, 301), (1029, 256, 700), (6000, 256, 300),
+                                   (5000, 256, 700), (8000, 256, 700), (5100, 256, 1000), (9001, 192, 700),
+                                   (12270, 128, 1001), (5, 192, 70)])
+def test_gemm_tiles(m, k, t):
+    # one shape per tile of the chunk GEMM (32 x 32 up to 256 x 192), ragged in both directions, an odd number of
+    # 64-value units among them; against its own definition, from f32 and from f16 activations, and a row's bits the
+    # same in a chunk of its own (the smallest tile)
+    r = orc.Rng(0x6E00 + m + t)
+    w = orc.random_q8_0_bytes(r, m * k // 32).reshape(-1, 34)
+    scales = (r.uniform_array(w.shape[0]) * 0.05 + 0.001).astype(np.float16)
+    w[:, :2] = scales.view(np.uint8).reshape(-1, 2)
+    w = w.ravel()
+    x = r.normal_array((t, k))
+    got = run_gemm(w, x, m, k, t)
+    want = f16_operand_reference(w, x, m, k)
+    assert np.max(np.abs(got - want)) < 2e-5 * np.sqrt(k) * max(1.0, np.abs(want).max() / 8)
+    y16 = torch.full((t, m), float("nan"), dtype=torch.float32, device="cuda")
+    attn.output_chunk_q8_0(dev(w), None, None, y16, m, k, t, dev(x).to(torch.float16))
+    torch.cuda.synchronize()
+    assert np.array_equal(host(y16), got)
+    for i in (0, t // 2, t - 1):
+        assert np.array_equal(run_gemm(w, x[i:i + 1], m, k, 1)[0], got[i])
