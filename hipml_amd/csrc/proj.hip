@@ -4,7 +4,8 @@
 // W is [m][k/32] blocks of 34 bytes (f16 scale d, 32 int8), row-major; y[r][row] = sum_k W[row][k] x[r][k]
 // (crates/hipml-core/src/quant.rs:653-675, crates/hipml-core/src/ops.rs:102-104,136-176).
 //
-// gemv_q8_rows_kernel: one or two activation rows, bound by streaming W once from HBM.
+// gemv_q8_rows_kernel: one or two activation rows over shapes the raw-row kernel does not take, bound by streaming W
+// once from HBM.
 //   All MFMAs are v_mfma_f32_16x16x32_f16 with A = x (activation rows), B = W (16 weight rows),
 //   one q8 block = one contraction, so the f16 block scale multiplies an exact integer dot product
 //   in fp32: acc += d * (x . q), as the CPU definition's d*q products summed in fp32.
@@ -22,9 +23,11 @@
 //   The waves of a workgroup split k; a wave requests the activations first, then two chunks of
 //   its weight blocks (all of them for k = 6144) before it waits for anything, and the partial sums
 //   meet in LDS in a fixed order (no atomics: the result does not depend on timing).
-// gemv_q8_tile_kernel (further down): the same stream for 3 to 128 rows, activations as full A tiles.
+// gemv_q8_dma_kernel: one to eight rows; gemv_q8_blocks_kernel: more (both further down).
 
 #include "q8_weights.h"
+
+#include <type_traits>
 
 namespace hipml {
 
@@ -36,13 +39,15 @@ __device__ __forceinline__ void split_hi_lo(const float4v &a, const float4v &b, 
         const float x0 = j < 2 ? a[2 * j] : b[2 * j - 4];
         const float x1 = j < 2 ? a[2 * j + 1] : b[2 * j - 3];
         const half2v h = __builtin_bit_cast(half2v, __builtin_amdgcn_cvt_pkrtz(x0, x1));
-        // x - h (exact: h holds the leading bits of x) in one mixed-precision instruction per value, which reads
-        // the f16 half in place; the compiler turns the same expression into a conversion and a subtraction
+        // x - h (exact: h holds the leading bits of x), rounded to f16 by the same instruction, which reads the f16
+        // half in place: one per value where the compiler makes two conversions and a subtraction
         const uint32_t hb = __builtin_bit_cast(uint32_t, h);
-        float r0, r1;
-        asm("v_fma_mix_f32 %0, -%1, 1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r0) : "v"(hb), "v"(x0));
-        asm("v_fma_mix_f32 %0, -%1, 1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r1) : "v"(hb), "v"(x1));
-        const half2v l = __builtin_bit_cast(half2v, __builtin_amdgcn_cvt_pkrtz(r0, r1));
+        uint32_t lb;
+        asm("v_fma_mixlo_f16 %0, -%1, 1.0, %2 op_sel_hi:[1,0,0]\n\t"
+            "v_fma_mixhi_f16 %0, -%1, 1.0, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]"
+            : "=&v"(lb)
+            : "v"(hb), "v"(x0), "v"(x1));
+        const half2v l = __builtin_bit_cast(half2v, lb);
         hi[2 * j] = h[0];
         hi[2 * j + 1] = h[1];
         lo[2 * j] = l[0];
@@ -661,216 +666,226 @@ __global__ void __launch_bounds__(64 * WAVES, 1) gemv_q8_dma_kernel(const uint8_
     }
 }
 
-// ---- gemv_q8_dma_tile_kernel: 10 to 128 activation rows over the same stream of raw weight rows, 64 a pass ------
+// ---- 9 to 128 activation rows (verify groups, batched decode): two kernels ---------------------------------------
 //
-// More rows than the kernel above holds operands for.  The workgroups are the same (rows_wg consecutive weight
-// rows, one workgroup per CU, eight waves), but the waves walk the chunks together: for a chunk of 256 values the
-// workgroup fetches its weight rows and the same 256 values of every activation row as raw f32 (1 KB per row, all
-// through global_load_lds_dwordx4, the requests dealt to the waves), and wave w multiplies block w of the chunk.  So
-// a workgroup reads every activation once, from LDS.
-// Lane (row lm, quarter lg) of an A tile reads its 8 floats and splits them into hi and lo halves in registers;
-// a block and tile is two chained MFMAs (hi, then lo into the same fp32 sums) per weight tile, the weights exactly as
-// f16 integers (1024 + u trick), the block scale applied to the fp32 dot product.  The activation rows lie 1,040
-// bytes apart in LDS, so the 16 rows of a tile start in 16 different banks.
-// Two rings: kDW chunks of weights and kDX chunks of activations are in flight, two barriers per chunk.  Vector
-// memory returns in order, so a wave that waits for its activation requests of a chunk also waits for every weight
-// request it made before them: the activations of chunk c + kDX are asked for before the weights of chunk c + kDW,
-// and the wait counts the activation requests behind it only.
-// A (row, weight row) result is the sum in wave order of eight chains (block b of every chunk belongs to chain b):
-// the same whatever the number of rows, and other bits than those of the kernel for up to 8 rows.
-constexpr int kTileRowPitch = 1040;
-// (chunks of activations / of weights in flight, measured at 5120 x 6144 over 16 / 24 / 32 / 64 rows: 2 / 3: 17.5 / 23.4 /
-// 23.5 / 39.8 us; 2 / 4: 17.9 / 29.0 / 29.1 / 41.4; 3 / 6: 18.3 / 25.5 / 25.6 / -; the tile kernel below: 19.6 / 25.8 / 29.7 /
-// 54.5.  The figures for 24 and 32 rows move between 23.4 and 29.6 us from run to run of the same build, those for 16 and 64
-// do not.  Two chunks a turn of the loop, half the barriers: 20.5 / 26.7 / 26.9 against 17.5 / 29.6 / 29.7 in one run; every
-// workgroup starting at another chunk, so that they do not all ask for the same activation bytes at once: 20.8 / 24.3 / 24.5 /
-// 39.2 against 17.4 / 23.4 / 23.5 / 39.7 in one run.  Not fetching the 8 rows of a last tile that has no more than 8 live
-// ones (HALF): 17 and 24 rows 21.9 us where 32 rows take 23.5, 33 and 40 rows 34.7 / 34.8 where 48 take 35.1.  Sixteen waves,
-// two per block of a chunk with one weight tile each: 18.4 / 24.9 / 45.9 us at 16 / 24 / 64 rows against 17.0 / 22.7 / 34.0.)
-constexpr int gemv_tile_dx(int) { return 2; }
-constexpr int gemv_tile_dw(int) { return 3; }
-inline int gemv_dma_tile_lds(int xt, int ni, int rows_wg)
-{
-    const int ring = gemv_tile_dw(xt) * rows_wg * 17 * 16 + gemv_tile_dx(xt) * 16 * xt * kTileRowPitch;
-    const int sums = 8 * xt * gemv_dma_tiles(ni) * 64 * 16;
-    return ring > sums ? ring : sums;
-}
+// More rows than the kernel above holds operands for.  In both, a workgroup takes RW weight rows and XT tiles of 16
+// activation rows; weights and f32 activations travel by global_load_lds as they lie in memory, into a ring, and from
+// there to registers while what came before them is multiplied.  A lane (row lm, quarter lg) splits its 8 floats of a
+// tile and block into hi and lo halves; a block and pair of tiles is two chained MFMAs (hi, then lo into the same fp32
+// sums), the weights exactly as f16 integers (1024 + u trick), the block scale applied to the fp32 dot product.  The
+// 16-byte pieces of an activation row lie in LDS at piece ^ row, so that the rows of a tile start in different banks
+// without padding.  A result is a sum over eight chains of blocks in fixed order: its bits depend on the shape of W
+// (which picks the kernel), not on the number of rows, tiles and weight rows per workgroup.
+//
+// What bounds them: vector instructions (bytes to f16, hi / lo split, scaling of block products: a single wave issues
+// one per 8 cycles, so a SIMD needs two), requests (~16 cycles of a CU each, whatever their size), and ~4 us of launch,
+// first data and final sum.
+//
+// gemv_q8_units_kernel (m up to 6,144; any k of whole 64-value units, W at a 4-byte boundary): no barrier, a wave
+// streams units of its own.  gemv_q8_blocks_kernel (more rows, k of whole 256-value chunks, W at a 16-byte boundary):
+// the workgroup walks chunks together and shares 16-byte requests for the weights, where units take four times as many
+// dword requests, which tell where a workgroup has 48 weight rows.  us over 24 rows, units / blocks / the kernel before
+// them (eight waves in step, a block of each chunk per wave, two barriers per chunk): 1024 x 5120 9.7 / 12.0 / 14.0,
+// 5120 x 6144 17.0 / 21.3 / 23.6, 12288 x 5120 26.1 / 23.4 / 38.6.
 
-template <int XT, int NI, bool HALF>
-__global__ void __launch_bounds__(512, 1) gemv_q8_dma_tile_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x,
-                                                                   float *__restrict__ y, int m, int k, int rows,
-                                                                   int rows_wg)
+template <int XT, int RW, bool HALF>
+struct BlocksShape {
+    static constexpr int kMT = (RW + 15) / 16;              // weight tiles
+    static constexpr int kXRows = 16 * XT - (HALF ? 8 : 0); // activation rows that are fetched
+    static constexpr int kWBytes = RW * kDmaChunkBytes;
+    static constexpr int kXWave = kXRows * 128;             // one wave's block of them
+    static constexpr int kSlot = kWBytes + 8 * kXWave;
+    static constexpr int kFit = (160 << 10) / kSlot;
+    static constexpr int kDepth = kFit < 5 ? kFit : 5; // chunks in flight
+    static constexpr int kSums = 8 * XT * kMT * 1024;
+    static constexpr int kRead = HALF ? 1024 : 0; // (a HALF tile's dead rows are read past the wave's block)
+    static constexpr int kLds = (kDepth * kSlot > kSums ? kDepth * kSlot : kSums) + kRead;
+    static_assert(kDepth >= 2 && kLds <= 160 << 10, "");
+};
+
+// Wave w multiplies block w of a chunk of 256 values.  One barrier per chunk: behind it chunk c + 1 has arrived for
+// everybody, and everybody has moved chunk c to registers, so that its place is asked for anew at once.  HALF: the last
+// tile has at most 8 live rows; the other 8 are never fetched, hold whatever the LDS held, and are never stored.
+template <int XT, int RW, bool HALF>
+__global__ void __launch_bounds__(512, 2) gemv_q8_blocks_kernel(const uint8_t *__restrict__ w,
+                                                                const float *__restrict__ x, float *__restrict__ y,
+                                                                int m, int k, int rows)
 {
-    constexpr int kNT = gemv_dma_tiles(NI);
-    constexpr int kXRows = 16 * XT;
-    constexpr int kDX = gemv_tile_dx(XT), kDW = gemv_tile_dw(XT);
-    static_assert(kDW > kDX, "a chunk's weights are asked for before its activations");
-    // activation requests of a wave per chunk: one per row, 16 XT rows, or 8 fewer (HALF: the last tile has at most
-    // 8 live rows; the other 8 are never fetched, hold whatever the ring held, and their sums are never stored)
-    constexpr int kNX = 2 * XT - (HALF ? 1 : 0);
-    constexpr int kWMost = (NI + 7) / 8;     // weight requests of a wave per chunk, or one less
+    typedef BlocksShape<XT, RW, HALF> S;
+    constexpr int MT = S::kMT, D = S::kDepth;
+    constexpr int NX = S::kXRows / 8;                     // activation requests per chunk and wave: eight rows each
+    constexpr int NW = (RW * 17 + 63) / 64;               // weight requests per chunk
+    constexpr int NWMost = (NW + 7) / 8;                  // of a wave, or one less
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int lane = threadIdx.x & 63;
     const int lm = lane & 15, lg = lane >> 4;
-    const int nb = k >> 5;
-    const int nchunk = nb >> 3;
+    const int nb = k >> 5, nchunk = (nb + 7) >> 3;
     const uint32_t row_bytes = (uint32_t)nb * kQ8Block;
-    const int m0 = blockIdx.x * rows_wg;
-    const int r0 = blockIdx.y * kXRows;
-    const int nrows = rows - r0 < kXRows ? rows - r0 : kXRows;
-    const int pieces = rows_wg * 17;
-    if ((pieces + 63) / 64 != NI)
-        return; // (the launcher's contract: a chunk of weights is NI requests)
-    const int wbytes = pieces * 16;
-    constexpr int kXBytes = kXRows * kTileRowPitch;
-    uint8_t *wring = lds, *xring = lds + kDW * wbytes;
-    const uint32_t wring_at = proj_lds_address(wring), xring_at = proj_lds_address(xring);
+    const int m0 = blockIdx.x * RW, r0 = blockIdx.y * (16 * XT);
+    const int nrows = rows - r0 < 16 * XT ? rows - r0 : 16 * XT;
+    const uint32_t ring_at = proj_lds_address(lds);
+    const uint8_t *wb = w + (size_t)m0 * row_bytes;
+    const uint8_t *xb = reinterpret_cast<const uint8_t *>(x + (size_t)r0 * k);
 
-    // weights of chunk c: request q = wave + 8 j < NI brings 64 pieces (piece p: row p / 17 of the workgroup, 16
-    // bytes p % 17 of its 272; rows past the end of the matrix repeat the last)
-    uint32_t woff[kWMost];
+    // piece p of a chunk of weights: row p / 17, 16 bytes p % 17 of its 272; rows past the matrix repeat the last
+    constexpr int kPieces = RW * 17;
+    uint32_t woff[NWMost], xoff[NX];
+    int wreq = 0;
 #pragma unroll
-    for (int j = 0; j < kWMost; j++) {
+    for (int j = 0; j < NWMost; j++) {
         const int p = (wave + 8 * j) * 64 + lane;
         const int pr = p / 17, pq = p - pr * 17;
-        const int row = m0 + pr < m ? m0 + pr : m - 1;
-        woff[j] = (uint32_t)row * row_bytes + (uint32_t)pq * 16u;
+        woff[j] = (uint32_t)(m0 + pr < m ? pr : m - 1 - m0) * row_bytes + (uint32_t)pq * 16u;
+        wreq += wave + 8 * j < NW ? 1 : 0;
     }
-    int wreq = 0; // weight requests of this wave per chunk
 #pragma unroll
-    for (int j = 0; j < kWMost; j++)
-        wreq += wave + 8 * j < NI ? 1 : 0;
-    auto issue_w = [&](int c) {
-        const uint32_t at = wring_at + (uint32_t)((c % kDW) * wbytes);
+    for (int j = 0; j < NX; j++) { // rows past the live ones repeat the last
+        const int r = 8 * j + (lane >> 3);
+        xoff[j] = (uint32_t)(r < nrows ? r : nrows - 1) * (uint32_t)k * 4u + (uint32_t)(((lane ^ r) & 7) * 16);
+    }
+    auto issue = [&](int c) {
+        const uint32_t at = ring_at + (uint32_t)((c % D) * S::kSlot);
+        const int b = 8 * c + wave < nb ? 8 * c + wave : nb - 1;
+        const uint8_t *xs = xb + (size_t)b * 128;
 #pragma unroll
-        for (int j = 0; j < kWMost; j++) {
+        for (int j = 0; j < NX; j++)
+            proj_dma16<false>(at + S::kWBytes + wave * S::kXWave + j * 1024, xs, xoff[j]);
+#pragma unroll
+        for (int j = 0; j < NWMost; j++) {
             const int q = wave + 8 * j;
-            if (q < NI && q * 64 + lane < pieces)
-                proj_dma16<true>(at + q * 1024, w, woff[j] + (uint32_t)c * kDmaChunkBytes);
+            if (q < NW && (kPieces % 64 == 0 || q * 64 + lane < kPieces))
+                proj_dma16<true>(at + q * 1024, wb, woff[j] + (uint32_t)c * kDmaChunkBytes);
         }
     };
-    // activations of chunk c: rows wave + 8 j of the pass (rows past the live ones repeat the last), 256 floats each
-    const uint8_t *xb = reinterpret_cast<const uint8_t *>(x + (size_t)r0 * k);
-    uint32_t xoff[kNX];
-#pragma unroll
-    for (int j = 0; j < kNX; j++) {
-        const int r = wave + 8 * j;
-        xoff[j] = (uint32_t)(r < nrows ? r : nrows - 1) * (uint32_t)k * 4u + lane * 16u;
-    }
-    auto issue_x = [&](int c) {
-        const uint32_t at = xring_at + (uint32_t)((c % kDX) * kXBytes);
-#pragma unroll
-        for (int j = 0; j < kNX; j++)
-            proj_dma16<false>(at + (wave + 8 * j) * kTileRowPitch, xb, xoff[j] + (uint32_t)c * 1024u);
+    // chunk c has arrived: only the chunks asked for behind it, `most` of them, are outstanding
+    auto wait_chunk = [&](int c, int most) {
+        const int newer = nchunk - 1 - c < most ? nchunk - 1 - c : most;
+        constexpr int a = NX + NWMost, b = NX + NWMost - 1; // requests of a chunk
+        static_assert(4 * a < 64, "vmcnt has six bits");
+        switch (newer) {
+        case 4: return wreq == NWMost ? wait_vm<4 * a>() : wait_vm<4 * b>();
+        case 3: return wreq == NWMost ? wait_vm<3 * a>() : wait_vm<3 * b>();
+        case 2: return wreq == NWMost ? wait_vm<2 * a>() : wait_vm<2 * b>();
+        case 1: return wreq == NWMost ? wait_vm<a>() : wait_vm<b>();
+        default: return wait_vm<0>();
+        }
     };
-#pragma unroll
-    for (int c = 0; c < kDW; c++)
-        if (c < nchunk)
-            issue_w(c);
-#pragma unroll
-    for (int c = 0; c < kDX; c++)
-        if (c < nchunk)
-            issue_x(c);
 
-    float4v acc[XT][kNT];
+    struct Regs {
+        float4v x[XT][2];
+        uint32_t q[MT][3];
+        uint16_t d[MT];
+    };
+    // block w: the lane's 8 bytes sit 2 bytes past a dword boundary in even blocks (three dwords, realigned below) and
+    // at one in odd blocks; rows of the last tile past RW repeat the last (never stored)
+    const uint32_t shift = wave & 1 ? 0 : 16;
+    int wrow[MT];
+#pragma unroll
+    for (int t = 0; t < MT; t++)
+        wrow[t] = (t * 16 + lm < RW ? t * 16 + lm : RW - 1) * kDmaChunkBytes + wave * kQ8Block;
+    auto load = [&](Regs &g, int c) {
+        const uint8_t *buf = lds + (c % D) * S::kSlot;
+        const uint8_t *xa = buf + S::kWBytes + wave * S::kXWave + lm * 128;
+#pragma unroll
+        for (int t = 0; t < MT; t++) {
+            const uint8_t *blk = buf + wrow[t];
+            const uint32_t *q = reinterpret_cast<const uint32_t *>(blk + (wave & 1) * 2 + lg * 8);
+#pragma unroll
+            for (int j = 0; j < 3; j++)
+                g.q[t][j] = q[j];
+            g.d[t] = *reinterpret_cast<const uint16_t *>(blk);
+        }
+#pragma unroll
+        for (int xt = 0; xt < XT; xt++)
+#pragma unroll
+            for (int h = 0; h < 2; h++)
+                g.x[xt][h] = *reinterpret_cast<const float4v *>(xa + xt * 2048 + (((lg * 2 + h) ^ lm) & 7) * 16);
+    };
+    float4v acc[XT][MT];
 #pragma unroll
     for (int xt = 0; xt < XT; xt++)
 #pragma unroll
-        for (int t = 0; t < kNT; t++)
+        for (int t = 0; t < MT; t++)
             acc[xt][t] = (float4v){0, 0, 0, 0};
-    int wrow[kNT]; // (rows of the second tile past rows_wg repeat the last: never stored)
+    auto multiply = [&](const Regs &g) {
+        half8 wv[MT], hi[XT], lo[XT];
+        float d[MT];
 #pragma unroll
-    for (int t = 0; t < kNT; t++)
-        wrow[t] = (t * 16 + lm < rows_wg ? t * 16 + lm : rows_wg - 1) * kDmaChunkBytes;
-    const int b = wave; // this wave's block of every chunk
-
-    for (int c = 0; c < nchunk; c++) {
-        // This wave's requests for chunk c have arrived once only those made after them are outstanding.  In the
-        // steady state these are, in order, the weights of chunk c + 1, then per chunk finished since (kDX of them)
-        // the activations and the weights asked for behind it: kDX - 1 sets of activations and kDX of weights in
-        // all.  Counting the activation sets alone waits for requests made a chunk ago as well; measured at 16 / 24 /
-        // 48 / 64 rows: 17.5 / 21.9 / 35.1 / 39.7 us so, 17.5 / 23.2 / 31.2 / 35.7 with the full count, hence the full
-        // count from three activation tiles on.  At the ends, where some of those chunks do not exist, only the
-        // activation sets that do are counted, which errs on the side of waiting.
-        {
-            static_assert(kDX == 2 && kDW == 3 && kWMost <= 2, "the counts below");
-            const int behind = nchunk - 1 - c < kDX - 1 ? nchunk - 1 - c : kDX - 1;
-            if (XT >= 3 && c >= kDX && c + kDW - 1 < nchunk) {
-                if (wreq == 0)
-                    wait_vm<kNX>();
-                else if (wreq == 1)
-                    wait_vm<kNX + kDX>();
-                else
-                    wait_vm<kNX + 2 * kDX>();
-            } else if (behind >= 1) {
-                wait_vm<kNX>();
-            } else {
-                wait_vm<0>();
-            }
-        }
-        __syncthreads(); // ... and every wave's
-        const uint8_t *wbuf = wring + (c % kDW) * wbytes;
-        const uint8_t *xa = xring + (c % kDX) * kXBytes + b * 128 + lg * 32;
-        half8 wv[kNT];
-        float d[kNT];
-#pragma unroll
-        for (int t = 0; t < kNT; t++) {
-            const uint8_t *blk = wbuf + wrow[t] + b * kQ8Block;
-            uint32_t q0, q1;
-            if ((b & 1) == 0) { // (uniform) even blocks sit 2 bytes past a dword boundary
-                const uint3a4 e = *reinterpret_cast<const uint3a4 *>(blk + lg * 8);
-                q0 = __builtin_amdgcn_alignbit(e[1], e[0], 16);
-                q1 = __builtin_amdgcn_alignbit(e[2], e[1], 16);
-            } else {
-                const uint2a4 o = *reinterpret_cast<const uint2a4 *>(blk + 2 + lg * 8);
-                q0 = o[0];
-                q1 = o[1];
-            }
-            d[t] = (float)*reinterpret_cast<const _Float16 *>(blk);
-            wv[t] = int8x8_to_f16(q0, q1);
+        for (int t = 0; t < MT; t++) {
+            wv[t] = int8x8_to_f16(__builtin_amdgcn_alignbit(g.q[t][1], g.q[t][0], shift),
+                                  __builtin_amdgcn_alignbit(g.q[t][2], g.q[t][1], shift));
+            d[t] = (float)__builtin_bit_cast(_Float16, g.d[t]);
         }
 #pragma unroll
-        for (int xt = 0; xt < XT; xt++) {
-            const uint8_t *src = xa + (xt * 16 + lm) * kTileRowPitch;
-            const float4v a4 = *reinterpret_cast<const float4v *>(src);
-            const float4v b4 = *reinterpret_cast<const float4v *>(src + 16);
-            half8 hi, lo;
-            split_hi_lo(a4, b4, hi, lo);
+        for (int xt = 0; xt < XT; xt++)
+            split_hi_lo(g.x[xt][0], g.x[xt][1], hi[xt], lo[xt]);
+        float4v p[XT][MT];
 #pragma unroll
-            for (int t = 0; t < kNT; t++) {
-                float4v p = {0, 0, 0, 0};
-                p = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi, wv[t], p, 0, 0, 0);
-                p = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo, wv[t], p, 0, 0, 0);
+        for (int xt = 0; xt < XT; xt++)
+#pragma unroll
+            for (int t = 0; t < MT; t++)
+                p[xt][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi[xt], wv[t], (float4v){0, 0, 0, 0}, 0, 0, 0);
+#pragma unroll
+        for (int xt = 0; xt < XT; xt++)
+#pragma unroll
+            for (int t = 0; t < MT; t++)
+                p[xt][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo[xt], wv[t], p[xt][t], 0, 0, 0);
+#pragma unroll
+        for (int xt = 0; xt < XT; xt++)
+#pragma unroll
+            for (int t = 0; t < MT; t++)
 #pragma unroll
                 for (int j = 0; j < 4; j++)
-                    acc[xt][t][j] = fmaf(d[t], p[j], acc[xt][t][j]);
-            }
-        }
-        __syncthreads(); // every wave is done with the chunk's entries: later chunks may land in them
-        if (c + kDX < nchunk)
-            issue_x(c + kDX);
-        if (c + kDW < nchunk)
-            issue_w(c + kDW);
+                    acc[xt][t][j] = fmaf(d[t], p[xt][t][j], acc[xt][t][j]);
+    };
+#pragma unroll
+    for (int c = 0; c < D; c++)
+        if (c < nchunk)
+            issue(c);
+    Regs even, odd;
+    wait_chunk(0, D - 1);
+    __syncthreads();
+    load(even, 0);
+    // chunk c is in `now`
+    auto turn = [&](Regs &now, Regs &next, int c) {
+        // (lgkmcnt(0), through the builtin: the compiler then knows that `now` is there and does not hold up its use for
+        // the reads of `next`, of which there are more than lgkmcnt can count)
+        __builtin_amdgcn_s_waitcnt(0xc07f);
+        if (c + 1 < nchunk)
+            wait_chunk(c + 1, D - 2);
+        __syncthreads();
+        if (c + D < nchunk)
+            issue(c + D);
+        if (c + 1 < nchunk)
+            load(next, c + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        if (8 * c + wave < nb)
+            multiply(now);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    for (int c = 0; c < nchunk; c += 2) {
+        turn(even, odd, c);
+        if (c + 1 < nchunk)
+            turn(odd, even, c + 1);
     }
 
-    // ---- the waves' sums meet in wave order (the rings are free: the loop ended on a barrier) --------------------
+    // ---- the waves' sums meet in wave order (the ring is free: the last turn's barrier stood behind its last reads) --
     float4v *red = reinterpret_cast<float4v *>(lds);
 #pragma unroll
     for (int xt = 0; xt < XT; xt++)
 #pragma unroll
-        for (int t = 0; t < kNT; t++)
-            red[((wave * XT + xt) * kNT + t) * 64 + lane] = acc[xt][t];
+        for (int t = 0; t < MT; t++)
+            red[((wave * XT + xt) * MT + t) * 64 + lane] = acc[xt][t];
     __syncthreads();
-    for (int e = threadIdx.x; e < XT * kNT * 64; e += 512) {
-        const int l = e & 63, xt_t = e >> 6;
-        const int xt = xt_t / kNT, t = xt_t - xt * kNT;
+    for (int e = threadIdx.x; e < XT * MT * 64; e += 512) {
+        const int l = e & 63, xt = (e >> 6) / MT, t = (e >> 6) - xt * MT;
         float4v s = red[e];
 #pragma unroll
         for (int u = 1; u < 8; u++)
-            s += red[u * (XT * kNT * 64) + e];
+            s += red[u * (XT * MT * 64) + e];
         const int wr = t * 16 + (l & 15);
-        if (wr < rows_wg && m0 + wr < m) {
+        if (wr < RW && m0 + wr < m) {
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 const int r = xt * 16 + (l >> 4) * 4 + j;
@@ -881,195 +896,224 @@ __global__ void __launch_bounds__(512, 1) gemv_q8_dma_tile_kernel(const uint8_t 
     }
 }
 
-// ---- gemv_q8_tile_kernel: 3 to 128 activation rows (batched decode, verify groups) --------------
-//
-// The same streaming of W as above, with the activations as full 16-row A tiles: A row = activation
-// row, hi and lo halves as two chained MFMAs, XT tiles (16 or 32 rows) per pass.  The rows' operands
-// no longer fit LDS, and need not: the waves of a workgroup split k, so no two of them want the same
-// activations; lane (lm, lg) loads the 8 f32 of row lm, k quarter lg of each block straight from
-// global memory (L2: the rows are a few hundred KB that every workgroup reads) and splits them in
-// registers.  A step (a pair of blocks: 16 XT registers of activations, 5 TILES of weights) is one
-// record; four records rotate, each refilled as soon as it has been consumed, activations before
-// weights in request order (the loads complete in order: a step then waits for nothing younger than
-// itself).  What the time is made of at 5120 x 6144 and 16 rows: 13.1 us with the activation loads
-// taken out (the arithmetic is hidden behind the weight stream), 16.1 with all of them hitting L1,
-// 19.8 as it is: every workgroup reads every row (393 KB through its CU's L1 for 208 KB of weights).
-// Four weight tiles per workgroup halve that and leave 80 workgroups, too few to keep HBM busy (27.5 us).
-template <int TILES, int XT>
-struct TileRec {
-    float4v x[XT][2][2]; // [tile][block of the pair][half of the 8 values]
-    uint3a4 e[TILES];
-    uint2a4 o[TILES];
+template <int XT, int RW, bool HALF>
+struct UnitsShape {
+    static constexpr int kMT = (RW + 15) / 16;              // weight tiles
+    static constexpr int kXRows = 16 * XT - (HALF ? 8 : 0); // activation rows that are fetched
+    static constexpr int kXBytes = kXRows * 256;
+    static constexpr int kSlot = kXBytes + (RW * 68 + 15) / 16 * 16; // a unit
+    static constexpr int kRead = HALF ? 2048 : 0;           // (a HALF tile's dead rows are read past the activations)
+    static constexpr int kRoom = (160 << 10) - kRead;
+    static constexpr int kWaves = kRoom / (8 * kSlot) >= 2 ? 8 : 4;
+    static constexpr int kFit = kRoom / (kWaves * kSlot);
+    static constexpr int kDepth = kFit < 4 ? kFit : 4; // units in flight per wave
+    static constexpr int kLds = kWaves * kDepth * kSlot + kRead;
+    static constexpr int kChains = 8 / kWaves; // of a wave
+    static_assert(kDepth >= 2 && kDepth * kSlot >= kChains * XT * kMT * 1024, "");
 };
+template <int XT, int RW, bool HALF>
+constexpr int kUnitsThreads = 64 * UnitsShape<XT, RW, HALF>::kWaves;
 
-template <int WAVES, int TILES, int XT, int STEPS>
-__global__ void __launch_bounds__(64 * WAVES, 1) gemv_q8_tile_kernel(const uint8_t *__restrict__ w,
-                                                                   const float *__restrict__ x,
-                                                                   float *__restrict__ y, int m, int k, int rows)
+__device__ __forceinline__ void proj_dma4(uint32_t lds_at, const uint8_t *base, uint32_t voff)
 {
-    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int lm = lane & 15, lg = lane >> 4; // MFMA operand lane: A row / weight row lm, k quarter lg
-    const int fr = lane >> 2, fg = lane & 3;  // fetch lane: weight row fr, k quarter fg
-    const int pull = (lm * 4 + lg) * 4;
-    const int nb = k >> 5;
-    const size_t row_bytes = (size_t)nb * kQ8Block;
-    const int m0 = blockIdx.x * (16 * TILES);
-    const int r0 = blockIdx.y * (16 * XT);
-    const int nu = nb >> 1; // steps: pairs of blocks
-    // The steps are dealt to the waves round-robin: the activation rows are a multiple of the L2's
-    // channel interleave apart, so the 16 rows of one load meet in one channel, and only the k
-    // offsets of requests in flight spread the traffic; eight neighbouring steps are 2 KB of a row.
-    // (With a contiguous slice of k per wave the activation loads cost 10 us on top of 13.)
-    float4v *red = reinterpret_cast<float4v *>(lds);
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
+                 :
+                 : "s"(lds_at), "v"(voff), "s"(base)
+                 : "memory");
+}
 
-    // rows past the end are clamped: loaded and multiplied, never stored
-    const float *xp[XT];
+// Wave w of WV streams units (pairs of blocks, 64 values of k) w, w + WV, ... of its rows through a ring of its own; unit
+// u belongs to chain u % 8, so four waves keep two sets of sums each.  HALF: as above.
+template <int XT, int RW, bool HALF>
+__global__ void __launch_bounds__((kUnitsThreads<XT, RW, HALF>), 2)
+    gemv_q8_units_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, float *__restrict__ y, int m, int k, int rows)
+{
+    typedef UnitsShape<XT, RW, HALF> S;
+    constexpr int MT = S::kMT, D = S::kDepth, WV = S::kWaves;
+    constexpr int NX = S::kXRows / 4;          // activation requests per unit: four rows of 256 bytes each
+    constexpr int NW = (RW * 17 + 63) / 64;    // weight requests: 64 dwords each
+    constexpr int REQ = NX + NW;
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int lane = threadIdx.x & 63;
+    const int lm = lane & 15, lg = lane >> 4;
+    const int nunits = k >> 6;
+    const uint32_t row_bytes = (uint32_t)(k >> 5) * kQ8Block;
+    const int m0 = blockIdx.x * RW, r0 = blockIdx.y * (16 * XT);
+    const int nrows = rows - r0 < 16 * XT ? rows - r0 : 16 * XT;
+    const int mine = wave < nunits ? (nunits - wave + WV - 1) / WV : 0;
+    uint8_t *ring = lds + wave * (D * S::kSlot);
+    const uint32_t ring_at = proj_lds_address(ring);
+    const uint8_t *wb = w + (size_t)m0 * row_bytes;
+    const uint8_t *xb = reinterpret_cast<const uint8_t *>(x + (size_t)r0 * k);
+    uint32_t woff[NW], xoff[NX]; // rows past the matrix, and past the live activation rows, repeat the last
 #pragma unroll
-    for (int t = 0; t < XT; t++) {
-        const int r = r0 + t * 16 + lm < rows ? r0 + t * 16 + lm : rows - 1;
-        xp[t] = x + (size_t)r * k + lg * 8;
+    for (int j = 0; j < NW; j++) {
+        const int p = j * 64 + lane;
+        const int pr = p / 17, pd = p - pr * 17;
+        woff[j] = (uint32_t)(m0 + pr < m ? pr : m - 1 - m0) * row_bytes + (uint32_t)pd * 4u;
     }
-    const uint8_t *wp[TILES];
 #pragma unroll
-    for (int t = 0; t < TILES; t++) {
-        const int row = m0 + t * 16 + fr < m ? m0 + t * 16 + fr : m - 1;
-        wp[t] = w + (size_t)row * row_bytes;
+    for (int j = 0; j < NX; j++) {
+        const int r = 4 * j + lg;
+        xoff[j] = (uint32_t)(r < nrows ? r : nrows - 1) * (uint32_t)k * 4u + (uint32_t)((lm ^ (r & 15)) * 16);
     }
-    typedef TileRec<TILES, XT> Rec;
-    auto fetch = [&](Rec &c, int u) {
-        const int uc = u < nu ? u : nu - 1;
+    auto issue = [&](int i) {
+        const uint32_t at = ring_at + (uint32_t)((i % D) * S::kSlot);
+        const uint32_t u = (uint32_t)(wave + WV * i);
+        const uint8_t *xs = xb + (size_t)u * 256, *ws = wb + (size_t)u * (2 * kQ8Block);
 #pragma unroll
-        for (int t = 0; t < XT; t++)
+        for (int j = 0; j < NX; j++)
+            proj_dma16<false>(at + j * 1024, xs, xoff[j]);
 #pragma unroll
-            for (int b = 0; b < 2; b++) {
-                const float *p = xp[t] + (size_t)uc * 64 + b * 32;
-                c.x[t][b][0] = *reinterpret_cast<const float4v *>(p);
-                c.x[t][b][1] = *reinterpret_cast<const float4v *>(p + 4);
-            }
-#pragma unroll
-        for (int t = 0; t < TILES; t++) {
-            const uint8_t *unit = wp[t] + (size_t)uc * (2 * kQ8Block);
-            c.e[t] = *reinterpret_cast<const uint3a4 *>(unit + fg * 8);
-            c.o[t] = *reinterpret_cast<const uint2a4 *>(unit + 36 + fg * 8);
+        for (int j = 0; j < NW; j++) {
+            if ((j + 1) * 64 <= RW * 17 || j * 64 + lane < RW * 17)
+                proj_dma4(at + S::kXBytes + j * 256, ws, woff[j]);
         }
     };
-    float4v acc[TILES][XT];
+    // unit i has arrived: only the units asked for behind it, `most` of them, are outstanding
+    auto wait_unit = [&](int i, int most) {
+        const int newer = mine - 1 - i < most ? mine - 1 - i : most;
+        if (newer >= 3 && D > 3)
+            wait_vm<(3 * REQ < 63 ? 3 * REQ : 63)>();
+        else if (newer >= 2 && D > 2)
+            wait_vm<(2 * REQ < 63 ? 2 * REQ : 63)>();
+        else if (newer >= 1)
+            wait_vm<REQ>();
+        else
+            wait_vm<0>();
+    };
+    struct Regs {
+        float4v x[XT][2][2];
+        uint32_t e[MT][3], o[MT][2];
+        uint16_t d[MT][2];
+    };
+    int wrow[MT]; // (rows of the last tile past RW repeat the last: never stored)
 #pragma unroll
-    for (int t = 0; t < TILES; t++)
+    for (int t = 0; t < MT; t++)
+        wrow[t] = (t * 16 + lm < RW ? t * 16 + lm : RW - 1) * (2 * kQ8Block);
+    auto load = [&](Regs &g, int i) {
+        const uint8_t *buf = ring + (i % D) * S::kSlot;
 #pragma unroll
-        for (int a = 0; a < XT; a++)
-            acc[t][a] = (float4v){0, 0, 0, 0};
-    auto consume = [&](const Rec &c, int u) {
-        const bool live = u < nu;
-        half8 hi[XT][2], lo[XT][2];
+        for (int t = 0; t < MT; t++) {
+            const uint8_t *unit = buf + S::kXBytes + wrow[t];
+            const uint32_t *e = reinterpret_cast<const uint32_t *>(unit + lg * 8);
 #pragma unroll
-        for (int a = 0; a < XT; a++)
+            for (int j = 0; j < 3; j++)
+                g.e[t][j] = e[j];
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+                g.o[t][j] = e[9 + j];
+            g.d[t][0] = *reinterpret_cast<const uint16_t *>(unit);
+            g.d[t][1] = *reinterpret_cast<const uint16_t *>(unit + kQ8Block);
+        }
+#pragma unroll
+        for (int xt = 0; xt < XT; xt++)
 #pragma unroll
             for (int b = 0; b < 2; b++)
-                split_hi_lo(c.x[a][b][0], c.x[a][b][1], hi[a][b], lo[a][b]);
 #pragma unroll
-        for (int t = 0; t < TILES; t++) {
-            const uint3a4 e = c.e[t];
-            const int e2_of_g3 = __builtin_amdgcn_update_dpp(0, (int)e[2], 0xFF, 0xf, 0xf, true);
-            const int sc = (int)((e[0] & 0xffffu) | ((uint32_t)e2_of_g3 & 0xffff0000u));
-            const uint32_t q0 = (uint32_t)__builtin_amdgcn_ds_bpermute(pull, (int)__builtin_amdgcn_alignbit(e[1], e[0], 16));
-            const uint32_t q1 = (uint32_t)__builtin_amdgcn_ds_bpermute(pull, (int)__builtin_amdgcn_alignbit(e[2], e[1], 16));
-            const uint32_t q2 = (uint32_t)__builtin_amdgcn_ds_bpermute(pull, (int)c.o[t][0]);
-            const uint32_t q3 = (uint32_t)__builtin_amdgcn_ds_bpermute(pull, (int)c.o[t][1]);
-            const uint32_t ds = (uint32_t)__builtin_amdgcn_ds_bpermute(lm * 16, sc);
-            const float d0 = live ? (float)__builtin_bit_cast(_Float16, (uint16_t)(ds & 0xffffu)) : 0.0f;
-            const float d1 = live ? (float)__builtin_bit_cast(_Float16, (uint16_t)(ds >> 16)) : 0.0f;
-            const half8 w0 = int8x8_to_f16(q0, q1), w1 = int8x8_to_f16(q2, q3);
+                for (int h = 0; h < 2; h++)
+                    g.x[xt][b][h] = *reinterpret_cast<const float4v *>(buf + (xt * 16 + lm) * 256 + ((b * 8 + lg * 2 + h) ^ lm) * 16);
+    };
+    float4v acc[S::kChains][XT][MT];
 #pragma unroll
-            for (int a = 0; a < XT; a++) {
-                float4v p0 = {0, 0, 0, 0}, p1 = {0, 0, 0, 0};
-                p0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi[a][0], w0, p0, 0, 0, 0);
-                p1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi[a][1], w1, p1, 0, 0, 0);
-                p0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo[a][0], w0, p0, 0, 0, 0);
-                p1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo[a][1], w1, p1, 0, 0, 0);
+    for (int s = 0; s < S::kChains; s++)
 #pragma unroll
-                for (int j = 0; j < 4; j++)
-                    acc[t][a][j] = fmaf(d1, p1[j], fmaf(d0, p0[j], acc[t][a][j]));
+        for (int xt = 0; xt < XT; xt++)
+#pragma unroll
+            for (int t = 0; t < MT; t++)
+                acc[s][xt][t] = (float4v){0, 0, 0, 0};
+    auto multiply = [&](const Regs &g, float4v (&sum)[XT][MT]) {
+#pragma unroll
+        for (int b = 0; b < 2; b++) {
+            half8 wv[MT], hi[XT], lo[XT];
+            float d[MT];
+#pragma unroll
+            for (int t = 0; t < MT; t++) {
+                const uint32_t q0 = b == 0 ? __builtin_amdgcn_alignbit(g.e[t][1], g.e[t][0], 16) : g.o[t][0];
+                const uint32_t q1 = b == 0 ? __builtin_amdgcn_alignbit(g.e[t][2], g.e[t][1], 16) : g.o[t][1];
+                wv[t] = int8x8_to_f16(q0, q1);
+                d[t] = (float)__builtin_bit_cast(_Float16, g.d[t][b]);
             }
+#pragma unroll
+            for (int xt = 0; xt < XT; xt++)
+                split_hi_lo(g.x[xt][b][0], g.x[xt][b][1], hi[xt], lo[xt]);
+            float4v p[XT][MT];
+#pragma unroll
+            for (int xt = 0; xt < XT; xt++)
+#pragma unroll
+                for (int t = 0; t < MT; t++)
+                    p[xt][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi[xt], wv[t], (float4v){0, 0, 0, 0}, 0, 0, 0);
+#pragma unroll
+            for (int xt = 0; xt < XT; xt++)
+#pragma unroll
+                for (int t = 0; t < MT; t++)
+                    p[xt][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo[xt], wv[t], p[xt][t], 0, 0, 0);
+#pragma unroll
+            for (int xt = 0; xt < XT; xt++)
+#pragma unroll
+                for (int t = 0; t < MT; t++)
+#pragma unroll
+                    for (int j = 0; j < 4; j++)
+                        sum[xt][t][j] = fmaf(d[t], p[xt][t][j], sum[xt][t][j]);
         }
     };
-    // STEPS > 0: every wave has exactly STEPS steps (the launcher checks) and the code is straight
-    // line, so each step waits for exactly its own loads.  Otherwise a loop of four steps per turn
-    // (the records keep their registers; the compiler waits for every outstanding load at the head
-    // of a turn); a fetch past the wave's last step repeats it and a step past it multiplies by a
-    // zero scale.  The scheduler may not move a step's arithmetic past the refill behind it, or the
-    // other way round: either makes the wave wait for loads it has only just asked for.
-    Rec c[4];
-    const int u_lo = wave;
-    fetch(c[0], u_lo);
-    fetch(c[1], u_lo + WAVES);
-    fetch(c[2], u_lo + 2 * WAVES);
-    fetch(c[3], u_lo + 3 * WAVES);
-    if (STEPS > 0) {
 #pragma unroll
-        for (int i = 0; i < STEPS; i++) {
-            __builtin_amdgcn_sched_barrier(0);
-            consume(c[i & 3], u_lo + i * WAVES);
-            __builtin_amdgcn_sched_barrier(0);
-            if (i + 4 < STEPS)
-                fetch(c[i & 3], u_lo + (i + 4) * WAVES);
+    for (int i = 0; i < D; i++)
+        if (i < mine)
+            issue(i);
+    Regs even, odd;
+    if (mine > 0) {
+        wait_unit(0, D - 1);
+        load(even, 0);
+    }
+    // unit i is in `now`
+    auto turn = [&](Regs &now, Regs &next, float4v (&sum)[XT][MT], int i) {
+        __builtin_amdgcn_s_waitcnt(0xc07f); // lgkmcnt(0), as above: unit i's place in the ring has been read
+        asm volatile("" ::: "memory");
+        if (i + D < mine)
+            issue(i + D);
+        if (i + 1 < mine) {
+            wait_unit(i + 1, D - 1);
+            load(next, i + 1);
         }
-    } else {
-        for (int u = u_lo; u < nu; u += 4 * WAVES) {
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(now, sum);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    for (int i = 0; i < mine; i += 2) {
+        turn(even, odd, acc[0], i);
+        if (i + 1 < mine)
+            turn(odd, even, acc[S::kChains - 1], i + 1);
+    }
+
+    // ---- the chains' sums meet in their order (a wave leaves its own at the head of its ring, which it has read) ------
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    constexpr int kTiles = XT * MT * 64;
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                __builtin_amdgcn_sched_barrier(0);
-                consume(c[i], u + i * WAVES);
-                __builtin_amdgcn_sched_barrier(0);
-                fetch(c[i], u + (i + 4) * WAVES);
+    for (int s = 0; s < S::kChains; s++)
+#pragma unroll
+        for (int xt = 0; xt < XT; xt++)
+#pragma unroll
+            for (int t = 0; t < MT; t++)
+                reinterpret_cast<float4v *>(ring)[s * kTiles + (xt * MT + t) * 64 + lane] = acc[s][xt][t];
+    __syncthreads();
+    for (int e = threadIdx.x; e < kTiles; e += 64 * WV) {
+        const int l = e & 63, xt = (e >> 6) / MT, t = (e >> 6) - xt * MT;
+        float4v s = reinterpret_cast<const float4v *>(lds)[e];
+#pragma unroll
+        for (int c = 1; c < 8; c++)
+            s += reinterpret_cast<const float4v *>(lds + (c % WV) * (D * S::kSlot))[(c / WV) * kTiles + e];
+        const int wr = t * 16 + (l & 15);
+        if (wr < RW && m0 + wr < m) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const int r = xt * 16 + (l >> 4) * 4 + j;
+                if (r < nrows)
+                    y[(size_t)(r0 + r) * m + m0 + wr] = s[j];
             }
         }
     }
-
-    // the k slices meet in a fixed order: C row 4 lg + j = activation row, column lm = weight row
-#pragma unroll
-    for (int t = 0; t < TILES; t++)
-#pragma unroll
-        for (int a = 0; a < XT; a++)
-            red[((wave * TILES + t) * XT + a) * 64 + lane] = acc[t][a];
-    __syncthreads();
-    for (int i = threadIdx.x; i < TILES * XT * 64; i += 64 * WAVES) {
-        float4v s = red[i];
-#pragma unroll
-        for (int u = 1; u < WAVES; u++)
-            s += red[u * TILES * XT * 64 + i];
-        const int l = i & 63, a = (i >> 6) % XT, t = (i >> 6) / XT;
-        const int row = m0 + t * 16 + (l & 15);
-        const int r = r0 + a * 16 + 4 * (l >> 4);
-        if (row < m) {
-#pragma unroll
-            for (int j = 0; j < 4; j++)
-                if (r + j < rows)
-                    y[(size_t)(r + j) * m + row] = s[j];
-        }
-    }
-}
-
-template <int WAVES, int TILES, int XT, int STEPS>
-static int launch_gemv_tile_steps(hipStream_t st, const uint8_t *w, const float *x, float *y, int m, int k, int rows)
-{
-    const size_t lds = (size_t)WAVES * TILES * XT * 64 * sizeof(float4v);
-    auto kern = gemv_q8_tile_kernel<WAVES, TILES, XT, STEPS>;
-    const dim3 grid((unsigned)((m + 16 * TILES - 1) / (16 * TILES)), (unsigned)((rows + 16 * XT - 1) / (16 * XT)), 1);
-    HIPML_LAUNCH(kern, grid, dim3(64 * WAVES, 1, 1), lds, st, w, x, y, m, k, rows);
-    return launched("gemv_q8_0_rows");
-}
-
-template <int WAVES, int TILES, int XT>
-static int launch_gemv_tile(hipStream_t st, const uint8_t *w, const float *x, float *y, int m, int k, int rows)
-{
-    // straight-line variants for the model's two inner sizes: 6144 (W_o) and 5120 (W_q, W_k, W_v)
-    if (k == 64 * WAVES * 12)
-        return launch_gemv_tile_steps<WAVES, TILES, XT, 12>(st, w, x, y, m, k, rows);
-    if (k == 64 * WAVES * 10)
-        return launch_gemv_tile_steps<WAVES, TILES, XT, 10>(st, w, x, y, m, k, rows);
-    return launch_gemv_tile_steps<WAVES, TILES, XT, 0>(st, w, x, y, m, k, rows);
 }
 
 template <int WAVES, int TILES, int CH, int XG>
@@ -1106,29 +1150,64 @@ static int gemv_dma_waves(int rp, int ni, int rows_wg, int k)
     return 0;
 }
 
-template <int RP, int NI>
-static int launch_gemv_dma(hipStream_t st, const uint8_t *w, const float *x, float *y, int m, int k, int rows, int rows_wg)
+// Weight rows per workgroup for a pass of rp activation rows, as requests per chunk (NI).
+struct DmaRows {
+    int rows_wg, ni;
+    bool four; // four waves even where the LDS of eight fits (several workgroups then share a CU)
+};
+static DmaRows gemv_dma_rows_wg(int m, int rp)
 {
-    const dim3 grid((unsigned)((m + rows_wg - 1) / rows_wg), (unsigned)((rows + RP - 1) / RP), 1);
-    const int waves = gemv_dma_waves(RP, NI, rows_wg, k);
-    const size_t lds = (size_t)gemv_dma_lds(RP, NI, waves, rows_wg, k);
-    if (waves == 8)
-        HIPML_LAUNCH((gemv_q8_dma_kernel<RP, NI, 8>), grid, dim3(512, 1, 1), lds, st, w, x, y, m, k, rows, rows_wg);
-    else
-        HIPML_LAUNCH((gemv_q8_dma_kernel<RP, NI, 4>), grid, dim3(256, 1, 1), lds, st, w, x, y, m, k, rows, rows_wg);
-    return launched("gemv_q8_0_rows");
+    // The fewest weight rows that make one round of the chip's 256 CUs, every CU the same bytes (us at 1024 x 5120 over
+    // 1 / 2 / 4 / 8 rows: 4 rows a workgroup 4.4 / 5.7 / 7.3 / 9.0, 16 rows 5.5 / 6.9 / 8.5 / 11.3; at 5120 x 6144: 20 rows
+    // 9.6 / 11.4 / 12.9 / 16.7, 16 rows 11.9 / 14.7 / 18.3 / 24.3).
+    static const DmaRows kOneRound[5] = {{4, 2, false}, {8, 3, false}, {16, 5, false}, {20, 6, false}, {24, 7, false}};
+    for (const DmaRows &r : kOneRound)
+        if ((m + r.rows_wg - 1) / r.rows_wg <= 256)
+            return r;
+    // Beyond, small workgroups of which two or three share a CU, so that one's start and end lie behind another's
+    // stream (12288 x 5120 over 1 / 2 / 4 rows: 14.8 / 16.7 / 20.3 us; one workgroup of 48 rows per CU 17.9 / 18.7 / 20.5;
+    // 32 rows, a round and a half, 19.4 / 20.4 / 24.4).  With eight activation rows their copies fill the LDS and 32
+    // weight rows share them best (28.6; 16 rows 32.4).
+    if (rp == 1)
+        return {12, 4, false};
+    if (rp <= 4)
+        return {16, 5, true};
+    return {32, 9, false};
 }
 
-template <int NI>
-static int launch_gemv_dma_rows(hipStream_t st, const uint8_t *w, const float *x, float *y, int m, int k, int rows, int rows_wg)
+// Calls f with the kernel of (RP, NI, waves).
+template <int RP, typename F>
+static void with_gemv_dma_kernel(int ni, int waves, F &&f)
 {
-    if (rows == 1)
-        return launch_gemv_dma<1, NI>(st, w, x, y, m, k, rows, rows_wg);
-    if (rows == 2)
-        return launch_gemv_dma<2, NI>(st, w, x, y, m, k, rows, rows_wg);
-    if (rows <= 4)
-        return launch_gemv_dma<4, NI>(st, w, x, y, m, k, rows, rows_wg);
-    return launch_gemv_dma<8, NI>(st, w, x, y, m, k, rows, rows_wg);
+#define HIPML_DMA(n)                                            \
+    case n:                                                     \
+        return waves == 8 ? f(&gemv_q8_dma_kernel<RP, n, 8>)    \
+                          : f(&gemv_q8_dma_kernel<RP, n, 4>)
+    switch (ni) {
+        HIPML_DMA(2);
+        HIPML_DMA(3);
+        HIPML_DMA(5);
+        HIPML_DMA(6);
+        HIPML_DMA(7);
+    default:
+        if (RP == 1)
+            return waves == 8 ? f(&gemv_q8_dma_kernel<1, 4, 8>) : f(&gemv_q8_dma_kernel<1, 4, 4>);
+        return waves == 8 ? f(&gemv_q8_dma_kernel<8, 9, 8>) : f(&gemv_q8_dma_kernel<8, 9, 4>);
+    }
+#undef HIPML_DMA
+}
+
+template <int RP>
+static int launch_gemv_dma(hipStream_t st, const uint8_t *w, const float *x, float *y, int m, int k, int rows)
+{
+    const DmaRows r = gemv_dma_rows_wg(m, RP);
+    const dim3 grid((unsigned)((m + r.rows_wg - 1) / r.rows_wg), (unsigned)((rows + RP - 1) / RP), 1);
+    const int waves = r.four ? 4 : gemv_dma_waves(RP, r.ni, r.rows_wg, k);
+    const size_t lds = (size_t)gemv_dma_lds(RP, r.ni, waves, r.rows_wg, k);
+    with_gemv_dma_kernel<RP>(r.ni, waves, [&](auto kernel) {
+        HIPML_LAUNCH(kernel, grid, dim3(64 * waves, 1, 1), lds, st, w, x, y, m, k, rows, r.rows_wg);
+    });
+    return launched("gemv_q8_0_rows");
 }
 
 // Up to eight rows over the raw-row kernel: rows of whole 256-value chunks at 16-byte boundaries, addressed with
@@ -1140,98 +1219,102 @@ static int try_gemv_dma(hipStream_t st, const uint8_t *w, const float *x, float 
         (reinterpret_cast<uintptr_t>(x) & 15) != 0 || (size_t)m * (k >> 5) * kQ8Block >= ((size_t)1 << 32) ||
         (size_t)rows * k * sizeof(float) >= ((size_t)1 << 32))
         return -1;
-    // the fewest weight rows per workgroup that make one round of the chip's 256 CUs
-    static const int kRowsWg[4] = {16, 20, 24, 32}, kNi[4] = {5, 6, 7, 9};
-    int v = 3;
-    for (int i = 0; i < 4; i++)
-        if ((m + kRowsWg[i] - 1) / kRowsWg[i] <= 256) {
-            v = i;
-            break;
-        }
-    for (int rp = 1; rp <= 8; rp *= 2)
-        if (gemv_dma_waves(rp, kNi[v], kRowsWg[v], k) == 0)
+    for (int rp = 1; rp <= 8; rp *= 2) {
+        const DmaRows r = gemv_dma_rows_wg(m, rp);
+        if (gemv_dma_waves(rp, r.ni, r.rows_wg, k) == 0)
             return -1;
-    switch (v) {
-    case 0: return launch_gemv_dma_rows<5>(st, w, x, y, m, k, rows, 16);
-    case 1: return launch_gemv_dma_rows<6>(st, w, x, y, m, k, rows, 20);
-    case 2: return launch_gemv_dma_rows<7>(st, w, x, y, m, k, rows, 24);
-    default: return launch_gemv_dma_rows<9>(st, w, x, y, m, k, rows, 32);
     }
+    if (rows == 1)
+        return launch_gemv_dma<1>(st, w, x, y, m, k, rows);
+    if (rows == 2)
+        return launch_gemv_dma<2>(st, w, x, y, m, k, rows);
+    if (rows <= 4)
+        return launch_gemv_dma<4>(st, w, x, y, m, k, rows);
+    return launch_gemv_dma<8>(st, w, x, y, m, k, rows);
 }
 
-static int gemv_tile_xt(int rows)
+// Calls f with the kernel of (XT, RW, HALF), its threads and its LDS bytes.
+template <typename F>
+static void with_gemv_blocks_kernel(int xt, int rw, bool half, F &&f)
 {
-    const int pass = rows > 64 ? (rows + 1) / 2 : rows;
-    return (pass + 15) / 16;
+#define HIPML_BLOCKS(X, R)                                                                                      \
+    if (xt == X && rw == R)                                                                                     \
+        return half ? f(&gemv_q8_blocks_kernel<X, R, true>, 512, BlocksShape<X, R, true>::kLds)                 \
+                    : f(&gemv_q8_blocks_kernel<X, R, false>, 512, BlocksShape<X, R, false>::kLds)
+    HIPML_BLOCKS(1, 32);
+    HIPML_BLOCKS(1, 48);
+    HIPML_BLOCKS(2, 32);
+    HIPML_BLOCKS(2, 48);
+    HIPML_BLOCKS(3, 32);
+    HIPML_BLOCKS(3, 48);
+    HIPML_BLOCKS(4, 32);
+    HIPML_BLOCKS(4, 48);
+#undef HIPML_BLOCKS
 }
-
-template <int XT, int NI>
-static int launch_gemv_dma_tile(hipStream_t st, const uint8_t *w, const float *x, float *y, int m, int k, int rows,
-                                int rows_wg)
+template <typename F>
+static void with_gemv_units_kernel(int xt, int rw, bool half, F &&f)
 {
-    const dim3 grid((unsigned)((m + rows_wg - 1) / rows_wg), (unsigned)((rows + 16 * XT - 1) / (16 * XT)), 1);
-    const size_t lds = (size_t)gemv_dma_tile_lds(XT, NI, rows_wg);
-    if (grid.y == 1 && rows <= 16 * XT - 8)
-        HIPML_LAUNCH((gemv_q8_dma_tile_kernel<XT, NI, true>), grid, dim3(512, 1, 1), lds, st, w, x, y, m, k, rows, rows_wg);
-    else
-        HIPML_LAUNCH((gemv_q8_dma_tile_kernel<XT, NI, false>), grid, dim3(512, 1, 1), lds, st, w, x, y, m, k, rows, rows_wg);
-    return launched("gemv_q8_0_rows");
+#define HIPML_UNITS(X, R)                                                                                       \
+    if (xt == X && rw == R)                                                                                     \
+        return half ? f(&gemv_q8_units_kernel<X, R, true>, kUnitsThreads<X, R, true>, UnitsShape<X, R, true>::kLds) \
+                    : f(&gemv_q8_units_kernel<X, R, false>, kUnitsThreads<X, R, false>, UnitsShape<X, R, false>::kLds)
+    HIPML_UNITS(1, 16);
+    HIPML_UNITS(1, 20);
+    HIPML_UNITS(1, 24);
+    HIPML_UNITS(1, 32);
+    HIPML_UNITS(1, 48);
+    HIPML_UNITS(2, 16);
+    HIPML_UNITS(2, 20);
+    HIPML_UNITS(2, 24);
+    HIPML_UNITS(2, 32);
+    HIPML_UNITS(2, 48);
+#undef HIPML_UNITS
 }
+static const int kBlocksRw[2] = {32, 48}, kUnitsRw[5] = {16, 20, 24, 32, 48};
 
-template <int NI>
-static int launch_gemv_dma_tiles(hipStream_t st, const uint8_t *w, const float *x, float *y, int m, int k, int rows,
-                                 int rows_wg)
+static int launch_gemv_tiles(hipStream_t st, const uint8_t *w, const float *x, float *y, int m, int k, int rows)
 {
-    // the activation tiles of a pass: as many as the rows need, up to four; more than 64 rows: two passes (the
-    // grid's second dimension) that share the rows evenly
-    const int xt = gemv_tile_xt(rows);
-    switch (xt) {
-    case 1: return launch_gemv_dma_tile<1, NI>(st, w, x, y, m, k, rows, rows_wg);
-    case 2: return launch_gemv_dma_tile<2, NI>(st, w, x, y, m, k, rows, rows_wg);
-    case 3: return launch_gemv_dma_tile<3, NI>(st, w, x, y, m, k, rows, rows_wg);
-    default: return launch_gemv_dma_tile<4, NI>(st, w, x, y, m, k, rows, rows_wg);
-    }
-}
-
-// 9 rows and more over the raw-row tile kernel, under the conditions of try_gemv_dma.  Returns -1 where the shape
-// does not qualify.
-static int try_gemv_dma_tile(hipStream_t st, const uint8_t *w, const float *x, float *y, int m, int k, int rows)
-{
-    if (k % 256 != 0 || (reinterpret_cast<uintptr_t>(w) & 15) != 0 || (reinterpret_cast<uintptr_t>(x) & 15) != 0 ||
-        (size_t)m * (k >> 5) * kQ8Block >= ((size_t)1 << 32) || (size_t)rows * k * sizeof(float) >= ((size_t)1 << 32))
-        return -1;
-    static const int kRowsWg[4] = {16, 20, 24, 32};
-    int v = 3;
-    for (int i = 0; i < 4; i++)
-        if ((m + kRowsWg[i] - 1) / kRowsWg[i] <= 256) {
-            v = i;
-            break;
+    // by the shape of W alone: a row has the same bits however many travel with it
+    const bool blocks = m > 6144 && k % 256 == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0;
+    // the tile that costs least: rounds of 256 workgroups x the cycles of a unit in the eight waves of a CU, as the sum
+    // of its vector instructions (two waves a SIMD, 4 cycles each) and its requests (16 cycles); within 20 % of the
+    // measured times less 4 us, and in their order, at 1024 / 5120 / 12288 weight rows over 9 to 100 rows
+    int xt = 0, rw = 0;
+    long long best = 0;
+    for (int cx = 1; cx <= (blocks ? 4 : 2) && 16 * (cx - 1) < rows; cx++)
+        for (int cr : kUnitsRw) {
+            if (blocks && cr < 32)
+                continue;
+            const int mt = (cr + 15) / 16, ty = (rows + 16 * cx - 1) / (16 * cx);
+            const long long rounds = ((long long)((m + cr - 1) / cr) * ty + 255) / 256;
+            const int valu = 26 * mt + 28 * cx + 8 * mt * cx + 20;
+            const int requests = 4 * cx + (cr * 17 + 63) / 64 / (blocks ? 4 : 1);
+            const long long cost = rounds * (8 * valu + 8 * 16 * requests);
+            if (best == 0 || cost < best) {
+                best = cost;
+                xt = cx;
+                rw = cr;
+            }
         }
-    static const int kNi[4] = {5, 6, 7, 9};
-    const int xt = gemv_tile_xt(rows);
-    if (gemv_dma_tile_lds(xt, kNi[v], kRowsWg[v]) > (160 << 10))
-        return -1;
-    switch (v) {
-    case 0: return launch_gemv_dma_tiles<5>(st, w, x, y, m, k, rows, 16);
-    case 1: return launch_gemv_dma_tiles<6>(st, w, x, y, m, k, rows, 20);
-    case 2: return launch_gemv_dma_tiles<7>(st, w, x, y, m, k, rows, 24);
-    default: return launch_gemv_dma_tiles<9>(st, w, x, y, m, k, rows, 32);
-    }
+    const dim3 grid((unsigned)((m + rw - 1) / rw), (unsigned)((rows + 16 * xt - 1) / (16 * xt)), 1);
+    const bool half = grid.y == 1 && rows <= 16 * xt - 8;
+    auto go = [&](auto kernel, int threads, int lds) {
+        HIPML_LAUNCH(kernel, grid, dim3((unsigned)threads, 1, 1), (size_t)lds, st, w, x, y, m, k, rows);
+    };
+    if (blocks)
+        with_gemv_blocks_kernel(xt, rw, half, go);
+    else
+        with_gemv_units_kernel(xt, rw, half, go);
+    return launched("gemv_q8_0_rows");
 }
 
 int launch_gemv_q8_rows(hipStream_t st, const uint8_t *w, const float *x, float *y, int m, int k, int rows)
 {
-    // (10 rows and more: the raw-row tile kernel, in two passes beyond 64; 9 rows measured slower there than in the
-    // tile kernel below: 17.2 against 16.0 us at 5120 x 6144)
-    const int dma = rows <= 8 ? try_gemv_dma(st, w, x, y, m, k, rows)
-                              : (rows >= 10 && rows <= 128 ? try_gemv_dma_tile(st, w, x, y, m, k, rows) : -1);
+    const int dma = rows <= 8 ? try_gemv_dma(st, w, x, y, m, k, rows) : -1;
     if (dma >= 0)
         return dma;
-    // three rows or more: full A tiles of 16 or 32 rows (measured at 5120 x 6144, 4 rows: 14.6 us
-    // against 16.7 us for the row kernel with two weight tiles per workgroup; 1 row: 13.6 against 12.1)
     if (rows > kGemvMaxRows)
-        return rows > 16 ? launch_gemv_tile<8, 2, 2>(st, w, x, y, m, k, rows)
-                         : launch_gemv_tile<8, 2, 1>(st, w, x, y, m, k, rows);
+        return launch_gemv_tiles(st, w, x, y, m, k, rows);
     int rp = gemv_rows_per_pass(k);
     if (rp < 1)
         return fail(HIPML_ATTN_E_RANGE, "k %d: one activation row does not fit the LDS operand buffer", k);
@@ -1264,28 +1347,24 @@ int proj_init()
         if (e == hipSuccess)
             e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 << 10);
     };
-#define HIPML_RAISE_DMA(ni) \
-    raise(reinterpret_cast<const void *>(&gemv_q8_dma_kernel<1, ni, 8>)); \
-    raise(reinterpret_cast<const void *>(&gemv_q8_dma_kernel<2, ni, 8>)); \
-    raise(reinterpret_cast<const void *>(&gemv_q8_dma_kernel<4, ni, 8>)); \
-    raise(reinterpret_cast<const void *>(&gemv_q8_dma_kernel<8, ni, 8>)); \
-    raise(reinterpret_cast<const void *>(&gemv_q8_dma_kernel<1, ni, 4>)); \
-    raise(reinterpret_cast<const void *>(&gemv_q8_dma_kernel<2, ni, 4>)); \
-    raise(reinterpret_cast<const void *>(&gemv_q8_dma_kernel<4, ni, 4>)); \
-    raise(reinterpret_cast<const void *>(&gemv_q8_dma_kernel<8, ni, 4>));
-    HIPML_RAISE_DMA(5) HIPML_RAISE_DMA(6) HIPML_RAISE_DMA(7) HIPML_RAISE_DMA(9)
-#undef HIPML_RAISE_DMA
-#define HIPML_RAISE_TILE(ni) \
-    raise(reinterpret_cast<const void *>(&gemv_q8_dma_tile_kernel<1, ni, false>)); \
-    raise(reinterpret_cast<const void *>(&gemv_q8_dma_tile_kernel<2, ni, false>)); \
-    raise(reinterpret_cast<const void *>(&gemv_q8_dma_tile_kernel<3, ni, false>)); \
-    raise(reinterpret_cast<const void *>(&gemv_q8_dma_tile_kernel<4, ni, false>)); \
-    raise(reinterpret_cast<const void *>(&gemv_q8_dma_tile_kernel<1, ni, true>)); \
-    raise(reinterpret_cast<const void *>(&gemv_q8_dma_tile_kernel<2, ni, true>)); \
-    raise(reinterpret_cast<const void *>(&gemv_q8_dma_tile_kernel<3, ni, true>)); \
-    raise(reinterpret_cast<const void *>(&gemv_q8_dma_tile_kernel<4, ni, true>));
-    HIPML_RAISE_TILE(5) HIPML_RAISE_TILE(6) HIPML_RAISE_TILE(7) HIPML_RAISE_TILE(9)
-#undef HIPML_RAISE_TILE
+    auto raise_dma = [&](auto rp) {
+        constexpr int RP = decltype(rp)::value;
+        for (int ni : {2, 3, 4, 5, 6, 7, 9})
+            for (int waves : {4, 8})
+                with_gemv_dma_kernel<RP>(ni, waves, [&](auto kernel) { raise(reinterpret_cast<const void *>(kernel)); });
+    };
+    raise_dma(std::integral_constant<int, 1>{});
+    raise_dma(std::integral_constant<int, 2>{});
+    raise_dma(std::integral_constant<int, 4>{});
+    raise_dma(std::integral_constant<int, 8>{});
+    for (int xt = 1; xt <= 4; xt++)
+        for (bool half : {false, true}) {
+            auto up = [&](auto kernel, int, int) { raise(reinterpret_cast<const void *>(kernel)); };
+            for (int rw : kBlocksRw)
+                with_gemv_blocks_kernel(xt, rw, half, up);
+            for (int rw : kUnitsRw)
+                with_gemv_units_kernel(xt, rw, half, up);
+        }
     if (e != hipSuccess)
         return fail((int)e, "hipFuncSetAttribute(projection LDS) failed: %d (%s)", (int)e, hipGetErrorString(e));
     return 0;

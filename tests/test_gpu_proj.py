@@ -336,3 +336,34 @@ def test_gemm_tiles(m, k, t):
     assert np.array_equal(host(y16), got)
     for i in (0, t // 2, t - 1):
         assert np.array_equal(run_gemm(w, x[i:i + 1], m, k, 1)[0], got[i])
+
+
+@pytest.mark.parametrize("m,k", [(1030, 512), (2100, 256), (12290, 512)])
+def test_raw_row_kernel_workgroup_sizes(m, k):
+    # 8 and 16 weight rows per workgroup, and the small workgroups of which several share a CU (12 rows for one
+    # activation row, 16 for two to four)
+    test_raw_row_kernel_over_ragged_shapes(m, k)
+
+
+@pytest.mark.parametrize("m,k", [(12290, 512), (6200, 2304), (300, 320), (5000, 64), (2050, 1088)])
+def test_row_tile_kernels(m, k):
+    # more rows than the raw-row kernel takes (or a k it does not take): the kernel in step over chunks (m above 6,144,
+    # k a multiple of 256) and the one whose waves stream units of their own, with idle waves, uneven shares, tiles
+    # half dead; every row's bits the same whatever travels with it
+    r = orc.Rng(0x711F + m + k)
+    w = orc.random_q8_0_bytes(r, m * k // 32).reshape(-1, 34)
+    scales = (r.uniform_array(w.shape[0]) * 0.05 + 0.001).astype(np.float16)
+    w[:, :2] = scales.view(np.uint8).reshape(-1, 2)
+    w = w.ravel()
+    x = r.normal_array((128, k), 0.25)
+    blocks = w.reshape(m, k // 32, 34)
+    dense = (blocks[:, :, :2].copy().view(np.float16).astype(np.float64)
+             * blocks[:, :, 2:].view(np.int8).astype(np.float64)).reshape(m, k)
+    exact = x.astype(np.float64) @ dense.T
+    full = run_gemv(w, x, m, k, 128)
+    assert np.max(np.abs(full - exact)) <= 2e-6 * np.max(np.abs(exact)) + 1e-5
+    for rows in (9, 16, 17, 24, 32, 33, 40, 64, 65, 100):
+        assert np.array_equal(run_gemv(w, x[:rows], m, k, rows), full[:rows]), f"rows={rows}"
+    if k % 256 != 0:
+        assert np.array_equal(run_gemv(w, x[:3], m, k, 3), full[:3])
+    assert np.array_equal(run_gemv(w, x[60:75], m, k, 15), full[60:75])
