@@ -2109,6 +2109,43 @@ int chunk_tiles_splits(int pos0, int tokens, int n_head, int n_kv, int slices)
     return slices + (int)((tiles + per_slice - 1) / per_slice);
 }
 
+// Slices that a long chunk over f16 tiles runs of the `most` its scratch holds.  The caller's count fills the last
+// round of 256 workgroups; what it leaves out is that every slice writes its partial rows and has them read again
+// (2 KB per token and head at about 5 TB/s), and that a round of fewer workgroups runs faster (the chip holds its
+// clock by power: 15 % between an empty and a full one).  In units of a key tile of a full round (3 us): rounds x
+// (tiles of a slice + 4) x (1 + 0.15 fill) + slices x what their partial rows cost; within 8 % of the measured call at
+// ten shapes with 2 to 16 slices each.  us with the caller's count / with this one: 1,024 tokens at depth 8,192 264
+// (8 slices) / 242 (5), 1,500 at 20,000 852 (12) / 713 (3), 700 at 10,000 232 (10) / 193 (3), 800 at 40,000 735 (10) /
+// 703 (3); 2,048 at 100,000 keeps its 4.  Only counts for which every block of tokens gets all slices and the 64-token
+// kernel runs; chunks for which tiles are not made keep the caller's count.
+static int chunk_tile_slices(int pos0, int tokens, int n_head, int n_kv, int most)
+{
+    const int group = n_head / n_kv, tiles = (pos0 + tokens + kKTile - 1) / kKTile;
+    const int first_tokens = tokens < 64 ? tokens : 64; // (of the first block: it must see enough tiles for every slice)
+    const int first_tiles = (pos0 + first_tokens + kKTile - 1) / kKTile;
+    const int block32 = ((tokens + kQTile - 1) / kQTile * group + kTasks - 1) / kTasks;
+    const int rem = tokens % kT64Tile;
+    const int task64 = (tokens / kT64Tile + (rem > 32 ? 1 : 0)) * group + (rem > 0 && rem <= 32 ? (group + 1) / 2 : 0);
+    const int block64 = (task64 + kT64Tasks - 1) / kT64Tasks;
+    const float per_slice = (float)tokens * (float)n_head * (2048.0f / 5.0e6f / 3.0f);
+    int best = most;
+    float best_cost = 0.0f;
+    for (int s = 2; s <= most; s++) {
+        const int slice_tiles = (tiles + s - 1) / s;
+        const int rounds = (n_kv * s * block64 + 255) / 256;
+        if ((first_tiles + slice_tiles - 1) / slice_tiles < s || (tiles + slice_tiles - 1) / slice_tiles < s ||
+            rounds > (n_kv * s * block32 + 255) / 256)
+            continue;
+        const float fill = (float)(n_kv * s * block64) / (256.0f * (float)rounds);
+        const float cost = (float)rounds * ((float)slice_tiles + 4.0f) * (1.0f + 0.15f * fill) + (float)s * per_slice;
+        if (best_cost == 0.0f || cost < best_cost) {
+            best = s;
+            best_cost = cost;
+        }
+    }
+    return best;
+}
+
 int launch_chunk_q8(hipStream_t st, const float *q, const uint8_t *kc, const uint8_t *vc,
                     float *out, int n_head, int n_kv, int pos0, int tokens, int stride,
                     float *part_acc, float *part_ml, int splits, const float *gate, int q4, void *out16,
@@ -2136,6 +2173,8 @@ int launch_chunk_q8(hipStream_t st, const float *q, const uint8_t *kc, const uin
                 splits = s;
         }
     }
+    if (kv_f16 != nullptr && splits > 2 && chunk_tiles_pay(pos0, tokens))
+        splits = chunk_tile_slices(pos0, tokens, n_head, n_kv, splits);
     // rope_tab != nullptr (splits == 0 only): q holds unrotated rows, the kernel rotates them as it loads them
     ChunkArgs a;
     // kv_f16 != nullptr: K and V are read from the f16 copy of the cache (kc, vc unused)
