@@ -21,12 +21,15 @@
 //    sum of both: 2,150 cycles against 1,500 (192 x 192: 146 -> 117 us; 256 x 192 over 1,024 tokens: 166 -> 144 us).
 //  * small tiles with longer steps (KU 2 and 4) and eight producer waves where there are too few outputs for large
 //    ones: a step's cost is then latency, not work (1024 x 5120 over 117 tokens: 32 x 32 tiles 15 us, 128 x 128 48 us).
+//  * weights by whole 64-byte sectors, one aligned request of a quad of lanes each, where their rows allow it.  A row's
+//    pair of blocks is 68 bytes: asked for as it lies (12 and 8 bytes a lane) it takes three requests, most of them
+//    across a sector boundary, and the weights of a step cost the vector memory path as much as the activations
+//    (192 x 192 over 672 tokens 121 -> 108 us, 64 x 128 over 117 48 -> 42, 64 x 64 31 -> 27).  Tried on it: two sectors
+//    of a line asked for together (no gain), activations non-temporal (10 % slower), deeper records (no gain).
 // Before (128 x 128 tiles for every shape) and now, us: 12288 x 5120 over 117 / 672 / 1,024 / 2,048 tokens 78 / 173 /
-// 217 / 432 -> 34 / 117 / 144 / 284; 1024 x 5120 over the same 54 / 56 / 58 / 60 -> 15 / 25 / 32 / 49; 5120 x 6144
-// (f16 activations) 50 / 58 / 111 / 172 -> 24 / 58 / 81 / 137.
+// 217 / 432 -> 42 / 108 / 144 / 284; 1024 x 5120 over the same 74 / 56 / 69 / 71 -> 15 / 23 / 31 / 49; 5120 x 6144
+// (f16 activations) 62 / 58 / 111 / 172 -> 25 / 58 / 80 / 134.
 //
-// Weight fetch: the four lanes of a quad take the quarters of a pair of blocks of one row, 12 bytes of the even block
-// (2 bytes in; the scales ride along in lanes 0 and 3) and 8 of the odd one, dword aligned.
 // A tile row in LDS is an odd number of 16-byte groups: 128-bit reads and writes of 16 consecutive rows touch every
 // bank once.
 
@@ -39,13 +42,6 @@ namespace hipml {
 constexpr int gemm_pitch(int ku) { return 128 * ku + 16; } // bytes of a tile row
 constexpr int gemm_lds(int tt, int tm, int ku) { return 2 * (tt + tm) * gemm_pitch(ku); } // double buffered
 
-template <int WN, int XN>
-struct GemmFetch {
-    uint3a4 e[WN]; // even-block quarter (+ scales in quad lanes 0 and 3)
-    uint2a4 o[WN]; // odd-block quarter
-    float4v x[XN]; // f32: 4 activations; f16: 8
-};
-
 __device__ __forceinline__ half8 dequant8(uint32_t w0, uint32_t w1, _Float16 d)
 {
     const half8 q = int8x8_to_f16(w0, w1);
@@ -54,11 +50,37 @@ __device__ __forceinline__ half8 dequant8(uint32_t w0, uint32_t w1, _Float16 d)
 }
 
 
-template <bool X16, int CT, int CM, int AT, int BT, int KU, int NW, int R>
+// The lane at quad position i gets the value of position i + 1, the last one that of position 0.
+__device__ __forceinline__ uint32_t quad_next(uint32_t v)
+{
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x39, 0xf, 0xf, true);
+}
+
+// ... position i - 1, the first one that of position 3.
+__device__ __forceinline__ uint32_t quad_prev(uint32_t v)
+{
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x93, 0xf, 0xf, true);
+}
+
+// The weights of one producer thread's rows, for rows of whole 64-byte sectors (k a multiple of 1,024, W at a 64-byte
+// boundary): the four lanes of a quad share a row and load a sector in one request, lane i its 16 bytes i.  A set is
+// the five sectors that hold four units: unit u (17 dwords) starts u % 16 dwords into sector u + u / 16.
+template <int WS, int SETS>
+struct WideWeights {
+    uint4v p[SETS][WS][5];
+};
+// The same for any k of whole units and W at a 4-byte boundary: a lane takes a quarter of a pair of blocks, 12 bytes
+// of the even block (2 bytes in; the scales ride along in lanes 0 and 3) and 8 of the odd one.
+template <int WP, int SETS>
+struct QuarterWeights {
+    uint3a4 e[SETS][WP];
+    uint2a4 o[SETS][WP];
+};
+
+template <bool X16, bool WIDE, int CT, int CM, int AT, int BT, int KU, int NW, int R>
 __global__ void __launch_bounds__(64 * (NW + CT * CM)) gemm_q8_f16_kernel(const uint8_t *__restrict__ w,
-                                                                              const void *__restrict__ xv,
-                                                                              float *__restrict__ y, int m, int k,
-                                                                              int tokens)
+                                                                          const void *__restrict__ xv,
+                                                                          float *__restrict__ y, int m, int k, int tokens)
 {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     constexpr int NT = 64 * NW; // producer threads
@@ -74,25 +96,13 @@ __global__ void __launch_bounds__(64 * (NW + CT * CM)) gemm_q8_f16_kernel(const 
     const int nsteps = k / kGemmK;
 
     if (producer) {
-        const uint32_t row_bytes = (uint32_t)(k >> 5) * kQ8Block;
-        constexpr int WP = TM * 4 * KU / NT; // weight (unit, row, quarter) triples per producer thread
-        static_assert(WP * NT == TM * 4 * KU, "");
-        constexpr int XELT = X16 ? 2 : 4;  // bytes per activation
-        constexpr int XV = 16 / XELT;      // activations per 16-byte piece
-        constexpr int XPR = kGemmK / XV;   // pieces per tile row
-        constexpr int XN = TT * XPR / NT;  // pieces per producer thread
+        // ---- activations: XN pieces of 16 bytes per thread and step, R steps on the way
+        constexpr int XELT = X16 ? 2 : 4; // bytes per activation
+        constexpr int XV = 16 / XELT;     // activations per piece
+        constexpr int XPR = kGemmK / XV;  // pieces per tile row
+        constexpr int XN = TT * XPR / NT;
         static_assert(XN * NT == TT * XPR, "");
-        constexpr int XROWS = NT / XPR;    // rows covered by one piece of the workgroup
-        const uint8_t *wb = w + (size_t)m0 * row_bytes;
-        uint32_t woff[WP], wlds[WP];
-#pragma unroll
-        for (int h = 0; h < WP; h++) {
-            const int rest = (h * NT + tid) >> 2, fg = tid & 3;
-            const int r = rest % TM, unit = rest / TM; // (four lanes share a row: its k quarters)
-            const int row = m0 + r < m ? r : m - 1 - m0;
-            woff[h] = (uint32_t)row * row_bytes + unit * (2 * kQ8Block) + fg * 8;
-            wlds[h] = kXTile + r * kGemmPitch + unit * 128 + fg * 16;
-        }
+        constexpr int XROWS = NT / XPR; // rows covered by one piece of the workgroup
         const int xr = tid / XPR, xc = tid % XPR;
         const uint8_t *xb = static_cast<const uint8_t *>(xv) + (size_t)t0 * k * XELT;
         uint32_t xoff[XN];
@@ -101,73 +111,158 @@ __global__ void __launch_bounds__(64 * (NW + CT * CM)) gemm_q8_f16_kernel(const 
             const int t = t0 + xr + XROWS * i < tokens ? xr + XROWS * i : tokens - 1 - t0;
             xoff[i] = (uint32_t)t * (uint32_t)(k * XELT) + xc * 16;
         }
-        typedef GemmFetch<WP, XN> Fetch;
-        // piece h of a record: WP of them, each one weight pair and its share of the activations
-        auto fetch_piece = [&](Fetch &f, int s, int h) {
-            const int sc = s < nsteps ? s : nsteps - 1;
-            const uint8_t *ws = wb + (size_t)sc * (2 * KU * kQ8Block);
-            const uint8_t *xs = xb + (size_t)sc * (kGemmK * XELT);
-            const uint8_t *unit = ws + woff[h];
-            f.e[h] = *reinterpret_cast<const uint3a4 *>(unit);
-            f.o[h] = *reinterpret_cast<const uint2a4 *>(unit + 36);
+        float4v xrec[R][XN]; // f32: 4 activations; f16: 8
+        auto fetch_x = [&](int r, int s) {
+            const uint8_t *xs = xb + (size_t)(s < nsteps ? s : nsteps - 1) * (kGemmK * XELT);
 #pragma unroll
-            for (int i = h * XN / WP; i < (h + 1) * XN / WP; i++)
-                f.x[i] = *reinterpret_cast<const float4v *>(xs + xoff[i]);
-        };
-        auto fetch = [&](Fetch &f, int s) {
-#pragma unroll
-            for (int h = 0; h < WP; h++)
-                fetch_piece(f, s, h);
+            for (int i = 0; i < XN; i++)
+                xrec[r][i] = *reinterpret_cast<const float4v *>(xs + xoff[i]);
         };
         uint8_t *xdst = lds + xr * kGemmPitch + xc * (X16 ? 16 : 8);
-        auto stage_piece = [&](const Fetch &f, int b, int h) {
-            const uint3a4 e = f.e[h];
-            const uint32_t s0 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)e[0], 0x00, 0xf, 0xf, true);
-            const uint32_t s1 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)e[2], 0xFF, 0xf, 0xf, true);
-            const _Float16 d0 = __builtin_bit_cast(_Float16, (uint16_t)(s0 & 0xffffu));
-            const _Float16 d1 = __builtin_bit_cast(_Float16, (uint16_t)(s1 >> 16));
-            const half8 v0 = dequant8(__builtin_amdgcn_alignbit(e[1], e[0], 16),
-                                      __builtin_amdgcn_alignbit(e[2], e[1], 16), d0);
-            const half8 v1 = dequant8(f.o[h][0], f.o[h][1], d1);
-            uint8_t *dw = lds + b * kBuf + wlds[h];
-            *reinterpret_cast<half8 *>(dw) = v0;      // k = fg*8 .. of the even block
-            *reinterpret_cast<half8 *>(dw + 64) = v1; // k = 32 + fg*8 .. (the odd block)
+        auto stage_x = [&](int r, int b) {
 #pragma unroll
-            for (int i = h * XN / WP; i < (h + 1) * XN / WP; i++) {
+            for (int i = 0; i < XN; i++) {
                 uint8_t *d = xdst + b * kBuf + XROWS * i * kGemmPitch;
                 if (X16)
-                    *reinterpret_cast<float4v *>(d) = f.x[i];
+                    *reinterpret_cast<float4v *>(d) = xrec[r][i];
                 else // round to nearest even: truncation would bias every product the same way
-                    *reinterpret_cast<half4v *>(d) = __builtin_convertvector(f.x[i], half4v);
+                    *reinterpret_cast<half4v *>(d) = __builtin_convertvector(xrec[r][i], half4v);
             }
         };
-        auto stage = [&](const Fetch &f, int b) {
+
+        // ---- weights
+        const uint32_t row_bytes = (uint32_t)(k >> 5) * kQ8Block;
+        const uint8_t *wb = w + (size_t)m0 * row_bytes;
+        constexpr int CS = WIDE ? 4 / KU : 1;                     // steps per set
+        constexpr int SETS = WIDE ? (KU == 1 ? 1 : 2) : R;
+        constexpr int WWAVES = WIDE && TM < 16 * NW ? TM / 16 : NW; // waves that carry weights
+        constexpr int WS = WIDE ? TM / (16 * WWAVES) : TM * 4 * KU / NT; // rows, or (unit, row, quarter) triples, per thread
+        static_assert(WIDE ? WS * 16 * WWAVES == TM : WS * NT == TM * 4 * KU, "");
+        typename std::conditional<WIDE, WideWeights<WS, SETS>, QuarterWeights<WS, SETS>>::type wrec;
+        uint32_t woff[WS], wlds[WS];
+        const int qi = tid & 3; // four lanes share a row
 #pragma unroll
-            for (int h = 0; h < WP; h++)
-                stage_piece(f, b, h);
+        for (int h = 0; h < WS; h++) {
+            const int rest = WIDE ? (h * 64 * WWAVES + tid) >> 2 : (h * NT + tid) >> 2;
+            const int r = rest % TM, unit = rest / TM;
+            const int row = m0 + r < m ? r : m - 1 - m0;
+            woff[h] = (uint32_t)row * row_bytes + (WIDE ? qi * 16 : unit * (2 * kQ8Block) + qi * 8);
+            wlds[h] = kXTile + r * kGemmPitch + (WIDE ? 0 : unit * 128 + qi * 16);
+        }
+        const int nsets = nsteps / CS;
+        // what staging position v (a step within the SETS sets) leaves free of set v / CS is asked for anew, SETS sets on
+        auto fetch_w = [&](int v, int s) {
+            const int set = v / CS % SETS, sub = v % CS;
+            if constexpr (WIDE) {
+                int c = (s + CS * SETS) / CS;
+                c = c < nsets ? c : nsets - 1;
+                const uint8_t *ws = wb + (size_t)(4 * c + (c >> 2)) * 64;
+#pragma unroll
+                for (int h = 0; h < WS; h++) {
+#pragma unroll
+                    for (int j = sub * KU; j < (sub + 1) * KU; j++)
+                        wrec.p[set][h][j] = *reinterpret_cast<const uint4v *>(ws + woff[h] + j * 64);
+                    if (sub == CS - 1)
+                        wrec.p[set][h][4] = *reinterpret_cast<const uint4v *>(ws + woff[h] + 256);
+                }
+            } else {
+                const int c = s + SETS < nsteps ? s + SETS : nsteps - 1;
+                const uint8_t *ws = wb + (size_t)c * (2 * KU * kQ8Block);
+#pragma unroll
+                for (int h = 0; h < WS; h++) {
+                    wrec.e[set][h] = *reinterpret_cast<const uint3a4 *>(ws + woff[h]);
+                    wrec.o[set][h] = *reinterpret_cast<const uint2a4 *>(ws + woff[h] + 36);
+                }
+            }
         };
-        Fetch rec[R];
-        constexpr int U = R & 1 ? 2 * R : R;
-        auto produce = [&](auto first) {
-            constexpr bool kLoadFirst = decltype(first)::value;
-            // records: step s + 1 .. s + R are on the way (load first: s + 1 .. s + R - 1, the newest is asked for at
-            // the head of the turn)
+        auto stage_w = [&](int v, int s, int b) {
+            const int set = v / CS % SETS, sub = v % CS;
+            if constexpr (WIDE) {
+                // Unit j of set c starts j dwords into the 16 bytes of lane q = c % 4 of sector j.  The lanes from q on,
+                // then those before it with the next sector, are the unit's logical lanes 0 .. 3: a logical lane's 16
+                // values are its own dwords j .. 3 and the first of the lane behind it (for the last, of the next sector
+                // of lane q).  Logical lanes 0 and 1 hold the even block, whose values start 2 bytes in, 2 and 3 the odd
+                // one, a dword further; the scales lie at the head of lane 0 and in the upper half of lane 2's first
+                // dword.
+                const int q = (s / CS) & 3, li = (qi - q) & 3;
+                const bool here = qi >= q, past = qi > q, odd = li >= 2;
+                const uint32_t pick = odd ? 0x07060504u : 0x05040302u, shift = odd ? 16u : 0u;
+                uint8_t *const dst0 = lds + b * kBuf + li * 32;
+#pragma unroll
+                for (int h = 0; h < WS; h++)
+#pragma unroll
+                    for (int u = 0; u < KU; u++) {
+                        const int j = sub * KU + u;
+                        const uint4v p0 = wrec.p[set][h][j], p1 = wrec.p[set][h][j + 1];
+                        uint32_t d[5];
+#pragma unroll
+                        for (int n = 0; n < 5; n++) {
+                            const int e = (j + n) & 3;
+                            d[n] = j + n < 4 ? (here ? p0[e] : p1[e]) : quad_next(past ? p0[e] : p1[e]);
+                        }
+                        const uint32_t prev = quad_prev(d[0]); // (outside the choice: every lane takes part)
+                        const uint32_t sc = ((li & 1) ? prev : d[0]) >> shift;
+                        const _Float16 scale = __builtin_bit_cast(_Float16, (uint16_t)sc);
+                        uint32_t q[4];
+#pragma unroll
+                        for (int n = 0; n < 4; n++)
+                            q[n] = __builtin_amdgcn_perm(d[n + 1], d[n], pick);
+                        uint8_t *dst = dst0 + wlds[h] + u * 128;
+                        *reinterpret_cast<half8 *>(dst) = dequant8(q[0], q[1], scale);
+                        *reinterpret_cast<half8 *>(dst + 16) = dequant8(q[2], q[3], scale);
+                    }
+            } else {
+#pragma unroll
+                for (int h = 0; h < WS; h++) {
+                    const uint3a4 e = wrec.e[set][h];
+                    const uint32_t s0 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)e[0], 0x00, 0xf, 0xf, true);
+                    const uint32_t s1 = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)e[2], 0xFF, 0xf, 0xf, true);
+                    const _Float16 d0 = __builtin_bit_cast(_Float16, (uint16_t)(s0 & 0xffffu));
+                    const _Float16 d1 = __builtin_bit_cast(_Float16, (uint16_t)(s1 >> 16));
+                    uint8_t *dst = lds + b * kBuf + wlds[h];
+                    *reinterpret_cast<half8 *>(dst) = dequant8(__builtin_amdgcn_alignbit(e[1], e[0], 16),
+                                                               __builtin_amdgcn_alignbit(e[2], e[1], 16), d0);
+                    *reinterpret_cast<half8 *>(dst + 64) = dequant8(wrec.o[set][h][0], wrec.o[set][h][1], d1);
+                }
+            }
+        };
+
+        constexpr int CYCLE = CS * SETS;
+        constexpr int U0 = R % 2 ? 2 * R : R, U = CYCLE > U0 ? CYCLE : U0;
+        static_assert(U % U0 == 0 && U % CYCLE == 0, "the records of a turn of the loop are named at compile time");
+        auto produce = [&](auto load_first, auto weights) {
+            constexpr bool kLoadFirst = decltype(load_first)::value, kWeights = decltype(weights)::value;
+            auto fetch = [&](int v, int s) { // what staging step s (position v) has left free
+                if (kWeights)
+                    fetch_w(v % CYCLE, s);
+                fetch_x(v % R, s + R);
+            };
+            auto stage = [&](int v, int s) {
+                if (kWeights)
+                    stage_w(v % CYCLE, s, v & 1);
+                stage_x(v % R, v & 1);
+            };
+            if (kWeights) {
+#pragma unroll
+                for (int v = 0; v < CYCLE; v++)
+                    fetch_w(v, v - CYCLE);
+            }
 #pragma unroll
             for (int r = 0; r < R; r++)
-                fetch(rec[r], r);
-            stage(rec[0], 0);
+                fetch_x(r, r);
+            stage(0, 0);
             if (!kLoadFirst)
-                fetch(rec[0], R);
+                fetch(0, 0);
             __syncthreads();
-            auto step = [&](int u, int s) {
+            auto step = [&](int u, int s) { // stage step s + 1 while step s is multiplied
                 if (kLoadFirst) {
-                    fetch(rec[u % R], s + R);
+                    fetch(u, s);
                     __builtin_amdgcn_sched_barrier(0);
-                    stage(rec[(u + 1) % R], (u + 1) & 1);
+                    stage(u + 1, s + 1);
                 } else {
-                    stage(rec[(u + 1) % R], (u + 1) & 1);
+                    stage(u + 1, s + 1);
                     __builtin_amdgcn_sched_barrier(0);
-                    fetch(rec[(u + 1) % R], s + 1 + R);
+                    fetch(u + 1, s + 1);
                 }
             };
             int s = 0;
@@ -187,10 +282,18 @@ __global__ void __launch_bounds__(64 * (NW + CT * CM)) gemm_q8_f16_kernel(const 
                     __syncthreads();
             }
         };
-        if (wave & 1)
-            produce(std::integral_constant<bool, true>{});
-        else
-            produce(std::integral_constant<bool, false>{});
+        const std::true_type yes;
+        const std::false_type no;
+        if (WWAVES < NW && wave >= WWAVES) {
+            if (wave & 1)
+                produce(yes, no);
+            else
+                produce(no, no);
+        } else if (wave & 1) {
+            produce(yes, yes);
+        } else {
+            produce(no, yes);
+        }
         return;
     }
     // consumer wave (wt, wm): tokens wt * 32 AT .., weight rows wm * 32 BT ..
@@ -296,35 +399,43 @@ __global__ void __launch_bounds__(256) gate_f16_kernel(const float4v *__restrict
 
 // ---- which tile ----------------------------------------------------------------------------------------------
 //
-// (token rows and weight rows of the tile, 64-value units per step, microseconds per unit and round of the chip's 256
-// CUs as measured with one round of workgroups at k = 5120)
+// (token rows and weight rows of the tile, 64-value units per step, sectors or quarters for the weights, microseconds
+// per unit and round of the chip's 256 CUs over f32 and over f16 activations: measured at k = 5120 and 6144, less 4 us
+// per launch, with the slow-down of a full chip below taken out)
 struct GemmTile {
     int tt, tm, ku;
-    float cost;
+    bool wide;
+    float cost, cost16;
 };
 constexpr GemmTile kGemmTiles[] = {
-    {32, 32, 4, 0.14f},    {32, 64, 4, 0.17f},    {64, 64, 2, 0.23f},    {64, 128, 2, 0.35f},
-    {128, 128, 1, 0.53f},  {192, 128, 1, 0.70f},  {128, 192, 1, 0.76f},  {192, 192, 1, 0.92f}, {256, 192, 1, 1.12f},
-    {64, 64, 1, 0.33f}, // (the smallest for an odd number of units)
+    {32, 32, 4, true, 0.13f, 0.13f},   {32, 64, 4, true, 0.165f, 0.139f},  {64, 64, 2, true, 0.23f, 0.19f},
+    {64, 128, 2, true, 0.35f, 0.28f},  {128, 128, 1, true, 0.52f, 0.405f}, {192, 128, 1, true, 0.72f, 0.55f},
+    {128, 192, 1, true, 0.71f, 0.62f}, {192, 192, 1, true, 0.87f, 0.78f},  {256, 192, 1, true, 0.0f, 0.98f},
+    // rows of weights that are not whole sectors (and the largest tile over f32 activations, whose registers do not
+    // hold both)
+    {256, 192, 1, false, 1.12f, 1.05f}, {192, 192, 1, false, 0.97f, 0.87f}, {128, 128, 1, false, 0.56f, 0.50f},
+    {64, 64, 2, false, 0.26f, 0.23f},   {64, 64, 1, false, 0.34f, 0.30f},
 };
 constexpr int kGemmNTiles = sizeof(kGemmTiles) / sizeof(kGemmTiles[0]);
 
 // The tile for a shape: the cheapest by rounds x cost, where a round of 256 workgroups slows down as it fills (they
 // share L2, HBM and the power budget: 1.5 times the cost of a lone workgroup when all CUs have one).  The estimate is
 // within 10 % of the measured time at 40 shapes, and picks the measured best or one within 5 % of it.
-static int gemm_tile(int m, int k, int tokens)
+static int gemm_tile(int m, int k, int tokens, bool sectors, bool x16)
 {
     int best = -1;
     float best_cost = 0.0f;
     for (int i = 0; i < kGemmNTiles; i++) {
         const GemmTile &g = kGemmTiles[i];
+        const float tile_cost = x16 ? g.cost16 : g.cost;
         // (a tile's rows are addressed with 32-bit offsets)
-        if (k % (64 * g.ku) != 0 || (uint64_t)(g.tt > g.tm ? g.tt : g.tm) * (uint64_t)k * 4 >= (1ull << 32))
+        if (k % (64 * g.ku) != 0 || (g.wide && !sectors) || tile_cost == 0.0f ||
+            (uint64_t)(g.tt > g.tm ? g.tt : g.tm) * (uint64_t)k * 4 >= (1ull << 32))
             continue;
         const long long wg = (long long)((m + g.tm - 1) / g.tm) * ((tokens + g.tt - 1) / g.tt);
         const long long rounds = (wg + 255) / 256;
         const float fill = (float)wg / (256.0f * (float)rounds);
-        const float cost = (float)rounds * g.cost * (1.0f + 0.5f * fill * fill);
+        const float cost = (float)rounds * tile_cost * (1.0f + 0.5f * fill * fill);
         if (best < 0 || cost < best_cost) {
             best = i;
             best_cost = cost;
@@ -337,24 +448,36 @@ static int gemm_tile(int m, int k, int tokens)
 template <bool X16, typename F>
 static bool with_gemm_kernel(int i, F &&f)
 {
-#define HIPML_GEMM(idx, CT, CM, AT, BT, KU, NW, R)                                                                     \
+#define HIPML_GEMM(idx, WIDE, CT, CM, AT, BT, KU, NW, R)                                                               \
     case idx: {                                                                                                       \
         constexpr int tt = 32 * AT * CT, tm = 32 * BT * CM;                                                           \
-        static_assert(kGemmTiles[idx].tt == tt && kGemmTiles[idx].tm == tm && kGemmTiles[idx].ku == KU, "the table"); \
-        return f(&gemm_q8_f16_kernel<X16, CT, CM, AT, BT, KU, NW, R>, 64 * (NW + CT * CM), tt, tm,                    \
+        static_assert(kGemmTiles[idx].tt == tt && kGemmTiles[idx].tm == tm && kGemmTiles[idx].ku == KU &&             \
+                          kGemmTiles[idx].wide == WIDE,                                                               \
+                      "the table");                                                                                   \
+        return f(&gemm_q8_f16_kernel<X16, WIDE, CT, CM, AT, BT, KU, NW, R>, 64 * (NW + CT * CM), tt, tm,               \
                  gemm_lds(tt, tm, KU));                                                                               \
     }
     switch (i) {
-        HIPML_GEMM(0, 1, 1, 1, 1, 4, 8, 2)
-        HIPML_GEMM(1, 1, 2, 1, 1, 4, 8, 2)
-        HIPML_GEMM(2, 2, 2, 1, 1, 2, 8, 2)
-        HIPML_GEMM(3, 2, 2, 1, 2, 2, 8, 2)
-        HIPML_GEMM(4, 2, 2, 2, 2, 1, 8, 4)
-        HIPML_GEMM(5, 2, 2, 3, 2, 1, 4, 2)
-        HIPML_GEMM(6, 2, 2, 2, 3, 1, 4, 2)
-        HIPML_GEMM(7, 2, 2, 3, 3, 1, 4, 2)
-        HIPML_GEMM(8, 2, 2, 4, 3, 1, 4, 2)
-        HIPML_GEMM(9, 2, 2, 1, 1, 1, 4, 4)
+        HIPML_GEMM(0, true, 1, 1, 1, 1, 4, 8, 2)
+        HIPML_GEMM(1, true, 1, 2, 1, 1, 4, 8, 2)
+        HIPML_GEMM(2, true, 2, 2, 1, 1, 2, 8, 2)
+        HIPML_GEMM(3, true, 2, 2, 1, 2, 2, 8, 2)
+        HIPML_GEMM(4, true, 2, 2, 2, 2, 1, 8, 2)
+        HIPML_GEMM(5, true, 2, 2, 3, 2, 1, 4, 2)
+        HIPML_GEMM(6, true, 2, 2, 2, 3, 1, 4, 2)
+        HIPML_GEMM(7, true, 2, 2, 3, 3, 1, 4, 2)
+    case 8: // (f16 activations only)
+        if constexpr (X16) {
+            switch (i) {
+                HIPML_GEMM(8, true, 2, 2, 4, 3, 1, 4, 2)
+            }
+        }
+        return false;
+        HIPML_GEMM(9, false, 2, 2, 4, 3, 1, 4, 2)
+        HIPML_GEMM(10, false, 2, 2, 3, 3, 1, 4, 2)
+        HIPML_GEMM(11, false, 2, 2, 2, 2, 1, 8, 4)
+        HIPML_GEMM(12, false, 2, 2, 1, 1, 2, 8, 2)
+        HIPML_GEMM(13, false, 2, 2, 1, 1, 1, 4, 4)
     default:
         return false;
     }
@@ -398,7 +521,9 @@ int launch_gemm_q8_f16(hipStream_t st, const uint8_t *w, const float *x, const f
                      dim3(threads, 1, 1), lds, st, w, act, y, m, k, tokens);
         return true;
     };
-    const int tile = gemm_tile(m, k, tokens);
+    // (rows of weights in whole 64-byte sectors)
+    const bool sectors = k % 1024 == 0 && (reinterpret_cast<uintptr_t>(w) & 63) == 0;
+    const int tile = gemm_tile(m, k, tokens, sectors, x16 != nullptr);
     if (tile < 0)
         return fail(HIPML_ATTN_E_RANGE, "k %d: 32 rows of activations exceed 4 GB", k);
     if (x16 != nullptr)

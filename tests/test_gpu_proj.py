@@ -314,12 +314,13 @@ def test_qkv_projection_shapes(m, k):
     assert ok
 
 
-@pytest.mark.parametrize("m,k,t", [(33, 256, 33), (1029, 512, 301), (1029, 256, 700), (6000, 256, 300),
-                                   (5000, 256, 700), (8000, 256, 700), (5100, 256, 1000), (9001, 192, 700),
-                                   (12270, 128, 1001), (5, 192, 70)])
+@pytest.mark.parametrize("m,k,t", [(33, 1024, 33), (1029, 1024, 301), (1029, 3072, 700), (6000, 1024, 300),
+                                   (5000, 1024, 700), (8000, 1024, 700), (9001, 2048, 700), (12270, 1024, 1001),
+                                   (1029, 512, 301), (6000, 256, 300), (9001, 192, 700), (12270, 128, 1001),
+                                   (5, 192, 70)])
 def test_gemm_tiles(m, k, t):
-    # one shape per tile of the chunk GEMM (32 x 32 up to 256 x 192), ragged in both directions, an odd number of
-    # 64-value units among them; against its own definition, from f32 and from f16 activations, and a row's bits the
+    # one shape per tile of the chunk GEMM (32 x 32 up to 256 x 192), ragged in both directions, weight rows of whole
+    # 64-byte sectors (k a multiple of 1,024) and others, an odd number of 64-value units among them; against its own definition, from f32 and from f16 activations, and a row's bits the
     # same in a chunk of its own (the smallest tile)
     r = orc.Rng(0x6E00 + m + t)
     w = orc.random_q8_0_bytes(r, m * k // 32).reshape(-1, 34)
