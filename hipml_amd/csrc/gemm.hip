@@ -27,8 +27,8 @@
 //    (192 x 192 over 672 tokens 121 -> 108 us, 64 x 128 over 117 48 -> 42, 64 x 64 31 -> 27).  Tried on it: two sectors
 //    of a line asked for together (no gain), activations non-temporal (10 % slower), deeper records (no gain).
 // Before (128 x 128 tiles for every shape) and now, us: 12288 x 5120 over 117 / 672 / 1,024 / 2,048 tokens 78 / 173 /
-// 217 / 432 -> 42 / 108 / 144 / 284; 1024 x 5120 over the same 74 / 56 / 69 / 71 -> 15 / 23 / 31 / 49; 5120 x 6144
-// (f16 activations) 62 / 58 / 111 / 172 -> 25 / 58 / 80 / 134.
+// 217 / 432 -> 39 / 108 / 144 / 284; 1024 x 5120 over the same 74 / 56 / 69 / 71 -> 15 / 23 / 31 / 49; 5120 x 6144
+// (f16 activations) 62 / 58 / 111 / 172 -> 24 / 58 / 80 / 134.
 //
 // A tile row in LDS is an odd number of 16-byte groups: 128-bit reads and writes of 16 consecutive rows touch every
 // bank once.
@@ -415,6 +415,8 @@ constexpr GemmTile kGemmTiles[] = {
     // hold both)
     {256, 192, 1, false, 1.12f, 1.05f}, {192, 192, 1, false, 0.97f, 0.87f}, {128, 128, 1, false, 0.56f, 0.50f},
     {64, 64, 2, false, 0.26f, 0.23f},   {64, 64, 1, false, 0.34f, 0.30f},
+    // cuts that fit 256 workgroups where those above do not (12,288 weight rows: 128 tiles of 96)
+    {64, 96, 2, true, 0.293f, 0.0f},    {64, 64, 4, true, 0.0f, 0.175f},
 };
 constexpr int kGemmNTiles = sizeof(kGemmTiles) / sizeof(kGemmTiles[0]);
 
@@ -467,9 +469,18 @@ static bool with_gemm_kernel(int i, F &&f)
         HIPML_GEMM(6, true, 2, 2, 2, 3, 1, 4, 2)
         HIPML_GEMM(7, true, 2, 2, 3, 3, 1, 4, 2)
     case 8: // (f16 activations only)
+    case 15:
         if constexpr (X16) {
             switch (i) {
                 HIPML_GEMM(8, true, 2, 2, 4, 3, 1, 4, 2)
+                HIPML_GEMM(15, true, 2, 2, 1, 1, 4, 8, 2)
+            }
+        }
+        return false;
+    case 14: // (f32 activations only)
+        if constexpr (!X16) {
+            switch (i) {
+                HIPML_GEMM(14, true, 2, 1, 1, 3, 2, 8, 2)
             }
         }
         return false;

@@ -315,13 +315,13 @@ def test_qkv_projection_shapes(m, k):
 
 
 @pytest.mark.parametrize("m,k,t", [(33, 1024, 33), (1029, 1024, 301), (1029, 3072, 700), (6000, 1024, 300),
-                                   (5000, 1024, 700), (8000, 1024, 700), (9001, 2048, 700), (12270, 1024, 1001),
-                                   (1029, 512, 301), (6000, 256, 300), (9001, 192, 700), (12270, 128, 1001),
-                                   (5, 192, 70)])
+                                   (5000, 1024, 700), (8000, 1024, 700), (12250, 1024, 100), (5100, 1024, 117),
+                                   (9001, 2048, 700), (12270, 1024, 1001), (1029, 512, 301), (6000, 256, 300),
+                                   (9001, 192, 700), (12270, 128, 1001), (5, 192, 70)])
 def test_gemm_tiles(m, k, t):
     # one shape per tile of the chunk GEMM (32 x 32 up to 256 x 192), ragged in both directions, weight rows of whole
-    # 64-byte sectors (k a multiple of 1,024) and others, an odd number of 64-value units among them; against its own definition, from f32 and from f16 activations, and a row's bits the
-    # same in a chunk of its own (the smallest tile)
+    # 64-byte sectors (k a multiple of 1,024) and others, an odd number of 64-value units among them; against its own
+    # definition, from f32 and from f16 activations, and a row's bits the same in a chunk of its own (a small tile)
     r = orc.Rng(0x6E00 + m + t)
     w = orc.random_q8_0_bytes(r, m * k // 32).reshape(-1, 34)
     scales = (r.uniform_array(w.shape[0]) * 0.05 + 0.001).astype(np.float16)
