@@ -924,8 +924,9 @@ __device__ __forceinline__ void proj_dma4(uint32_t lds_at, const uint8_t *base, 
 
 // Wave w of WV streams units (pairs of blocks, 64 values of k) w, w + WV, ... of its rows through a ring of its own; unit
 // u belongs to chain u % 8, so four waves keep two sets of sums each.  HALF: as above.
+// (One wave a SIMD may use all 512 registers: held to 256, two sets of 2 x 3 tiles spill, 200 us instead of 28.)
 template <int XT, int RW, bool HALF>
-__global__ void __launch_bounds__((kUnitsThreads<XT, RW, HALF>), 2)
+__global__ void __launch_bounds__((kUnitsThreads<XT, RW, HALF>), (UnitsShape<XT, RW, HALF>::kWaves / 4))
     gemv_q8_units_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, float *__restrict__ y, int m, int k, int rows)
 {
     typedef UnitsShape<XT, RW, HALF> S;
