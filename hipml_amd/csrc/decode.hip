@@ -128,6 +128,7 @@ struct DecodeArgs {
     const float *gate;
     unsigned int *tickets;
     int merge;
+    int direct; // the one split of every item writes the output rows, gated: no partials, no second launch
     // Work items (grid.y).  A slot whose rows x heads fit the columns of one workgroup (16; the raw-row
     // kernel runs items of up to 8 columns through its narrow body and wider ones through its wide
     // one) is one item; a wider one (2-4 MTP rows x 6 heads) is cut by heads into
@@ -1236,8 +1237,14 @@ __device__ __forceinline__ void decode_body_dma(const DecodeArgs &a, const Front
         if ((int)threadIdx.x < nvalid) {
             const int col = threadIdx.x / group;
             const int head = hbase + (threadIdx.x - col * group);
-            float *pm = a.part_ml + (size_t)(row0 + col) * a.ml_slot + ((size_t)head * f.splits + split) * 2;
-            store_dev(pm, (float2){-INFINITY, 0.0f});
+            if (a.direct) {
+                float *o = a.out + (size_t)(row0 + col) * a.q_slot + (size_t)head * kHeadDim;
+                for (int d = 0; d < kHeadDim; d += 4)
+                    *reinterpret_cast<float4v *>(o + d) = (float4v){0, 0, 0, 0};
+            } else {
+                float *pm = a.part_ml + (size_t)(row0 + col) * a.ml_slot + ((size_t)head * f.splits + split) * 2;
+                store_dev(pm, (float2){-INFINITY, 0.0f});
+            }
         }
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // nothing may land in LDS after the wave has gone
         return; // uniform over the workgroup
@@ -1679,6 +1686,8 @@ __device__ __forceinline__ void decode_body_dma(const DecodeArgs &a, const Front
             const int head = hbase + (nc - col * group);
             const size_t slice = (size_t)head * f.splits + split;
             float *pa = a.part_acc + (size_t)(row0 + col) * a.acc_slot + slice * kHeadDim + d0;
+            const size_t out_at = (size_t)(row0 + col) * a.q_slot + (size_t)head * kHeadDim + d0;
+            const float inv = lsum > 0.0f ? 1.0f / lsum : 0.0f; // (direct: the merge kernels' expressions)
 #pragma unroll
             for (int dd = 0; dd < kRun; dd += 4) {
                 float4v acc = {0, 0, 0, 0};
@@ -1691,12 +1700,21 @@ __device__ __forceinline__ void decode_body_dma(const DecodeArgs &a, const Front
                     const float2 x1 = *reinterpret_cast<const float2 *>(row + col0 + dd + 2);
                     acc += ((float4v){x0.x, x0.y, x1.x, x1.y} - off) * wgt[w];
                 }
-                if (a.merge > 0)
+                if (a.direct) {
+                    float4v r = acc * inv;
+                    if (!(lsum > 0.0f))
+                        r = (float4v){0, 0, 0, 0};
+                    if (a.gate != nullptr) {
+                        const float4v gt = *reinterpret_cast<const float4v *>(a.gate + out_at + dd);
+                        r = (float4v){gated(r[0], gt[0]), gated(r[1], gt[1]), gated(r[2], gt[2]), gated(r[3], gt[3])};
+                    }
+                    *reinterpret_cast<float4v *>(a.out + out_at + dd) = r;
+                } else if (a.merge > 0)
                     store_dev(pa + dd, acc);
                 else
                     *reinterpret_cast<float4v *>(pa + dd) = acc;
             }
-            if (threadIdx.x % kDRuns == 0) {
+            if (!a.direct && threadIdx.x % kDRuns == 0) {
                 float *pm = a.part_ml + (size_t)(row0 + col) * a.ml_slot + slice * 2;
                 if (a.merge > 0)
                     store_dev(pm, (float2){ms, lsum});
@@ -2535,7 +2553,10 @@ int launch_decode_q8(hipStream_t st, const DecodeLaunch &given)
     a.gate = L.gate;
     a.tickets = nullptr;
     a.merge = 0;
-    if (raw_rows && !L.q4 && L.slots == 1 && a.workers == 0 && L.splits <= kMergeMaxSplits) {
+    // One split (up to 128 rows by the split policy) has nothing to merge: 6.6 us instead of 9.1.  Longer sequences
+    // keep their splits: every further tile of a wave costs 2.3 us (256 rows 9.06 in one split, 9.06 in two).
+    a.direct = raw_rows && L.splits == 1 && a.workers == 0 ? 1 : 0;
+    if (!a.direct && raw_rows && !L.q4 && L.slots == 1 && a.workers == 0 && L.splits <= kMergeMaxSplits) {
         const int ngroup = (L.splits + kMergeGroup - 1) / kMergeGroup;
         a.tickets = decode_tickets(st, items * L.n_kv * (ngroup + 1));
         a.merge = a.tickets != nullptr ? kMergeGroup : 0;
@@ -2559,7 +2580,7 @@ int launch_decode_q8(hipStream_t st, const DecodeLaunch &given)
     else
         HIPML_LAUNCH((decode_staged_kernel<false, true>), grid, dim3(kThreads, 1, 1), decode_lds_bytes(1), st, a);
     int rc = launched(L.q4 ? "attn_decode_kv_q4" : "attn_decode_kv_q8");
-    if (rc || a.merge > 0)
+    if (rc || a.merge > 0 || a.direct)
         return rc;
     // Up to 128 splits (every launch the split policies make): the one-barrier merge.  One sequence
     // (a query row, or the rows of a verify group: the same merge, so that a column of a group is

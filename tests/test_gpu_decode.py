@@ -306,3 +306,46 @@ def test_gated_batch_with_mtp_slots():
                                                  stride=stride), gate[row].ravel())
             assert orc.compare(want, host(one)[row].ravel(), *KERNEL_CLASS)[0], (s, j)
             row += 1
+
+
+@pytest.mark.parametrize("dtype", [0, 1])
+@pytest.mark.parametrize("seq", [0, 1, 31, 33, 127, 128, 300])
+def test_one_split_writes_the_rows_itself(seq, dtype):
+    # a launch with one split has nothing to merge: it writes the (gated) rows, and a verify group's columns have the
+    # bits of their plain decodes; no key at all: zeros; the scratch is not touched
+    stride = 320
+    r = orc.Rng(0x0D1E + seq * 2 + dtype)
+    q = r.normal_array((3, N_HEADS, HD))
+    gate = r.normal_array((N_HEADS, HD))
+    kb = orc.quantize(dtype, r.normal_array((N_KV, stride, HD))).reshape(N_KV, stride, -1)
+    vb = orc.quantize(dtype, r.normal_array((N_KV, stride, HD))).reshape(N_KV, stride, -1)
+    acc, ml = decode_scratch(N_HEADS, 1, 3)
+    acc.fill_(float("nan")), ml.fill_(float("nan"))
+    kd, vd = dev(kb), dev(vb)
+
+    def one(c, n, g=None):
+        out = torch.full((N_HEADS, HD), float("nan"), dtype=torch.float32, device="cuda")
+        args = (step_buffer(max(n - 1, 0), n), dtype, dev(q[c]), kd, vd, acc, ml, out)
+        rest = (N_HEADS, N_KV, HD, stride, SCALE, 1)
+        attn.attn_decode_kv(*args, *rest) if g is None else attn.attn_decode_kv_gate(*args, dev(g), *rest)
+        torch.cuda.synchronize()
+        return out
+
+    plain = one(0, seq)
+    if seq == 0:
+        assert not plain.any()
+    else:
+        want = orc.attn_decode_kv(q[0], kb, vb, N_HEADS, N_KV, HD, seq, SCALE, stride=stride, dtype=dtype)
+        ok, _, _ = report(f"one split, seq {seq}, dtype {dtype}", want.ravel(), host(plain).ravel(), *GATE)
+        assert ok
+    two = plain.clone()
+    attn.q_gate(two, dev(gate), two, N_HEADS * HD)
+    assert torch.equal(one(0, seq, gate), two)
+    pos = torch.tensor([[seq + c, seq + c + 1] for c in range(3)], dtype=torch.int32, device="cuda")
+    cols = torch.full((3, N_HEADS, HD), float("nan"), dtype=torch.float32, device="cuda")
+    attn.attn_decode_kv_cols(dtype, pos, dev(q), kd, vd, acc, ml, cols, N_HEADS, N_KV, HD, stride, SCALE, 1, 3,
+                             N_HEADS * HD, N_HEADS * 2, N_HEADS * HD)
+    torch.cuda.synchronize()
+    for c in range(3):
+        assert torch.equal(cols[c], one(c, seq + c + 1))
+    assert bool(acc.isnan().all()) and bool(ml.isnan().all())
