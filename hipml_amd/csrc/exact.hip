@@ -12,6 +12,64 @@
 
 namespace hipml {
 
+// ---- lane exchanges ------------------------------------------------------------
+//
+// In registers (DPP, row swaps): an exchange through the LDS crossbar (__shfl_xor) has ~120 cycles of latency, and the
+// launches below that handle few rows are chains of them (one token's pass over a q8_0 cache 56.4 -> 56.1 us, over a
+// q4_0 cache 56.1 -> 55.3, 16 slots of 3 rows 145.7 -> 144.7).  A maximum may meet in any order, so mirrors serve as
+// the wider steps inside 16 lanes.
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v)
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+}
+constexpr int kXor1 = 0xB1, kXor2 = 0x4E, kHalfMirror = 0x141, kMirror = 0x140, kRor4 = 0x124, kRor8 = 0x128;
+
+// (v of the even, v of the odd row of 16) of every pair of rows; (.. lower, .. upper) half of the wave
+__device__ __forceinline__ float2 row_pair(float v)
+{
+    const uint32_t x = __builtin_bit_cast(uint32_t, v);
+    const auto r = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+    const uint32_t a = r[0], b = r[1];
+    return make_float2(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b));
+}
+__device__ __forceinline__ float2 half_pair(float v)
+{
+    const uint32_t x = __builtin_bit_cast(uint32_t, v);
+    const auto r = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+    const uint32_t a = r[0], b = r[1];
+    return make_float2(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b));
+}
+
+// the largest of 8 neighbouring lanes; of the 32 lanes of a half wave
+__device__ __forceinline__ float max8(float m)
+{
+    m = fmaxf(m, dpp<kXor1>(m));
+    m = fmaxf(m, dpp<kXor2>(m));
+    return fmaxf(m, dpp<kHalfMirror>(m));
+}
+__device__ __forceinline__ float max32(float m)
+{
+    m = max8(m);
+    m = fmaxf(m, dpp<kMirror>(m));
+    const float2 r = row_pair(m);
+    return fmaxf(r.x, r.y);
+}
+
+// The halving tree v[l] += v[l ^ off], off = 32 .. 1, of a wave: IEEE addition commutes, so the row swaps give the
+// first two levels in every lane, and once lanes 8 (4) apart agree a rotation by 4 is the exchange with lane ^ 4.
+__device__ __forceinline__ float tree_sum64(float v)
+{
+    float2 r = half_pair(v);
+    v = r.x + r.y;
+    r = row_pair(v);
+    v = r.x + r.y;
+    v += dpp<kRor8>(v);
+    v += dpp<kRor4>(v);
+    v += dpp<kXor2>(v);
+    return v + dpp<kXor1>(v);
+}
+
 // ---- q8_0 quantize + append ---------------------------------------------------
 //
 // One workgroup per (kv head, unit); thread t owns value t of the head row.  A
@@ -24,11 +82,7 @@ namespace hipml {
 
 __device__ __forceinline__ float half_wave_amax(float x)
 {
-    float m = fabsf(x);
-#pragma unroll
-    for (int bit = 16; bit > 0; bit >>= 1)
-        m = fmaxf(m, __shfl_xor(m, bit));
-    return m;
+    return max32(fabsf(x));
 }
 
 __device__ __forceinline__ void q8_encode_store(float x, uint8_t *dst_block, int lane32)
@@ -73,29 +127,22 @@ __global__ void __launch_bounds__(256) kv_encode_q8_kernel(
 // id = 1/d or 0, q = clamp(round(x*id) + 8, 0, 15); byte j of the block holds q[j] in its low and
 // q[j+16] in its high nibble.  Same thread layout as the q8_0 kernel: 32 lanes per block.
 
-__device__ __forceinline__ float half_wave_vmax(float x, int lane32)
+__device__ __forceinline__ float half_wave_vmax(float x)
 {
     float mag = fabsf(x);
     if (!(mag == mag))
         mag = -1.0f; // NaN: below every real magnitude, like a failed `>`
-    float val = x;
-    int idx = lane32;
-#pragma unroll
-    for (int bit = 16; bit > 0; bit >>= 1) {
-        const float om = __shfl_xor(mag, bit);
-        const float ov = __shfl_xor(val, bit);
-        const int oi = __shfl_xor(idx, bit);
-        const bool take = om > mag || (om == mag && oi < idx);
-        mag = take ? om : mag;
-        val = take ? ov : val;
-        idx = take ? oi : idx;
-    }
-    return mag > 0.0f ? val : 0.0f; // nothing beat the fold's initial +0
+    const float most = max32(mag);
+    // the first lane of the half wave that holds it
+    const uint64_t all = __ballot(mag == most);
+    const uint32_t holders = (threadIdx.x & 32) ? (uint32_t)(all >> 32) : (uint32_t)all;
+    const float val = __shfl(x, (int)(threadIdx.x & 32) | (__ffs((int)holders) - 1));
+    return most > 0.0f ? val : 0.0f; // nothing beat the fold's initial +0
 }
 
 __device__ __forceinline__ void q4_encode_store(float x, uint8_t *dst_block, int lane32)
 {
-    const float vmax = half_wave_vmax(x, lane32);
+    const float vmax = half_wave_vmax(x);
     const float d = -vmax / 8.0f;
     const float id = d != 0.0f ? 1.0f / d : 0.0f;
     const float t = roundf(x * id) + 8.0f;
@@ -305,9 +352,7 @@ typedef float float4e __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ void q8_encode_store4(const float4e x, uint8_t *dst_block, int l8)
 {
     float m = fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3])));
-#pragma unroll
-    for (int bit = 4; bit > 0; bit >>= 1)
-        m = fmaxf(m, __shfl_xor(m, bit));
+    m = max8(m);
     const float d = m / 127.0f;
     const float id = d > 0.0f ? 1.0f / d : 0.0f;
     uint32_t pk = 0;
@@ -604,10 +649,7 @@ __global__ void __launch_bounds__(256) front_kernel(
     }
     const float a0 = x[0] * x[0] + x[2] * x[2]; // off = 128
     const float a1 = x[1] * x[1] + x[3] * x[3];
-    float sum = a0 + a1;                        // off = 64
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1)
-        sum += __shfl_xor(sum, off);
+    const float sum = tree_sum64(a0 + a1);      // off = 64, then 32 .. 1
     const float mean_sq = sum / (float)kHeadDim;
     const float scale = 1.0f / sqrtf(mean_sq + eps);
 #pragma unroll
