@@ -31,28 +31,36 @@
 
 namespace hipml {
 
-// 8 f32 -> hi and lo f16 halves with hi + lo = x to ~22 bits.
+// 8 f32 -> hi and lo f16 halves with hi + lo = x to ~22 bits (up to 65,504; beyond, lo holds what it can, and from 131,008
+// on the sum stays there).
 __device__ __forceinline__ void split_hi_lo(const float4v &a, const float4v &b, half8 &hi, half8 &lo)
 {
+    uint4v h, l;
+    float d[8];
 #pragma unroll
     for (int j = 0; j < 4; j++) {
         const float x0 = j < 2 ? a[2 * j] : b[2 * j - 4];
         const float x1 = j < 2 ? a[2 * j + 1] : b[2 * j - 3];
-        const half2v h = __builtin_bit_cast(half2v, __builtin_amdgcn_cvt_pkrtz(x0, x1));
-        // x - h (exact: h holds the leading bits of x), rounded to f16 by the same instruction, which reads the f16
-        // half in place: one per value where the compiler makes two conversions and a subtraction
-        const uint32_t hb = __builtin_bit_cast(uint32_t, h);
-        uint32_t lb;
-        asm("v_fma_mixlo_f16 %0, -%1, 1.0, %2 op_sel_hi:[1,0,0]\n\t"
-            "v_fma_mixhi_f16 %0, -%1, 1.0, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]"
-            : "=&v"(lb)
-            : "v"(hb), "v"(x0), "v"(x1));
-        const half2v l = __builtin_bit_cast(half2v, lb);
-        hi[2 * j] = h[0];
-        hi[2 * j + 1] = h[1];
-        lo[2 * j] = l[0];
-        lo[2 * j + 1] = l[1];
+        h[j] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(x0, x1));
+        // x - h (exact: h holds the leading bits of x) by the instruction that reads the f16 half in place: one per value
+        // where the compiler makes a conversion and a subtraction
+        asm("v_fma_mix_f32 %0, -%1, 1.0, %2 op_sel_hi:[1,0,0]" : "=v"(d[2 * j]) : "v"(h[j]), "v"(x0));
+        asm("v_fma_mix_f32 %0, -%1, 1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(d[2 * j + 1]) : "v"(h[j]), "v"(x1));
     }
+    // To f16, to nearest, with MODE bit 23 on: an overflow gives +-65,504 and not infinity (which a weight of 0 makes NaN).
+    // For these conversions alone: under it an MFMA of infinities gives large finite numbers.  us over 5120 x 6144 and 24 /
+    // 40 / 128 rows: 18.4 / 28.9 / 55.5; without the bit 18.3 / 28.0 / 53.4, the rounded difference by v_fma_mixlo_f16 and
+    // v_fma_mixhi_f16 18.5 / 28.5 / 54.4, x clamped by v_med3_f32 first 19.3 / 30.7 / 58.4.
+    asm("s_setreg_imm32_b32 hwreg(HW_REG_MODE, 23, 1), 1\n\t"
+        "v_cvt_pk_f16_f32 %0, %4, %5\n\t"
+        "v_cvt_pk_f16_f32 %1, %6, %7\n\t"
+        "v_cvt_pk_f16_f32 %2, %8, %9\n\t"
+        "v_cvt_pk_f16_f32 %3, %10, %11\n\t"
+        "s_setreg_imm32_b32 hwreg(HW_REG_MODE, 23, 1), 0"
+        : "=&v"(l[0]), "=&v"(l[1]), "=&v"(l[2]), "=&v"(l[3])
+        : "v"(d[0]), "v"(d[1]), "v"(d[2]), "v"(d[3]), "v"(d[4]), "v"(d[5]), "v"(d[6]), "v"(d[7]));
+    hi = __builtin_bit_cast(half8, h);
+    lo = __builtin_bit_cast(half8, l);
 }
 
 // One chunk of a wave's steps, as fetched.  A step is a pair of blocks of one weight row (68 bytes,

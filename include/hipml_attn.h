@@ -505,7 +505,8 @@ int hipml_kv_rows_copy(hipml_stream_t stream, int dtype, const void *k_src, cons
  * f16 scale, 32 int8) at a 4-byte aligned address, x is f32 [rows][k] (16-byte aligned), y is f32
  * [rows][m]; k a multiple of 64 up to 32768, 1 <= rows <= 128.
  * fp32 accumulation of exact integer block products (the activations enter as hi + lo f16 halves), so
- * every row has the precision class of the reference's f32 GEMV kernels.  Up to 8 rows W streams from
+ * every row has the precision class of the reference's f32 GEMV kernels.  Finite activations are taken up to a
+ * magnitude of 131,008 (two f16 halves; ~22 bits up to 65,504, to the nearest 32 above) and as that value beyond.  Up to 8 rows W streams from
  * memory once and a row's result has the same bits whatever `rows` is and whichever rows travel with it:
  * the rows of a verify group match their plain decodes, as the reference's batched GEMVs do
  * (crates/hipml-kernels/src/attn_gpu.rs:930-932).  From 10 to 128 rows W streams once per pass of up to 64 rows

@@ -195,6 +195,32 @@ def test_weights_at_a_4_byte_aligned_address(rows):
     assert ok
 
 
+@pytest.mark.parametrize("m,k,rows", [(96, 1024, 1), (96, 1024, 3), (96, 1024, 8), (96, 320, 2), (96, 1024, 12),
+                                      (6200, 512, 12)])
+def test_activations_beyond_two_f16_halves_saturate(m, k, rows):
+    # every kernel that splits activations into hi + lo f16 halves: finite magnitudes beyond 131,008 count as 131,008
+    # (weights of 0 under them too), an infinite one reaches its own row only
+    r = orc.Rng(0x5A70 + m + rows)
+    w = orc.random_q8_0_bytes(r, m * k // 32).reshape(m, k // 32, 34)
+    w[::3, :, 2:] = 0
+    x = r.normal_array((rows, k))
+    x[0, :6] = (131_000.0, 131_023.0, -131_024.0, 1.0e6, -3.0e38, 100_000.0)
+    blocks = w[:, :, :2].copy().view(np.float16).astype(np.float64) * w[:, :, 2:].view(np.int8)
+    dense = blocks.reshape(m, k)
+    scale = np.repeat(w[:, :, :2].copy().view(np.float16).astype(np.float64), 32, axis=2).reshape(m, k)
+    taken = np.clip(x.astype(np.float64), -131_008.0, 131_008.0)
+    got = run_gemv(w.ravel(), x, m, k, rows)
+    assert np.isfinite(got).all()
+    # lo halves of 32,768 to 65,504 lie 32 apart; else ~21 bits of the terms and fp32 sums of them; up to 8 rows the
+    # weights enter as 128 + q, whose 128 comes out again in fp32
+    bound = 16 * np.abs(dense[:, :6]).sum(axis=1)[None, :] * (np.arange(rows) == 0)[:, None]
+    bound = bound + 4e-6 * (np.abs(taken) @ np.abs(dense).T) + 3e-7 * 128 * (np.abs(taken) @ scale.T) + 1e-5
+    assert np.all(np.abs(got - taken @ dense.T) <= bound)
+    x[0, 7] = np.inf
+    inf = run_gemv(w.ravel(), x, m, k, rows)
+    assert not np.isfinite(inf[0]).any() and np.array_equal(inf[1:], got[1:])
+
+
 def test_argument_errors():
     w = torch.zeros(34 * 4, dtype=torch.uint8, device="cuda")
     x = torch.zeros(64, device="cuda")
