@@ -19,6 +19,9 @@
 //  * half of the producer waves ask for the next record before they stage, the other half behind it.  Asked for by all
 //    of them at once the loads queue up (one request per ~25 cycles and CU) while no wave stages, and a step costs the
 //    sum of both: 2,150 cycles against 1,500 (192 x 192: 146 -> 117 us; 256 x 192 over 1,024 tokens: 166 -> 144 us).
+//    Not so for 128 x 128 tiles over f16 activations, whose step has the fewest loads for its eight producer waves: there
+//    all of them stage first and four records cover the loads (5120 x 6144 over 512 / 672 tokens 50.8 -> 47.5 / 62.6 ->
+//    58.6 us).
 //  * small tiles with longer steps (KU 2 and 4) and eight producer waves where there are too few outputs for large
 //    ones: a step's cost is then latency, not work (1024 x 5120 over 117 tokens: 32 x 32 tiles 15 us, 128 x 128 48 us).
 //  * weights by whole 64-byte sectors, one aligned request of a quad of lanes each, where their rows allow it.  A row's
@@ -26,9 +29,9 @@
 //    across a sector boundary, and the weights of a step cost the vector memory path as much as the activations
 //    (192 x 192 over 672 tokens 121 -> 108 us, 64 x 128 over 117 48 -> 42, 64 x 64 31 -> 27).  Tried on it: two sectors
 //    of a line asked for together (no gain), activations non-temporal (10 % slower), deeper records (no gain).
-// Before (128 x 128 tiles for every shape) and now, us: 12288 x 5120 over 117 / 672 / 1,024 / 2,048 tokens 78 / 173 /
-// 217 / 432 -> 39 / 108 / 144 / 284; 1024 x 5120 over the same 74 / 56 / 69 / 71 -> 15 / 23 / 31 / 49; 5120 x 6144
-// (f16 activations) 62 / 58 / 111 / 172 -> 24 / 58 / 80 / 134.
+// The kernel before this one (128 x 128 tiles for every shape) and this one, us: 12288 x 5120 over 117 / 672 / 1,024 /
+// 2,048 tokens 76 / 178 / 202 / 397 -> 40 / 114 / 144 / 282; 1024 x 5120 over the same 52 / 55 / 58 / 63 -> 16 / 24 / 28 /
+// 51; 5120 x 6144 (f16 activations) 44 / 58 / 102 / 166 -> 23 / 58 / 80 / 131.
 //
 // A tile row in LDS is an odd number of 16-byte groups: 128-bit reads and writes of 16 consecutive rows touch every
 // bank once.
@@ -77,7 +80,9 @@ struct QuarterWeights {
     uint2a4 o[SETS][WP];
 };
 
-template <bool X16, bool WIDE, int CT, int CM, int AT, int BT, int KU, int NW, int R>
+// TURNS: half of the producer waves ask for the next record before they stage (above); else all of them stage first,
+// activations ahead of weights, and R records cover the loads.
+template <bool X16, bool WIDE, int CT, int CM, int AT, int BT, int KU, int NW, int R, bool TURNS = true>
 __global__ void __launch_bounds__(64 * (NW + CT * CM)) gemm_q8_f16_kernel(const uint8_t *__restrict__ w,
                                                                           const void *__restrict__ xv,
                                                                           float *__restrict__ y, int m, int k, int tokens)
@@ -238,9 +243,12 @@ __global__ void __launch_bounds__(64 * (NW + CT * CM)) gemm_q8_f16_kernel(const 
                 fetch_x(v % R, s + R);
             };
             auto stage = [&](int v, int s) {
+                if (!TURNS)
+                    stage_x(v % R, v & 1);
                 if (kWeights)
                     stage_w(v % CYCLE, s, v & 1);
-                stage_x(v % R, v & 1);
+                if (TURNS)
+                    stage_x(v % R, v & 1);
             };
             if (kWeights) {
 #pragma unroll
@@ -285,11 +293,11 @@ __global__ void __launch_bounds__(64 * (NW + CT * CM)) gemm_q8_f16_kernel(const 
         const std::true_type yes;
         const std::false_type no;
         if (WWAVES < NW && wave >= WWAVES) {
-            if (wave & 1)
+            if (TURNS && (wave & 1))
                 produce(yes, no);
             else
                 produce(no, no);
-        } else if (wave & 1) {
+        } else if (TURNS && (wave & 1)) {
             produce(yes, yes);
         } else {
             produce(no, yes);
@@ -307,50 +315,55 @@ __global__ void __launch_bounds__(64 * (NW + CT * CM)) gemm_q8_f16_kernel(const 
 #pragma unroll
             for (int i = 0; i < 16; i++)
                 acc[a][b][i] = 0.0f;
-    auto multiply = [&](const uint8_t *buf) {
-        const uint8_t *xa = buf + (wt_ * 32 * AT + ln) * kGemmPitch + lh * 16;
-        const uint8_t *wb = buf + kXTile + (wm_ * 32 * BT + ln) * kGemmPitch + lh * 16;
+    // operands of 16 values of k are read while those of the 16 before them are multiplied: one MFMA and one read in turn.
+    // A step's barrier stands where its last operands have been read, in front of the last MFMAs, behind which the next
+    // step's first operands are read: the barrier and the first reads behind it cost little MFMA time (with the barrier at
+    // the end of the step the large tiles take 1 to 3 % more: 12288 x 5120 over 1,024 tokens 146.5 us, here 143.5).
+    const uint8_t *xa = lds + (wt_ * 32 * AT + ln) * kGemmPitch + lh * 16;
+    const uint8_t *wb = lds + kXTile + (wm_ * 32 * BT + ln) * kGemmPitch + lh * 16;
+    half8 A[2][AT], B[2][BT];
+    auto read = [&](int kk) {
+#pragma unroll
+        for (int a = 0; a < AT; a++)
+            A[kk & 1][a] = *reinterpret_cast<const half8 *>(xa + a * 32 * kGemmPitch + kk * 32);
+#pragma unroll
+        for (int b = 0; b < BT; b++)
+            B[kk & 1][b] = *reinterpret_cast<const half8 *>(wb + b * 32 * kGemmPitch + kk * 32);
+    };
+    auto multiply = [&](int kk) {
         constexpr int per = AT + BT, mf = AT * BT, rr = (per + mf - 1) / mf;
         constexpr int pairs = per < mf ? per : mf;
-        // operands of 16 values of k are read while those of the 16 before them are multiplied: one MFMA and one
-        // read in turn
-        half8 A[2][AT], B[2][BT];
-        auto read = [&](int kk) {
 #pragma unroll
-            for (int a = 0; a < AT; a++)
-                A[kk & 1][a] = *reinterpret_cast<const half8 *>(xa + a * 32 * kGemmPitch + kk * 32);
+        for (int a = 0; a < AT; a++)
 #pragma unroll
             for (int b = 0; b < BT; b++)
-                B[kk & 1][b] = *reinterpret_cast<const half8 *>(wb + b * 32 * kGemmPitch + kk * 32);
-        };
-        read(0);
-        __builtin_amdgcn_sched_barrier(0);
+                acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[kk & 1][a], B[kk & 1][b], acc[a][b], 0, 0, 0);
 #pragma unroll
-        for (int kk = 0; kk < 4 * KU; kk++) {
-            if (kk + 1 < 4 * KU)
-                read(kk + 1);
-#pragma unroll
-            for (int a = 0; a < AT; a++)
-#pragma unroll
-                for (int b = 0; b < BT; b++)
-                    acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[kk & 1][a], B[kk & 1][b], acc[a][b], 0, 0, 0);
-            if (kk + 1 < 4 * KU) {
-#pragma unroll
-                for (int i = 0; i < pairs; i++) {
-                    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                    __builtin_amdgcn_sched_group_barrier(0x100, rr, 0);
-                }
-                if (mf > pairs)
-                    __builtin_amdgcn_sched_group_barrier(0x008, mf - pairs, 0);
-            }
-            __builtin_amdgcn_sched_barrier(0);
+        for (int i = 0; i < pairs; i++) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x100, rr, 0);
         }
+        if (mf > pairs)
+            __builtin_amdgcn_sched_group_barrier(0x008, mf - pairs, 0);
+        __builtin_amdgcn_sched_barrier(0);
     };
+    constexpr int kSlices = 4 * KU; // of 16 values of k in a step: an even number
     __syncthreads();
+    read(0);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll 1
     for (int s = 0; s < nsteps; s++) {
-        multiply(lds + (s & 1) * kBuf);
+#pragma unroll
+        for (int kk = 0; kk + 1 < kSlices; kk++) {
+            read(kk + 1);
+            multiply(kk);
+        }
         __syncthreads();
+        const int other = s & 1 ? -kBuf : kBuf;
+        xa += other;
+        wb += other;
+        read(0); // (behind the last step: whatever the other buffer holds, not used)
+        multiply(kSlices - 1);
     }
 
     // C tile: lane holds column ln (weight row), rows (i/4)*8 + lh*4 + i%4 (tokens)
@@ -399,39 +412,45 @@ __global__ void __launch_bounds__(256) gate_f16_kernel(const float4v *__restrict
 
 // ---- which tile ----------------------------------------------------------------------------------------------
 //
-// (token rows and weight rows of the tile, 64-value units per step, sectors or quarters for the weights, microseconds
-// per unit and round of the chip's 256 CUs over f32 and over f16 activations: measured at k = 5120 and 6144, less 4 us
-// per launch, with the slow-down of a full chip below taken out)
+// (token rows and weight rows of the tile, 64-value units per step, sectors or quarters for the weights; microseconds
+// per unit and round of the chip's 256 CUs where weight rows are whole sectors, over f32 and over f16 activations, and
+// where they are not; 0: not for these.  Less 4 us per launch, with the slow-down of a full chip below taken out)
 struct GemmTile {
     int tt, tm, ku;
     bool wide;
-    float cost, cost16;
+    float sectors, sectors16, other, other16;
 };
 constexpr GemmTile kGemmTiles[] = {
-    {32, 32, 4, true, 0.13f, 0.13f},   {32, 64, 4, true, 0.165f, 0.139f},  {64, 64, 2, true, 0.23f, 0.19f},
-    {64, 128, 2, true, 0.35f, 0.28f},  {128, 128, 1, true, 0.52f, 0.405f}, {192, 128, 1, true, 0.72f, 0.55f},
-    {128, 192, 1, true, 0.71f, 0.62f}, {192, 192, 1, true, 0.87f, 0.78f},  {256, 192, 1, true, 0.0f, 0.98f},
-    // rows of weights that are not whole sectors (and the largest tile over f32 activations, whose registers do not
-    // hold both)
-    {256, 192, 1, false, 1.12f, 1.05f}, {192, 192, 1, false, 0.97f, 0.87f}, {128, 128, 1, false, 0.56f, 0.50f},
-    {64, 64, 2, false, 0.26f, 0.23f},   {64, 64, 1, false, 0.34f, 0.30f},
-    // cuts that fit 256 workgroups where those above do not (12,288 weight rows: 128 tiles of 96)
-    {64, 96, 2, true, 0.293f, 0.0f},    {64, 64, 4, true, 0.0f, 0.175f},
+    {32, 32, 4, true, 0.115f, 0.105f, 0.0f, 0.0f},   {32, 64, 4, true, 0.155f, 0.14f, 0.0f, 0.0f},
+    {64, 64, 2, true, 0.214f, 0.0f, 0.0f, 0.0f},     {64, 128, 2, true, 0.344f, 0.312f, 0.0f, 0.0f},
+    {128, 128, 1, true, 0.497f, 0.0f, 0.0f, 0.0f},   {192, 128, 1, true, 0.725f, 0.59f, 0.0f, 0.0f},
+    {128, 192, 1, true, 0.725f, 0.646f, 0.0f, 0.0f}, {192, 192, 1, true, 0.929f, 0.82f, 0.0f, 0.0f},
+    {256, 192, 1, true, 0.0f, 0.98f, 0.0f, 0.0f},
+    // quarters: the largest tile over f32 activations, whose registers do not hold sectors too; 128 x 128 over f16
+    // activations, which they serve better; rows of weights that are not whole sectors
+    {256, 192, 1, false, 1.174f, 0.0f, 1.35f, 1.152f}, {192, 192, 1, false, 0.0f, 0.0f, 1.054f, 0.902f},
+    {128, 128, 1, false, 0.0f, 0.419f, 0.616f, 0.465f}, {64, 64, 2, false, 0.0f, 0.0f, 0.208f, 0.174f},
+    {64, 64, 1, false, 0.0f, 0.0f, 0.229f, 0.184f},
+    // cuts that fit 256 workgroups where those above do not (12,288 weight rows: 128 tiles of 96); over f16 activations
+    // the 64 x 64 tile of longer steps stands for that of shorter ones
+    {64, 96, 2, true, 0.291f, 0.0f, 0.0f, 0.0f},     {64, 64, 4, true, 0.0f, 0.18f, 0.0f, 0.0f},
 };
 constexpr int kGemmNTiles = sizeof(kGemmTiles) / sizeof(kGemmTiles[0]);
 
 // The tile for a shape: the cheapest by rounds x cost, where a round of 256 workgroups slows down as it fills (they
-// share L2, HBM and the power budget: 1.5 times the cost of a lone workgroup when all CUs have one).  The estimate is
-// within 10 % of the measured time at 40 shapes, and picks the measured best or one within 5 % of it.
+// share L2, HBM and the power budget: 1.5 times the cost of a lone workgroup when all CUs have one).  The costs are fitted
+// to every tile's time at 143 shapes (1,024 to 12,288 weight rows, k of 576 to 6,144, 24 to 2,048 tokens) over each type of
+// activations: the tile picked is the measured best or within 5 % of it at 284 of the 286 (8192 x 2176 over 1,500 tokens:
+// 92.5 us, best 84.8; 4096 x 576 over 450: 10.2, best 8.9), 0.1 % behind it on average.
 static int gemm_tile(int m, int k, int tokens, bool sectors, bool x16)
 {
     int best = -1;
     float best_cost = 0.0f;
     for (int i = 0; i < kGemmNTiles; i++) {
         const GemmTile &g = kGemmTiles[i];
-        const float tile_cost = x16 ? g.cost16 : g.cost;
+        const float tile_cost = sectors ? (x16 ? g.sectors16 : g.sectors) : (x16 ? g.other16 : g.other);
         // (a tile's rows are addressed with 32-bit offsets)
-        if (k % (64 * g.ku) != 0 || (g.wide && !sectors) || tile_cost == 0.0f ||
+        if (k % (64 * g.ku) != 0 || tile_cost == 0.0f ||
             (uint64_t)(g.tt > g.tm ? g.tt : g.tm) * (uint64_t)k * 4 >= (1ull << 32))
             continue;
         const long long wg = (long long)((m + g.tm - 1) / g.tm) * ((tokens + g.tt - 1) / g.tt);
@@ -450,13 +469,14 @@ static int gemm_tile(int m, int k, int tokens, bool sectors, bool x16)
 template <bool X16, typename F>
 static bool with_gemm_kernel(int i, F &&f)
 {
-#define HIPML_GEMM(idx, WIDE, CT, CM, AT, BT, KU, NW, R)                                                               \
+#define HIPML_GEMM(idx, WIDE, CT, CM, AT, BT, KU, NW, R, ...)                                                          \
     case idx: {                                                                                                       \
         constexpr int tt = 32 * AT * CT, tm = 32 * BT * CM;                                                           \
         static_assert(kGemmTiles[idx].tt == tt && kGemmTiles[idx].tm == tm && kGemmTiles[idx].ku == KU &&             \
                           kGemmTiles[idx].wide == WIDE,                                                               \
                       "the table");                                                                                   \
-        return f(&gemm_q8_f16_kernel<X16, WIDE, CT, CM, AT, BT, KU, NW, R>, 64 * (NW + CT * CM), tt, tm,               \
+        return f(&gemm_q8_f16_kernel<X16, WIDE, CT, CM, AT, BT, KU, NW, R __VA_OPT__(, ) __VA_ARGS__>,               \
+                 64 * (NW + CT * CM), tt, tm,                                                                         \
                  gemm_lds(tt, tm, KU));                                                                               \
     }
     switch (i) {
@@ -464,7 +484,6 @@ static bool with_gemm_kernel(int i, F &&f)
         HIPML_GEMM(1, true, 1, 2, 1, 1, 4, 8, 2)
         HIPML_GEMM(2, true, 2, 2, 1, 1, 2, 8, 2)
         HIPML_GEMM(3, true, 2, 2, 1, 2, 2, 8, 2)
-        HIPML_GEMM(4, true, 2, 2, 2, 2, 1, 8, 2)
         HIPML_GEMM(5, true, 2, 2, 3, 2, 1, 4, 2)
         HIPML_GEMM(6, true, 2, 2, 2, 3, 1, 4, 2)
         HIPML_GEMM(7, true, 2, 2, 3, 3, 1, 4, 2)
@@ -477,16 +496,18 @@ static bool with_gemm_kernel(int i, F &&f)
             }
         }
         return false;
-    case 14: // (f32 activations only)
+    case 4: // (f32 activations only)
+    case 14:
         if constexpr (!X16) {
             switch (i) {
+                HIPML_GEMM(4, true, 2, 2, 2, 2, 1, 8, 2)
                 HIPML_GEMM(14, true, 2, 1, 1, 3, 2, 8, 2)
             }
         }
         return false;
         HIPML_GEMM(9, false, 2, 2, 4, 3, 1, 4, 2)
         HIPML_GEMM(10, false, 2, 2, 3, 3, 1, 4, 2)
-        HIPML_GEMM(11, false, 2, 2, 2, 2, 1, 8, 4)
+        HIPML_GEMM(11, false, 2, 2, 2, 2, 1, 8, 4, !X16)
         HIPML_GEMM(12, false, 2, 2, 1, 1, 2, 8, 2)
         HIPML_GEMM(13, false, 2, 2, 1, 1, 1, 4, 4)
     default:
