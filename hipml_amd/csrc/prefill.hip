@@ -2109,16 +2109,16 @@ int chunk_tiles_splits(int pos0, int tokens, int n_head, int n_kv, int slices)
     return slices + (int)((tiles + per_slice - 1) / per_slice);
 }
 
-// Slices that a long chunk over f16 tiles runs of the `most` its scratch holds.  The caller's count fills the last
-// round of 256 workgroups; what it leaves out is that every slice writes its partial rows and has them read again
-// (2 KB per token and head at about 5 TB/s), and that a round of fewer workgroups runs faster (the chip holds its
-// clock by power: 15 % between an empty and a full one).  In units of a key tile of a full round (3 us): rounds x
-// (tiles of a slice + 4) x (1 + 0.15 fill) + slices x what their partial rows cost; within 8 % of the measured call at
-// ten shapes with 2 to 16 slices each.  us with the caller's count / with this one: 1,024 tokens at depth 8,192 264
-// (8 slices) / 242 (5), 1,500 at 20,000 852 (12) / 713 (3), 700 at 10,000 232 (10) / 193 (3), 800 at 40,000 735 (10) /
-// 703 (3); 2,048 at 100,000 keeps its 4.  Only counts for which every block of tokens gets all slices and the 64-token
-// kernel runs; chunks for which tiles are not made keep the caller's count.
-static int chunk_tile_slices(int pos0, int tokens, int n_head, int n_kv, int most)
+// Slices for a long chunk over f16 tiles, of at most `most` (the count that fills the last round of 256 workgroups).  What
+// that count leaves out is that every slice writes its partial rows and has them read again (2 KB per token and head), and
+// that a round of fewer workgroups runs a little faster.  In units of a key tile of a round (2.6 us): rounds x (tiles of a
+// slice + 6) x (1 + 0.05 fill) + slices x what their partial rows cost at 4 TB/s.  Fitted to 2 to 16 slices at 14 shapes
+// and checked at 12 others: it picks the fastest count or one within 2.7 % of it at all 26 (the times themselves are 10 %
+// under to 25 % over).  us with the filling count / with this one: 1,024 tokens at depth 8,192 255 (8 slices) / 222 (2),
+// 1,500 at 20,000 829 (12) / 688 (3), 700 at 10,000 226 (10) / 186 (3), 800 at 40,000 709 (10) / 669 (3), 2,048 at 2,048
+// 219 (4) / 204 (2); 672 at 8,192 and 2,048 at 100,000 keep their 4.  Only counts for which every block of tokens gets all
+// slices and the 64-token kernel runs.
+int chunk_tile_slices(int pos0, int tokens, int n_head, int n_kv, int most)
 {
     const int group = n_head / n_kv, tiles = (pos0 + tokens + kKTile - 1) / kKTile;
     const int first_tokens = tokens < 64 ? tokens : 64; // (of the first block: it must see enough tiles for every slice)
@@ -2127,7 +2127,7 @@ static int chunk_tile_slices(int pos0, int tokens, int n_head, int n_kv, int mos
     const int rem = tokens % kT64Tile;
     const int task64 = (tokens / kT64Tile + (rem > 32 ? 1 : 0)) * group + (rem > 0 && rem <= 32 ? (group + 1) / 2 : 0);
     const int block64 = (task64 + kT64Tasks - 1) / kT64Tasks;
-    const float per_slice = (float)tokens * (float)n_head * (2048.0f / 5.0e6f / 3.0f);
+    const float per_slice = (float)tokens * (float)n_head * (2048.0f / 4.0e6f / 2.6f);
     int best = most;
     float best_cost = 0.0f;
     for (int s = 2; s <= most; s++) {
@@ -2137,7 +2137,7 @@ static int chunk_tile_slices(int pos0, int tokens, int n_head, int n_kv, int mos
             rounds > (n_kv * s * block32 + 255) / 256)
             continue;
         const float fill = (float)(n_kv * s * block64) / (256.0f * (float)rounds);
-        const float cost = (float)rounds * ((float)slice_tiles + 4.0f) * (1.0f + 0.15f * fill) + (float)s * per_slice;
+        const float cost = (float)rounds * ((float)slice_tiles + 6.0f) * (1.0f + 0.05f * fill) + (float)s * per_slice;
         if (best_cost == 0.0f || cost < best_cost) {
             best = s;
             best_cost = cost;
@@ -2165,16 +2165,17 @@ int launch_chunk_q8(hipStream_t st, const float *q, const uint8_t *kc, const uin
         }
         // A count that was meant to hold the tiles but does not (hipml_attn_chunk_splits assumes 6 heads per KV
         // head; fewer make the partial rows, and with them the room per slice, smaller): the extra slices are
-        // not slices to run.  The kernel that dequantizes for itself gets the count it would have been given.
+        // not slices to run.  The kernel that dequantizes for itself gets the count it would have been given, within
+        // what the scratch holds.
         if (kv_f16 == nullptr && rope_tab == nullptr && splits >= 3 && chunk_tiles_pay(pos0, tokens) &&
             n_head / n_kv < 6) {
             const int s = hipml_attn_chunk_slices(pos0, tokens, n_kv);
-            if (s >= 2 && s < splits && splits == chunk_tiles_splits(pos0, tokens, 6 * n_kv, n_kv, s))
-                splits = s;
+            if (s >= 2 && s < splits && splits == chunk_tiles_splits(pos0, tokens, 6 * n_kv, n_kv, s)) {
+                const int fill = chunk_fill_slices(pos0, tokens, n_kv);
+                splits = fill < splits ? fill : splits;
+            }
         }
     }
-    if (kv_f16 != nullptr && splits > 2 && chunk_tiles_pay(pos0, tokens))
-        splits = chunk_tile_slices(pos0, tokens, n_head, n_kv, splits);
     // rope_tab != nullptr (splits == 0 only): q holds unrotated rows, the kernel rotates them as it loads them
     ChunkArgs a;
     // kv_f16 != nullptr: K and V are read from the f16 copy of the cache (kc, vc unused)

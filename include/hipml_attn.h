@@ -107,8 +107,9 @@ int hipml_attn_batch_splits(int stride, int n_kv, int slots);
  * NOTE: unlike the reference's split_count, which is at least 1, this returns 0 near position 0. */
 int hipml_attn_chunk_splits(int pos0, int tokens, int n_kv);
 /* The slice count (>= 1) for callers that want the sliced kernel whatever the shape, and for
- * hipml_attn_chunk_kv_f16, which has no in-workgroup variant: what hipml_attn_chunk_splits
- * returns where it does not return 0. */
+ * hipml_attn_chunk_kv_f16, which has no in-workgroup variant: the count that fills the chip's last round
+ * of workgroups, and for the long chunks named above the count that runs fastest over f16 tiles, often
+ * fewer (1,024 tokens at depth 8,192: 2, 1,500 at 20,000: 3, 2,048 at 100,000: 4). */
 int hipml_attn_chunk_slices(int pos0, int tokens, int n_kv);
 
 /* ---- RoPE ----------------------------------------------------------------

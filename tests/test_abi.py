@@ -70,6 +70,20 @@ def test_split_policies(lib):
     assert attn.chunk_slices(0, 672, 4) >= 2
 
 
+@pytest.mark.parametrize("tok,pos0,slices,splits", [
+    (1024, 8192, 2, 4), (1500, 20_000, 3, 6), (2048, 2048, 2, 3), (700, 10_000, 3, 6), (800, 40_000, 3, 13),
+    (672, 8192, 4, 7), (2048, 32_768, 4, 8), (2048, 100_000, 4, 13), (2048, 200_000, 4, 22), (2048, 400_000, 4, 40),
+    (2048, 800_000, 4, 4),              # the tiles would need more than 64 slices' room: the count of the kernel over the cache
+    (6000, 10_000, 1, 1),               # enough task blocks to fill the chip by themselves
+    (1023, 1022, 2, 2), (639, 100_000, 4, 4), (768, 767, 4, 0)])  # too short, or too short a prefix, for tiles
+def test_slice_counts_of_long_chunks(lib, tok, pos0, slices, splits):
+    from hipml_amd import attn
+    assert (attn.chunk_slices(pos0, tok, 4), attn.chunk_splits(pos0, tok, 4)) == (slices, splits)
+    if splits > slices:  # room for the tiles behind the partial rows, and no slice more than that takes
+        per_slice, tiles = (tok + 31) // 32 * 32 * 24 * 1024, 4 * ((pos0 + tok + 63) // 64) * 70_656
+        assert (splits - slices - 1) * per_slice < tiles <= (splits - slices) * per_slice
+
+
 def test_rope_table_on_the_host_is_the_f64_definition(lib):
     theta, n_rot, max_pos = 1e7, 64, 300
     nbytes = lib.hipml_rope_table_bytes(n_rot, max_pos)

@@ -124,6 +124,27 @@ def test_against_the_oracle(tok, pos0, pad, splits, n_heads, n_kv):
     assert ok
 
 
+@pytest.mark.parametrize("splits", [2, 3, 5, 8, 10])
+def test_the_callers_count_runs(splits):
+    # a long chunk, for which the library by itself takes 3 slices: with an explicit count that many write their
+    # partial rows, no more, and the values are those of the single pass
+    tok, pos0, n_heads, n_kv = 700, 6000, 24, 4
+    q, kb, vb, stride = inputs(0x7641_0C07, tok, pos0, 4, n_heads, n_kv)
+    copy = attn.kv_f16_alloc(stride, n_kv)
+    attn.kv_f16_rows(0, dev(kb), dev(vb), copy, n_kv, HD, stride, 0, pos0 + tok)
+    rows, most = (tok + 31) // 32 * 32, 11
+    acc = torch.full((most * rows * n_heads * HD,), float("nan"), dtype=torch.float32, device="cuda")
+    ml = torch.full((most, rows, n_heads, 2), float("nan"), dtype=torch.float32, device="cuda")
+    out = torch.full((2, tok, n_heads, HD), float("nan"), dtype=torch.float32, device="cuda")
+    for i, n in enumerate((splits, 1)):
+        attn.chunk_attention_kv_f16(dev(q), copy, None, out[i], None, n_heads, n_kv, HD, pos0, tok, stride, acc, ml, n)
+    torch.cuda.synchronize()
+    written = ~ml[:, :tok].isnan().flatten(1)
+    assert written[:splits].any(1).all() and written[0].all() and not written[splits:].any()
+    ok, _, _ = report(f"{splits} slices vs the single pass", host(out[1]), host(out[0]), *SAME_OPERANDS)
+    assert ok
+
+
 def test_gate_is_applied_by_the_merge():
     tok, pos0, splits, n_heads, n_kv = 130, 4000, 4, 24, 4
     assert uniform(tok, pos0, splits, n_heads // n_kv)
