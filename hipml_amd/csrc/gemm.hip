@@ -421,15 +421,15 @@ struct GemmTile {
     float sectors, sectors16, other, other16;
 };
 constexpr GemmTile kGemmTiles[] = {
-    {32, 32, 4, true, 0.115f, 0.105f, 0.0f, 0.0f},   {32, 64, 4, true, 0.155f, 0.14f, 0.0f, 0.0f},
-    {64, 64, 2, true, 0.214f, 0.0f, 0.0f, 0.0f},     {64, 128, 2, true, 0.344f, 0.312f, 0.0f, 0.0f},
-    {128, 128, 1, true, 0.497f, 0.0f, 0.0f, 0.0f},   {192, 128, 1, true, 0.725f, 0.59f, 0.0f, 0.0f},
-    {128, 192, 1, true, 0.725f, 0.646f, 0.0f, 0.0f}, {192, 192, 1, true, 0.929f, 0.82f, 0.0f, 0.0f},
-    {256, 192, 1, true, 0.0f, 0.98f, 0.0f, 0.0f},
+    {32, 32, 4, true, 0.117f, 0.105f, 0.0f, 0.0f},   {32, 64, 4, true, 0.156f, 0.14f, 0.0f, 0.0f},
+    {64, 64, 2, true, 0.216f, 0.0f, 0.0f, 0.0f},     {64, 128, 2, true, 0.341f, 0.311f, 0.0f, 0.0f},
+    {128, 128, 1, true, 0.504f, 0.0f, 0.0f, 0.0f},   {192, 128, 1, true, 0.729f, 0.585f, 0.0f, 0.0f},
+    {128, 192, 1, true, 0.725f, 0.642f, 0.0f, 0.0f}, {192, 192, 1, true, 0.931f, 0.814f, 0.0f, 0.0f},
+    {256, 192, 1, true, 0.0f, 0.972f, 0.0f, 0.0f},
     // quarters: the largest tile over f32 activations, whose registers do not hold sectors too; 128 x 128 over f16
     // activations, which they serve better; rows of weights that are not whole sectors
-    {256, 192, 1, false, 1.174f, 0.0f, 1.35f, 1.152f}, {192, 192, 1, false, 0.0f, 0.0f, 1.054f, 0.902f},
-    {128, 128, 1, false, 0.0f, 0.419f, 0.616f, 0.465f}, {64, 64, 2, false, 0.0f, 0.0f, 0.208f, 0.174f},
+    {256, 192, 1, false, 1.171f, 0.0f, 1.35f, 1.152f}, {192, 192, 1, false, 0.0f, 0.0f, 1.054f, 0.902f},
+    {128, 128, 1, false, 0.0f, 0.417f, 0.616f, 0.465f}, {64, 64, 2, false, 0.0f, 0.0f, 0.208f, 0.174f},
     {64, 64, 1, false, 0.0f, 0.0f, 0.229f, 0.184f},
     // cuts that fit 256 workgroups where those above do not (12,288 weight rows: 128 tiles of 96); over f16 activations
     // the 64 x 64 tile of longer steps stands for that of shorter ones
@@ -439,9 +439,9 @@ constexpr int kGemmNTiles = sizeof(kGemmTiles) / sizeof(kGemmTiles[0]);
 
 // The tile for a shape: the cheapest by rounds x cost, where a round of 256 workgroups slows down as it fills (they
 // share L2, HBM and the power budget: 1.5 times the cost of a lone workgroup when all CUs have one).  The costs are fitted
-// to every tile's time at 143 shapes (1,024 to 12,288 weight rows, k of 576 to 6,144, 24 to 2,048 tokens) over each type of
-// activations: the tile picked is the measured best or within 5 % of it at 284 of the 286 (8192 x 2176 over 1,500 tokens:
-// 92.5 us, best 84.8; 4096 x 576 over 450: 10.2, best 8.9), 0.1 % behind it on average.
+// to every tile's time at 173 shapes (1,024 to 12,288 weight rows, k of 576 to 6,144, 24 to 2,048 tokens), 346 with the
+// types of activations: the tile picked is the measured best or within 5 % of it at 340 of them, 14 % behind it at most
+// (1024 x 5120 over 1,400 tokens: 42.4 us, best 37.1), 0.2 % on average.
 static int gemm_tile(int m, int k, int tokens, bool sectors, bool x16)
 {
     int best = -1;
