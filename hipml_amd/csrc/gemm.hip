@@ -482,7 +482,6 @@ static bool with_gemm_kernel(int i, F &&f)
     switch (i) {
         HIPML_GEMM(0, true, 1, 1, 1, 1, 4, 8, 2)
         HIPML_GEMM(1, true, 1, 2, 1, 1, 4, 8, 2)
-        HIPML_GEMM(2, true, 2, 2, 1, 1, 2, 8, 2)
         HIPML_GEMM(3, true, 2, 2, 1, 2, 2, 8, 2)
         HIPML_GEMM(5, true, 2, 2, 3, 2, 1, 4, 2)
         HIPML_GEMM(6, true, 2, 2, 2, 3, 1, 4, 2)
@@ -496,10 +495,12 @@ static bool with_gemm_kernel(int i, F &&f)
             }
         }
         return false;
-    case 4: // (f32 activations only)
+    case 2: // (f32 activations only)
+    case 4:
     case 14:
         if constexpr (!X16) {
             switch (i) {
+                HIPML_GEMM(2, true, 2, 2, 1, 1, 2, 8, 2)
                 HIPML_GEMM(4, true, 2, 2, 2, 2, 1, 8, 2)
                 HIPML_GEMM(14, true, 2, 1, 1, 3, 2, 8, 2)
             }

@@ -366,10 +366,11 @@ __device__ __forceinline__ half8 int8x8_to_f16_sub(uint32_t w0, uint32_t w1)
 // (rows_wg x 17 pieces), which also says how many 16-row tiles cover rows_wg.
 constexpr bool gemv_dma_front(int rp) { return rp == 1; }
 constexpr int gemv_dma_tiles(int ni) { return ni > 5 ? 2 : 1; }
+constexpr int gemv_dma_rows(int ni) { return 4 * (ni - 1); } // weight rows of a workgroup, as the rule below picks them
 constexpr int kDmaDepth = 2; // chunks in flight per wave (three measured no faster)
 // a ring entry: the chunk's weights as they arrive (rows_wg x 272 bytes) and, behind them, its activations
-inline int gemv_dma_entry(int rp, int rows_wg) { return rows_wg * kDmaChunkBytes + (gemv_dma_front(rp) ? 0 : rp * 1024); }
-inline int gemv_dma_lds(int rp, int ni, int waves, int rows_wg, int k)
+constexpr int gemv_dma_entry(int rp, int rows_wg) { return rows_wg * kDmaChunkBytes + (gemv_dma_front(rp) ? 0 : rp * 1024); }
+constexpr int gemv_dma_lds(int rp, int ni, int waves, int rows_wg, int k)
 {
     const int per_wave = ((k >> 8) + waves - 1) / waves; // chunks of a wave
     // rings (at least the 1 KB per chain and tile in which the chains' sums meet at the end); front: the waves'
@@ -728,7 +729,7 @@ __global__ void __launch_bounds__(512, 2) gemv_q8_blocks_kernel(const uint8_t *_
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int lane = threadIdx.x & 63;
     const int lm = lane & 15, lg = lane >> 4;
-    const int nb = k >> 5, nchunk = (nb + 7) >> 3;
+    const int nb = k >> 5, nchunk = nb >> 3;
     const uint32_t row_bytes = (uint32_t)nb * kQ8Block;
     const int m0 = blockIdx.x * RW, r0 = blockIdx.y * (16 * XT);
     const int nrows = rows - r0 < 16 * XT ? rows - r0 : 16 * XT;
@@ -754,8 +755,7 @@ __global__ void __launch_bounds__(512, 2) gemv_q8_blocks_kernel(const uint8_t *_
     }
     auto issue = [&](int c) {
         const uint32_t at = ring_at + (uint32_t)((c % D) * S::kSlot);
-        const int b = 8 * c + wave < nb ? 8 * c + wave : nb - 1;
-        const uint8_t *xs = xb + (size_t)b * 128;
+        const uint8_t *xs = xb + (size_t)(8 * c + wave) * 128;
 #pragma unroll
         for (int j = 0; j < NX; j++)
             proj_dma16<false>(at + S::kWBytes + wave * S::kXWave + j * 1024, xs, xoff[j]);
@@ -868,8 +868,7 @@ __global__ void __launch_bounds__(512, 2) gemv_q8_blocks_kernel(const uint8_t *_
         if (c + 1 < nchunk)
             load(next, c + 1);
         __builtin_amdgcn_sched_barrier(0);
-        if (8 * c + wave < nb)
-            multiply(now);
+        multiply(now);
         __builtin_amdgcn_sched_barrier(0);
     };
     for (int c = 0; c < nchunk; c += 2) {
@@ -1184,26 +1183,35 @@ static DmaRows gemv_dma_rows_wg(int m, int rp)
     return {32, 9, false};
 }
 
-// Calls f with the kernel of (RP, NI, waves).
+// Calls f with the kernel of (RP, NI, waves).  Eight waves exist where their LDS fits, four where eight may not fit (with one
+// activation row the LDS grows with k) and where the rule above asks for them.
+template <int RP, int NI, typename F>
+static void with_gemv_dma_waves(int waves, F &&f)
+{
+    constexpr bool kEight = gemv_dma_lds(RP, NI, 8, gemv_dma_rows(NI), 256) <= (160 << 10);
+    constexpr bool kFour = RP == 1 || !kEight || (NI == 5 && RP <= 4);
+    if constexpr (kEight)
+        if (waves == 8)
+            f(&gemv_q8_dma_kernel<RP, NI, 8>);
+    if constexpr (kFour)
+        if (waves == 4)
+            f(&gemv_q8_dma_kernel<RP, NI, 4>);
+}
 template <int RP, typename F>
 static void with_gemv_dma_kernel(int ni, int waves, F &&f)
 {
-#define HIPML_DMA(n)                                            \
-    case n:                                                     \
-        return waves == 8 ? f(&gemv_q8_dma_kernel<RP, n, 8>)    \
-                          : f(&gemv_q8_dma_kernel<RP, n, 4>)
     switch (ni) {
-        HIPML_DMA(2);
-        HIPML_DMA(3);
-        HIPML_DMA(5);
-        HIPML_DMA(6);
-        HIPML_DMA(7);
-    default:
-        if (RP == 1)
-            return waves == 8 ? f(&gemv_q8_dma_kernel<1, 4, 8>) : f(&gemv_q8_dma_kernel<1, 4, 4>);
-        return waves == 8 ? f(&gemv_q8_dma_kernel<8, 9, 8>) : f(&gemv_q8_dma_kernel<8, 9, 4>);
+    case 2: return with_gemv_dma_waves<RP, 2>(waves, f);
+    case 3: return with_gemv_dma_waves<RP, 3>(waves, f);
+    case 5: return with_gemv_dma_waves<RP, 5>(waves, f);
+    case 6: return with_gemv_dma_waves<RP, 6>(waves, f);
+    case 7: return with_gemv_dma_waves<RP, 7>(waves, f);
+    default: // the small and the large workgroups of matrices beyond a round
+        if constexpr (RP == 1)
+            with_gemv_dma_waves<RP, 4>(waves, f);
+        else if constexpr (RP == 8)
+            with_gemv_dma_waves<RP, 9>(waves, f);
     }
-#undef HIPML_DMA
 }
 
 template <int RP>
