@@ -465,6 +465,12 @@ static int gemm_tile(int m, int k, int tokens, bool sectors, bool x16)
     return best;
 }
 
+// For the tests: the tile (its place in the table) that a call takes.
+extern "C" int hipml_test_gemm_tile(int m, int k, int tokens, int sectors, int x16)
+{
+    return gemm_tile(m, k, tokens, sectors != 0, x16 != 0);
+}
+
 // Calls f with the kernel of tile i and its launch figures: (kernel, threads, tile tokens, tile rows, LDS bytes).
 template <bool X16, typename F>
 static bool with_gemm_kernel(int i, F &&f)

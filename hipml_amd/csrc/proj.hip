@@ -1150,17 +1150,17 @@ static int launch_gemv_variant(hipStream_t st, const uint8_t *w, const float *x,
 }
 
 // the most waves (8, else 4) whose rings and tables fit a CU's LDS; 0: none
-static int gemv_dma_waves(int rp, int ni, int rows_wg, int k)
+static int gemv_dma_waves(int rp, int ni, int k)
 {
     for (int waves = 8; waves >= 4; waves -= 4)
-        if (gemv_dma_lds(rp, ni, waves, rows_wg, k) <= (160 << 10))
+        if (gemv_dma_lds(rp, ni, waves, gemv_dma_rows(ni), k) <= (160 << 10))
             return waves;
     return 0;
 }
 
 // Weight rows per workgroup for a pass of rp activation rows, as requests per chunk (NI).
 struct DmaRows {
-    int rows_wg, ni;
+    int ni;
     bool four; // four waves even where the LDS of eight fits (several workgroups then share a CU)
 };
 static DmaRows gemv_dma_rows_wg(int m, int rp)
@@ -1168,19 +1168,19 @@ static DmaRows gemv_dma_rows_wg(int m, int rp)
     // The fewest weight rows that make one round of the chip's 256 CUs, every CU the same bytes (us at 1024 x 5120 over
     // 1 / 2 / 4 / 8 rows: 4 rows a workgroup 4.4 / 5.7 / 7.3 / 9.0, 16 rows 5.5 / 6.9 / 8.5 / 11.3; at 5120 x 6144: 20 rows
     // 9.6 / 11.4 / 12.9 / 16.7, 16 rows 11.9 / 14.7 / 18.3 / 24.3).
-    static const DmaRows kOneRound[5] = {{4, 2, false}, {8, 3, false}, {16, 5, false}, {20, 6, false}, {24, 7, false}};
+    static const DmaRows kOneRound[5] = {{2, false}, {3, false}, {5, false}, {6, false}, {7, false}};
     for (const DmaRows &r : kOneRound)
-        if ((m + r.rows_wg - 1) / r.rows_wg <= 256)
+        if ((m + gemv_dma_rows(r.ni) - 1) / gemv_dma_rows(r.ni) <= 256)
             return r;
     // Beyond, small workgroups of which two or three share a CU, so that one's start and end lie behind another's
     // stream (12288 x 5120 over 1 / 2 / 4 rows: 14.8 / 16.7 / 20.3 us; one workgroup of 48 rows per CU 17.9 / 18.7 / 20.5;
     // 32 rows, a round and a half, 19.4 / 20.4 / 24.4).  With eight activation rows their copies fill the LDS and 32
     // weight rows share them best (28.6; 16 rows 32.4).
     if (rp == 1)
-        return {12, 4, false};
+        return {4, false};
     if (rp <= 4)
-        return {16, 5, true};
-    return {32, 9, false};
+        return {5, true};
+    return {9, false};
 }
 
 // Calls f with the kernel of (RP, NI, waves).  Eight waves exist where their LDS fits, four where eight may not fit (with one
@@ -1214,41 +1214,12 @@ static void with_gemv_dma_kernel(int ni, int waves, F &&f)
     }
 }
 
-template <int RP>
-static int launch_gemv_dma(hipStream_t st, const uint8_t *w, const float *x, float *y, int m, int k, int rows)
-{
-    const DmaRows r = gemv_dma_rows_wg(m, RP);
-    const dim3 grid((unsigned)((m + r.rows_wg - 1) / r.rows_wg), (unsigned)((rows + RP - 1) / RP), 1);
-    const int waves = r.four ? 4 : gemv_dma_waves(RP, r.ni, r.rows_wg, k);
-    const size_t lds = (size_t)gemv_dma_lds(RP, r.ni, waves, r.rows_wg, k);
-    with_gemv_dma_kernel<RP>(r.ni, waves, [&](auto kernel) {
-        HIPML_LAUNCH(kernel, grid, dim3(64 * waves, 1, 1), lds, st, w, x, y, m, k, rows, r.rows_wg);
-    });
-    return launched("gemv_q8_0_rows");
-}
-
-// Up to eight rows over the raw-row kernel: rows of whole 256-value chunks at 16-byte boundaries, addressed with
-// 32-bit offsets, and LDS room for every row count (so that all of them take this kernel, or none).  Returns -1
-// where the shape does not qualify (the kernels above serve it).
-static int try_gemv_dma(hipStream_t st, const uint8_t *w, const float *x, float *y, int m, int k, int rows)
-{
-    if (rows > 8 || k % 256 != 0 || (reinterpret_cast<uintptr_t>(w) & 15) != 0 ||
-        (reinterpret_cast<uintptr_t>(x) & 15) != 0 || (size_t)m * (k >> 5) * kQ8Block >= ((size_t)1 << 32) ||
-        (size_t)rows * k * sizeof(float) >= ((size_t)1 << 32))
-        return -1;
-    for (int rp = 1; rp <= 8; rp *= 2) {
-        const DmaRows r = gemv_dma_rows_wg(m, rp);
-        if (gemv_dma_waves(rp, r.ni, r.rows_wg, k) == 0)
-            return -1;
-    }
-    if (rows == 1)
-        return launch_gemv_dma<1>(st, w, x, y, m, k, rows);
-    if (rows == 2)
-        return launch_gemv_dma<2>(st, w, x, y, m, k, rows);
-    if (rows <= 4)
-        return launch_gemv_dma<4>(st, w, x, y, m, k, rows);
-    return launch_gemv_dma<8>(st, w, x, y, m, k, rows);
-}
+// Which kernel a call takes, and its variant: kRows: -; kDma: activation rows per pass, requests per chunk, waves; kBlocks
+// and kUnits: activation tiles, weight rows per workgroup, whether the last tile is half dead.
+struct RowsPick {
+    enum { kRows, kDma, kBlocks, kUnits } kernel;
+    int a, b, c;
+};
 
 // Calls f with the kernel of (XT, RW, HALF), its threads and its LDS bytes.
 template <typename F>
@@ -1289,10 +1260,10 @@ static void with_gemv_units_kernel(int xt, int rw, bool half, F &&f)
 }
 static const int kBlocksRw[2] = {32, 48}, kUnitsRw[5] = {16, 20, 24, 32, 48};
 
-static int launch_gemv_tiles(hipStream_t st, const uint8_t *w, const float *x, float *y, int m, int k, int rows)
+static RowsPick pick_tiles(int m, int k, int rows, bool w16)
 {
     // by the shape of W alone: a row has the same bits however many travel with it
-    const bool blocks = m > 6144 && k % 256 == 0 && (reinterpret_cast<uintptr_t>(w) & 15) == 0;
+    const bool blocks = m > 6144 && k % 256 == 0 && w16;
     // the tile that costs least: rounds of 256 workgroups x the cycles of a unit in the eight waves of a CU, as the sum
     // of its vector instructions (two waves a SIMD, 4 cycles each) and its requests (16 cycles); within 20 % of the
     // measured times less 4 us, and in their order, at 1024 / 5120 / 12288 weight rows over 9 to 100 rows
@@ -1313,35 +1284,88 @@ static int launch_gemv_tiles(hipStream_t st, const uint8_t *w, const float *x, f
                 rw = cr;
             }
         }
+    return {blocks ? RowsPick::kBlocks : RowsPick::kUnits, xt, rw, rows <= 16 * xt - 8 ? 1 : 0};
+}
+
+static RowsPick pick_rows(int m, int k, int rows, bool w16)
+{
+    // Up to eight rows over the raw-row kernel: rows of whole 256-value chunks at 16-byte boundaries, addressed with
+    // 32-bit offsets, and LDS room for every row count (so that all of them take this kernel, or none).
+    bool dma = rows <= 8 && k % 256 == 0 && w16 && (size_t)m * (k >> 5) * kQ8Block < ((size_t)1 << 32) &&
+               (size_t)rows * k * sizeof(float) < ((size_t)1 << 32);
+    RowsPick p = {RowsPick::kDma, 0, 0, 0};
+    for (int rp = 1; dma && rp <= 8; rp *= 2) {
+        const DmaRows r = gemv_dma_rows_wg(m, rp);
+        const int waves = gemv_dma_waves(rp, r.ni, k);
+        dma = waves != 0;
+        if (p.a < rows) {
+            p.a = rp;
+            p.b = r.ni;
+            p.c = r.four ? 4 : waves;
+        }
+    }
+    if (dma)
+        return p;
+    return rows > kGemvMaxRows ? pick_tiles(m, k, rows, w16) : RowsPick{RowsPick::kRows, 0, 0, 0};
+}
+
+template <int RP>
+static void launch_gemv_dma(hipStream_t st, const uint8_t *w, const float *x, float *y, int m, int k, int rows,
+                            const RowsPick &p)
+{
+    const int rows_wg = gemv_dma_rows(p.b), waves = p.c;
+    const dim3 grid((unsigned)((m + rows_wg - 1) / rows_wg), (unsigned)((rows + RP - 1) / RP), 1);
+    const size_t lds = (size_t)gemv_dma_lds(RP, p.b, waves, rows_wg, k);
+    with_gemv_dma_kernel<RP>(p.b, waves, [&](auto kernel) {
+        HIPML_LAUNCH(kernel, grid, dim3(64 * waves, 1, 1), lds, st, w, x, y, m, k, rows, rows_wg);
+    });
+}
+
+static bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
+
+// (x at a 16-byte boundary: the caller has checked it)
+int launch_gemv_q8_rows(hipStream_t st, const uint8_t *w, const float *x, float *y, int m, int k, int rows)
+{
+    const RowsPick p = pick_rows(m, k, rows, aligned16(w));
+    if (p.kernel == RowsPick::kRows) {
+        int rp = gemv_rows_per_pass(k);
+        if (rp < 1)
+            return fail(HIPML_ATTN_E_RANGE, "k %d: one activation row does not fit the LDS operand buffer", k);
+        rp = rows < rp ? rows : rp;
+        // One 16-row weight tile per workgroup keeps the kernel inside 128 registers, so two workgroups
+        // share a CU and the 320 workgroups of a 5120-row matrix start together (workgroups start in
+        // windows of as many as fit the chip; a second window opens when the first has drained).
+        return launch_gemv_variant<8, 1, 6>(st, w, x, y, m, k, rows, rp);
+    }
+    if (p.kernel == RowsPick::kDma) {
+        if (p.a == 1)
+            launch_gemv_dma<1>(st, w, x, y, m, k, rows, p);
+        else if (p.a == 2)
+            launch_gemv_dma<2>(st, w, x, y, m, k, rows, p);
+        else if (p.a == 4)
+            launch_gemv_dma<4>(st, w, x, y, m, k, rows, p);
+        else
+            launch_gemv_dma<8>(st, w, x, y, m, k, rows, p);
+        return launched("gemv_q8_0_rows");
+    }
+    const int xt = p.a, rw = p.b;
     const dim3 grid((unsigned)((m + rw - 1) / rw), (unsigned)((rows + 16 * xt - 1) / (16 * xt)), 1);
-    const bool half = grid.y == 1 && rows <= 16 * xt - 8;
     auto go = [&](auto kernel, int threads, int lds) {
         HIPML_LAUNCH(kernel, grid, dim3((unsigned)threads, 1, 1), (size_t)lds, st, w, x, y, m, k, rows);
     };
-    if (blocks)
-        with_gemv_blocks_kernel(xt, rw, half, go);
+    if (p.kernel == RowsPick::kBlocks)
+        with_gemv_blocks_kernel(xt, rw, p.c, go);
     else
-        with_gemv_units_kernel(xt, rw, half, go);
+        with_gemv_units_kernel(xt, rw, p.c, go);
     return launched("gemv_q8_0_rows");
 }
 
-int launch_gemv_q8_rows(hipStream_t st, const uint8_t *w, const float *x, float *y, int m, int k, int rows)
+// For the tests: the kernel that a call takes, as kernel * 10^6 + a * 10^4 + b * 100 + c of its RowsPick.
+extern "C" int hipml_test_rows_kernel(int m, int k, int rows, int w_aligned16)
 {
-    const int dma = rows <= 8 ? try_gemv_dma(st, w, x, y, m, k, rows) : -1;
-    if (dma >= 0)
-        return dma;
-    if (rows > kGemvMaxRows)
-        return launch_gemv_tiles(st, w, x, y, m, k, rows);
-    int rp = gemv_rows_per_pass(k);
-    if (rp < 1)
-        return fail(HIPML_ATTN_E_RANGE, "k %d: one activation row does not fit the LDS operand buffer", k);
-    rp = rows < rp ? rows : rp;
-    // One 16-row weight tile per workgroup keeps the kernel inside 128 registers, so two workgroups
-    // share a CU and the 320 workgroups of a 5120-row matrix start together (workgroups start in
-    // windows of as many as fit the chip; a second window opens when the first has drained).
-    return launch_gemv_variant<8, 1, 6>(st, w, x, y, m, k, rows, rp);
+    const RowsPick p = pick_rows(m, k, rows, w_aligned16 != 0);
+    return p.kernel * 1000000 + p.a * 10000 + p.b * 100 + p.c;
 }
-
 
 template <int WAVES, int TILES, int CH>
 static hipError_t raise_gemv_lds()

@@ -1,0 +1,40 @@
+"""Shapes that between them run every variant of the projection kernels, as the library itself names the variant a call
+takes (test_proj_instances.py holds that none is missing, test_gpu_proj_instances.py runs them)."""
+from hipml_amd import attn
+
+
+def row_kernel(m, k, rows):
+    """kernel * 10^6 + a * 10^4 + b * 100 + c: 0 the row kernel, 1 raw rows (activation rows a pass, requests, waves), 2
+    blocks and 3 units (activation tiles, weight rows, last tile half dead); W at a 16-byte boundary."""
+    return attn.lib().hipml_test_rows_kernel(m, k, rows, 1)
+
+
+def gemm_tile(m, k, tokens, x16):
+    """(place in the table of tiles, whole sectors of weights), W at a 64-byte boundary."""
+    sectors = int(k % 1024 == 0)
+    return attn.lib().hipml_test_gemm_tile(m, k, tokens, sectors, x16), sectors
+
+
+# (weight rows, k, activation rows): ragged in the rows of a workgroup, k of 19 chunks or 37 units (uneven shares of the
+# waves, several turns of every ring); the depths that leave no LDS for eight waves or for the raw-row kernel at all
+ROWS = [
+    (3, 2368, 1), (3, 34560, 1), (3, 4864, 1), (1032, 32768, 1), (1032, 4864, 1), (6156, 4864, 1), (2069, 4864, 1),
+    (4143, 4864, 1), (5180, 4864, 1), (3, 4864, 2), (1032, 4864, 2), (6156, 4864, 2), (2069, 4864, 2),
+    (4143, 4864, 2), (5180, 4864, 2), (3, 4864, 3), (1032, 4864, 3), (6156, 4864, 3), (2069, 4864, 3),
+    (4143, 4864, 3), (5180, 4864, 3), (3, 4864, 5), (1032, 4864, 5), (2069, 4864, 5), (4143, 4864, 5),
+    (5180, 4864, 5), (6156, 4864, 5), (6156, 4864, 9), (6156, 32768, 3), (8230, 4864, 9), (8230, 32768, 3),
+    (6156, 4864, 25), (6156, 4864, 17), (8230, 4864, 25), (8230, 4864, 17), (6156, 4864, 41), (6156, 4864, 33),
+    (8230, 4864, 41), (8230, 4864, 33), (6156, 4864, 57), (6156, 4864, 49), (8230, 4864, 57), (8230, 4864, 49),
+    (3, 2368, 9), (3, 2368, 3), (2069, 2368, 17), (4143, 2368, 3), (2618, 2368, 17), (5180, 2368, 3),
+    (3106, 2368, 17), (6156, 2368, 3), (8230, 2368, 9), (8230, 2368, 3), (2069, 2368, 49), (4143, 2368, 17),
+    (2740, 2368, 33), (5180, 2368, 17), (4082, 2368, 33), (6156, 2368, 17), (4143, 2368, 33), (8230, 2368, 17),
+]
+# (weight rows, k, tokens, f16 activations)
+TILES = [
+    (12380, 704, 580, 0), (10996, 704, 258, 0), (10996, 704, 143, 0), (239, 1408, 51, 0), (239, 704, 51, 0),
+    (12380, 704, 649, 1), (10996, 704, 258, 1), (7190, 704, 212, 1), (239, 1408, 51, 1), (239, 704, 51, 1),
+    (239, 3072, 51, 0), (2173, 3072, 97, 0), (5460, 3072, 74, 0), (12380, 3072, 74, 0), (10996, 3072, 143, 0),
+    (6671, 3072, 534, 0), (10996, 3072, 258, 0), (12380, 3072, 396, 0), (12380, 3072, 649, 0), (8228, 3072, 74, 0),
+    (239, 3072, 51, 1), (2173, 3072, 97, 1), (8228, 3072, 74, 1), (10996, 3072, 258, 1), (10996, 3072, 396, 1),
+    (12380, 3072, 396, 1), (7363, 3072, 985, 1), (10996, 3072, 143, 1), (3730, 3072, 97, 1),
+]

@@ -1,0 +1,67 @@
+"""Every variant of the projection kernels once, at the shapes of proj_instances.py: against the definition in 64 bits, with
+nothing written past the outputs, and a row's bits those it has in other company."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+import proj_instances as inst  # noqa: E402
+from hipml_amd import attn  # noqa: E402
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _init():
+    attn.init(0)
+
+
+def inputs(m, k, rows):
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(m * 1_000_003 + k * 131 + rows)
+    q = torch.randint(-128, 128, (m, k // 32, 32), device="cuda", dtype=torch.int8, generator=gen)
+    d = (torch.rand((m, k // 32, 1), device="cuda", generator=gen) * 0.05 + 0.001).to(torch.float16)
+    w = torch.cat((d.view(torch.uint8), q.view(torch.uint8)), dim=2).contiguous()
+    return w, d, q, torch.randn((rows, k), device="cuda", generator=gen) * 0.25
+
+
+def padded(rows, m):
+    return torch.full((rows + 1, m), float("nan"), device="cuda")
+
+
+@pytest.mark.parametrize("m,k,rows", inst.ROWS)
+def test_row_kernel(m, k, rows):
+    w, d, q, x = inputs(m, k, rows)
+    y = padded(rows, m)
+    attn.gemv_q8_0_rows(w, x, y, m, k, rows)
+    assert bool(y[rows].isnan().all())
+    exact = x.double() @ (d.double() * q.double()).reshape(m, k).T
+    err = (y[:rows] - exact).abs().max().item()
+    # activations to ~22 bits, fp32 sums over eight chains; the raw-row kernel's 128 + q, whose 128 comes out in fp32
+    assert err <= 2e-6 * exact.abs().max().item() * max(1.0, (k / 8192) ** 0.5) + 1e-5, err
+    # the last row among others: the same bits where those take kernels of the same class
+    kernel = inst.row_kernel(m, k, rows) // 1_000_000
+    for more in (2 * rows, rows + 9, 128):
+        if more <= 128 and more > rows and inst.row_kernel(m, k, more) // 1_000_000 == kernel:
+            company = torch.cat((torch.randn((more - 1, k), device="cuda"), x[-1:]))
+            z = padded(more, m)
+            attn.gemv_q8_0_rows(w, company, z, m, k, more)
+            assert torch.equal(z[more - 1], y[rows - 1]) and bool(z[more].isnan().all())
+
+
+@pytest.mark.parametrize("m,k,tokens,x16", inst.TILES)
+def test_tile(m, k, tokens, x16):
+    w, d, q, x = inputs(m, k, tokens)
+    h = x.to(torch.float16)
+    y, one = padded(tokens, m), padded(1, m)
+    if x16:
+        attn.output_chunk_q8_0(w, None, None, y, m, k, tokens, h)
+    else:
+        attn.gemm_q8_0_f16(w, x, y, m, k, tokens)
+    attn.gemm_q8_0_f16(w, x[tokens // 2:], one, m, k, 1)
+    assert bool(y[tokens].isnan().all()) and bool(one[1].isnan().all())
+    # f16 operands, the weights f16(d * q); 2^-24 of every term for each of about sqrt(k) roundings of the fp32 sum
+    dense = (d.float() * q.float()).to(torch.float16).double().reshape(m, k)
+    terms = h.double().norm(dim=1)[:, None] * dense.norm(dim=1)[None, :]
+    err = ((y[:tokens] - h.double() @ dense.T).abs() / terms).max().item()
+    assert err <= 2.0 ** -24 * np.sqrt(k), err
+    assert torch.equal(y[tokens // 2], one[0])

@@ -1,0 +1,30 @@
+"""That tests/proj_instances.py names a shape for every variant of the projection kernels that any call can take."""
+import pytest
+
+import proj_instances as inst
+
+M = sorted({*range(1, 400, 13), *range(400, 20_000, 197), *range(20_000, 130_000, 7_777), 1024, 2048, 5120, 6144, 12_288})
+
+
+@pytest.mark.parametrize("k", [64, 256, 1088, 5120, 32_768, 34_560, 36_096])
+def test_every_row_kernel_has_a_shape(k):
+    named = {inst.row_kernel(*shape) for shape in inst.ROWS}
+    assert len(named) == len(inst.ROWS)
+    taken = {inst.row_kernel(m, k, rows): (m, rows) for m in M for rows in range(1, 129)}
+    assert not {c: s for c, s in taken.items() if c not in named}
+
+
+@pytest.mark.parametrize("x16", [0, 1])
+@pytest.mark.parametrize("k", [64, 128, 1024])
+def test_every_tile_has_a_shape(k, x16):
+    named = {(inst.gemm_tile(m, k_, t, h), h) for m, k_, t, h in inst.TILES}
+    assert len(named) == len(inst.TILES)
+    tokens = [*range(1, 700, 17), *range(700, 4200, 83)]
+    taken = {(inst.gemm_tile(m, k, t, x16), x16): (m, t) for m in M for t in tokens}
+    assert not {c: s for c, s in taken.items() if c not in named}
+
+
+@pytest.mark.parametrize("m,k", [(12_288, 5120), (1024, 5120), (5120, 6144)])
+def test_the_models_projections_are_among_them(m, k):
+    named = {inst.row_kernel(*shape) for shape in inst.ROWS}
+    assert all(inst.row_kernel(m, k, rows) in named for rows in range(1, 129))
