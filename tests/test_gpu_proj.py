@@ -84,7 +84,7 @@ def test_output_projection_shape(rows):
             assert np.array_equal(run_gemv(w, x[r], m, k, 1)[0], got[r])
     if rows == 8:
         assert np.array_equal(run_gemv(w, x[2:5], m, k, 3)[1], got[3])
-    # 10 to 128 rows share one kernel (two passes of it beyond 64), 9 rows take another
+    # 9 to 128 rows share one kernel, whatever its tiles
     if rows in (24, 64, 70, 128):
         assert np.array_equal(run_gemv(w, x[3:13], m, k, 10)[2], got[5])
         assert np.array_equal(run_gemv(w, x[rows - 10:], m, k, 10)[9], got[rows - 1])
@@ -96,8 +96,8 @@ def test_ragged_shapes_and_scales():
     # reference bounds such cases with LARGE_TOL (2e-3 / 3e-2, quant_parity.rs:20-25); on top of that
     # the kernel must be as close to the float64 value as the sequential fp32 sum is.
     r = orc.Rng(0x7A66)
-    # rows 1-2 take the row kernel; more rows take full 16- or 32-row tiles (k = 5120 and 6144 in
-    # straight-line code, any other k in a loop; k = 64 leaves seven of eight waves without a step)
+    # rows 1-2 take the row kernel or, like 3-8, the raw-row kernel where k allows it; more rows (and 3-8 where it does
+    # not) take tiles of 16 rows (k = 64 leaves seven of eight waves without a step)
     for m, k, rows in ((1, 64, 1), (33, 192, 2), (1000, 320, 7), (50, 4096, 16), (7, 64, 5),
                        (40, 5120, 9), (130, 704, 33), (64, 1024, 128), (20, 6144, 47)):
         w = orc.random_q8_0_bytes(r, m * k // 32).reshape(-1, 34)
@@ -148,10 +148,10 @@ def test_raw_row_kernel_over_ragged_shapes(m, k):
 
 @pytest.mark.parametrize("m,k", [(100, 2304), (5121, 1024), (300, 8192)])
 def test_raw_row_tile_kernel_over_row_counts(m, k):
-    # 10 to 128 rows over the tile kernel that moves the weight rows into LDS as they lie: one to four activation
-    # tiles, a last tile with at most 8 live rows (whose other rows are not fetched), two passes beyond 64 rows with
-    # a short second pass; real scales.  Every row count against the oracle, and a row's bits the same whatever
-    # travels with it and whichever pass and tile it falls in.
+    # 10 to 128 rows over the kernel whose waves stream units of their own: one or two activation tiles a workgroup, a
+    # last tile with at most 8 live rows (whose other rows are not fetched), several passes with a short last one; real
+    # scales.  Every row count against the oracle, and a row's bits the same whatever travels with it and whichever
+    # pass and tile it falls in.
     r = orc.Rng(0x711E + m + k)
     w = orc.random_q8_0_bytes(r, m * k // 32).reshape(-1, 34)
     scales = (r.uniform_array(w.shape[0]) * 0.05 + 0.001).astype(np.float16)
@@ -345,9 +345,10 @@ def test_qkv_projection_shapes(m, k):
                                    (9001, 2048, 700), (12270, 1024, 1001), (1029, 512, 301), (6000, 256, 300),
                                    (9001, 192, 700), (12270, 128, 1001), (5, 192, 70)])
 def test_gemm_tiles(m, k, t):
-    # one shape per tile of the chunk GEMM (32 x 32 up to 256 x 192), ragged in both directions, weight rows of whole
-    # 64-byte sectors (k a multiple of 1,024) and others, an odd number of 64-value units among them; against its own
-    # definition, from f32 and from f16 activations, and a row's bits the same in a chunk of its own (a small tile)
+    # shapes across the tiles of the chunk GEMM, ragged in both directions, weight rows of whole 64-byte sectors (k a
+    # multiple of 1,024) and others, an odd number of 64-value units among them; against its own definition, from f32
+    # and from f16 activations, and a row's bits the same in a chunk of its own (a small tile).  Which tile a shape takes
+    # is a matter of costs: test_gpu_proj_instances.py has one for each.
     r = orc.Rng(0x6E00 + m + t)
     w = orc.random_q8_0_bytes(r, m * k // 32).reshape(-1, 34)
     scales = (r.uniform_array(w.shape[0]) * 0.05 + 0.001).astype(np.float16)
