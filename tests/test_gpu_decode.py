@@ -349,3 +349,44 @@ def test_one_split_writes_the_rows_itself(seq, dtype):
     for c in range(3):
         assert torch.equal(cols[c], one(c, seq + c + 1))
     assert bool(acc.isnan().all()) and bool(ml.isnan().all())
+
+
+@pytest.mark.parametrize("dtype", [0, 1])
+@pytest.mark.parametrize("slots,n_kv", [(40, 8), (66, 4)])
+def test_one_split_over_a_batch_too_large_for_a_window(slots, n_kv, dtype):
+    # more items than a window of workers serves: the plain grid, where one split writes the rows itself; slots of one to
+    # three rows, slots of different depth, one without any key: the bits of each row's plain decode, gated or not, the
+    # oracle's values on some, and no scratch touched
+    stride = 160
+    r = orc.Rng(0x0D1F + slots + dtype)
+    cols = [(1, 3, 1, 2)[s % 4] for s in range(slots)]
+    depths = [(5, 31, 32, 64, 127, 128, 150)[s % 7] for s in range(slots)]
+    kb = orc.quantize(dtype, r.normal_array((slots, n_kv, stride, HD))).reshape(slots, n_kv, stride, -1)
+    vb = orc.quantize(dtype, r.normal_array((slots, n_kv, stride, HD))).reshape(slots, n_kv, stride, -1)
+    pos = [(d + c, d + c + 1) for d, n in zip(depths, cols) for c in range(n)]
+    pos[0] = (0, 0)  # slot 0 has no key
+    slot_of = [s for s, n in enumerate(cols) for _ in range(n)]
+    rows = len(pos)
+    assert 2 * slots > 512 // n_kv and rows <= 128
+    q, gate = r.normal_array((rows, N_HEADS, HD)), dev(r.normal_array((rows, N_HEADS, HD)))
+    kd, vd, qd = dev(kb), dev(vb), dev(q)
+    acc, ml = decode_scratch(N_HEADS, 1, rows)
+    acc.fill_(float("nan")), ml.fill_(float("nan"))
+    args = (N_HEADS, n_kv, HD, stride, SCALE, 1, kd[0].numel(), N_HEADS * HD, N_HEADS * 2, N_HEADS * HD, cols)
+    p = torch.tensor(pos, dtype=torch.int32, device="cuda")
+    out = torch.full((3, rows, N_HEADS, HD), float("nan"), device="cuda")
+    attn.attn_decode_batch_cols(dtype, p, qd, kd, vd, acc, ml, out[0], *args)
+    attn.attn_decode_batch_cols_gate(dtype, p, qd, kd, vd, acc, ml, out[1], gate, *args)
+    attn.q_gate(out[0], gate, out[2])
+    assert torch.equal(out[1], out[2]) and not out[0][0].any()
+    one = torch.full((rows, N_HEADS, HD), float("nan"), device="cuda")
+    for i, (at, seq) in enumerate(pos):
+        attn.attn_decode_kv(step_buffer(at, seq), dtype, qd[i], kd[slot_of[i]], vd[slot_of[i]], acc, ml, one[i], N_HEADS, n_kv,
+                            HD, stride, SCALE, 1)
+    torch.cuda.synchronize()
+    assert torch.equal(out[0], one)
+    assert bool(acc.isnan().all()) and bool(ml.isnan().all())
+    for i in (1, 2, 3, rows // 2, rows - 1):
+        want = orc.attn_decode_kv(q[i], kb[slot_of[i]], vb[slot_of[i]], N_HEADS, n_kv, HD, pos[i][1], SCALE, stride=stride,
+                                  dtype=dtype)
+        assert report(f"row {i} of {slots} slots, one split", want.ravel(), host(out[0][i]).ravel(), *GATE)[0]
