@@ -693,9 +693,18 @@ __global__ void __launch_bounds__(64 * WAVES, 1) gemv_q8_dma_kernel(const uint8_
 // gemv_q8_units_kernel (m up to 6,144; any k of whole 64-value units, W at a 4-byte boundary): no barrier, a wave
 // streams units of its own.  gemv_q8_blocks_kernel (more rows, k of whole 256-value chunks, W at a 16-byte boundary):
 // the workgroup walks chunks together and shares 16-byte requests for the weights, where units take four times as many
-// dword requests, which tell where a workgroup has 48 weight rows.  us over 24 rows, units / blocks / the kernel before
-// them (eight waves in step, a block of each chunk per wave, two barriers per chunk): 1024 x 5120 9.7 / 12.0 / 14.0,
-// 5120 x 6144 17.0 / 21.3 / 23.6, 12288 x 5120 26.1 / 23.4 / 38.6.
+// dword requests, which tell where a workgroup has 48 weight rows.  The kernels before them had eight waves in step, a
+// block of each chunk per wave and two barriers per chunk.  us over 9 / 24 / 32 / 48 / 64 / 128 rows (k 5120, for 5,120
+// weight rows 6144; before / units / blocks):
+//    1,024 weight rows  11.2  8.9 14.7 | 14.5  9.1 14.7 | 15.7  9.2 15.1 | 20.7  9.3 15.1 | 24.5  9.6 15.4 | 24.8 12.7 15.7
+//    4,096              11.4  9.3 14.8 | 15.2 12.5 15.2 | 16.3 12.6 15.4 | 21.3 19.4 18.0 | 25.6 19.8 18.4 | 49.2 37.2 29.9
+//    5,120              14.8 13.3 17.1 | 23.5 18.4 22.3 | 22.3 20.5 23.1 | 29.7 29.1 27.3 | 34.2 29.7 28.6 | 68.4 55.3 40.7
+//    6,144              12.8 13.5 15.2 | 21.0 17.2 18.3 | 20.2 18.5 18.6 | 26.5 25.0 21.3 | 30.7 25.7 22.3 | 58.2 48.5 33.5
+//    7,168              14.7 15.4 15.4 | 19.1 19.2 17.6 | 22.0 22.4 18.9 | 26.6 33.4 28.0 | 30.1 38.7 30.9 | 57.6 70.6 61.3
+//    8,192              14.8 15.7 16.1 | 19.3 19.7 17.9 | 22.3 22.8 19.3 | 27.2 39.9 28.2 | 30.4 40.7 31.2 | 59.7 71.6 59.9
+//   12,288              26.9 20.7 20.7 | 36.8 25.8 22.6 | 41.2 29.7 26.0 | 50.6 51.4 32.8 | 57.6 52.2 35.5 | 88.0 97.8 69.6
+// The choice must not depend on the number of rows (their bits would), so the line lies where the row counts of verify
+// groups and batched decode, 9 to 32, change sides; over more rows the blocks would win from 4,096 weight rows on.
 
 template <int XT, int RW, bool HALF>
 struct BlocksShape {
@@ -1265,8 +1274,9 @@ static RowsPick pick_tiles(int m, int k, int rows, bool w16)
     // by the shape of W alone: a row has the same bits however many travel with it
     const bool blocks = m > 6144 && k % 256 == 0 && w16;
     // the tile that costs least: rounds of 256 workgroups x the cycles of a unit in the eight waves of a CU, as the sum
-    // of its vector instructions (two waves a SIMD, 4 cycles each) and its requests (16 cycles); within 20 % of the
-    // measured times less 4 us, and in their order, at 1024 / 5120 / 12288 weight rows over 9 to 100 rows
+    // of its vector instructions (two waves a SIMD, 4 cycles each) and its requests (16 cycles).  At ten matrices of 1,024
+    // to 12,288 weight rows over 9 to 128 rows it picks the fastest tile or one within 5 %, but for 9 % at 7,168 weight
+    // rows over 100 (60.3 us, best 55.2)
     int xt = 0, rw = 0;
     long long best = 0;
     for (int cx = 1; cx <= (blocks ? 4 : 2) && 16 * (cx - 1) < rows; cx++)
