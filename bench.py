@@ -790,6 +790,21 @@ def random_q8_0_weights(torch, m, k, gen):
     return w.reshape(-1)
 
 
+def row_kernel_name(attn, m, k, rows):
+    """The kernel that the row projection takes, as the profiler names it."""
+    code = attn.lib().hipml_dbg_rows_kernel(m, k, rows, 1)
+    kernel, a, b, c = code // 1000000, code // 10000 % 100, code // 100 % 100, code % 100
+    if kernel == 0:
+        return "gemv_q8_rows_kernel"
+    if kernel == 1:
+        return f"gemv_q8_dma_kernel<{a}, {b}, {c}>"
+    return f"gemv_q8_{'blocks' if kernel == 2 else 'units'}_kernel<{a}, {b}, {'true' if c else 'false'}>"
+
+
+# W_o over 672 tokens: 128 x 128 tiles over f16 activations (the tile with this place in the library's table)
+GEMM672_TILE, GEMM672_KERNEL = 11, "gemm_q8_f16_kernel<true, false, 2, 2, 2, 2, 1, 8, 4, false>"
+
+
 def bench_gemv(torch, attn, rows, steps, layers, m=5120, k=6144):
     """Output projection W_o (Q8_0, 6144 -> 5120) over `rows` activation rows, rotating over
     `layers` distinct matrices (33.4 MB each) so the weights come from HBM."""
@@ -812,10 +827,8 @@ def bench_gemv(torch, attn, rows, steps, layers, m=5120, k=6144):
             "roofline": {"bound": "hbm", "achieved": gbs, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                          "frac": gbs / HBM_PEAK_GBS,
                          "traffic": measured_traffic({1: "gemv1", 24: "gemv24"}.get(rows, ""),
-                                                     ["gemv_q8_dma_kernel", "gemv_q8_dma_tile_kernel", "gemv_q8_rows_kernel",
-                                                      "gemv_q8_tile_kernel"]),
-                         "kernel": ("gemv_q8_dma_kernel" if rows <= 8 else
-                                    "gemv_q8_dma_tile_kernel" if rows >= 10 else "gemv_q8_tile_kernel"),
+                                                     [row_kernel_name(attn, m, k, rows)]),
+                         "kernel": row_kernel_name(attn, m, k, rows),
                          "bytes_per_launch": nbytes, "launch_us": us}}
 
 
@@ -836,7 +849,7 @@ def bench_gemm(torch, attn, tokens, steps, layers, m=5120, k=6144, mfma=None):
     us = ms * 1e3
     flop = 2.0 * tokens * m * k
     tf = flop / (us * 1e-6) / 1e12
-    wl = "gemm672" if tokens == 672 else ""
+    wl = "gemm672" if attn.lib().hipml_dbg_gemm_tile(m, k, tokens, 1, 1) == GEMM672_TILE and tokens == 672 else ""
     return {"workload": f"W_o projection of a chunk, Q8_0 {m}x{k}, {tokens} tokens",
             "us_per_layer": us, "timed_ms": total, "steps_timed": n, "us_per_layer_f32_rows_no_gate": t32 * 1e3,
             "flop": flop, "layers_rotated": layers,
@@ -844,8 +857,9 @@ def bench_gemm(torch, attn, tokens, steps, layers, m=5120, k=6144, mfma=None):
                          "frac": tf / MFMA_F16_PEAK_TF,
                          "achievable": None if mfma is None else mfma["tflops"],
                          "frac_of_achievable": None if mfma is None else tf / mfma["tflops"],
-                         **counters(wl, "gemm_q8_f16_kernel<true"),
-                         "traffic": measured_traffic(wl, ["gate_f16_kernel", "gemm_q8_f16_kernel<true"]),
+                         **counters(wl, GEMM672_KERNEL),
+                         "traffic": None if not counters(wl, GEMM672_KERNEL) else
+                                    measured_traffic(wl, ["gate_f16_kernel", GEMM672_KERNEL]),
                          "kernel": "gate_f16_kernel + gemm_q8_f16_kernel",
                          "flop_per_launch": flop, "launch_us": us}}
 

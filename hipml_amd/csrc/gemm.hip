@@ -465,8 +465,8 @@ static int gemm_tile(int m, int k, int tokens, bool sectors, bool x16)
     return best;
 }
 
-// For the tests: the tile (its place in the table) that a call takes.
-extern "C" int hipml_test_gemm_tile(int m, int k, int tokens, int sectors, int x16)
+// For tests and the benchmark: the tile (its place in the table) that a call takes.
+extern "C" int hipml_dbg_gemm_tile(int m, int k, int tokens, int sectors, int x16)
 {
     return gemm_tile(m, k, tokens, sectors != 0, x16 != 0);
 }

@@ -1275,8 +1275,8 @@ static RowsPick pick_tiles(int m, int k, int rows, bool w16)
     const bool blocks = m > 6144 && k % 256 == 0 && w16;
     // the tile that costs least: rounds of 256 workgroups x the cycles of a unit in the eight waves of a CU, as the sum
     // of its vector instructions (two waves a SIMD, 4 cycles each) and its requests (16 cycles).  At ten matrices of 1,024
-    // to 12,288 weight rows over 9 to 128 rows it picks the fastest tile or one within 5 %, but for 9 % at 7,168 weight
-    // rows over 100 (60.3 us, best 55.2)
+    // to 12,288 weight rows over 9 to 128 rows it picks the fastest tile or one within 5 %, but for 7 % at 3,072 weight
+    // rows over 64 (16.2 us, best 15.1) and 9 % at 7,168 over 100 (60.3, best 55.2)
     int xt = 0, rw = 0;
     long long best = 0;
     for (int cx = 1; cx <= (blocks ? 4 : 2) && 16 * (cx - 1) < rows; cx++)
@@ -1370,8 +1370,8 @@ int launch_gemv_q8_rows(hipStream_t st, const uint8_t *w, const float *x, float 
     return launched("gemv_q8_0_rows");
 }
 
-// For the tests: the kernel that a call takes, as kernel * 10^6 + a * 10^4 + b * 100 + c of its RowsPick.
-extern "C" int hipml_test_rows_kernel(int m, int k, int rows, int w_aligned16)
+// For tests and the benchmark: the kernel that a call takes, as kernel * 10^6 + a * 10^4 + b * 100 + c of its RowsPick.
+extern "C" int hipml_dbg_rows_kernel(int m, int k, int rows, int w_aligned16)
 {
     const RowsPick p = pick_rows(m, k, rows, w_aligned16 != 0);
     return p.kernel * 1000000 + p.a * 10000 + p.b * 100 + p.c;

@@ -6,13 +6,13 @@ from hipml_amd import attn
 def row_kernel(m, k, rows):
     """kernel * 10^6 + a * 10^4 + b * 100 + c: 0 the row kernel, 1 raw rows (activation rows a pass, requests, waves), 2
     blocks and 3 units (activation tiles, weight rows, last tile half dead); W at a 16-byte boundary."""
-    return attn.lib().hipml_test_rows_kernel(m, k, rows, 1)
+    return attn.lib().hipml_dbg_rows_kernel(m, k, rows, 1)
 
 
 def gemm_tile(m, k, tokens, x16):
     """(place in the table of tiles, whole sectors of weights), W at a 64-byte boundary."""
     sectors = int(k % 1024 == 0)
-    return attn.lib().hipml_test_gemm_tile(m, k, tokens, sectors, x16), sectors
+    return attn.lib().hipml_dbg_gemm_tile(m, k, tokens, sectors, x16), sectors
 
 
 # (weight rows, k, activation rows): ragged in the rows of a workgroup, k of 19 chunks or 37 units (uneven shares of the
