@@ -91,8 +91,8 @@ int hipml_attn_batch_splits(int stride, int n_kv, int slots);
  * than the number of slices that run (hipml_attn_chunk_slices): the chunk entry points then write the
  * live rows of the cache as f16 tiles (70,656 bytes per KV head and 64 rows) into the tail of part_acc
  * and run the attention over those, which is faster than dequantizing inside the attention (2,048 tokens
- * at depth 100,000: n = 13 for 4 slices, 654 MB of scratch, 4.1 against 4.7 ms).  A caller that passes a
- * smaller n (the reference's own policy gives 8) gets n slices of the kernel that dequantizes for itself:
+ * at depth 100,000: n = 13 for 4 slices, 654 MB of scratch, 4.1 against 4.7 ms).  A caller that passes fewer
+ * than that (the reference's own policy gives 8) gets so many slices of the kernel that dequantizes for itself:
  * the scratch is never written beyond the n slices it was sized for.
  * How that count grows: the partial rows are ceil32(tokens) * n_heads * 1,024 bytes per slice (50.3 MB at
  * 2,048 tokens and 24 heads), the tiles n_kv * ceil((pos0 + tokens) / 64) * 70,656 bytes (4.4 MB per 1,000
@@ -100,7 +100,8 @@ int hipml_attn_batch_splits(int stride, int n_kv, int slots);
  * at depth 32,768 / 100,000 / 200,000 / 400,000: 8 / 13 / 22 / 40, i.e. 0.40 / 0.65 / 1.1 / 2.0 GB.  The
  * reference caps its scratch at 1 GiB (crates/hipml-model/src/gpu/prefill.rs:159-166); an engine that keeps
  * that cap passes the count its allocation holds, and from ~195,000 positions on that is the kernel that
- * dequantizes for itself again.  Counts above 64 are never returned (the plain slice count is, instead).
+ * dequantizes for itself again.  Counts above 64 are never returned (a slice count
+ * for the kernel that dequantizes for itself is, instead).
  * An engine that registers its caches with hipml_kv_f16_attach needs none of this: the tiles then live
  * in the cache's own shadow, the count only has to cover the slices that run (hipml_attn_chunk_slices:
  * 4 at these shapes), and 8 is always enough.
@@ -507,13 +508,13 @@ int hipml_kv_rows_copy(hipml_stream_t stream, int dtype, const void *k_src, cons
  * [rows][m]; k a multiple of 64 up to 32768, 1 <= rows <= 128.
  * fp32 accumulation of exact integer block products (the activations enter as hi + lo f16 halves), so
  * every row has the precision class of the reference's f32 GEMV kernels.  Finite activations are taken up to a
- * magnitude of 131,008 (two f16 halves; ~22 bits up to 65,504, to the nearest 32 above) and as that value beyond.  Up to 8 rows W streams from
- * memory once and a row's result has the same bits whatever `rows` is and whichever rows travel with it:
- * the rows of a verify group match their plain decodes, as the reference's batched GEMVs do
- * (crates/hipml-kernels/src/attn_gpu.rs:930-932).  From 10 to 128 rows W streams once per pass of up to 64 rows
- * (two passes beyond 64) and a row's bits are the same for every such `rows`; 9 rows take a kernel of their own.
- * The three classes differ from each other in the last bits.
- * (W at a 16-byte aligned address and k a multiple of 256 take the fastest road.)
+ * magnitude of 131,008 (two f16 halves; ~22 bits up to 65,504, to the nearest 32 above) and as that value beyond.  Up to 8
+ * rows W streams from memory once and a row's result has the same bits whatever `rows` is and whichever rows travel with
+ * it: the rows of a verify group match their plain decodes, as the reference's batched GEMVs do
+ * (crates/hipml-kernels/src/attn_gpu.rs:930-932).  From 9 to 128 rows W streams once per pass of 16 to 64 rows, and a row's
+ * bits are the same for every such `rows`.  The two classes differ from each other in the last bits.  (W at a 16-byte
+ * aligned address and k a multiple of 256 take the fastest road; where they do not, 1 and 2 rows are a class of their own
+ * and 3 to 8 belong to the second.)
  * Replaces AttnLayer::gemv / gemv_rows / gemv_batched over a Q8_0 ResidentMat (the output
  * projection of apply_output / output_rows, and W_q, W_k, W_v in prepare_rows),
  * crates/hipml-kernels/src/attn_gpu.rs:843-846,967-1023,1066-1117 -> gemv_q8_0 / gemv_q8_0_b,
