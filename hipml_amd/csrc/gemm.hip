@@ -23,7 +23,7 @@
 //    all of them stage first and four records cover the loads (5120 x 6144 over 512 / 672 tokens 50.8 -> 47.5 / 62.6 ->
 //    58.6 us).
 //  * small tiles with longer steps (KU 2 and 4) and eight producer waves where there are too few outputs for large
-//    ones: a step's cost is then latency, not work (1024 x 5120 over 117 tokens: 32 x 32 tiles 15 us, 128 x 128 48 us).
+//    ones: a step's cost is then latency, not work (1024 x 5120 over 117 tokens: 32 x 32 tiles 16 us, 128 x 128 44 us).
 //  * weights by whole 64-byte sectors, one aligned request of a quad of lanes each, where their rows allow it.  A row's
 //    pair of blocks is 68 bytes: asked for as it lies (12 and 8 bytes a lane) it takes three requests, most of them
 //    across a sector boundary, and the weights of a step cost the vector memory path as much as the activations

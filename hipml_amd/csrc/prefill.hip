@@ -2117,7 +2117,8 @@ int chunk_tiles_splits(int pos0, int tokens, int n_head, int n_kv, int slices)
 // under to 25 % over).  us with the filling count / with this one: 1,024 tokens at depth 8,192 255 (8 slices) / 222 (2),
 // 1,500 at 20,000 829 (12) / 688 (3), 700 at 10,000 226 (10) / 186 (3), 800 at 40,000 709 (10) / 669 (3), 2,048 at 2,048
 // 219 (4) / 204 (2); 672 at 8,192 and 2,048 at 100,000 keep their 4.  Only counts for which every block of tokens gets all
-// slices and the 64-token kernel runs.
+// slices and the 64-token kernel runs (and none above `most`: 1,024 at 1,024 takes 74 us with its 2, 67 with 3 slices of the
+// other kernel).
 int chunk_tile_slices(int pos0, int tokens, int n_head, int n_kv, int most)
 {
     const int group = n_head / n_kv, tiles = (pos0 + tokens + kKTile - 1) / kKTile;

@@ -23,7 +23,7 @@
 //   The waves of a workgroup split k; a wave requests the activations first, then two chunks of
 //   its weight blocks (all of them for k = 6144) before it waits for anything, and the partial sums
 //   meet in LDS in a fixed order (no atomics: the result does not depend on timing).
-// gemv_q8_dma_kernel: one to eight rows; gemv_q8_blocks_kernel: more (both further down).
+// gemv_q8_dma_kernel: one to eight rows; gemv_q8_units_kernel, gemv_q8_blocks_kernel: more (all further down).
 
 #include "q8_weights.h"
 
