@@ -797,7 +797,7 @@ def row_kernel_name(attn, m, k, rows):
     if kernel == 0:
         return "gemv_q8_rows_kernel"
     if kernel == 1:
-        return f"gemv_q8_dma_kernel<{a}, {b}, {c}>"
+        return f"gemv_q8_digits_kernel<{a}, {b}>"
     return f"gemv_q8_{'blocks' if kernel == 2 else 'units'}_kernel<{a}, {b}, {'true' if c else 'false'}>"
 
 

@@ -23,7 +23,7 @@
 //   The waves of a workgroup split k; a wave requests the activations first, then two chunks of
 //   its weight blocks (all of them for k = 6144) before it waits for anything, and the partial sums
 //   meet in LDS in a fixed order (no atomics: the result does not depend on timing).
-// gemv_q8_dma_kernel: one to eight rows; gemv_q8_units_kernel, gemv_q8_blocks_kernel: more (all further down).
+// gemv_q8_digits_kernel: one to eight rows; gemv_q8_units_kernel, gemv_q8_blocks_kernel: more (all further down).
 
 #include "q8_weights.h"
 
@@ -292,35 +292,40 @@ __global__ void __launch_bounds__(64 * WAVES, TILES == 1 ? 2 : 1) gemv_q8_rows_k
     }
 }
 
-// ---- gemv_q8_dma_kernel: one to eight activation rows, the weight rows moved into LDS as they lie in memory ----
+// ---- gemv_q8_digits_kernel: one to eight activation rows, int8 matrix instructions over the weights as they are ----
 //
-// The row kernel above asks for its weights in 12- and 8-byte pieces per lane, which the memory pipeline serves
-// at 10.0 us for the 33.4 MB of a 5120 x 6144 matrix; the same bytes as whole pieces of rows through
-// global_load_lds_dwordx4 need no registers while they travel and arrive sooner.  A workgroup takes `rows_wg`
-// consecutive weight rows (m / 256 where that is 16..32: one workgroup per CU and every CU the same bytes; one or
-// two MFMA tiles of 16 rows); its waves deal the rows' chunks of 256 values (8 blocks, 272 bytes: the smallest
-// piece of a row that starts and ends at a 16-byte boundary) round-robin, and a wave keeps two chunks in flight
-// into a ring of two buffers.  Nothing is shared between the waves until their sums meet, so the loop has no
-// barrier.
-// The activations take the same road as raw f32 and become MFMA operands in place (the 128 bytes of a block's 32
-// floats of one row become 64 bytes of f16 hi halves and 64 of lo halves, x = hi + lo to ~22 bits): with one row,
-// all of a wave's chunks before the loop, while the first weights travel; with more rows, a chunk's values ride
-// behind its weights in the ring and are converted when the chunk has arrived.
-// One v_mfma_f32_16x16x32_f16 per block and tile with A = activations (A rows 0..7 the hi halves of rows 0..7, A
-// rows 8..15 the lo halves), B = 16 weight rows.  Lane (lm, lg) reads its 8 bytes of weight row lm, quarter lg of
-// the block, from the raw rows with dword-aligned reads (even blocks sit 2 bytes past a boundary and are
-// realigned; LDS reads at 2-byte alignment measured four times slower).  The weight bytes enter the MFMA as the
-// f16 subnormals (b + 128) x 2^-24, one v_perm_b32 per pair: exact, and the offset 128 comes out again as
-// 128 x 2^-24 x (sum of the block's activation halves), a number the wave forms once per block and chunk.  The
-// block's scale multiplies the corrected fp32 dot product, as the CPU definition's d * q products summed in
-// fp32; 2^24 multiplies the final sum.
-// A (row, weight row) result is the sum, in a fixed order, of eight chains (chunk c belongs to chain c % 8, a
-// chain adds its blocks in order), hi and lo halves apart until the end: the same operations in the same order
-// whatever RP, the wave count and rows_wg are and whichever rows travel with it, so a verify group's rows have the
-// bits of their plain decodes (crates/hipml-kernels/src/attn_gpu.rs:930-932).
-constexpr int kDmaChunkBytes = 8 * kQ8Block; // 272: one row's share of a chunk
-constexpr int kDmaChains = 8;
-constexpr float kTwo24f = 16777216.0f;
+// (a result) = sum over blocks of d * (sum of q x over the block).  The activations of a block become whole numbers: x =
+// s X with s a power of two and |X| < 2^30, so that the block's largest value keeps all its 24 bits and every other one is
+// cut at 2^-30 of it; X = X0 + 256 X1 + 65536 X2 + 2^24 X3 with digits in [-128, 127].  v_mfma_i32_16x16x64_i8 then
+// multiplies the weight bytes as they lie in memory with the digits, exactly, and a block's four digit sums become one
+// float.  Compared with f16 operands (x = hi + lo, the bytes made f16 numbers first) that is a third of the vector
+// instructions for one row and half of them for four.
+//
+// B operand (weights): lane (lm, lg) holds 16 bytes of weight row lm, block lg of a group of four, so that a lane reads its
+// whole block at once (9 dwords from the first dword boundary, realigned by v_perm_b32; the scale is among them).  A operand
+// (activations): row 4 b + i is digit i of block b and holds zeros for the other three blocks, so that the contraction
+// over the lanes lg keeps the blocks apart: C row 4 lg + j, digit j of block lg, meets in lane (lm, lg) the block's scale
+// that this lane has read.  A lane's sum is thus one float for its weight row, its blocks and an activation row.
+// Three and four activation rows fill the operand without zeros: v_mfma_i32_16x16x32_i8 over one block, A row 4 r + i digit
+// i of row r, lane (lm, lg) holding 8 bytes of weight row lm and, in C, the digit sums of activation row lg; it adds the
+// blocks 0 .. 3 of a group of four apart, as the lanes lg above do, so that a row's bits are the same.
+//
+// A workgroup takes `ng` groups of GR weight rows (up to 16).  Wave v of V owns the runs v, v + V, ... of 512 values of k (544
+// bytes of each row: with runs of 272 a pass over 12288 x 5120 reads 1 us slower) for all of them, makes the digits of its
+// activations while its first weights travel, and then streams the groups' rows of its run through a place of its own by
+// global_load_lds_dwordx4: a group's bytes move to registers, the next group is asked for, and the registers are
+// multiplied.  Nothing is shared between the waves until their sums meet, so there is no barrier before that.
+// A result is the sum over the waves in order, of which each adds its runs in order, blocks 0 .. 3 of a group of four apart
+// and (0 + 2) + (1 + 3) behind them; V follows from k: the same operations in the same order whatever R is and whichever rows travel with it, so a
+// verify group's rows have the bits of their plain decodes (crates/hipml-kernels/src/attn_gpu.rs:930-932).
+constexpr int kChunkBytes = 8 * kQ8Block; // 272: a row's share of 256 values, which starts and ends at a 16-byte boundary
+constexpr int kRunBytes = 2 * kChunkBytes;
+constexpr int kDigitLds = 160 << 10;
+constexpr int kDigitMaxWaves = 12;
+
+typedef int int4v __attribute__((ext_vector_type(4)));
+typedef uint32_t uint2v __attribute__((ext_vector_type(2)));
+typedef uint32_t uint4a4 __attribute__((ext_vector_type(4), aligned(4)));
 
 __device__ __forceinline__ uint32_t proj_lds_address(const void *p)
 {
@@ -350,328 +355,346 @@ __device__ __forceinline__ void wait_vm()
     asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory");
 }
 
-// 8 int8 (two dwords) -> 8 f16 subnormals (b + 128) x 2^-24, exactly
-__device__ __forceinline__ half8 int8x8_to_f16_sub(uint32_t w0, uint32_t w1)
+
+
+// LDS of a wave: a group's rows of a run; the digits of its activations of the run, 2 KB a row, and their scales (four rows
+// exchange those by ds_bpermute: they leave no room for the table), whose place takes the wave's sums when they are in
+// registers, unless a wave has several runs; behind the waves 64 zero bytes.
+constexpr int gemv_digit_x(int r) { return (r < 4 ? 2048 + 64 : 2048) * r; }
+constexpr int gemv_digit_wave(int r, int gr, int ng, bool more)
 {
-    const uint32_t x0 = w0 ^ 0x80808080u, x1 = w1 ^ 0x80808080u;
-    uint4v r;
-    r[0] = __builtin_amdgcn_perm(0u, x0, 0x0c010c00u);
-    r[1] = __builtin_amdgcn_perm(0u, x0, 0x0c030c02u);
-    r[2] = __builtin_amdgcn_perm(0u, x1, 0x0c010c00u);
-    r[3] = __builtin_amdgcn_perm(0u, x1, 0x0c030c02u);
-    return __builtin_bit_cast(half8, r);
+    const int sums = ng * r * 64, x = gemv_digit_x(r);
+    return gr * kRunBytes + (more ? x + sums : (x > sums ? x : sums));
+}
+static_assert(kDigitMaxWaves * gemv_digit_wave(4, 4, 12, true) + 64 <= kDigitLds, "groups of four rows always fit");
+
+// acc + ds * (p[0] + 2^8 p[1] + 2^16 p[2] + 2^24 p[3]); a digit sum is at most 2^19, so that both pairs are exact
+__device__ __forceinline__ float add_digits(const int4v &p, float ds, float acc)
+{
+    const float lo = (float)(p[0] + p[1] * 256), hi = (float)(p[2] + p[3] * 256);
+    return fmaf(fmaf(hi, 65536.0f, lo), ds, acc);
 }
 
-// The variants: RP activation rows per pass on WAVES waves; NI requests of 64 x 16 bytes per chunk of weights
-// (rows_wg x 17 pieces), which also says how many 16-row tiles cover rows_wg.
-constexpr bool gemv_dma_front(int rp) { return rp == 1; }
-constexpr int gemv_dma_tiles(int ni) { return ni > 5 ? 2 : 1; }
-constexpr int gemv_dma_rows(int ni) { return 4 * (ni - 1); } // weight rows of a workgroup, as the rule below picks them
-constexpr int kDmaDepth = 2; // chunks in flight per wave (three measured no faster)
-// a ring entry: the chunk's weights as they arrive (rows_wg x 272 bytes) and, behind them, its activations
-constexpr int gemv_dma_entry(int rp, int rows_wg) { return rows_wg * kDmaChunkBytes + (gemv_dma_front(rp) ? 0 : rp * 1024); }
-constexpr int gemv_dma_lds(int rp, int ni, int waves, int rows_wg, int k)
+// s + the s of lane ^ 16, and of lane ^ 32
+__device__ __forceinline__ float sum_lanes16(float s)
 {
-    const int per_wave = ((k >> 8) + waves - 1) / waves; // chunks of a wave
-    // rings (at least the 1 KB per chain and tile in which the chains' sums meet at the end); front: the waves'
-    // activations, 1 KB per chunk; the waves' offset tables [8 blocks][2 rp] floats per chunk (front: every chunk,
-    // else the ring's two)
-    int ring = kDmaDepth * gemv_dma_entry(rp, rows_wg);
-    const int sums = kDmaChains / waves * gemv_dma_tiles(ni) * 64 * 16;
-    ring = ring > sums ? ring : sums;
-    return waves * ring + (gemv_dma_front(rp) ? waves * per_wave * (1024 + 64) : waves * 2 * 64 * rp);
+    const auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, s), __builtin_bit_cast(uint32_t, s), false, false);
+    return __builtin_bit_cast(float, (uint32_t)r[0]) + __builtin_bit_cast(float, (uint32_t)r[1]);
+}
+__device__ __forceinline__ float sum_lanes32(float s)
+{
+    const auto r = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, s), __builtin_bit_cast(uint32_t, s), false, false);
+    return __builtin_bit_cast(float, (uint32_t)r[0]) + __builtin_bit_cast(float, (uint32_t)r[1]);
 }
 
-template <int RP, int NI, int WAVES>
-__global__ void __launch_bounds__(64 * WAVES, 1) gemv_q8_dma_kernel(const uint8_t *__restrict__ w,
-                                                                                 const float *__restrict__ x,
-                                                                                 float *__restrict__ y, int m, int k,
-                                                                                 int rows, int rows_wg)
+template <int R, int GR>
+__global__ void __launch_bounds__(64 * kDigitMaxWaves) gemv_q8_digits_kernel(const uint8_t *__restrict__ w,
+                                                                             const float *__restrict__ x,
+                                                                             float *__restrict__ y, int m, int k, int rows,
+                                                                             int ng)
 {
-    static_assert(RP == 1 || RP == 2 || RP == 4 || RP == 8, "activation rows per pass");
-    static_assert(WAVES == 4 || WAVES == 8, "the eight chains are dealt to four or eight waves");
-    constexpr int kWaves = WAVES;
-    constexpr int kNCh = kDmaChains / kWaves; // chains of a wave
-    constexpr int kNT = gemv_dma_tiles(NI);
-    constexpr bool kFront = gemv_dma_front(RP);
-    constexpr int kDepth = kDmaDepth;
-    constexpr int kReq = NI + (kFront ? 0 : RP); // requests per chunk
-    constexpr int kNJ = RP < 4 ? RP : 4;         // accumulator rows a lane needs
-    constexpr int kUnits = 32 * RP;              // (block, row, quarter) units of 8 activations per chunk
-    constexpr int kPasses = (kUnits + 63) / 64;
+    constexpr int kPerRow = kRunBytes / 16, kPieces = GR * kPerRow; // 16-byte pieces of a unit: a group's rows of a run
+    constexpr int NI = (kPieces + 63) / 64;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int waves = (int)(blockDim.x >> 6);
     const int lane = threadIdx.x & 63;
     const int lm = lane & 15, lg = lane >> 4;
-    const int nb = k >> 5;
-    const int nchunk = nb >> 3;
-    const uint32_t row_bytes = (uint32_t)nb * kQ8Block;
-    const int m0 = blockIdx.x * rows_wg;
-    const int r0 = blockIdx.y * RP;
-    const int nrows = rows - r0 < RP ? rows - r0 : RP;
-    const int pieces = rows_wg * 17;
-    if ((pieces + 63) / 64 != NI)
-        return; // (the launcher's contract: the waits below count NI requests per chunk of weights)
-    const int mine = wave < nchunk ? (nchunk - wave + kWaves - 1) / kWaves : 0; // chunks wave, wave + kWaves, ...
-    const int per_wave = (nchunk + kWaves - 1) / kWaves;
+    const int nchunk = k >> 8, nrun = (nchunk + 1) >> 1;
+    const uint32_t row_bytes = (uint32_t)(k >> 5) * kQ8Block;
+    const int m0 = blockIdx.x * (ng * GR);
+    const int r0 = blockIdx.y * R;
+    const int nrows = rows - r0 < R ? rows - r0 : R;
+    const bool more = nrun > waves;
+    const int area = gemv_digit_wave(R, GR, ng, more);
+    uint8_t *const place = lds + wave * area;
+    uint8_t *const xdig = place + kPieces * 16; // [chunk][row][block][digit][32], then the scales [chunk][row][block]
+    uint32_t *const scales = reinterpret_cast<uint32_t *>(xdig + 2048 * R);
+    auto sums_of = [&](int v) { return reinterpret_cast<float *>(lds + v * area + kPieces * 16 + (more ? gemv_digit_x(R) : 0)); };
+    uint8_t *const zeros = lds + waves * area;
+    const uint32_t place_at = proj_lds_address(place), xdig_at = proj_lds_address(xdig);
+    const uint8_t *const xb = reinterpret_cast<const uint8_t *>(x + (size_t)r0 * k);
 
-    const int entry = pieces * 16 + (kFront ? 0 : RP * 1024);
-    constexpr int kSums = kNCh * kNT * 64 * 16; // where this wave's chains leave their sums: the head of its ring
-    const int ring_bytes = kDepth * entry > kSums ? kDepth * entry : kSums;
-    uint8_t *ring = lds + wave * ring_bytes;
-    uint8_t *xfront = lds + kWaves * ring_bytes + wave * per_wave * 1024; // (front only)
-    uint8_t *after_x = lds + kWaves * ring_bytes + (kFront ? kWaves * per_wave * 1024 : 0);
-    float *offs = reinterpret_cast<float *>(after_x + wave * (kFront ? per_wave * 64 : 2 * 64 * RP));
-    const uint32_t ring_at = proj_lds_address(ring);
-
-    // ---- requests ---------------------------------------------------------------------------------------------
-    // weights: piece p = 64 j + lane of the chunk: row p / 17 of the workgroup, 16 bytes p % 17 of its 272; rows
-    // past the end of the matrix repeat the last one (never stored)
+    // ---- requests (a chunk past the end of k repeats the one before it, rows past the end the last: never used) ----------
+    auto issue_x = [&](int run) {
+#pragma unroll
+        for (int cc = 0; cc < 2; cc++) {
+            const int c = 2 * run + cc < nchunk ? 2 * run + cc : nchunk - 1;
+#pragma unroll
+            for (int r = 0; r < R; r++)
+                proj_dma16<false>(xdig_at + (cc * R + r) * 1024u, xb + (size_t)(r < nrows ? r : nrows - 1) * ((size_t)k * 4) + (size_t)c * 1024,
+                                  lane * 16u);
+        }
+    };
+    // piece p = 64 j + lane of a unit: row p / kPerRow of the group, 16 bytes p % kPerRow of its run
     uint32_t woff[NI];
 #pragma unroll
     for (int j = 0; j < NI; j++) {
-        const int p = j * 64 + lane;
-        const int pr = p / 17, pq = p - pr * 17;
-        const int row = m0 + pr < m ? m0 + pr : m - 1;
-        woff[j] = (uint32_t)row * row_bytes + (uint32_t)pq * 16u;
+        const uint32_t p = (uint32_t)(j * 64 + lane), pr = p / (uint32_t)kPerRow;
+        woff[j] = pr * row_bytes + (p - pr * kPerRow) * 16u;
     }
-    const uint8_t *xb = reinterpret_cast<const uint8_t *>(x + (size_t)r0 * k);
-    auto issue = [&](int i) {
-        const uint32_t at = ring_at + (uint32_t)((i % kDepth) * entry);
-        const uint32_t c = (uint32_t)(wave + i * kWaves);
-        // activations behind the weights: one request per row, its 256 floats of the chunk as they lie in memory;
-        // rows past the live ones repeat the last
-        if (!kFront) {
+    auto issue_w = [&](int run, int g) {
+        const int row = m0 + g * GR < m ? m0 + g * GR : m - 1;
+        const uint8_t *const src = w + (size_t)row * row_bytes + (size_t)run * kRunBytes;
+        if (row + GR <= m && 2 * run + 2 <= nchunk) {
 #pragma unroll
-            for (int r = 0; r < RP; r++) {
-                const uint32_t rr = (uint32_t)(r < nrows ? r : nrows - 1);
-                proj_dma16<false>(at + pieces * 16 + r * 1024, xb, rr * (uint32_t)k * 4u + c * 1024u + lane * 16u);
+            for (int j = 0; j < NI; j++)
+                if ((j + 1) * 64 <= kPieces || j * 64 + lane < kPieces)
+                    proj_dma16<true>(place_at + j * 1024, src, woff[j]);
+        } else {
+            int l = lane;
+            asm volatile("" : "+v"(l)); // (what follows is worked out here, where it is seldom needed, and not kept in registers)
+#pragma unroll
+            for (int j = 0; j < NI; j++) {
+                const uint32_t p = (uint32_t)(j * 64 + l), pr = p / (uint32_t)kPerRow, pq = p - pr * kPerRow;
+                const int past = row + (int)pr - (m - 1);
+                const uint32_t back = (past > 0 ? (uint32_t)past * row_bytes : 0u) + (2 * run + 2 > nchunk && pq >= 17 ? kChunkBytes : 0);
+                if ((j + 1) * 64 <= kPieces || j * 64 + lane < kPieces)
+                    proj_dma16<true>(place_at + j * 1024, src, woff[j] - back);
             }
         }
-        // (NI = ceil(pieces / 64): every request has a live lane, so each chunk counts NI requests)
-#pragma unroll
-        for (int j = 0; j < NI; j++) {
-            if (j * 64 + lane < pieces)
-                proj_dma16<true>(at + j * 1024, w, woff[j] + c * kDmaChunkBytes);
-        }
     };
-    if (kFront) {
-        for (int i = 0; i < mine; i++)
-            proj_dma16<false>(proj_lds_address(xfront) + i * 1024, xb, (uint32_t)(wave + i * kWaves) * 1024u + lane * 16u);
+    if (wave < nrun) {
+        issue_x(wave);
+        issue_w(wave, 0);
     }
-#pragma unroll
-    for (int i = 0; i < kDepth; i++)
-        if (i < mine)
-            issue(i);
-    // all but the newest `newer` chunks (at most kDepth - 1) have arrived: requests return in order
-    auto wait_chunks = [&](int newer) {
-        if (newer >= 2 && kDepth > 2)
-            wait_vm<(kDepth > 2 ? 2 : 0) * kReq>();
-        else if (newer >= 1)
-            wait_vm<kReq>();
+    if (lane < 16) // (every wave writes the same zeros)
+        reinterpret_cast<uint32_t *>(zeros)[lane] = 0;
+
+    constexpr bool kDense = R > 2, kTable = R < 4;
+    // (not dense) lanes lg = 0 .. 3 take the blocks 0, 2, 1, 3 of a group of four: their first dwords then start in different
+    // banks; payload dwords start 2 bytes into the first dword, or at the next; A row lm is a digit of the block of lanes
+    // lm / 4.  (Rows past a group's repeat its last: never stored.)
+    const uint32_t odd = (uint32_t)lg >> 1;
+    const int blk = 2 * (lg & 1) + (int)odd;
+    const uint32_t pick = odd ? 0x07060504u : 0x05040302u;
+    const bool live = (lm >> 2) == lg;
+    const uint8_t *const wrow = place + (lm < GR ? lm : GR - 1) * kRunBytes;
+    const uint8_t *const wlane = kDense ? wrow + lg * 8 : wrow + blk * kQ8Block - 2 * (int)odd;
+    const uint8_t *const xlane = kDense  ? xdig + ((lm >> 2) < R ? lm >> 2 : R - 1) * 1024 + (lm & 3) * 32 + lg * 8
+                                 : live ? xdig + blk * 128 + (lm & 3) * 32
+                                        : zeros;
+    const int xstep = kDense || live ? 1 : 0;
+
+    for (int run = wave; run < nrun; run += waves) {
+        const bool two = 2 * run + 1 < nchunk; // (the last run may be one chunk)
+        if (run == wave)
+            wait_vm<NI>(); // (the first weights are still travelling)
         else
             wait_vm<0>();
-    };
-
-    // ---- activations -> operands, in place: unit ((block b, row r), quarter q): 8 floats -> 8 hi and 8 lo halves in
-    // the operand order of the block, and the block's offset terms.  Every unit of an area is read before any is
-    // written (one wave, LDS in program order).
-    auto unit_write = [&](uint8_t *area, float *off, int b, int r, int q, bool on, const float4v &a4, const float4v &b4) {
-        half8 hi, lo;
-        split_hi_lo(a4, b4, hi, lo);
-        float sh = 0.0f, sl = 0.0f;
+        // ---- digits, in place: four values a lane, eight lanes a block ----------------------------------------------
+        float4v f[2 * R];
 #pragma unroll
-        for (int e = 0; e < 8; e++) {
-            sh += (float)hi[e];
-            sl += (float)lo[e];
-        }
-        // over the unit's four quarters (the lanes of a quad)
-        sh += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, sh), 0xB1, 0xf, 0xf, true));
-        sl += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, sl), 0xB1, 0xf, 0xf, true));
-        sh += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, sh), 0x4E, 0xf, 0xf, true));
-        sl += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, sl), 0x4E, 0xf, 0xf, true));
-        if (on) {
-            uint8_t *blk = area + b * (RP * 128) + q * 16;
-            *reinterpret_cast<half8 *>(blk + r * 64) = hi;
-            *reinterpret_cast<half8 *>(blk + (RP + r) * 64) = lo;
-            if (q == 0) {
-                off[b * 2 * RP + r] = sh * (128.0f / kTwo24f);
-                off[b * 2 * RP + RP + r] = sl * (128.0f / kTwo24f);
+        for (int e = 0; e < 2 * R; e++)
+            f[e] = *reinterpret_cast<const float4v *>(xdig + e * 1024 + lane * 16);
+        asm volatile("" ::: "memory"); // (one wave: every lane has read before any writes)
+        __builtin_amdgcn_wave_barrier();
+        uint32_t sbits[kTable ? 1 : 2 * R]; // of block lane / 8
+#pragma unroll
+        for (int e = 0; e < 2 * R; e++) {
+            uint32_t b[4];
+            float v[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                v[i] = f[e][i]; // (__builtin_bit_cast of a vector's element itself takes element 0)
+                b[i] = __builtin_bit_cast(uint32_t, v[i]) & 0x7fffffffu;
             }
-        }
-    };
-    if (kFront) {
-        // two chunks per pass: lanes 0..31 the units of chunk 2 ps, lanes 32..63 those of chunk 2 ps + 1
-        constexpr int kFrontPasses = 2;
-        // only weights are still travelling
-        if (mine >= 2)
-            wait_vm<2 * NI>();
-        else
-            wait_vm<NI>();
-        for (int i0 = 0; i0 < mine; i0 += 2 * kFrontPasses) {
-            float4v a4[kFrontPasses], b4[kFrontPasses];
+            // the block's largest magnitude, as bits (infinities and NaN above all numbers)
+            uint32_t top = b[0] > b[1] ? b[0] : b[1];
+            top = top > b[2] ? top : b[2];
+            top = top > b[3] ? top : b[3];
+            uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)top, 0xB1, 0xf, 0xf, true); // lane ^ 1
+            top = o > top ? o : top;
+            o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)top, 0x4E, 0xf, 0xf, true); // lane ^ 2
+            top = o > top ? o : top;
+            o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)top, 0x141, 0xf, 0xf, true); // lane 7 - i of eight
+            top = o > top ? o : top;
+            const uint32_t most = 0x47ffe000u; // 131,008: beyond it activations count as that much
+            uint32_t bad = 0;
+            if (__builtin_amdgcn_ballot_w64(top > most) != 0) { // (in no block of the wave, as a rule)
+                bad = top >= 0x7f800000u ? 0x7fc00000u : 0u;
+                top = top < most ? top : most;
 #pragma unroll
-            for (int ps = 0; ps < kFrontPasses; ps++) {
-                const int i = i0 + 2 * ps + (lane >> 5);
-                const uint8_t *src = xfront + (i < mine ? i : 0) * 1024 + (lane & 31) * 32;
-                a4[ps] = *reinterpret_cast<const float4v *>(src);
-                b4[ps] = *reinterpret_cast<const float4v *>(src + 16);
+                for (int i = 0; i < 4; i++)
+                    v[i] = __builtin_amdgcn_fmed3f(v[i], -131008.0f, 131008.0f);
             }
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-            __builtin_amdgcn_wave_barrier();
+            uint32_t ex = top & 0x7f800000u; // |x| < 2^(ex - 126)
+            ex = ex > (30u << 23) ? ex : 30u << 23;
+            const float up = __builtin_bit_cast(float, (283u << 23) - ex); // 2^(156 - ex)
+            uint32_t z[4];
 #pragma unroll
-            for (int ps = 0; ps < kFrontPasses; ps++) {
-                const int i = i0 + 2 * ps + (lane >> 5);
-                unit_write(xfront + i * 1024, offs + i * 16, (lane & 31) >> 2, 0, lane & 3, i < mine, a4[ps], b4[ps]);
+            for (int i = 0; i < 4; i++) // X + 0x808080: the three low digits, each 128 up, and the fourth
+                z[i] = (uint32_t)(int)fmaf(v[i], up, 8421504.0f);
+            const uint32_t p0 = __builtin_amdgcn_perm(z[1], z[0], 0x05010400u), p1 = __builtin_amdgcn_perm(z[3], z[2], 0x05010400u);
+            const uint32_t p2 = __builtin_amdgcn_perm(z[1], z[0], 0x07030602u), p3 = __builtin_amdgcn_perm(z[3], z[2], 0x07030602u);
+            uint32_t *const dst = reinterpret_cast<uint32_t *>(xdig + e * 1024 + (lane >> 3) * 128 + (lane & 7) * 4);
+            dst[0] = __builtin_amdgcn_perm(p1, p0, 0x05040100u) ^ 0x80808080u;
+            dst[8] = __builtin_amdgcn_perm(p1, p0, 0x07060302u) ^ 0x80808080u;
+            dst[16] = __builtin_amdgcn_perm(p3, p2, 0x05040100u) ^ 0x80808080u;
+            dst[24] = __builtin_amdgcn_perm(p3, p2, 0x07060302u);
+            const uint32_t scale = (ex - (29u << 23)) | bad; // 2^(ex - 156), or NaN
+            if (!kTable)
+                sbits[kTable ? 0 : e] = scale;
+            else if ((lane & 7) == 0)
+                scales[e * 8 + (lane >> 3)] = scale;
+        }
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_wave_barrier();
+        int4v a[kDense ? 1 : 2 * R][2][2];
+        uint2v ad[kDense ? 2 : 1][8];
+        float sx[kDense ? 2 : 2 * R][kDense ? 8 : 2];
+        if constexpr (kDense) {
+#pragma unroll
+            for (int cc = 0; cc < 2; cc++)
+#pragma unroll
+                for (int q = 0; q < 8; q++) {
+                    ad[cc][q] = *reinterpret_cast<const uint2v *>(xlane + cc * (R * 1024) + q * 128);
+                    uint32_t t; // of row lg
+                    if constexpr (kTable) {
+                        t = scales[(cc * R + (lg < R ? lg : R - 1)) * 8 + q];
+                    } else {
+                        t = (uint32_t)__builtin_amdgcn_ds_bpermute(q * 32, (int)sbits[cc * R]);
+#pragma unroll
+                        for (int r = 1; r < R; r++) {
+                            const uint32_t u = (uint32_t)__builtin_amdgcn_ds_bpermute(q * 32, (int)sbits[cc * R + r]);
+                            t = lg == r ? u : t;
+                        }
+                    }
+                    sx[cc][q] = __builtin_bit_cast(float, t);
+                }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 2 * R; e++)
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+#pragma unroll
+                    for (int j = 0; j < 2; j++)
+                        a[e][h][j] = *reinterpret_cast<const int4v *>(xlane + (e * 1024 + h * 512) * xstep + j * 16);
+                    sx[e][h] = __builtin_bit_cast(float, scales[e * 8 + h * 4 + blk]);
+                }
+        }
+        // ---- the groups ---------------------------------------------------------------------------------------------
+#pragma unroll 1
+        for (int g = 0; g < ng; g++) {
+            wait_vm<0>();
+            auto ask = [&]() { // the unit, and the activations before it, are in registers
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+                if (g + 1 < ng) {
+                    issue_w(run, g + 1);
+                } else if (run + waves < nrun) {
+                    issue_x(run + waves);
+                    issue_w(run + waves, 0);
+                }
+            };
+            if constexpr (kDense) {
+                float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f}; // blocks 0 .. 3 of a group of four
+#pragma unroll
+                for (int cc = 0; cc < 2; cc++) {
+                    uint32_t q0[8], q1[8], q2[4];
+                    _Float16 dh[8];
+#pragma unroll
+                    for (int q = 0; q < 8; q++) {
+                        const uint8_t *const src = wlane + cc * kChunkBytes + q * kQ8Block;
+                        if ((q & 1) == 0) { // (the lane's 8 bytes start 2 bytes past a dword boundary)
+                            const uint3a4 v = *reinterpret_cast<const uint3a4 *>(src);
+                            q0[q] = v[0];
+                            q1[q] = v[1];
+                            q2[q >> 1] = v[2];
+                        } else {
+                            const uint2a4 v = *reinterpret_cast<const uint2a4 *>(src + 2);
+                            q0[q] = v[0];
+                            q1[q] = v[1];
+                        }
+                        dh[q] = *reinterpret_cast<const _Float16 *>(wrow + cc * kChunkBytes + q * kQ8Block);
+                    }
+                    if (cc == 1) {
+                        ask();
+                        if (!two)
+                            break;
+                    }
+#pragma unroll
+                    for (int q = 0; q < 8; q++) {
+                        uint2v v = {q0[q], q1[q]};
+                        if ((q & 1) == 0) {
+                            v[0] = __builtin_amdgcn_alignbit(q1[q], q0[q], 16);
+                            v[1] = __builtin_amdgcn_alignbit(q2[q >> 1], q1[q], 16);
+                        }
+                        int4v p = {0, 0, 0, 0};
+                        p = __builtin_amdgcn_mfma_i32_16x16x32_i8(__builtin_bit_cast(long, ad[cc][q]), __builtin_bit_cast(long, v), p, 0, 0, 0);
+                        acc[q & 3] = add_digits(p, (float)dh[q] * sx[cc][q], acc[q & 3]);
+                    }
+                }
+                const float s = (acc[0] + acc[2]) + (acc[1] + acc[3]);
+                float *const to = sums_of(wave) + (g * R + lg) * 16 + lm;
+                if (lg < R)
+                    *to = run == wave ? s : *to + s;
+            } else {
+                float acc[R];
+#pragma unroll
+                for (int r = 0; r < R; r++)
+                    acc[r] = 0.0f;
+#pragma unroll
+                for (int cc = 0; cc < 2; cc++) {
+                    uint4v d0[2], d1[2];
+                    uint32_t d2[2];
+#pragma unroll
+                    for (int h = 0; h < 2; h++) {
+                        const uint8_t *const src = wlane + cc * kChunkBytes + h * (4 * kQ8Block);
+                        d0[h] = *reinterpret_cast<const uint4a4 *>(src);
+                        d1[h] = *reinterpret_cast<const uint4a4 *>(src + 16);
+                        d2[h] = *reinterpret_cast<const uint32_t *>(src + 32);
+                    }
+                    if (cc == 1) {
+                        ask();
+                        if (!two)
+                            break;
+                    }
+#pragma unroll
+                    for (int h = 0; h < 2; h++) {
+                        const uint4v u0 = d0[h], u1 = d1[h];
+                        int4v w0, w1;
+                        w0[0] = (int)__builtin_amdgcn_perm(u0[1], u0[0], pick);
+                        w0[1] = (int)__builtin_amdgcn_perm(u0[2], u0[1], pick);
+                        w0[2] = (int)__builtin_amdgcn_perm(u0[3], u0[2], pick);
+                        w0[3] = (int)__builtin_amdgcn_perm(u1[0], u0[3], pick);
+                        w1[0] = (int)__builtin_amdgcn_perm(u1[1], u1[0], pick);
+                        w1[1] = (int)__builtin_amdgcn_perm(u1[2], u1[1], pick);
+                        w1[2] = (int)__builtin_amdgcn_perm(u1[3], u1[2], pick);
+                        w1[3] = (int)__builtin_amdgcn_perm(d2[h], u1[3], pick);
+                        const float d = (float)__builtin_bit_cast(_Float16, (uint16_t)(u0[0] >> (odd * 16)));
+#pragma unroll
+                        for (int r = 0; r < R; r++) {
+                            const int e = cc * R + r;
+                            int4v p = {0, 0, 0, 0};
+                            p = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[e][h][0], w0, p, 0, 0, 0);
+                            p = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[e][h][1], w1, p, 0, 0, 0);
+                            acc[r] = add_digits(p, d * sx[e][h], acc[r]);
+                        }
+                    }
+                }
+                // the lane's four fellows of a weight row: blocks (0 + 2) + (1 + 3)
+#pragma unroll
+                for (int r = 0; r < R; r++) {
+                    float s = acc[r];
+                    s = sum_lanes16(s);
+                    s = sum_lanes32(s);
+                    float *const to = sums_of(wave) + (g * R + r) * 16 + lm;
+                    if (lg == 0)
+                        *to = run == wave ? s : *to + s;
+                }
             }
         }
     }
-
-    float4v acc[kNCh][kNT];
-#pragma unroll
-    for (int s = 0; s < kNCh; s++)
-#pragma unroll
-        for (int t = 0; t < kNT; t++)
-            acc[s][t] = (float4v){0, 0, 0, 0};
-    // A row lm: half lm / 8 (hi, lo) of activation row lm % 8; rows past the live ones repeat a valid slot
-    // (their products are never read)
-    const int arow = (lm & 7) < nrows ? (lm & 7) : nrows - 1;
-    const int xslot = (((lm >> 3) * RP + arow) * 4 + lg) * 16;
-    // the lane's accumulators are C rows 4 lg + j: half lg / 2, activation rows 4 (lg % 2) + j
-    const int obase = (lg >> 1) * RP + ((lg & 1) * 4 < RP ? (lg & 1) * 4 : 0);
-    int wrow[kNT]; // (rows of the second tile past rows_wg repeat the last: never stored)
-#pragma unroll
-    for (int t = 0; t < kNT; t++)
-        wrow[t] = (t * 16 + lm < rows_wg ? t * 16 + lm : rows_wg - 1) * kDmaChunkBytes;
-
-    auto chunk = [&](int i, float4v (&sum)[kNT]) {
-        wait_chunks(mine - 1 - i < kDepth - 1 ? mine - 1 - i : kDepth - 1);
-        uint8_t *buf = ring + (i % kDepth) * entry;
-        uint8_t *xa = kFront ? xfront + i * 1024 : buf + pieces * 16;
-        float *off = offs + (kFront ? i : (i & 1)) * (16 * RP);
-        if (!kFront) {
-            float4v a4[kPasses], b4[kPasses];
-#pragma unroll
-            for (int ps = 0; ps < kPasses; ps++) {
-                const int u = ps * 64 + lane;
-                const int br = u >> 2, q = u & 3;
-                const int b = br / RP, r = br - b * RP;
-                const uint8_t *src = xa + (u < kUnits ? r * 1024 + b * 128 + q * 32 : 0);
-                a4[ps] = *reinterpret_cast<const float4v *>(src);
-                b4[ps] = *reinterpret_cast<const float4v *>(src + 16);
-            }
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-            __builtin_amdgcn_wave_barrier();
-#pragma unroll
-            for (int ps = 0; ps < kPasses; ps++) {
-                const int u = ps * 64 + lane;
-                const int br = u >> 2, q = u & 3;
-                const int b = br / RP, r = br - b * RP;
-                unit_write(xa, off, b, r, q, u < kUnits, a4[ps], b4[ps]);
-            }
-        }
-        // ---- the chunk's 8 blocks, in two halves: the reads of the second travel while the first is multiplied
-        half8 xop[8];
-        float ofs[8][kNJ];
-        uint32_t qa[8][kNT], qb[8][kNT], qc[4][kNT];
-        _Float16 dh[8][kNT];
-        auto read_block = [&](int b) {
-            xop[b] = *reinterpret_cast<const half8 *>(xa + b * (RP * 128) + xslot);
-#pragma unroll
-            for (int j = 0; j < kNJ; j++)
-                ofs[b][j] = off[b * 2 * RP + obase + j];
-#pragma unroll
-            for (int t = 0; t < kNT; t++) {
-                const uint8_t *blk = buf + wrow[t] + b * kQ8Block;
-                // the lane's 8 bytes sit 2 bytes past a dword boundary in even blocks (three dwords, realigned
-                // below) and at one in odd blocks
-                if ((b & 1) == 0) {
-                    const uint3a4 e = *reinterpret_cast<const uint3a4 *>(blk + lg * 8);
-                    qa[b][t] = e[0];
-                    qb[b][t] = e[1];
-                    qc[b >> 1][t] = e[2];
-                } else {
-                    const uint2a4 o = *reinterpret_cast<const uint2a4 *>(blk + 2 + lg * 8);
-                    qa[b][t] = o[0];
-                    qb[b][t] = o[1];
-                }
-                dh[b][t] = *reinterpret_cast<const _Float16 *>(blk);
-            }
-        };
-        auto math_block = [&](int b) {
-#pragma unroll
-            for (int t = 0; t < kNT; t++) {
-                uint32_t q0 = qa[b][t], q1 = qb[b][t];
-                if ((b & 1) == 0) {
-                    q0 = __builtin_amdgcn_alignbit(qb[b][t], qa[b][t], 16);
-                    q1 = __builtin_amdgcn_alignbit(qc[b >> 1][t], qb[b][t], 16);
-                }
-                const float d = (float)dh[b][t];
-                const half8 wv = int8x8_to_f16_sub(q0, q1);
-                float4v p = {0, 0, 0, 0};
-                p = __builtin_amdgcn_mfma_f32_16x16x32_f16(xop[b], wv, p, 0, 0, 0);
-#pragma unroll
-                for (int j = 0; j < kNJ; j++)
-                    sum[t][j] = fmaf(d, p[j] - ofs[b][j], sum[t][j]);
-            }
-        };
-#pragma unroll
-        for (int b = 0; b < 4; b++)
-            read_block(b);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int b = 4; b < 8; b++)
-            read_block(b);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int b = 0; b < 4; b++)
-            math_block(b);
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int b = 4; b < 8; b++)
-            math_block(b);
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // the wave's reads of this entry are done
-        if (i + kDepth < mine)
-            issue(i + kDepth);
-    };
-    // chunk wave + i kWaves belongs to chain wave + (i % kNCh) kWaves
-    for (int i0 = 0; i0 < mine; i0 += kNCh) {
-#pragma unroll
-        for (int s = 0; s < kNCh; s++)
-            if (i0 + s < mine)
-                chunk(i0 + s, acc[s]);
-    }
-
-    // ---- the chains' sums meet in their order; lanes lg = 0, 1 hold the hi products of activation rows 4 lg + j,
-    // lanes lg = 2, 3 the lo products ----------------------------------------------------------------------------
-    // (a wave leaves its chains' sums at the head of its own ring, which it has finished reading)
-    auto sums_of = [&](int chain, int t) {
-        return reinterpret_cast<float4v *>(lds + (chain % kWaves) * ring_bytes) + ((chain / kWaves) * kNT + t) * 64;
-    };
-#pragma unroll
-    for (int s = 0; s < kNCh; s++)
-#pragma unroll
-        for (int t = 0; t < kNT; t++)
-            sums_of(wave + s * kWaves, t)[lane] = acc[s][t];
     __syncthreads();
-    if (threadIdx.x < 32 * kNT) {
-        const int t = threadIdx.x >> 5, l = threadIdx.x & 31; // (weight row 16 t + l % 16, activation rows 4 (l / 16) + j)
-        float4v hi = sums_of(0, t)[l], lo = sums_of(0, t)[32 + l];
-#pragma unroll
-        for (int c = 1; c < kDmaChains; c++) {
-            hi += sums_of(c, t)[l];
-            lo += sums_of(c, t)[32 + l];
-        }
-        const float4v s = (hi + lo) * kTwo24f;
-        const int wr = t * 16 + (l & 15);
-        if (wr < rows_wg && m0 + wr < m) {
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const int r = (l >> 4) * 4 + j;
-                if (r < nrows)
-                    y[(size_t)(r0 + r) * m + m0 + wr] = s[j];
-            }
-        }
+    const int used = nrun < waves ? nrun : waves;
+    for (int e = threadIdx.x; e < ng * R * 16; e += 64 * waves) {
+        const int wr = e & 15, e4 = e >> 4, g = e4 / R, r = e4 - g * R;
+        float s = sums_of(0)[e];
+        for (int v = 1; v < used; v++)
+            s += sums_of(v)[e];
+        const int row = m0 + g * GR + wr;
+        if (wr < GR && row < m && r < nrows)
+            y[(size_t)(r0 + r) * m + row] = s;
     }
 }
 
@@ -710,7 +733,7 @@ template <int XT, int RW, bool HALF>
 struct BlocksShape {
     static constexpr int kMT = (RW + 15) / 16;              // weight tiles
     static constexpr int kXRows = 16 * XT - (HALF ? 8 : 0); // activation rows that are fetched
-    static constexpr int kWBytes = RW * kDmaChunkBytes;
+    static constexpr int kWBytes = RW * kChunkBytes;
     static constexpr int kXWave = kXRows * 128;             // one wave's block of them
     static constexpr int kSlot = kWBytes + 8 * kXWave;
     static constexpr int kFit = (160 << 10) / kSlot;
@@ -772,7 +795,7 @@ __global__ void __launch_bounds__(512, 2) gemv_q8_blocks_kernel(const uint8_t *_
         for (int j = 0; j < NWMost; j++) {
             const int q = wave + 8 * j;
             if (q < NW && (kPieces % 64 == 0 || q * 64 + lane < kPieces))
-                proj_dma16<true>(at + q * 1024, wb, woff[j] + (uint32_t)c * kDmaChunkBytes);
+                proj_dma16<true>(at + q * 1024, wb, woff[j] + (uint32_t)c * kChunkBytes);
         }
     };
     // chunk c has arrived: only the chunks asked for behind it, `most` of them, are outstanding
@@ -800,7 +823,7 @@ __global__ void __launch_bounds__(512, 2) gemv_q8_blocks_kernel(const uint8_t *_
     int wrow[MT];
 #pragma unroll
     for (int t = 0; t < MT; t++)
-        wrow[t] = (t * 16 + lm < RW ? t * 16 + lm : RW - 1) * kDmaChunkBytes + wave * kQ8Block;
+        wrow[t] = (t * 16 + lm < RW ? t * 16 + lm : RW - 1) * kChunkBytes + wave * kQ8Block;
     auto load = [&](Regs &g, int c) {
         const uint8_t *buf = lds + (c % D) * S::kSlot;
         const uint8_t *xa = buf + S::kWBytes + wave * S::kXWave + lm * 128;
@@ -1158,75 +1181,55 @@ static int launch_gemv_variant(hipStream_t st, const uint8_t *w, const float *x,
     return launch_gemv_xg<WAVES, TILES, CH, 8>(st, w, x, y, m, k, rows, rp);
 }
 
-// the most waves (8, else 4) whose rings and tables fit a CU's LDS; 0: none
-static int gemv_dma_waves(int rp, int ni, int k)
-{
-    for (int waves = 8; waves >= 4; waves -= 4)
-        if (gemv_dma_lds(rp, ni, waves, gemv_dma_rows(ni), k) <= (160 << 10))
-            return waves;
-    return 0;
-}
-
-// Weight rows per workgroup for a pass of rp activation rows, as requests per chunk (NI).
-struct DmaRows {
-    int ni;
-    bool four; // four waves even where the LDS of eight fits (several workgroups then share a CU)
+// How a call of `rows` activation rows is cut: R rows a pass, waves, ng groups of gr weight rows per workgroup.
+struct DigitsCut {
+    int r, waves, gr, ng, lds;
 };
-static DmaRows gemv_dma_rows_wg(int m, int rp)
+// One round of the chip's 256 CUs, every CU the same bytes, up to 48 weight rows per workgroup and several such rounds
+// beyond; of the groups that fit the LDS the one that pads the rows least.  A unit is what a wave has in flight: 10 and 8
+// weight rows keep the stream evener than 12 and 16 (12288 x 5120, one row, 4 / 8 / 10 / 12 / 16 weight rows: 15.3 / 12.8 /
+// 12.8 / 13.7 / 14.6 us), but with three and four rows a unit's fixed work tells (three: 19.4 / 15.8 / 15.8 / 15.3 / 16.2).
+static const int kDigitGroups[] = {12, 10, 8, 4};
+static DigitsCut gemv_digits_cut(int m, int k, int rows)
 {
-    // The fewest weight rows that make one round of the chip's 256 CUs, every CU the same bytes (us at 1024 x 5120 over
-    // 1 / 2 / 4 / 8 rows: 4 rows a workgroup 4.4 / 5.7 / 7.3 / 9.0, 16 rows 5.5 / 6.9 / 8.5 / 11.3; at 5120 x 6144: 20 rows
-    // 9.6 / 11.4 / 12.9 / 16.7, 16 rows 11.9 / 14.7 / 18.3 / 24.3).
-    static const DmaRows kOneRound[5] = {{2, false}, {3, false}, {5, false}, {6, false}, {7, false}};
-    for (const DmaRows &r : kOneRound)
-        if ((m + gemv_dma_rows(r.ni) - 1) / gemv_dma_rows(r.ni) <= 256)
-            return r;
-    // Beyond, small workgroups of which two or three share a CU, so that one's start and end lie behind another's
-    // stream (12288 x 5120 over 1 / 2 / 4 rows: 14.8 / 16.7 / 20.3 us; one workgroup of 48 rows per CU 17.9 / 18.7 / 20.5;
-    // 32 rows, a round and a half, 19.4 / 20.4 / 24.4).  With eight activation rows their copies fill the LDS and 32
-    // weight rows share them best (28.6; 16 rows 32.4).
-    if (rp == 1)
-        return {4, false};
-    if (rp <= 4)
-        return {5, true};
-    return {9, false};
-}
-
-// Calls f with the kernel of (RP, NI, waves).  Eight waves exist where their LDS fits, four where eight may not fit (with one
-// activation row the LDS grows with k) and where the rule above asks for them.
-template <int RP, int NI, typename F>
-static void with_gemv_dma_waves(int waves, F &&f)
-{
-    constexpr bool kEight = gemv_dma_lds(RP, NI, 8, gemv_dma_rows(NI), 256) <= (160 << 10);
-    constexpr bool kFour = RP == 1 || !kEight || (NI == 5 && RP <= 4);
-    if constexpr (kEight)
-        if (waves == 8)
-            f(&gemv_q8_dma_kernel<RP, NI, 8>);
-    if constexpr (kFour)
-        if (waves == 4)
-            f(&gemv_q8_dma_kernel<RP, NI, 4>);
-}
-template <int RP, typename F>
-static void with_gemv_dma_kernel(int ni, int waves, F &&f)
-{
-    switch (ni) {
-    case 2: return with_gemv_dma_waves<RP, 2>(waves, f);
-    case 3: return with_gemv_dma_waves<RP, 3>(waves, f);
-    case 5: return with_gemv_dma_waves<RP, 5>(waves, f);
-    case 6: return with_gemv_dma_waves<RP, 6>(waves, f);
-    case 7: return with_gemv_dma_waves<RP, 7>(waves, f);
-    default: // the small and the large workgroups of matrices beyond a round
-        if constexpr (RP == 1)
-            with_gemv_dma_waves<RP, 4>(waves, f);
-        else if constexpr (RP == 8)
-            with_gemv_dma_waves<RP, 9>(waves, f);
+    DigitsCut c = {0, 0, 0, 0, 0};
+    // (the waves follow from k alone: a row's bits depend on them)
+    const int nrun = ((k >> 8) + 1) >> 1, passes = (nrun + kDigitMaxWaves - 1) / kDigitMaxWaves;
+    c.waves = (nrun + passes - 1) / passes;
+    c.r = rows < 4 ? rows : 4;
+    const long long all = (long long)m * ((rows + c.r - 1) / c.r), most = 256 * 48;
+    const long long round = 256 * ((all + most - 1) / most);
+    const int n = (int)((all + round - 1) / round);
+    for (int gr : kDigitGroups) {
+        const int ng = (n + gr - 1) / gr;
+        const int lds = c.waves * gemv_digit_wave(c.r, gr, ng, passes > 1) + 64;
+        if (lds <= kDigitLds && (c.r > 2 || gr < 12) && (c.ng == 0 || ng * gr < c.ng * c.gr)) {
+            c.gr = gr;
+            c.ng = ng;
+            c.lds = lds;
+        }
     }
+    return c;
 }
 
-// Which kernel a call takes, and its variant: kRows: -; kDma: activation rows per pass, requests per chunk, waves; kBlocks
+// Calls f with the kernel of (R, GR).
+template <int R, typename F>
+static void with_gemv_digits_kernel(int gr, F &&f)
+{
+    if (gr == 4)
+        return f(&gemv_q8_digits_kernel<R, 4>);
+    if (gr == 8)
+        return f(&gemv_q8_digits_kernel<R, 8>);
+    if (gr == 10)
+        return f(&gemv_q8_digits_kernel<R, 10>);
+    if constexpr (R > 2)
+        f(&gemv_q8_digits_kernel<R, 12>);
+}
+
+// Which kernel a call takes, and its variant: kRows: -; kDigits: activation rows a pass, weight rows of a group, -; kBlocks
 // and kUnits: activation tiles, weight rows per workgroup, whether the last tile is half dead.
 struct RowsPick {
-    enum { kRows, kDma, kBlocks, kUnits } kernel;
+    enum { kRows, kDigits, kBlocks, kUnits } kernel;
     int a, b, c;
 };
 
@@ -1238,8 +1241,9 @@ static void with_gemv_blocks_kernel(int xt, int rw, bool half, F &&f)
     if (xt == X && rw == R)                                                                                     \
         return half ? f(&gemv_q8_blocks_kernel<X, R, true>, 512, BlocksShape<X, R, true>::kLds)                 \
                     : f(&gemv_q8_blocks_kernel<X, R, false>, 512, BlocksShape<X, R, false>::kLds)
-    HIPML_BLOCKS(1, 32);
-    HIPML_BLOCKS(1, 48);
+    if (xt == 1) // (nine rows and more: never half dead)
+        return rw == 32 ? f(&gemv_q8_blocks_kernel<1, 32, false>, 512, BlocksShape<1, 32, false>::kLds)
+                        : f(&gemv_q8_blocks_kernel<1, 48, false>, 512, BlocksShape<1, 48, false>::kLds);
     HIPML_BLOCKS(2, 32);
     HIPML_BLOCKS(2, 48);
     HIPML_BLOCKS(3, 32);
@@ -1299,35 +1303,21 @@ static RowsPick pick_tiles(int m, int k, int rows, bool w16)
 
 static RowsPick pick_rows(int m, int k, int rows, bool w16)
 {
-    // Up to eight rows over the raw-row kernel: rows of whole 256-value chunks at 16-byte boundaries, addressed with
-    // 32-bit offsets, and LDS room for every row count (so that all of them take this kernel, or none).
-    bool dma = rows <= 8 && k % 256 == 0 && w16 && (size_t)m * (k >> 5) * kQ8Block < ((size_t)1 << 32) &&
-               (size_t)rows * k * sizeof(float) < ((size_t)1 << 32);
-    RowsPick p = {RowsPick::kDma, 0, 0, 0};
-    for (int rp = 1; dma && rp <= 8; rp *= 2) {
-        const DmaRows r = gemv_dma_rows_wg(m, rp);
-        const int waves = gemv_dma_waves(rp, r.ni, k);
-        dma = waves != 0;
-        if (p.a < rows) {
-            p.a = rp;
-            p.b = r.ni;
-            p.c = r.four ? 4 : waves;
-        }
+    // Up to eight rows over the digits kernel: weight rows of whole 256-value chunks at 16-byte boundaries.
+    if (rows <= 8 && k % 256 == 0 && w16) {
+        const DigitsCut c = gemv_digits_cut(m, k, rows);
+        return {RowsPick::kDigits, c.r, c.gr, 0};
     }
-    if (dma)
-        return p;
     return rows > kGemvMaxRows ? pick_tiles(m, k, rows, w16) : RowsPick{RowsPick::kRows, 0, 0, 0};
 }
 
-template <int RP>
-static void launch_gemv_dma(hipStream_t st, const uint8_t *w, const float *x, float *y, int m, int k, int rows,
-                            const RowsPick &p)
+template <int R>
+static void launch_gemv_digits(hipStream_t st, const uint8_t *w, const float *x, float *y, int m, int k, int rows)
 {
-    const int rows_wg = gemv_dma_rows(p.b), waves = p.c;
-    const dim3 grid((unsigned)((m + rows_wg - 1) / rows_wg), (unsigned)((rows + RP - 1) / RP), 1);
-    const size_t lds = (size_t)gemv_dma_lds(RP, p.b, waves, rows_wg, k);
-    with_gemv_dma_kernel<RP>(p.b, waves, [&](auto kernel) {
-        HIPML_LAUNCH(kernel, grid, dim3(64 * waves, 1, 1), lds, st, w, x, y, m, k, rows, rows_wg);
+    const DigitsCut c = gemv_digits_cut(m, k, rows);
+    const dim3 grid((unsigned)((m + c.ng * c.gr - 1) / (c.ng * c.gr)), (unsigned)((rows + R - 1) / R), 1);
+        with_gemv_digits_kernel<R>(c.gr, [&](auto kernel) {
+        HIPML_LAUNCH(kernel, grid, dim3(64 * c.waves, 1, 1), (size_t)c.lds, st, w, x, y, m, k, rows, c.ng);
     });
 }
 
@@ -1347,15 +1337,13 @@ int launch_gemv_q8_rows(hipStream_t st, const uint8_t *w, const float *x, float 
         // windows of as many as fit the chip; a second window opens when the first has drained).
         return launch_gemv_variant<8, 1, 6>(st, w, x, y, m, k, rows, rp);
     }
-    if (p.kernel == RowsPick::kDma) {
-        if (p.a == 1)
-            launch_gemv_dma<1>(st, w, x, y, m, k, rows, p);
-        else if (p.a == 2)
-            launch_gemv_dma<2>(st, w, x, y, m, k, rows, p);
-        else if (p.a == 4)
-            launch_gemv_dma<4>(st, w, x, y, m, k, rows, p);
-        else
-            launch_gemv_dma<8>(st, w, x, y, m, k, rows, p);
+    if (p.kernel == RowsPick::kDigits) {
+        switch (p.a) {
+        case 1: launch_gemv_digits<1>(st, w, x, y, m, k, rows); break;
+        case 2: launch_gemv_digits<2>(st, w, x, y, m, k, rows); break;
+        case 3: launch_gemv_digits<3>(st, w, x, y, m, k, rows); break;
+        default: launch_gemv_digits<4>(st, w, x, y, m, k, rows);
+        }
         return launched("gemv_q8_0_rows");
     }
     const int xt = p.a, rw = p.b;
@@ -1398,16 +1386,15 @@ int proj_init()
         if (e == hipSuccess)
             e = hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 160 << 10);
     };
-    auto raise_dma = [&](auto rp) {
-        constexpr int RP = decltype(rp)::value;
-        for (int ni : {2, 3, 4, 5, 6, 7, 9})
-            for (int waves : {4, 8})
-                with_gemv_dma_kernel<RP>(ni, waves, [&](auto kernel) { raise(reinterpret_cast<const void *>(kernel)); });
+    auto raise_digits = [&](auto r) {
+        for (int gr : kDigitGroups)
+            with_gemv_digits_kernel<decltype(r)::value>(
+                gr, [&](auto kernel) { raise(reinterpret_cast<const void *>(kernel)); });
     };
-    raise_dma(std::integral_constant<int, 1>{});
-    raise_dma(std::integral_constant<int, 2>{});
-    raise_dma(std::integral_constant<int, 4>{});
-    raise_dma(std::integral_constant<int, 8>{});
+    raise_digits(std::integral_constant<int, 1>{});
+    raise_digits(std::integral_constant<int, 2>{});
+    raise_digits(std::integral_constant<int, 3>{});
+    raise_digits(std::integral_constant<int, 4>{});
     for (int xt = 1; xt <= 4; xt++)
         for (bool half : {false, true}) {
             auto up = [&](auto kernel, int, int) { raise(reinterpret_cast<const void *>(kernel)); };

@@ -4,7 +4,7 @@ from hipml_amd import attn
 
 
 def row_kernel(m, k, rows):
-    """kernel * 10^6 + a * 10^4 + b * 100 + c: 0 the row kernel, 1 raw rows (activation rows a pass, requests, waves), 2
+    """kernel * 10^6 + a * 10^4 + b * 100 + c: 0 the row kernel, 1 digits (activation rows a pass, weight rows of a group), 2
     blocks and 3 units (activation tiles, weight rows, last tile half dead); W at a 16-byte boundary."""
     return attn.lib().hipml_dbg_rows_kernel(m, k, rows, 1)
 
@@ -16,13 +16,11 @@ def gemm_tile(m, k, tokens, x16):
 
 
 # (weight rows, k, activation rows): ragged in the rows of a workgroup, k of 19 chunks or 37 units (uneven shares of the
-# waves, several turns of every ring); the depths that leave no LDS for eight waves or for the raw-row kernel at all
+# waves, several turns of every ring, a last run of one chunk), more runs than waves, one chunk in all
 ROWS = [
-    (3, 2368, 1), (3, 34560, 1), (3, 4864, 1), (1032, 32768, 1), (1032, 4864, 1), (6156, 4864, 1), (2069, 4864, 1),
-    (4143, 4864, 1), (5180, 4864, 1), (3, 4864, 2), (1032, 4864, 2), (6156, 4864, 2), (2069, 4864, 2),
-    (4143, 4864, 2), (5180, 4864, 2), (3, 4864, 3), (1032, 4864, 3), (6156, 4864, 3), (2069, 4864, 3),
-    (4143, 4864, 3), (5180, 4864, 3), (3, 4864, 5), (1032, 4864, 5), (2069, 4864, 5), (4143, 4864, 5),
-    (5180, 4864, 5), (6156, 4864, 5), (6156, 4864, 9), (6156, 32768, 3), (8230, 4864, 9), (8230, 32768, 3),
+    (3, 2368, 1), (3, 34560, 1), (1032, 32768, 1), (5117, 4864, 1), (6156, 256, 2), (5180, 4864, 2), (2069, 4864, 2),
+    (3, 4864, 3), (1032, 4864, 3), (2069, 4864, 3), (12281, 4864, 3), (1003, 34560, 4), (597, 4864, 5), (5117, 6144, 4),
+    (12281, 4864, 5), (6156, 4864, 9), (8230, 4864, 9),
     (6156, 4864, 25), (6156, 4864, 17), (8230, 4864, 25), (8230, 4864, 17), (6156, 4864, 41), (6156, 4864, 33),
     (8230, 4864, 41), (8230, 4864, 33), (6156, 4864, 57), (6156, 4864, 49), (8230, 4864, 57), (8230, 4864, 49),
     (3, 2368, 9), (3, 2368, 3), (2069, 2368, 17), (4143, 2368, 3), (2618, 2368, 17), (5180, 2368, 3),
