@@ -358,15 +358,16 @@ __device__ __forceinline__ void wait_vm()
 
 
 // LDS of a wave: a group's rows of a run; the digits of its activations of the run, 2 KB a row, and their scales (four rows
-// exchange those by ds_bpermute: they leave no room for the table), whose place takes the wave's sums when they are in
+// beside groups of ten, which twelve waves have no room for, exchange those by ds_bpermute: 0.6 us), whose place takes the wave's sums when they are in
 // registers, unless a wave has several runs; behind the waves 64 zero bytes.
-constexpr int gemv_digit_x(int r) { return (r < 4 ? 2048 + 64 : 2048) * r; }
+constexpr bool gemv_digit_table(int r, int gr) { return r < 4 || gr != 10; }
+constexpr int gemv_digit_x(int r, int gr) { return (gemv_digit_table(r, gr) ? 2048 + 64 : 2048) * r; }
 constexpr int gemv_digit_wave(int r, int gr, int ng, bool more)
 {
-    const int sums = ng * r * 64, x = gemv_digit_x(r);
+    const int sums = ng * r * 64, x = gemv_digit_x(r, gr);
     return gr * kRunBytes + (more ? x + sums : (x > sums ? x : sums));
 }
-static_assert(kDigitMaxWaves * gemv_digit_wave(4, 4, 12, true) + 64 <= kDigitLds, "groups of four rows always fit");
+static_assert(kDigitMaxWaves * gemv_digit_wave(4, 4, 11, true) + 64 <= kDigitLds, "groups of four rows always fit");
 
 // acc + ds * (p[0] + 2^8 p[1] + 2^16 p[2] + 2^24 p[3]); a digit sum is at most 2^19, so that both pairs are exact
 __device__ __forceinline__ float add_digits(const int4v &p, float ds, float acc)
@@ -410,12 +411,12 @@ __global__ void __launch_bounds__(64 * kDigitMaxWaves) gemv_q8_digits_kernel(con
     uint8_t *const place = lds + wave * area;
     uint8_t *const xdig = place + kPieces * 16; // [chunk][row][block][digit][32], then the scales [chunk][row][block]
     uint32_t *const scales = reinterpret_cast<uint32_t *>(xdig + 2048 * R);
-    auto sums_of = [&](int v) { return reinterpret_cast<float *>(lds + v * area + kPieces * 16 + (more ? gemv_digit_x(R) : 0)); };
+    auto sums_of = [&](int v) { return reinterpret_cast<float *>(lds + v * area + kPieces * 16 + (more ? gemv_digit_x(R, GR) : 0)); };
     uint8_t *const zeros = lds + waves * area;
     const uint32_t place_at = proj_lds_address(place), xdig_at = proj_lds_address(xdig);
     const uint8_t *const xb = reinterpret_cast<const uint8_t *>(x + (size_t)r0 * k);
 
-    // ---- requests (a chunk past the end of k repeats the one before it, rows past the end the last: never used) ----------
+    // ---- requests (a chunk past the end of k repeats the one before it, rows past the live ones the last: never used) ----
     auto issue_x = [&](int run) {
 #pragma unroll
         for (int cc = 0; cc < 2; cc++) {
@@ -433,26 +434,17 @@ __global__ void __launch_bounds__(64 * kDigitMaxWaves) gemv_q8_digits_kernel(con
         const uint32_t p = (uint32_t)(j * 64 + lane), pr = p / (uint32_t)kPerRow;
         woff[j] = pr * row_bytes + (p - pr * kPerRow) * 16u;
     }
+    const uint8_t *const w_last = w + (size_t)m * row_bytes - 16;
     auto issue_w = [&](int run, int g) {
         const int row = m0 + g * GR < m ? m0 + g * GR : m - 1;
         const uint8_t *const src = w + (size_t)row * row_bytes + (size_t)run * kRunBytes;
-        if (row + GR <= m && 2 * run + 2 <= nchunk) {
+        // pieces past the matrix repeat its last one; a run cut short by the end of k goes on into the next row (never used)
+        const size_t room = (size_t)(w_last - src);
+        const uint32_t most = room < 0xfffffff0u ? (uint32_t)room : 0xfffffff0u;
 #pragma unroll
-            for (int j = 0; j < NI; j++)
-                if ((j + 1) * 64 <= kPieces || j * 64 + lane < kPieces)
-                    proj_dma16<true>(place_at + j * 1024, src, woff[j]);
-        } else {
-            int l = lane;
-            asm volatile("" : "+v"(l)); // (what follows is worked out here, where it is seldom needed, and not kept in registers)
-#pragma unroll
-            for (int j = 0; j < NI; j++) {
-                const uint32_t p = (uint32_t)(j * 64 + l), pr = p / (uint32_t)kPerRow, pq = p - pr * kPerRow;
-                const int past = row + (int)pr - (m - 1);
-                const uint32_t back = (past > 0 ? (uint32_t)past * row_bytes : 0u) + (2 * run + 2 > nchunk && pq >= 17 ? kChunkBytes : 0);
-                if ((j + 1) * 64 <= kPieces || j * 64 + lane < kPieces)
-                    proj_dma16<true>(place_at + j * 1024, src, woff[j] - back);
-            }
-        }
+        for (int j = 0; j < NI; j++)
+            if ((j + 1) * 64 <= kPieces || j * 64 + lane < kPieces)
+                proj_dma16<true>(place_at + j * 1024, src, woff[j] < most ? woff[j] : most);
     };
     if (wave < nrun) {
         issue_x(wave);
@@ -461,7 +453,7 @@ __global__ void __launch_bounds__(64 * kDigitMaxWaves) gemv_q8_digits_kernel(con
     if (lane < 16) // (every wave writes the same zeros)
         reinterpret_cast<uint32_t *>(zeros)[lane] = 0;
 
-    constexpr bool kDense = R > 2, kTable = R < 4;
+    constexpr bool kDense = R > 2, kTable = gemv_digit_table(R, GR);
     // (not dense) lanes lg = 0 .. 3 take the blocks 0, 2, 1, 3 of a group of four: their first dwords then start in different
     // banks; payload dwords start 2 bytes into the first dword, or at the next; A row lm is a digit of the block of lanes
     // lm / 4.  (Rows past a group's repeat its last: never stored.)
@@ -1185,10 +1177,11 @@ static int launch_gemv_variant(hipStream_t st, const uint8_t *w, const float *x,
 struct DigitsCut {
     int r, waves, gr, ng, lds;
 };
-// One round of the chip's 256 CUs, every CU the same bytes, up to 48 weight rows per workgroup and several such rounds
-// beyond; of the groups that fit the LDS the one that pads the rows least.  A unit is what a wave has in flight: 10 and 8
-// weight rows keep the stream evener than 12 and 16 (12288 x 5120, one row, 4 / 8 / 10 / 12 / 16 weight rows: 15.3 / 12.8 /
-// 12.8 / 13.7 / 14.6 us), but with three and four rows a unit's fixed work tells (three: 19.4 / 15.8 / 15.8 / 15.3 / 16.2).
+// One round of the chip's 256 CUs, every CU the same bytes, up to 48 weight rows per workgroup (44 where a wave has several
+// runs and keeps its sums apart) and several such rounds beyond; of the groups that fit the LDS the one that pads the rows
+// least.  A unit is what a wave has in flight: 10 and 8 weight rows keep the stream evener than 12 and 16 (12288 x 5120, one
+// row, 4 / 8 / 10 / 12 / 16 weight rows: 15.3 / 12.8 / 12.8 / 13.7 / 14.6 us), but with three and four rows a unit's fixed
+// work tells (three: 19.4 / 15.8 / 15.8 / 15.3 / 16.2).
 static const int kDigitGroups[] = {12, 10, 8, 4};
 static DigitsCut gemv_digits_cut(int m, int k, int rows)
 {
@@ -1197,7 +1190,7 @@ static DigitsCut gemv_digits_cut(int m, int k, int rows)
     const int nrun = ((k >> 8) + 1) >> 1, passes = (nrun + kDigitMaxWaves - 1) / kDigitMaxWaves;
     c.waves = (nrun + passes - 1) / passes;
     c.r = rows < 4 ? rows : 4;
-    const long long all = (long long)m * ((rows + c.r - 1) / c.r), most = 256 * 48;
+    const long long all = (long long)m * ((rows + c.r - 1) / c.r), most = 256 * (passes > 1 ? 44 : 48);
     const long long round = 256 * ((all + most - 1) / most);
     const int n = (int)((all + round - 1) / round);
     for (int gr : kDigitGroups) {
