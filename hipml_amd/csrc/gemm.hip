@@ -23,14 +23,15 @@
 //    all of them stage first and four records cover the loads (5120 x 6144 over 512 / 672 tokens 50.8 -> 47.5 / 62.6 ->
 //    58.6 us).
 //  * small tiles with longer steps (KU 2 and 4) and eight producer waves where there are too few outputs for large
-//    ones: a step's cost is then latency, not work (1024 x 5120 over 117 tokens: 32 x 32 tiles 16 us, 128 x 128 44 us).
+//    ones: a step's cost is then latency, not work (1024 x 5120 over 117 tokens: 64 x 64 tiles 23 us, 128 x 128 44 us; the
+//    smallest tiles are gemm_q8_few_kernel's).
 //  * weights by whole 64-byte sectors, one aligned request of a quad of lanes each, where their rows allow it.  A row's
 //    pair of blocks is 68 bytes: asked for as it lies (12 and 8 bytes a lane) it takes three requests, most of them
 //    across a sector boundary, and the weights of a step cost the vector memory path as much as the activations
 //    (192 x 192 over 672 tokens 121 -> 108 us, 64 x 128 over 117 48 -> 42, 64 x 64 31 -> 27).  Tried on it: two sectors
 //    of a line asked for together (no gain), activations non-temporal (10 % slower), deeper records (no gain).
 // The kernel before this one (128 x 128 tiles for every shape) and this one, us: 12288 x 5120 over 117 / 672 / 1,024 /
-// 2,048 tokens 76 / 178 / 202 / 397 -> 40 / 114 / 144 / 282; 1024 x 5120 over the same 52 / 55 / 58 / 63 -> 16 / 24 / 28 /
+// 2,048 tokens 76 / 178 / 202 / 397 -> 40 / 114 / 144 / 282; 1024 x 5120 over the same 52 / 55 / 58 / 63 -> 11 / 24 / 28 /
 // 51; 5120 x 6144 (f16 activations) 44 / 58 / 102 / 166 -> 23 / 58 / 80 / 131.
 //
 // A tile row in LDS is an odd number of 16-byte groups: 128-bit reads and writes of 16 consecutive rows touch every
@@ -79,6 +80,34 @@ struct QuarterWeights {
     uint3a4 e[SETS][WP];
     uint2a4 o[SETS][WP];
 };
+
+// Unit j of a set from the sectors it starts in and behind, into a row of the LDS tile.  In set c it starts j dwords into
+// the 16 bytes of lane q = c % 4 of sector j.  The lanes from q on, then those before it with the next sector, are the
+// unit's logical lanes 0 .. 3 (this one is lane (qi - q) % 4, and dst its place): a logical lane's 16 values are its own
+// dwords j .. 3 and the first of the lane behind it (for the last, of the next sector of lane q).  Logical lanes 0 and 1
+// hold the even block, whose values start 2 bytes in, 2 and 3 the odd one, a dword further; the scales lie at the head of
+// lane 0 and in the upper half of lane 2's first dword.
+__device__ __forceinline__ void stage_unit(const uint4v p0, const uint4v p1, const int j, int qi, int q, uint8_t *dst)
+{
+    const int li = (qi - q) & 3;
+    const bool here = qi >= q, past = qi > q, odd = li >= 2;
+    const uint32_t pick = odd ? 0x07060504u : 0x05040302u, shift = odd ? 16u : 0u;
+    uint32_t d[5];
+#pragma unroll
+    for (int n = 0; n < 5; n++) {
+        const int e = (j + n) & 3;
+        d[n] = j + n < 4 ? (here ? p0[e] : p1[e]) : quad_next(past ? p0[e] : p1[e]);
+    }
+    const uint32_t prev = quad_prev(d[0]); // (outside the choice: every lane takes part)
+    const uint32_t sc = ((li & 1) ? prev : d[0]) >> shift;
+    const _Float16 scale = __builtin_bit_cast(_Float16, (uint16_t)sc);
+    uint32_t v[4];
+#pragma unroll
+    for (int n = 0; n < 4; n++)
+        v[n] = __builtin_amdgcn_perm(d[n + 1], d[n], pick);
+    *reinterpret_cast<half8 *>(dst) = dequant8(v[0], v[1], scale);
+    *reinterpret_cast<half8 *>(dst + 16) = dequant8(v[2], v[3], scale);
+}
 
 // TURNS: half of the producer waves ask for the next record before they stage (above); else all of them stage first,
 // activations ahead of weights, and R records cover the loads.
@@ -183,38 +212,14 @@ __global__ void __launch_bounds__(64 * (NW + CT * CM)) gemm_q8_f16_kernel(const 
         auto stage_w = [&](int v, int s, int b) {
             const int set = v / CS % SETS, sub = v % CS;
             if constexpr (WIDE) {
-                // Unit j of set c starts j dwords into the 16 bytes of lane q = c % 4 of sector j.  The lanes from q on,
-                // then those before it with the next sector, are the unit's logical lanes 0 .. 3: a logical lane's 16
-                // values are its own dwords j .. 3 and the first of the lane behind it (for the last, of the next sector
-                // of lane q).  Logical lanes 0 and 1 hold the even block, whose values start 2 bytes in, 2 and 3 the odd
-                // one, a dword further; the scales lie at the head of lane 0 and in the upper half of lane 2's first
-                // dword.
-                const int q = (s / CS) & 3, li = (qi - q) & 3;
-                const bool here = qi >= q, past = qi > q, odd = li >= 2;
-                const uint32_t pick = odd ? 0x07060504u : 0x05040302u, shift = odd ? 16u : 0u;
-                uint8_t *const dst0 = lds + b * kBuf + li * 32;
+                const int q = (s / CS) & 3;
+                uint8_t *const dst0 = lds + b * kBuf + ((qi - q) & 3) * 32;
 #pragma unroll
                 for (int h = 0; h < WS; h++)
 #pragma unroll
                     for (int u = 0; u < KU; u++) {
                         const int j = sub * KU + u;
-                        const uint4v p0 = wrec.p[set][h][j], p1 = wrec.p[set][h][j + 1];
-                        uint32_t d[5];
-#pragma unroll
-                        for (int n = 0; n < 5; n++) {
-                            const int e = (j + n) & 3;
-                            d[n] = j + n < 4 ? (here ? p0[e] : p1[e]) : quad_next(past ? p0[e] : p1[e]);
-                        }
-                        const uint32_t prev = quad_prev(d[0]); // (outside the choice: every lane takes part)
-                        const uint32_t sc = ((li & 1) ? prev : d[0]) >> shift;
-                        const _Float16 scale = __builtin_bit_cast(_Float16, (uint16_t)sc);
-                        uint32_t q[4];
-#pragma unroll
-                        for (int n = 0; n < 4; n++)
-                            q[n] = __builtin_amdgcn_perm(d[n + 1], d[n], pick);
-                        uint8_t *dst = dst0 + wlds[h] + u * 128;
-                        *reinterpret_cast<half8 *>(dst) = dequant8(q[0], q[1], scale);
-                        *reinterpret_cast<half8 *>(dst + 16) = dequant8(q[2], q[3], scale);
+                        stage_unit(wrec.p[set][h][j], wrec.p[set][h][j + 1], j, qi, q, dst0 + wlds[h] + u * 128);
                     }
             } else {
 #pragma unroll
@@ -381,6 +386,177 @@ __global__ void __launch_bounds__(64 * (NW + CT * CM)) gemm_q8_f16_kernel(const 
         }
 }
 
+// ---- gemm_q8_few_kernel: 16 AT tokens x 32 weight rows ------------------------------------------------------------
+//
+// The same product for calls with few outputs, where a step of the kernel above is latency: 1024 x 5120 over 16 tokens
+// took as long as over 200 (15.6 and 16.6 us for some 5 us of loads).  Here a workgroup's waves each have one short thing
+// to do per step of 256 values of k: four weight waves stage 16 rows x 128 values each (three sectors asked for, two units
+// dequantized; a wave of the kernel above had 16 rows x 256 values, its longest chain), four the activations, and two
+// consumer waves multiply with v_mfma_f32_16x16x32_f16, whose chain takes as long for 32 values of k as that of
+// v_mfma_f32_32x32x16_f16 for 16 (and gives its bits).  16 tokens a tile also make twice the workgroups of 32 x 32.
+// R steps are on the way in registers: three with AT = 1, two with 2 (three need more registers than ten waves have).
+// Weights as WIDE above (whole sectors, k a multiple of 1,024).
+// Tile 0 of the kernel above before, us over f32 / f16 activations: 1024 x 5120 over 16 / 117 / 200 tokens 15.7 / 16.2 / 16.9
+// and 15.5 / 15.9 / 16.4, here 9.7 / 10.9 / 14.0 and 9.4 / 10.3 / 12.2; 5120 x 6144 over 16 tokens 19.3 and 18.8, here 15.6
+// and 12.5.  Tried on it: 16 x 64, 32 x 64, 64 x 32 and 64 x 64 tiles (behind the kernel above wherever they beat 32 x 32);
+// weights by quarters of a pair of blocks instead of whole sectors (10 % slower); 16 x 32 with two steps on the way (6 to
+// 30 % slower).
+template <bool X16, int AT, int R>
+__global__ void __launch_bounds__(640) gemm_q8_few_kernel(const uint8_t *__restrict__ w, const void *__restrict__ xv,
+                                                          float *__restrict__ y, int m, int k, int tokens)
+{
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    constexpr int KU = 4, NC = 2, NA = 4, TT = 16 * AT, TM = 32;
+    constexpr int kPitch = gemm_pitch(KU), kXTile = TT * kPitch, kBuf = (TT + TM) * kPitch;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int m0 = blockIdx.x * TM, t0 = blockIdx.y * TT;
+    const int nsteps = k / (64 * KU);
+
+    if (wave >= NC) {
+        constexpr int U = R % 2 ? 2 * R : R;
+        auto produce = [&](auto fetch, auto stage) { // fetch(record, step); stage(record, step, buffer)
+#pragma unroll
+            for (int r = 0; r < R; r++)
+                fetch(r, r);
+            stage(0, 0, 0);
+            fetch(0, R);
+            __syncthreads();
+            int s = 0;
+#pragma unroll 1
+            for (; s + U < nsteps; s += U) {
+#pragma unroll
+                for (int u = 0; u < U; u++) { // stage step s + u + 1 while step s + u is multiplied
+                    stage((u + 1) % R, s + u + 1, (u + 1) & 1);
+                    __builtin_amdgcn_sched_barrier(0);
+                    fetch((u + 1) % R, s + u + 1 + R);
+                    __syncthreads();
+                }
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                if (s + u + 1 < nsteps) {
+                    stage((u + 1) % R, s + u + 1, (u + 1) & 1);
+                    if (u + 1 + R < U)
+                        fetch((u + 1) % R, s + u + 1 + R);
+                }
+                if (s + u < nsteps)
+                    __syncthreads();
+            }
+        };
+        if (wave < NC + NA) {
+            // ---- weights: units 2 H and 2 H + 1 of a step's four of 16 rows, as WideWeights above
+            const uint32_t row_bytes = (uint32_t)(k >> 5) * kQ8Block;
+            const int qi = lane & 3, r = (wave - NC) / 2 * 16 + (lane >> 2);
+            const int row = m0 + r < m ? r : m - 1 - m0;
+            auto weights = [&](auto half_) {
+                constexpr int H = decltype(half_)::value;
+                const uint8_t *const wb = w + (size_t)m0 * row_bytes;
+                const uint32_t woff = (uint32_t)row * row_bytes + (uint32_t)(qi * 16 + H * 128);
+                uint8_t *const wdst = lds + kXTile + r * kPitch + H * 256;
+                uint4v rec[R][3];
+                auto fetch = [&](int v, int s) {
+                    const int c = s < nsteps ? s : nsteps - 1;
+                    const uint8_t *const ws = wb + (size_t)(4 * c + (c >> 2)) * 64;
+#pragma unroll
+                    for (int j = 0; j < 3; j++)
+                        rec[v][j] = *reinterpret_cast<const uint4v *>(ws + woff + j * 64);
+                };
+                auto stage = [&](int v, int s, int b) {
+                    const int q = s & 3, li = (qi - q) & 3;
+#pragma unroll
+                    for (int u = 0; u < 2; u++)
+                        stage_unit(rec[v][u], rec[v][u + 1], 2 * H + u, qi, q, wdst + b * kBuf + li * 32 + u * 128);
+                };
+                produce(fetch, stage);
+            };
+            if (wave & 1)
+                weights(std::integral_constant<int, 1>{});
+            else
+                weights(std::integral_constant<int, 0>{});
+        } else {
+            // ---- activations: XN pieces of 16 bytes per thread
+            constexpr int XELT = X16 ? 2 : 4, XPR = 64 * KU * XELT / 16, XROWS = 256 / XPR, XN = TT / XROWS;
+            const int xt = threadIdx.x - 64 * (NC + NA), xr = xt / XPR, xc = xt % XPR;
+            const uint8_t *const xb = static_cast<const uint8_t *>(xv) + (size_t)t0 * k * XELT;
+            uint32_t xoff[XN];
+#pragma unroll
+            for (int i = 0; i < XN; i++) {
+                const int t = t0 + xr + XROWS * i < tokens ? xr + XROWS * i : tokens - 1 - t0;
+                xoff[i] = (uint32_t)t * (uint32_t)(k * XELT) + xc * 16;
+            }
+            uint8_t *const xdst = lds + xr * kPitch + xc * (X16 ? 16 : 8);
+            float4v rec[R][XN];
+            auto fetch = [&](int v, int s) {
+                const uint8_t *const xs = xb + (size_t)(s < nsteps ? s : nsteps - 1) * (64 * KU * XELT);
+#pragma unroll
+                for (int i = 0; i < XN; i++)
+                    rec[v][i] = *reinterpret_cast<const float4v *>(xs + xoff[i]);
+            };
+            auto stage = [&](int v, int, int b) {
+#pragma unroll
+                for (int i = 0; i < XN; i++) {
+                    uint8_t *const d = xdst + b * kBuf + XROWS * i * kPitch;
+                    if (X16)
+                        *reinterpret_cast<float4v *>(d) = rec[v][i];
+                    else // (rounded as the kernel above rounds)
+                        *reinterpret_cast<half4v *>(d) = __builtin_convertvector(rec[v][i], half4v);
+                }
+            };
+            produce(fetch, stage);
+        }
+        return;
+    }
+    // consumer wave: 16 weight rows
+    const int lm = lane & 15, lg = lane >> 4;
+    float4v acc[AT];
+#pragma unroll
+    for (int a = 0; a < AT; a++)
+        acc[a] = (float4v){0.0f, 0.0f, 0.0f, 0.0f};
+    const uint8_t *xa = lds + lm * kPitch + lg * 16;
+    const uint8_t *wb = lds + kXTile + (wave * 16 + lm) * kPitch + lg * 16;
+    half8 A[2][AT], B[2];
+    auto read = [&](int kk) {
+#pragma unroll
+        for (int a = 0; a < AT; a++)
+            A[kk & 1][a] = *reinterpret_cast<const half8 *>(xa + a * 16 * kPitch + kk * 64);
+        B[kk & 1] = *reinterpret_cast<const half8 *>(wb + kk * 64);
+    };
+    auto multiply = [&](int kk) {
+#pragma unroll
+        for (int a = 0; a < AT; a++)
+            acc[a] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A[kk & 1][a], B[kk & 1], acc[a], 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    constexpr int kSlices = 2 * KU; // of 32 values of k in a step: an even number
+    __syncthreads();
+    read(0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll 1
+    for (int s = 0; s < nsteps; s++) {
+#pragma unroll
+        for (int kk = 0; kk + 1 < kSlices; kk++) {
+            read(kk + 1);
+            multiply(kk);
+        }
+        __syncthreads();
+        const int other = s & 1 ? -kBuf : kBuf;
+        xa += other;
+        wb += other;
+        read(0); // (behind the last step: whatever the other buffer holds, not used)
+        multiply(kSlices - 1);
+    }
+    // C tile: lane holds column lm (weight row), rows 4 lg + j (tokens)
+    const int row = m0 + wave * 16 + lm;
+#pragma unroll
+    for (int a = 0; a < AT; a++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int t = t0 + a * 16 + lg * 4 + j;
+            if (t < tokens && row < m)
+                y[(size_t)t * m + row] = acc[a][j];
+        }
+}
+
 // x16[i] = f16(x[i] * sigmoid(gate[i])) (gate may be null: plain conversion), 8 values per thread.
 // The gate is the expression every gating kernel of this library uses, the rounding the one the
 // f32-activation GEMM applies when it stages x: the two routes give the same bits.
@@ -421,7 +597,7 @@ struct GemmTile {
     float sectors, sectors16, other, other16;
 };
 constexpr GemmTile kGemmTiles[] = {
-    {32, 32, 4, true, 0.117f, 0.105f, 0.0f, 0.0f},   {32, 64, 4, true, 0.156f, 0.14f, 0.0f, 0.0f},
+    {32, 32, 4, true, 0.101f, 0.086f, 0.0f, 0.0f},   {32, 64, 4, true, 0.145f, 0.13f, 0.0f, 0.0f},
     {64, 64, 2, true, 0.216f, 0.0f, 0.0f, 0.0f},     {64, 128, 2, true, 0.341f, 0.311f, 0.0f, 0.0f},
     {128, 128, 1, true, 0.504f, 0.0f, 0.0f, 0.0f},   {192, 128, 1, true, 0.729f, 0.585f, 0.0f, 0.0f},
     {128, 192, 1, true, 0.725f, 0.642f, 0.0f, 0.0f}, {192, 192, 1, true, 0.931f, 0.814f, 0.0f, 0.0f},
@@ -434,6 +610,9 @@ constexpr GemmTile kGemmTiles[] = {
     // cuts that fit 256 workgroups where those above do not (12,288 weight rows: 128 tiles of 96); over f16 activations
     // the 64 x 64 tile of longer steps stands for that of shorter ones
     {64, 96, 2, true, 0.291f, 0.0f, 0.0f, 0.0f},     {64, 64, 4, true, 0.0f, 0.18f, 0.0f, 0.0f},
+    // gemm_q8_few_kernel, as tile 0: the costs of both and of tile 1 are fitted to these three and their neighbours at 468
+    // shapes of 8 to 382 tokens (0.7 % behind the best of them on average; 16 shapes more than 5 %)
+    {16, 32, 4, true, 0.074f, 0.06f, 0.0f, 0.0f},
 };
 constexpr int kGemmNTiles = sizeof(kGemmTiles) / sizeof(kGemmTiles[0]);
 
@@ -485,8 +664,15 @@ static bool with_gemm_kernel(int i, F &&f)
                  64 * (NW + CT * CM), tt, tm,                                                                         \
                  gemm_lds(tt, tm, KU));                                                                               \
     }
+#define HIPML_GEMM_FEW(idx, AT, R)                                                                                     \
+    case idx:                                                                                                         \
+        static_assert(kGemmTiles[idx].tt == 16 * AT && kGemmTiles[idx].tm == 32 && kGemmTiles[idx].ku == 4 &&         \
+                          kGemmTiles[idx].wide,                                                                       \
+                      "the table");                                                                                   \
+        return f(&gemm_q8_few_kernel<X16, AT, R>, 640, 16 * AT, 32, gemm_lds(16 * AT, 32, 4));
     switch (i) {
-        HIPML_GEMM(0, true, 1, 1, 1, 1, 4, 8, 2)
+        HIPML_GEMM_FEW(0, 2, 2)
+        HIPML_GEMM_FEW(16, 1, 3)
         HIPML_GEMM(1, true, 1, 2, 1, 1, 4, 8, 2)
         HIPML_GEMM(3, true, 2, 2, 1, 2, 2, 8, 2)
         HIPML_GEMM(5, true, 2, 2, 3, 2, 1, 4, 2)
@@ -521,6 +707,7 @@ static bool with_gemm_kernel(int i, F &&f)
         return false;
     }
 #undef HIPML_GEMM
+#undef HIPML_GEMM_FEW
 }
 
 int gemm_init()

@@ -31,8 +31,9 @@ ROWS = [
 TILES = [
     (12380, 704, 580, 0), (10996, 704, 258, 0), (10996, 704, 143, 0), (239, 1408, 51, 0), (239, 704, 51, 0),
     (12380, 704, 649, 1), (10996, 704, 258, 1), (7190, 704, 212, 1), (239, 1408, 51, 1), (239, 704, 51, 1),
-    (239, 3072, 51, 0), (2173, 3072, 97, 0), (5460, 3072, 74, 0), (12380, 3072, 74, 0), (10996, 3072, 143, 0),
+    (239, 5120, 51, 0), (2173, 3072, 97, 0), (5460, 3072, 74, 0), (12380, 3072, 74, 0), (10996, 3072, 143, 0),
     (6671, 3072, 534, 0), (10996, 3072, 258, 0), (12380, 3072, 396, 0), (12380, 3072, 649, 0), (8228, 3072, 74, 0),
-    (239, 3072, 51, 1), (2173, 3072, 97, 1), (8228, 3072, 74, 1), (10996, 3072, 258, 1), (10996, 3072, 396, 1),
-    (12380, 3072, 396, 1), (7363, 3072, 985, 1), (10996, 3072, 143, 1), (3730, 3072, 97, 1),
+    (1069, 3072, 210, 0),
+    (239, 1024, 51, 1), (2173, 3072, 97, 1), (7363, 3072, 97, 1), (10996, 3072, 258, 1), (10996, 3072, 396, 1),
+    (12380, 3072, 396, 1), (7363, 3072, 985, 1), (10996, 3072, 143, 1), (1069, 3072, 210, 1), (7363, 3072, 210, 1),
 ]
