@@ -801,8 +801,8 @@ def row_kernel_name(attn, m, k, rows):
     return f"gemv_q8_{'blocks' if kernel == 2 else 'units'}_kernel<{a}, {b}, {'true' if c else 'false'}>"
 
 
-# W_o over 672 tokens: 128 x 128 tiles over f16 activations (the tile with this place in the library's table)
-GEMM672_TILE, GEMM672_KERNEL = 11, "gemm_q8_f16_kernel<true, false, 2, 2, 2, 2, 1, 8, 4, false>"
+# W_o over 672 gated tokens: packed rows, 256 x 64 tiles (100 x route + place in the library's table of tiles)
+GEMM672_CHOICE, GEMM672_KERNEL = 307, "gemm_q8_direct_kernel<4, 4, 4, 4, 4, 2>"
 
 
 def bench_gemv(torch, attn, rows, steps, layers, m=5120, k=6144):
@@ -849,7 +849,7 @@ def bench_gemm(torch, attn, tokens, steps, layers, m=5120, k=6144, mfma=None):
     us = ms * 1e3
     flop = 2.0 * tokens * m * k
     tf = flop / (us * 1e-6) / 1e12
-    wl = "gemm672" if attn.lib().hipml_dbg_gemm_tile(m, k, tokens, 1, 1) == GEMM672_TILE and tokens == 672 else ""
+    wl = "gemm672" if attn.lib().hipml_dbg_gemm_choice(m, k, tokens, 1, 1) == GEMM672_CHOICE and tokens == 672 else ""
     return {"workload": f"W_o projection of a chunk, Q8_0 {m}x{k}, {tokens} tokens",
             "us_per_layer": us, "timed_ms": total, "steps_timed": n, "us_per_layer_f32_rows_no_gate": t32 * 1e3,
             "flop": flop, "layers_rotated": layers,
@@ -859,8 +859,8 @@ def bench_gemm(torch, attn, tokens, steps, layers, m=5120, k=6144, mfma=None):
                          "frac_of_achievable": None if mfma is None else tf / mfma["tflops"],
                          **counters(wl, GEMM672_KERNEL),
                          "traffic": None if not counters(wl, GEMM672_KERNEL) else
-                                    measured_traffic(wl, ["gate_f16_kernel", GEMM672_KERNEL]),
-                         "kernel": "gate_f16_kernel + gemm_q8_f16_kernel",
+                                    measured_traffic(wl, ["pack_f16_kernel", GEMM672_KERNEL]),
+                         "kernel": "pack_f16_kernel + gemm_q8_direct_kernel" if wl else "chunk projection",
                          "flop_per_launch": flop, "launch_us": us}}
 
 

@@ -36,7 +36,8 @@ EXPORTS = [
     "hipml_attn_decode_kv_gate", "hipml_attn_decode_batch_cols_gate",
     "hipml_attn_chunk_q8_split", "hipml_attn_chunk_q8_split_gate", "hipml_q_gate_f32",
     "hipml_attn_front_f32", "hipml_attn_chunk_front_f32",
-    "hipml_gemv_q8_0_rows", "hipml_gemm_q8_0_f16", "hipml_attn_output_chunk_q8_0",
+    "hipml_gemv_q8_0_rows", "hipml_gemm_q8_0_f16", "hipml_gemm_q8_0_f16_scratch",
+    "hipml_attn_output_chunk_q8_0",
     "hipml_kv_rows_copy", "hipml_rope_encode_chunk_f32",
     "hipml_attn_front_encode_f32", "hipml_attn_chunk_front_encode_f32",
     "hipml_attn_chunk_q8_split_gate_f16", "hipml_attn_chunk_rope_q8",
@@ -133,6 +134,7 @@ def lib() -> C.CDLL:
             "hipml_rope_encode_chunk_f32": (i, [vp, vp, vp, vp, vp, vp, i, i, i, i, f, i, i, i, i]),
             "hipml_gemv_q8_0_rows": (i, [vp, vp, vp, vp, i, i, i]),
             "hipml_gemm_q8_0_f16": (i, [vp, vp, vp, vp, i, i, i]),
+            "hipml_gemm_q8_0_f16_scratch": (sz, [i, i, i]),
             "hipml_attn_output_chunk_q8_0": (i, [vp, vp, vp, vp, vp, i, i, i, vp]),
         }
         for name, (res, args) in sig.items():
@@ -524,7 +526,19 @@ def gemv_q8_0_rows(w, x, y, m, k, rows, stream=None):
 
 def gemm_q8_0_f16(w, x, y, m, k, tokens, stream=None):
     """`AttnLayer::apply_output_chunk`'s tiled GEMM (after the gate) over a Q8_0 weight matrix:
-    y[tokens][m], f16 operands."""
+    y[tokens][m], f16 operands.  On the current stream the library's scratch for the rows as f16, where it
+    asks for one, comes from torch's allocator, which keeps it for that stream; not under capture, where the memory
+    would be free again before the graph is replayed, and not for a stream the allocator is not told of."""
+    if stream is None and x is not None:
+        nbytes = lib().hipml_gemm_q8_0_f16_scratch(m, k, tokens)
+        if nbytes and x.data_ptr() and not torch.cuda.is_current_stream_capturing():
+            try:
+                x16 = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+            except torch.cuda.OutOfMemoryError:
+                x16 = None
+            if x16 is not None:
+                _check(lib().hipml_attn_output_chunk_q8_0(_stream(), _p(w), _p(x), 0, _p(y), m, k, tokens, _p(x16)))
+                return
     _check(lib().hipml_gemm_q8_0_f16(_stream(stream), _p(w), _p(x), _p(y), m, k, tokens))
 
 

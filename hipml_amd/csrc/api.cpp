@@ -1329,6 +1329,13 @@ int hipml_gemm_q8_0_f16(hipml_stream_t stream, const void *w, const float *x, fl
                               tokens, nullptr);
 }
 
+size_t hipml_gemm_q8_0_f16_scratch(int m, int k, int tokens)
+{
+    if (m < 1 || k < 64 || k % 64 != 0 || tokens < 1)
+        return 0;
+    return gemm_wants_scratch(m, k, tokens) ? (size_t)tokens * (size_t)k * 2 : 0;
+}
+
 int hipml_attn_output_chunk_q8_0(hipml_stream_t stream, const void *wo, const float *attn_out,
                                  const float *gate, float *y, int m, int k, int tokens, void *x16)
 {

@@ -156,9 +156,12 @@ int launch_kv_f16_rows(hipStream_t st, const uint8_t *kc, const uint8_t *vc, voi
 int launch_gemv_q8_rows(hipStream_t st, const uint8_t *w, const float *x, float *y, int m, int k, int rows);
 // The same product for a prefill chunk: f16 operands on MFMA, fp32 accumulation (gemm.hip).
 // With a scratch of tokens*k f16 (x16) the activations are gated (gate may be null) and converted once
-// by a first kernel; without it the GEMM converts the f32 activations itself (gate must be null).
+// by a first kernel where that is faster or there is a gate; without it the GEMM converts the f32 activations itself
+// (gate must be null).
 int launch_gemm_q8_f16(hipStream_t st, const uint8_t *w, const float *x, const float *gate, float *y, int m,
                        int k, int tokens, void *x16);
+// Whether a scratch makes the product without a gate faster.
+bool gemm_wants_scratch(int m, int k, int tokens);
 // Raise the projection kernels' dynamic LDS limit (once per process; called by hipml_attn_init).
 int proj_init();
 int gemm_init();

@@ -386,6 +386,41 @@ __global__ void __launch_bounds__(64 * (NW + CT * CM)) gemm_q8_f16_kernel(const 
         }
 }
 
+// A producer wave's turns in the two kernels below: R steps on the way, step s + 1 staged while step s is multiplied.
+// fetch(record, step), past the last step too; stage(record, step, buffer).
+template <int R, typename F, typename S>
+__device__ __forceinline__ void produce_steps(int nsteps, F &&fetch, S &&stage)
+{
+    constexpr int U = R % 2 ? 2 * R : R;
+#pragma unroll
+    for (int r = 0; r < R; r++)
+        fetch(r, r);
+    stage(0, 0, 0);
+    fetch(0, R);
+    __syncthreads();
+    int s = 0;
+#pragma unroll 1
+    for (; s + U < nsteps; s += U) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            stage((u + 1) % R, s + u + 1, (u + 1) & 1);
+            __builtin_amdgcn_sched_barrier(0);
+            fetch((u + 1) % R, s + u + 1 + R);
+            __syncthreads();
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+        if (s + u + 1 < nsteps) {
+            stage((u + 1) % R, s + u + 1, (u + 1) & 1);
+            if (u + 1 + R < U)
+                fetch((u + 1) % R, s + u + 1 + R);
+        }
+        if (s + u < nsteps)
+            __syncthreads();
+    }
+}
+
 // ---- gemm_q8_few_kernel: 16 AT tokens x 32 weight rows ------------------------------------------------------------
 //
 // The same product for calls with few outputs, where a step of the kernel above is latency: 1024 x 5120 over 16 tokens
@@ -413,36 +448,6 @@ __global__ void __launch_bounds__(640) gemm_q8_few_kernel(const uint8_t *__restr
     const int nsteps = k / (64 * KU);
 
     if (wave >= NC) {
-        constexpr int U = R % 2 ? 2 * R : R;
-        auto produce = [&](auto fetch, auto stage) { // fetch(record, step); stage(record, step, buffer)
-#pragma unroll
-            for (int r = 0; r < R; r++)
-                fetch(r, r);
-            stage(0, 0, 0);
-            fetch(0, R);
-            __syncthreads();
-            int s = 0;
-#pragma unroll 1
-            for (; s + U < nsteps; s += U) {
-#pragma unroll
-                for (int u = 0; u < U; u++) { // stage step s + u + 1 while step s + u is multiplied
-                    stage((u + 1) % R, s + u + 1, (u + 1) & 1);
-                    __builtin_amdgcn_sched_barrier(0);
-                    fetch((u + 1) % R, s + u + 1 + R);
-                    __syncthreads();
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < U; u++) {
-                if (s + u + 1 < nsteps) {
-                    stage((u + 1) % R, s + u + 1, (u + 1) & 1);
-                    if (u + 1 + R < U)
-                        fetch((u + 1) % R, s + u + 1 + R);
-                }
-                if (s + u < nsteps)
-                    __syncthreads();
-            }
-        };
         if (wave < NC + NA) {
             // ---- weights: units 2 H and 2 H + 1 of a step's four of 16 rows, as WideWeights above
             const uint32_t row_bytes = (uint32_t)(k >> 5) * kQ8Block;
@@ -467,7 +472,7 @@ __global__ void __launch_bounds__(640) gemm_q8_few_kernel(const uint8_t *__restr
                     for (int u = 0; u < 2; u++)
                         stage_unit(rec[v][u], rec[v][u + 1], 2 * H + u, qi, q, wdst + b * kBuf + li * 32 + u * 128);
                 };
-                produce(fetch, stage);
+                produce_steps<R>(nsteps, fetch, stage);
             };
             if (wave & 1)
                 weights(std::integral_constant<int, 1>{});
@@ -502,7 +507,7 @@ __global__ void __launch_bounds__(640) gemm_q8_few_kernel(const uint8_t *__restr
                         *reinterpret_cast<half4v *>(d) = __builtin_convertvector(rec[v][i], half4v);
                 }
             };
-            produce(fetch, stage);
+            produce_steps<R>(nsteps, fetch, stage);
         }
         return;
     }
@@ -557,6 +562,209 @@ __global__ void __launch_bounds__(640) gemm_q8_few_kernel(const uint8_t *__restr
         }
 }
 
+// ---- gemm_q8_direct_kernel: activations from L2 straight into operand registers -----------------------------------
+//
+// In the kernel above every activation passes through LDS once as it is staged and is read back by CM consumer waves: at
+// 12288 x 5120 that, and the producers' loads behind it, cost as much as the MFMAs.  Here pack_f16_kernel has rounded the
+// activations to f16 (after the gate, if any) and laid them out as the MFMA's operand: for each 32 values of k and 16
+// tokens the 64 lanes' 16 bytes in a row.  A consumer wave loads its 16 AT tokens' operands from L2 with one request a
+// KB, P slices of 32 k ahead, and no other wave of the workgroup reads them; only the weights, which every consumer wave
+// needs, go through LDS, KU = 4 units a step, staged by NP producer waves (each half of a step's units of BT / (NP / 2) groups
+// of 16 rows, SETS steps ahead).  Consumers: 16 AT tokens x 16 BT weight rows each, NC of them side by side in tokens.
+// Loaded from the row-major rows instead it is slower than the kernel above: 16 rows 10,240 bytes apart lie in two of
+// L2's channels.
+// What bounds it (12288 x 5120 over 672 tokens, 384 x 96 tiles, timing-only builds): MFMAs and LDS reads alone 72 us, all
+// of it 86, packing 5.  The kernel above with f32 rows before, this one with packing, us: 12288 x 5120 over 96 / 117 / 200 /
+// 382 / 672 / 1,500 / 2,048 tokens 37.1 / 39.6 / 58.3 / 85.3 / 115 / 227 / 290 -> 32.4 / 33.8 / 47.8 / 60.2 / 96.7 / 184 /
+// 252; after a gate 5120 x 6144 over 200 / 382 / 672 / 1,024 / 1,500 42.4 / 50.7 / 69.0 / 94.8 / 128 -> 33.5 / 43.3 / 62.3 /
+// 82.7 / 110.  Tried on it: weights by LDS DMA and dequantized by the consumers (behind the kernel above), weights loaded
+// non-temporally (20 % slower), three or four steps of weights on the way (no gain).
+// Layout of the packed activations: slice s (k from 32 s) starts at s * tokens * 64 bytes, its tokens from 16 t at t * 1024;
+// there value k = 32 s + 8 g + e of token 16 t + i at (g * n + i) * 16 + 2 e, with n = 16, or what is left of the tokens.
+// That is tokens * k * 2 bytes in all.
+
+// One wave: 16 tokens x 128 values of k, each lane 8 values of 4 slices.
+__global__ void __launch_bounds__(256) pack_f16_kernel(const float *__restrict__ x, const float *__restrict__ gate,
+                                                       uint8_t *__restrict__ x16, int k, int tokens)
+{
+    const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
+    const int t0 = blockIdx.x * 16, n = tokens - t0 < 16 ? tokens - t0 : 16;
+    const int s0 = (blockIdx.y * 4 + (threadIdx.x >> 6)) * 4;
+    if (i >= n)
+        return;
+    const size_t from = (size_t)(t0 + i) * k + g * 8;
+    float4v a[4][2], ga[4][2];
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+        if (s0 + u < k / 32)
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                a[u][h] = *reinterpret_cast<const float4v *>(x + from + (s0 + u) * 32 + h * 4);
+                if (gate != nullptr)
+                    ga[u][h] = *reinterpret_cast<const float4v *>(gate + from + (s0 + u) * 32 + h * 4);
+            }
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+        if (s0 + u < k / 32) {
+            half8 v;
+#pragma unroll
+            for (int h = 0; h < 2; h++) {
+                float4v f = a[u][h];
+                if (gate != nullptr)
+#pragma unroll
+                    for (int j = 0; j < 4; j++)
+                        f[j] = gated(f[j], ga[u][h][j]);
+                const half4v r = __builtin_convertvector(f, half4v); // (rounded as gate_f16_kernel rounds)
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    v[4 * h + j] = r[j];
+            }
+            *reinterpret_cast<half8 *>(x16 + (size_t)(s0 + u) * tokens * 64 + (size_t)t0 * 64 + (g * n + i) * 16) = v;
+        }
+}
+
+template <int NC, int AT, int BT, int NP, int P, int SETS>
+__global__ void __launch_bounds__(64 * (NP + NC)) gemm_q8_direct_kernel(const uint8_t *__restrict__ w,
+                                                                        const void *__restrict__ xv,
+                                                                        float *__restrict__ y, int m, int k, int tokens)
+{
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    constexpr int KU = 4, TM = 16 * BT, TT = 16 * AT * NC;
+    constexpr int kPitch = gemm_pitch(KU), kBuf = TM * kPitch;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int m0 = blockIdx.x * TM, t0 = blockIdx.y * TT;
+    const int nsteps = k / (64 * KU);
+
+    if (wave >= NC) {
+        const int pw = wave - NC;
+        constexpr int G = BT / (NP / 2); // groups of 16 weight rows of a wave
+        static_assert(G * (NP / 2) == BT && NP % 2 == 0, "");
+        const uint32_t row_bytes = (uint32_t)(k >> 5) * kQ8Block;
+        const uint8_t *const wb = w + (size_t)m0 * row_bytes;
+        const int qi = lane & 3;
+        auto produce = [&](auto half_) {
+            constexpr int H = decltype(half_)::value; // units 2 H and 2 H + 1 of a step's four
+            uint32_t woff[G], wlds[G];
+#pragma unroll
+            for (int g = 0; g < G; g++) {
+                const int r = ((pw >> 1) * G + g) * 16 + (lane >> 2);
+                const int row = m0 + r < m ? r : m - 1 - m0;
+                woff[g] = (uint32_t)row * row_bytes + (uint32_t)(qi * 16 + H * 128);
+                wlds[g] = (uint32_t)(r * kPitch + H * 256);
+            }
+            uint4v rec[SETS][G][3];
+            auto fetch = [&](int v, int s) {
+                const int c = s < nsteps ? s : nsteps - 1;
+                const uint8_t *const ws = wb + (size_t)(4 * c + (c >> 2)) * 64;
+#pragma unroll
+                for (int g = 0; g < G; g++)
+#pragma unroll
+                    for (int j = 0; j < 3; j++)
+                        rec[v][g][j] = *reinterpret_cast<const uint4v *>(ws + woff[g] + j * 64);
+            };
+            auto stage = [&](int v, int s, int b) {
+                const int q = s & 3;
+                uint8_t *const dst0 = lds + b * kBuf + ((qi - q) & 3) * 32;
+#pragma unroll
+                for (int g = 0; g < G; g++)
+#pragma unroll
+                    for (int u = 0; u < 2; u++)
+                        stage_unit(rec[v][g][u], rec[v][g][u + 1], 2 * H + u, qi, q, dst0 + wlds[g] + u * 128);
+            };
+            produce_steps<SETS>(nsteps, fetch, stage);
+        };
+        if (pw & 1)
+            produce(std::integral_constant<int, 1>{});
+        else
+            produce(std::integral_constant<int, 0>{});
+        return;
+    }
+    const int lm = lane & 15, lg = lane >> 4;
+    const int tw = t0 / 16 + wave * AT; // the wave's first 16 tokens
+    float4v acc[AT][BT];
+#pragma unroll
+    for (int a = 0; a < AT; a++)
+#pragma unroll
+        for (int b = 0; b < BT; b++)
+            acc[a][b] = (float4v){0.0f, 0.0f, 0.0f, 0.0f};
+    uint32_t xoff[AT]; // (tokens past the last: the last one's)
+#pragma unroll
+    for (int a = 0; a < AT; a++) {
+        const int last = (tokens - 1) >> 4, t = tw + a < last ? tw + a : last;
+        const int n = tokens - 16 * t < 16 ? tokens - 16 * t : 16;
+        xoff[a] = (uint32_t)(t * 64 + lg * n + (lm < n ? lm : n - 1)) * 16u;
+    }
+    const uint8_t *const xb = static_cast<const uint8_t *>(xv);
+    const size_t xstep = (size_t)tokens * 64;
+    const int nslice = k / 32;
+    half8 X[P][AT], W[2][BT];
+    auto load = [&](int v, int s) {
+        const uint8_t *const xs = xb + (size_t)(s < nslice ? s : nslice - 1) * xstep;
+#pragma unroll
+        for (int a = 0; a < AT; a++)
+            X[v][a] = *reinterpret_cast<const half8 *>(xs + xoff[a]);
+    };
+    const uint8_t *wl = lds + lm * kPitch + lg * 16;
+    auto read = [&](int kk) {
+#pragma unroll
+        for (int b = 0; b < BT; b++)
+            W[kk & 1][b] = *reinterpret_cast<const half8 *>(wl + b * 16 * kPitch + kk * 64);
+    };
+    auto multiply = [&](int kk) { // (weights as the first operand: a lane's four sums are one token's)
+#pragma unroll
+        for (int b = 0; b < BT; b++)
+#pragma unroll
+            for (int a = 0; a < AT; a++)
+                acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(W[kk & 1][b], X[kk % P][a], acc[a][b], 0, 0, 0);
+    };
+    constexpr int kSlices = 2 * KU;
+    static_assert(kSlices % P == 0, "the records of a step are named at compile time");
+#pragma unroll
+    for (int v = 0; v < P; v++)
+        load(v, v);
+    __syncthreads();
+    read(0);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll 1
+    for (int s = 0; s < nsteps; s++) {
+#pragma unroll
+        for (int kk = 0; kk + 1 < kSlices; kk++) {
+            read(kk + 1);
+            multiply(kk);
+            load(kk % P, s * kSlices + kk + P);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        __syncthreads();
+        wl += s & 1 ? -kBuf : kBuf;
+        read(0); // (behind the last step: whatever the other buffer holds, not used)
+        multiply(kSlices - 1);
+        load((kSlices - 1) % P, s * kSlices + kSlices - 1 + P);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    // C tile: lane holds column lm (token), rows 4 lg + j (weight rows)
+    const bool wide = (m & 3) == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0;
+#pragma unroll
+    for (int a = 0; a < AT; a++) {
+        const int t = (tw + a) * 16 + lm;
+        if (t < tokens) {
+            float *const yt = y + (size_t)t * m;
+#pragma unroll
+            for (int b = 0; b < BT; b++) {
+                const int row = m0 + 16 * b + 4 * lg;
+                if (wide) {
+                    if (row < m)
+                        *reinterpret_cast<float4v *>(yt + row) = acc[a][b];
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 4; j++)
+                        if (row + j < m)
+                            yt[row + j] = acc[a][b][j];
+                }
+            }
+        }
+    }
+}
+
 // x16[i] = f16(x[i] * sigmoid(gate[i])) (gate may be null: plain conversion), 8 values per thread.
 // The gate is the expression every gating kernel of this library uses, the rounding the one the
 // f32-activation GEMM applies when it stages x: the two routes give the same bits.
@@ -597,7 +805,7 @@ struct GemmTile {
     float sectors, sectors16, other, other16;
 };
 constexpr GemmTile kGemmTiles[] = {
-    {32, 32, 4, true, 0.101f, 0.086f, 0.0f, 0.0f},   {32, 64, 4, true, 0.145f, 0.13f, 0.0f, 0.0f},
+    {32, 32, 4, true, 0.101f, 0.086f, 0.0f, 0.0f},   {32, 64, 4, true, 0.145f, 0.119f, 0.0f, 0.0f},
     {64, 64, 2, true, 0.216f, 0.0f, 0.0f, 0.0f},     {64, 128, 2, true, 0.341f, 0.311f, 0.0f, 0.0f},
     {128, 128, 1, true, 0.504f, 0.0f, 0.0f, 0.0f},   {192, 128, 1, true, 0.729f, 0.585f, 0.0f, 0.0f},
     {128, 192, 1, true, 0.725f, 0.642f, 0.0f, 0.0f}, {192, 192, 1, true, 0.931f, 0.814f, 0.0f, 0.0f},
@@ -616,12 +824,21 @@ constexpr GemmTile kGemmTiles[] = {
 };
 constexpr int kGemmNTiles = sizeof(kGemmTiles) / sizeof(kGemmTiles[0]);
 
+// Rounds of a tile over the chip's 256 CUs, a full one weighing 1 + slope.
+static float tile_rounds(int m, int tokens, int tt, int tm, float slope)
+{
+    const long long wg = (long long)((m + tm - 1) / tm) * ((tokens + tt - 1) / tt);
+    const long long rounds = (wg + 255) / 256;
+    const float fill = (float)wg / (256.0f * (float)rounds);
+    return (float)rounds * (1.0f + slope * fill * fill);
+}
+
 // The tile for a shape: the cheapest by rounds x cost, where a round of 256 workgroups slows down as it fills (they
 // share L2, HBM and the power budget: 1.5 times the cost of a lone workgroup when all CUs have one).  The costs are fitted
 // to every tile's time at 173 shapes (1,024 to 12,288 weight rows, k of 576 to 6,144, 24 to 2,048 tokens), 346 with the
 // types of activations: the tile picked is the measured best or within 5 % of it at 340 of them, 14 % behind it at most
 // (1024 x 5120 over 1,400 tokens: 42.4 us, best 37.1), 0.2 % on average.
-static int gemm_tile(int m, int k, int tokens, bool sectors, bool x16)
+static int gemm_tile(int m, int k, int tokens, bool sectors, bool x16, float *cost_of_unit)
 {
     int best = -1;
     float best_cost = 0.0f;
@@ -632,22 +849,21 @@ static int gemm_tile(int m, int k, int tokens, bool sectors, bool x16)
         if (k % (64 * g.ku) != 0 || tile_cost == 0.0f ||
             (uint64_t)(g.tt > g.tm ? g.tt : g.tm) * (uint64_t)k * 4 >= (1ull << 32))
             continue;
-        const long long wg = (long long)((m + g.tm - 1) / g.tm) * ((tokens + g.tt - 1) / g.tt);
-        const long long rounds = (wg + 255) / 256;
-        const float fill = (float)wg / (256.0f * (float)rounds);
-        const float cost = (float)rounds * tile_cost * (1.0f + 0.5f * fill * fill);
+        const float cost = tile_cost * tile_rounds(m, tokens, g.tt, g.tm, 0.5f);
         if (best < 0 || cost < best_cost) {
             best = i;
             best_cost = cost;
         }
     }
+    if (cost_of_unit != nullptr)
+        *cost_of_unit = best_cost;
     return best;
 }
 
 // For tests and the benchmark: the tile (its place in the table) that a call takes.
 extern "C" int hipml_dbg_gemm_tile(int m, int k, int tokens, int sectors, int x16)
 {
-    return gemm_tile(m, k, tokens, sectors != 0, x16 != 0);
+    return gemm_tile(m, k, tokens, sectors != 0, x16 != 0, nullptr);
 }
 
 // Calls f with the kernel of tile i and its launch figures: (kernel, threads, tile tokens, tile rows, LDS bytes).
@@ -710,6 +926,45 @@ static bool with_gemm_kernel(int i, F &&f)
 #undef HIPML_GEMM_FEW
 }
 
+// The packed route's tiles (tokens and weight rows; microseconds as in the table above, with a full chip's slow-down of 1.1
+// instead of 1.5) and its kernels.
+struct DirectTile {
+    int tt, tm;
+    float cost;
+};
+constexpr DirectTile kDirectTiles[] = {
+    {128, 32, 0.21f}, {128, 48, 0.248f}, {128, 64, 0.281f},  {128, 96, 0.366f},  {192, 48, 0.298f}, {192, 96, 0.522f},
+    {192, 128, 0.691f}, {256, 64, 0.476f}, {256, 96, 0.668f}, {256, 128, 0.807f}, {384, 96, 0.825f},
+};
+constexpr int kDirectNTiles = sizeof(kDirectTiles) / sizeof(kDirectTiles[0]);
+
+template <typename F>
+static bool with_direct_kernel(int i, F &&f)
+{
+#define HIPML_DIRECT(idx, NC, AT, BT, NP, P)                                                                           \
+    case idx: {                                                                                                       \
+        constexpr int tt = 16 * AT * NC, tm = 16 * BT;                                                                \
+        static_assert(kDirectTiles[idx].tt == tt && kDirectTiles[idx].tm == tm, "the table");                         \
+        return f(&gemm_q8_direct_kernel<NC, AT, BT, NP, P, 2>, 64 * (NP + NC), tt, tm, 2 * tm * gemm_pitch(4));       \
+    }
+    switch (i) {
+        HIPML_DIRECT(0, 4, 2, 2, 4, 8)
+        HIPML_DIRECT(1, 4, 2, 3, 6, 8)
+        HIPML_DIRECT(2, 4, 2, 4, 4, 4)
+        HIPML_DIRECT(3, 4, 2, 6, 4, 4)
+        HIPML_DIRECT(4, 4, 3, 3, 6, 4)
+        HIPML_DIRECT(5, 4, 3, 6, 4, 4)
+        HIPML_DIRECT(6, 4, 3, 8, 4, 4)
+        HIPML_DIRECT(7, 4, 4, 4, 4, 4)
+        HIPML_DIRECT(8, 4, 4, 6, 4, 4)
+        HIPML_DIRECT(9, 4, 4, 8, 4, 2)
+        HIPML_DIRECT(10, 8, 3, 6, 4, 4)
+    default:
+        return false;
+    }
+#undef HIPML_DIRECT
+}
+
 int gemm_init()
 {
     hipError_t e = hipSuccess;
@@ -722,17 +977,92 @@ int gemm_init()
         with_gemm_kernel<false>(i, raise);
         with_gemm_kernel<true>(i, raise);
     }
+    for (int i = 0; i < kDirectNTiles; i++)
+        with_direct_kernel(i, raise);
     if (e != hipSuccess)
         return fail((int)e, "hipFuncSetAttribute(chunk projection LDS) failed: %d (%s)", (int)e, hipGetErrorString(e));
     return 0;
 }
 
-// x16 != nullptr: gate (optional) and convert into x16 first, then the GEMM over f16 activations;
-// x == nullptr: x16 already holds them.
+// How f32 rows are multiplied where the caller gives scratch for them as f16: as they lie (only without a gate), rounded
+// into the scratch row by row, or packed into it for the direct kernel (weights in whole sectors only).  The cheapest by
+// the tiles' costs and that of the pass that fills the scratch: 3 us (a launch 2, scratch from an allocator 1) and the
+// rows read and written (3.4 M / 10.5 M values: 5.0 / 9.8 us in all, alone).  As they lie, too, below a k of 2,048, where
+// the pass is not paid back (6000 x 1024 over 1,024 / 2,048 tokens: 24.3 / 39.3 us, with scratch 25.6 / 41.4).  The costs
+// are fitted like the table above at 253 shapes (1,024 to 16,384 weight rows, 32 to 2,048 tokens): 1 % behind the best of
+// all routes and tiles on average, 11 % at most; 12 % ahead of the tiles over the rows as they lie, at 3 shapes more than
+// 2 % behind them.
+enum class GemmRoute { kNone, kRows, kRowsF16, kPacked };
+struct GemmChoice {
+    GemmRoute route;
+    int tile;
+};
+static GemmChoice gemm_choice(int m, int k, int tokens, bool sectors, bool gated_rows)
+{
+    GemmChoice best = {GemmRoute::kNone, -1};
+    float best_cost = 0.0f;
+    auto offer = [&](GemmRoute route, int tile, float cost) {
+        if (tile >= 0 && (best.tile < 0 || cost < best_cost)) {
+            best = {route, tile};
+            best_cost = cost;
+        }
+    };
+    const float units = (float)(k / 64), pass = 3.0f + 0.75e-6f * (float)tokens * (float)k;
+    float cost = 0.0f;
+    if (!gated_rows) {
+        const int tile = gemm_tile(m, k, tokens, sectors, false, &cost);
+        offer(GemmRoute::kRows, tile, units * cost);
+        if (k < 2048)
+            return best;
+    }
+    const int tile = gemm_tile(m, k, tokens, sectors, true, &cost);
+    offer(GemmRoute::kRowsF16, tile, units * cost + pass);
+    // (32-bit offsets in a tile's weights and in a slice of the activations, and the passes' grids)
+    if (sectors && tile >= 0 && k <= 1 << 23 && tokens <= 1 << 22)
+        for (int i = 0; i < kDirectNTiles; i++) {
+            const DirectTile &g = kDirectTiles[i];
+            offer(GemmRoute::kPacked, i, units * g.cost * tile_rounds(m, tokens, g.tt, g.tm, 0.1f) + pass);
+        }
+    return best;
+}
+
+// For tests and the benchmark: 100 x route (1 as they lie, 2 rounded, 3 packed) + tile of a call with scratch.
+extern "C" int hipml_dbg_gemm_choice(int m, int k, int tokens, int sectors, int gated_rows)
+{
+    const GemmChoice c = gemm_choice(m, k, tokens, sectors != 0, gated_rows != 0);
+    return c.tile < 0 ? -1 : 100 * (int)c.route + c.tile;
+}
+
+// Whether scratch for the rows as f16 makes hipml_gemm_q8_0_f16's product faster (W at a 64-byte boundary).
+bool gemm_wants_scratch(int m, int k, int tokens)
+{
+    const GemmChoice c = gemm_choice(m, k, tokens, k % 1024 == 0, false);
+    return c.tile >= 0 && c.route != GemmRoute::kRows;
+}
+
+// x16 != nullptr: scratch for the rows as f16 (the gate, if any, applied first); x == nullptr: x16 already holds them, row
+// by row.
 int launch_gemm_q8_f16(hipStream_t st, const uint8_t *w, const float *x, const float *gate, float *y, int m,
                        int k, int tokens, void *x16)
 {
-    if (x16 != nullptr && x != nullptr) {
+    // (rows of weights in whole 64-byte sectors)
+    const bool sectors = k % 1024 == 0 && (reinterpret_cast<uintptr_t>(w) & 63) == 0;
+    GemmChoice c;
+    if (x != nullptr && x16 != nullptr)
+        c = gemm_choice(m, k, tokens, sectors, gate != nullptr);
+    else
+        c = {x != nullptr ? GemmRoute::kRows : GemmRoute::kRowsF16,
+             gemm_tile(m, k, tokens, sectors, x == nullptr, nullptr)};
+    if (c.tile < 0)
+        return fail(HIPML_ATTN_E_RANGE, "k %d: 32 rows of activations exceed 4 GB", k);
+    const void *act = c.route == GemmRoute::kRows ? static_cast<const void *>(x) : x16;
+    if (c.route == GemmRoute::kPacked) {
+        HIPML_LAUNCH(pack_f16_kernel, dim3((unsigned)((tokens + 15) / 16), (unsigned)((k / 32 + 15) / 16), 1),
+                     dim3(256, 1, 1), 0, st, x, gate, static_cast<uint8_t *>(x16), k, tokens);
+        int rc = launched("pack_f16");
+        if (rc)
+            return rc;
+    } else if (c.route == GemmRoute::kRowsF16 && x != nullptr) {
         const size_t n8 = (size_t)tokens * k / 8;
         HIPML_LAUNCH(gate_f16_kernel, dim3((unsigned)((n8 + 255) / 256), 1, 1), dim3(256, 1, 1), 0, st,
                            reinterpret_cast<const float4v *>(x), reinterpret_cast<const float4v *>(gate),
@@ -741,21 +1071,17 @@ int launch_gemm_q8_f16(hipStream_t st, const uint8_t *w, const float *x, const f
         if (rc)
             return rc;
     }
-    const void *act = x16 != nullptr ? x16 : x;
     auto go = [&](auto kernel, int threads, int tt, int tm, int lds) {
         HIPML_LAUNCH(kernel, dim3((unsigned)((m + tm - 1) / tm), (unsigned)((tokens + tt - 1) / tt), 1),
                      dim3(threads, 1, 1), lds, st, w, act, y, m, k, tokens);
         return true;
     };
-    // (rows of weights in whole 64-byte sectors)
-    const bool sectors = k % 1024 == 0 && (reinterpret_cast<uintptr_t>(w) & 63) == 0;
-    const int tile = gemm_tile(m, k, tokens, sectors, x16 != nullptr);
-    if (tile < 0)
-        return fail(HIPML_ATTN_E_RANGE, "k %d: 32 rows of activations exceed 4 GB", k);
-    if (x16 != nullptr)
-        with_gemm_kernel<true>(tile, go);
+    if (c.route == GemmRoute::kPacked)
+        with_direct_kernel(c.tile, go);
+    else if (c.route == GemmRoute::kRowsF16)
+        with_gemm_kernel<true>(c.tile, go);
     else
-        with_gemm_kernel<false>(tile, go);
+        with_gemm_kernel<false>(c.tile, go);
     return launched("gemm_q8_0_f16");
 }
 

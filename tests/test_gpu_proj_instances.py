@@ -65,3 +65,43 @@ def test_tile(m, k, tokens, x16):
     err = ((y[:tokens] - h.double() @ dense.T).abs() / terms).max().item()
     assert err <= 2.0 ** -24 * np.sqrt(k), err
     assert torch.equal(y[tokens // 2], one[0])
+
+
+@pytest.mark.parametrize("m,k,tokens,gated", inst.PACKED)
+def test_packed_tile(m, k, tokens, gated):
+    w, _, _, x = inputs(m, k, tokens)
+    gate = torch.randn((tokens, k), device="cuda") if gated else None
+    rows = x
+    if gated:
+        rows = torch.empty_like(x)
+        attn.q_gate(x, gate, rows, tokens * k)
+    y, want = padded(tokens, m), padded(tokens, m)
+    x16 = torch.full((tokens + 1, k), 3.0, dtype=torch.float16, device="cuda")
+    attn.output_chunk_q8_0(w, x, gate, y, m, k, tokens, x16)
+    attn.gemm_q8_0_f16(w, rows, want, m, k, tokens, stream=torch.cuda.current_stream())  # (no scratch: test_tile's kernels)
+    assert torch.equal(y[:tokens], want[:tokens]) and bool(y[tokens].isnan().all())
+    assert bool((x16[tokens] == 3.0).all())
+
+
+def test_scratch_of_a_call_on_the_current_stream_and_under_capture():
+    m, k, tokens = 12380, 3072, 392
+    assert attn.lib().hipml_gemm_q8_0_f16_scratch(m, k, tokens) == tokens * k * 2
+    w, _, _, x = inputs(m, k, tokens)
+    want, y = padded(tokens, m), padded(tokens, m)
+    attn.gemm_q8_0_f16(w, x, want, m, k, tokens, stream=torch.cuda.current_stream())
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        for _ in range(3):  # (the scratch of one call is the next one's)
+            attn.gemm_q8_0_f16(w, x, y, m, k, tokens)
+    torch.cuda.current_stream().wait_stream(side)
+    assert torch.equal(y[:tokens], want[:tokens])
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        attn.gemm_q8_0_f16(w, x, y, m, k, tokens)
+    for _ in range(3):
+        y.fill_(float("nan"))
+        junk = torch.randn((tokens, k), device="cuda")  # (eager work in memory that was free at the capture)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y[:tokens], want[:tokens]) and bool(junk.isfinite().all())

@@ -24,6 +24,14 @@ def test_every_tile_has_a_shape(k, x16):
     assert not {c: s for c, s in taken.items() if c not in named}
 
 
+def test_every_packed_tile_has_a_shape():
+    named = {inst.gemm_choice(*shape) for shape in inst.PACKED}
+    assert len(named) == len(inst.PACKED) and min(named) >= 300
+    tokens = [*range(1, 700, 17), *range(700, 4200, 83)]
+    taken = {inst.gemm_choice(m, k, t, g): (m, k, t, g) for m in M for t in tokens for k in (1024, 5120) for g in (0, 1)}
+    assert not {c: s for c, s in taken.items() if c >= 300 and c not in named}
+
+
 @pytest.mark.parametrize("m,k", [(12_288, 5120), (1024, 5120), (5120, 6144)])
 def test_the_models_projections_are_among_them(m, k):
     named = {inst.row_kernel(*shape) for shape in inst.ROWS}
