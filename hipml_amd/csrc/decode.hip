@@ -330,6 +330,18 @@ struct Work {
     int hbase, nvalid;                      // first head overall, (row, head) columns of the item
 };
 
+// Sum over the lanes up to and including this one, without LDS (every lane active).
+__device__ __forceinline__ int wave_scan(int v)
+{
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true); // within 16 lanes: from 1, 2, 4 and 8 lanes before
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false); // lane 15's to lanes 16 .. 31, lane 47's to 48 .. 63
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false); // lane 31's to lanes 32 .. 63
+    return v;
+}
+
 // Returns false when this workgroup has nothing to do (uniform over the workgroup).
 __device__ __forceinline__ bool find_work(const DecodeArgs &a, const Front &f, int lane, Work &wk)
 {
@@ -345,6 +357,7 @@ __device__ __forceinline__ bool find_work(const DecodeArgs &a, const Front &f, i
     // tiles per worker for which these add up to no more than `workers` (the launcher keeps
     // items <= workers), i.e. no worker has more than T tiles.
     int kvh, split, item, nsp;
+    int slot, row0, ncols, group, head0; // group = heads of this item: columns are (row, head) pairs over them
     // The scalar arguments span two 64-byte lines of the kernel-argument segment, both cold when a
     // workgroup starts.  Left alone the compiler fetches `workers` (second line) here and the first
     // line only where the pointers are first used: two memory round trips one after the other.  A
@@ -359,31 +372,31 @@ __device__ __forceinline__ bool find_work(const DecodeArgs &a, const Front &f, i
         // argument struct would make the compiler copy its arrays to scratch
         typedef const __attribute__((address_space(4))) uint8_t *KargBytes;
         typedef const __attribute__((address_space(4))) uint16_t *KargHalves;
-        const KargBytes ka = (KargBytes)__builtin_amdgcn_kernarg_segment_ptr();
-        const KargHalves t_row0 = (KargHalves)(ka + f.karg_at + offsetof(DecodeArgs, row0));
-        const KargBytes t_cols = ka + f.karg_at + offsetof(DecodeArgs, cols);
-        int tiles = 0;
-        if (lane < f.items) {
-            const int r0 = t_row0[lane], nc = t_cols[lane];
-            int sm = 0;
-            for (int c = 0; c < nc; c++) {
-                int v = f.pos[(size_t)(r0 + c) * 2 + 1];
-                v = v < 0 ? 0 : (v > f.stride ? f.stride : v);
-                sm = v > sm ? v : sm;
-            }
-            tiles = (sm + kTileKeys - 1) / kTileKeys;
+        const KargBytes ka = (KargBytes)__builtin_amdgcn_kernarg_segment_ptr() + f.karg_at;
+        // All of the lane's item in one round trip, then the live lengths of its rows in another; the sums over lanes by
+        // DPP.  (Lengths one after the other, the found item's fields in a third round trip behind the search, and thirty
+        // LDS shuffles: 32 items of 115 to 2,026 rows had their work item after 2.7 us and their first requests out after
+        // 4.2, now 1.4 and 2.8; the launch 22.5 -> 20.6 us.)
+        const int mine = lane < f.items ? lane : f.items - 1;
+        const int l_row0 = ((KargHalves)(ka + offsetof(DecodeArgs, row0)))[mine], l_cols = ka[offsetof(DecodeArgs, cols) + mine];
+        const int l_slot = ka[offsetof(DecodeArgs, kvslot) + mine], l_head0 = ka[offsetof(DecodeArgs, head0) + mine];
+        const int l_nhead = ka[offsetof(DecodeArgs, nhead) + mine];
+        int sm = 0;
+        int len[kMaxCols];
+#pragma unroll
+        for (int c = 0; c < kMaxCols; c++)
+            len[c] = f.pos[(size_t)(l_row0 + (c < l_cols ? c : 0)) * 2 + 1];
+#pragma unroll
+        for (int c = 0; c < kMaxCols; c++) {
+            const int v = len[c] < 0 ? 0 : (len[c] > f.stride ? f.stride : len[c]);
+            sm = v > sm ? v : sm;
         }
+        const int tiles = lane < f.items ? (sm + kTileKeys - 1) / kTileKeys : 0;
         // the smallest number T of tiles per worker for which the items' shares ceil(tiles / T)
         // (at least one worker each, at most `splits`) fit the workers there are: no worker then has
         // more than T tiles, whatever the mix of depths (shares proportional to the tiles and rounded
         // down left some items with half as many workers again as they needed)
-        int tmax = tiles, total = tiles;
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) {
-            const int o = __shfl_xor(tmax, off);
-            tmax = o > tmax ? o : tmax;
-            total += __shfl_xor(total, off);
-        }
+        const int total = __builtin_amdgcn_readlane(wave_scan(tiles), 63);
         auto share_at = [&](int t) {
             int sh = 0;
             if (lane < f.items) {
@@ -397,39 +410,32 @@ __device__ __forceinline__ bool find_work(const DecodeArgs &a, const Front &f, i
             return sh;
         };
         // T lies between total / workers and total / (workers - items) (each share is below
-        // tiles / T + 1), so the search is a few steps
+        // tiles / T + 1, and the launcher keeps 2 items <= workers), so the search is a few steps
         const int spare = f.workers - f.items;
         int lo = (total + f.workers - 1) / f.workers;
         lo = lo < 1 ? 1 : lo;
-        int hi = spare > 0 ? (total + spare - 1) / spare : (tmax > 1 ? tmax : 1);
+        int hi = (total + spare - 1) / spare;
         hi = hi < lo ? lo : hi;
         while (lo < hi) { // uniform over the wave
             const int mid = (lo + hi) >> 1;
-            int need = share_at(mid);
-#pragma unroll
-            for (int off = 32; off > 0; off >>= 1)
-                need += __shfl_xor(need, off);
-            if (need <= f.workers)
+            if (__builtin_amdgcn_readlane(wave_scan(share_at(mid)), 63) <= f.workers)
                 hi = mid;
             else
                 lo = mid + 1;
         }
         const int share = share_at(lo);
-        int end = share; // inclusive prefix sum over lanes
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-            const int up = __shfl_up(end, off);
-            end += lane >= off ? up : 0;
-        }
+        const int end = wave_scan(share);
         const unsigned long long hit = __ballot(lane < f.items && w >= end - share && w < end);
         if (hit == 0)
             return false; // more workers than the shares add up to (uniform over the workgroup)
-        item = __builtin_ctzll(hit);
-        nsp = __shfl(share, item);
-        split = w - (__shfl(end, item) - nsp);
-        item = __builtin_amdgcn_readfirstlane(item);
-        nsp = __builtin_amdgcn_readfirstlane(nsp);
-        split = __builtin_amdgcn_readfirstlane(split);
+        item = __builtin_amdgcn_readfirstlane(__builtin_ctzll(hit));
+        nsp = __builtin_amdgcn_readlane(share, item);
+        split = w - (__builtin_amdgcn_readlane(end, item) - nsp);
+        slot = __builtin_amdgcn_readlane(l_slot, item);
+        row0 = __builtin_amdgcn_readlane(l_row0, item);
+        ncols = __builtin_amdgcn_readlane(l_cols, item);
+        group = __builtin_amdgcn_readlane(l_nhead, item);
+        head0 = __builtin_amdgcn_readlane(l_head0, item);
     } else {
         kvh = blockIdx.x / f.splits;
         split = blockIdx.x - kvh * f.splits;
@@ -441,8 +447,9 @@ __device__ __forceinline__ bool find_work(const DecodeArgs &a, const Front &f, i
     // makes the wave wait for them here, while nothing else is outstanding: the (conditional) Q loads
     // below come later in the same in-order queue, so a first use behind them would wait for the Q
     // rows as well, and the first tile could only be requested once those had arrived.
-    int slot, row0, ncols, group, head0; // group = heads of this item: columns are (row, head) pairs over them
-    if (f.items == 1) {
+    if (worker_launch) {
+        // (known from the search)
+    } else if (f.items == 1) {
         slot = f.i0_slot;
         row0 = f.i0_row0;
         ncols = f.i0_cols;
@@ -457,19 +464,6 @@ __device__ __forceinline__ bool find_work(const DecodeArgs &a, const Front &f, i
     }
     const int hbase = kvh * f.group + head0;
     const int nvalid = ncols * group;
-    if (f.workers > 0 && split == 0 && nsp < f.splits) {
-        // the splits of this item that no worker takes: empty partials, which the merge skips
-        const int empty = f.splits - nsp;
-        for (int e = threadIdx.x; e < nvalid * empty; e += (int)blockDim.x) {
-            const int n = e / empty, sp = nsp + (e - n * empty);
-            const int col = n / group;
-            const int head = hbase + (n - col * group);
-            float *pm = a.part_ml + (size_t)(row0 + col) * a.ml_slot + ((size_t)head * f.splits + sp) * 2;
-            pm[0] = -INFINITY;
-            pm[1] = 0.0f;
-        }
-    }
-
     wk.kvh = kvh;
     wk.split = split;
     wk.nsp = nsp;
@@ -482,6 +476,22 @@ __device__ __forceinline__ bool find_work(const DecodeArgs &a, const Front &f, i
     wk.hbase = hbase;
     wk.nvalid = nvalid;
     return true;
+}
+
+// Worker launches: the splits of an item that no worker takes get empty partials, which the merge skips.
+__device__ __forceinline__ void leave_empty_splits(const DecodeArgs &a, const Front &f, const Work &wk)
+{
+    if (f.workers > 0 && wk.split == 0 && wk.nsp < f.splits) {
+        const int empty = f.splits - wk.nsp;
+        for (int e = threadIdx.x; e < wk.nvalid * empty; e += (int)blockDim.x) {
+            const int n = e / empty, sp = wk.nsp + (e - n * empty);
+            const int col = n / wk.group;
+            const int head = wk.hbase + (n - col * wk.group);
+            float *pm = a.part_ml + (size_t)(wk.row0 + col) * a.ml_slot + ((size_t)head * f.splits + sp) * 2;
+            pm[0] = -INFINITY;
+            pm[1] = 0.0f;
+        }
+    }
 }
 
 template <int NT, bool Q4, bool PLO>
@@ -504,6 +514,7 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &a)
     Work wk;
     if (!find_work(a, f, lane, wk))
         return;
+    leave_empty_splits(a, f, wk);
     const int kvh = wk.kvh, split = wk.split, nsp = wk.nsp, slot = wk.slot, row0 = wk.row0, ncols = wk.ncols,
               group = wk.group, hbase = wk.hbase, nvalid = wk.nvalid;
 
@@ -1889,11 +1900,13 @@ __global__ void __launch_bounds__(kThreads, 2)
     HIPML_STAMP(stamps_, 1); // work item found
     if (wk.nvalid > 8) { // uniform over the workgroup
         decode_body_dma<true>(a, f, wk HIPML_STAMPS_PASS);
+        leave_empty_splits(a, f, wk);
         HIPML_STAMP(stamps_, 7); // partial stored (not yet acknowledged)
         if (a.merge > 0)
             decode_merge_tail<true>(a, wk HIPML_STAMPS_PASS);
     } else {
         decode_body_dma<false>(a, f, wk HIPML_STAMPS_PASS);
+        leave_empty_splits(a, f, wk);
         HIPML_STAMP(stamps_, 7);
         if (a.merge > 0)
             decode_merge_tail<false>(a, wk HIPML_STAMPS_PASS);
@@ -1918,6 +1931,7 @@ __global__ void __launch_bounds__(kThreads, 2)
     if (!find_work(a, f, threadIdx.x & 63, wk))
         return;
     decode_body_dma<false, true>(a, f, wk HIPML_STAMPS_PASS);
+    leave_empty_splits(a, f, wk);
 }
 
 // Wave-wide reductions without LDS: DPP inside a row of 16 lanes, then the two row-swap

@@ -351,6 +351,39 @@ def test_one_split_writes_the_rows_itself(seq, dtype):
     assert bool(acc.isnan().all()) and bool(ml.isnan().all())
 
 
+@pytest.mark.parametrize("slots", [2, 17, 33, 64])
+def test_window_of_workers_divides_itself_among_the_slots(slots):
+    # every worker finds its slot from the live lengths, one lane per work item: up to the 64 a wave has lanes for; slots
+    # without a key, of one key, around a tile and deep enough for several workers
+    stride, n_kv = 900, 4
+    r = orc.Rng(0x0D2F + slots)
+    cols = [2 if slots < 64 and s % 5 == 3 else 1 for s in range(slots)]  # (two rows of six heads: two items)
+    depths = [(880, 0, 31, 500, 32, 640, 5)[s % 7] for s in range(slots)]
+    kb = orc.quantize(0, r.normal_array((slots, n_kv, stride, HD))).reshape(slots, n_kv, stride, -1)
+    vb = orc.quantize(0, r.normal_array((slots, n_kv, stride, HD))).reshape(slots, n_kv, stride, -1)
+    pos = [(d + c, d + c + 1) for d, n in zip(depths, cols) for c in range(n)]
+    pos[1] = (0, 0)  # slot 1 has no key
+    slot_of = [s for s, n in enumerate(cols) for _ in range(n)]
+    rows, items = len(pos), sum(n for n in cols)
+    assert 2 * items <= 512 // n_kv
+    splits = attn.batch_splits(stride, n_kv, slots)
+    q = r.normal_array((rows, N_HEADS, HD))
+    kd, vd, qd = dev(kb), dev(vb), dev(q)
+    acc, ml = decode_scratch(N_HEADS, splits, rows)
+    acc.fill_(float("nan")), ml.fill_(float("nan"))
+    out = torch.full((rows, N_HEADS, HD), float("nan"), device="cuda")
+    attn.attn_decode_batch_cols(0, torch.tensor(pos, dtype=torch.int32, device="cuda"), qd, kd, vd, acc, ml, out, N_HEADS, n_kv,
+                                HD, stride, SCALE, splits, kd[0].numel(), N_HEADS * splits * HD, N_HEADS * splits * 2,
+                                N_HEADS * HD, cols)
+    torch.cuda.synchronize()
+    got = host(out)
+    assert not got[1].any()
+    for i in range(rows):
+        if pos[i][1] > 0:
+            want = orc.attn_decode_kv(q[i], kb[slot_of[i]], vb[slot_of[i]], N_HEADS, n_kv, HD, pos[i][1], SCALE, stride=stride)
+            assert report(f"row {i} of {slots} slots", want.ravel(), got[i].ravel(), *KERNEL_CLASS)[0]
+
+
 @pytest.mark.parametrize("dtype", [0, 1])
 @pytest.mark.parametrize("slots,n_kv", [(40, 8), (66, 4)])
 def test_one_split_over_a_batch_too_large_for_a_window(slots, n_kv, dtype):
