@@ -564,7 +564,10 @@ __global__ void __launch_bounds__(256) front_kernel(
     float eps, const float *__restrict__ tab, int tab_rows, const FrontAppend ap)
 {
     __shared__ float buf[4][kHeadDim];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    // (the wave's number as a scalar: row, head and addresses are scalar arithmetic then.  us over 1 / 16 / 672 / 1,024 / 2,048
+    // rows 3.26 / 3.58 / 15.9 / 23.4 / 40.8 -> 3.15 / 3.48 / 15.4 / 23.0 / 39.6.  Tried: 16 bytes a lane for the q rows, 17.3 us
+    // over 672: the tree's exchanges four times over)
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int per_row = n_heads + n_kv;
     const int idx = blockIdx.x * 4 + wave;
     const int nfront = per_row * rows;
