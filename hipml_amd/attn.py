@@ -37,6 +37,7 @@ EXPORTS = [
     "hipml_attn_chunk_q8_split", "hipml_attn_chunk_q8_split_gate", "hipml_q_gate_f32",
     "hipml_attn_front_f32", "hipml_attn_chunk_front_f32",
     "hipml_gemv_q8_0_rows", "hipml_gemm_q8_0_f16", "hipml_gemm_q8_0_f16_scratch",
+    "hipml_gemm_q8_0_f16_rows", "hipml_gemm_q8_0_f16_rows_scratch",
     "hipml_attn_output_chunk_q8_0",
     "hipml_kv_rows_copy", "hipml_rope_encode_chunk_f32",
     "hipml_attn_front_encode_f32", "hipml_attn_chunk_front_encode_f32",
@@ -135,6 +136,8 @@ def lib() -> C.CDLL:
             "hipml_gemv_q8_0_rows": (i, [vp, vp, vp, vp, i, i, i]),
             "hipml_gemm_q8_0_f16": (i, [vp, vp, vp, vp, i, i, i]),
             "hipml_gemm_q8_0_f16_scratch": (sz, [i, i, i]),
+            "hipml_gemm_q8_0_f16_rows": (i, [vp, vp, vp, vp, i, i, i, vp]),
+            "hipml_gemm_q8_0_f16_rows_scratch": (sz, [i, i, i]),
             "hipml_attn_output_chunk_q8_0": (i, [vp, vp, vp, vp, vp, i, i, i, vp]),
         }
         for name, (res, args) in sig.items():
@@ -524,27 +527,38 @@ def gemv_q8_0_rows(w, x, y, m, k, rows, stream=None):
     _check(lib().hipml_gemv_q8_0_rows(_stream(stream), _p(w), _p(x), _p(y), m, k, rows))
 
 
+def _scratch(nbytes):
+    """`nbytes` from torch's allocator for launches on the current stream, which the allocator then keeps them for; None where
+    there is nothing to ask for, under capture (the memory would be free again before the graph is replayed) and
+    where the device has no more."""
+    if not nbytes or torch.cuda.is_current_stream_capturing():
+        return None
+    try:
+        return torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+    except torch.cuda.OutOfMemoryError:
+        return None
+
+
 def gemm_q8_0_f16(w, x, y, m, k, tokens, stream=None):
     """`AttnLayer::apply_output_chunk`'s tiled GEMM (after the gate) over a Q8_0 weight matrix:
-    y[tokens][m], f16 operands.  On the current stream the library's scratch for the rows as f16, where it
-    asks for one, comes from torch's allocator, which keeps it for that stream; not under capture, where the memory
-    would be free again before the graph is replayed, and not for a stream the allocator is not told of."""
-    if stream is None and x is not None:
-        nbytes = lib().hipml_gemm_q8_0_f16_scratch(m, k, tokens)
-        if nbytes and x.data_ptr() and not torch.cuda.is_current_stream_capturing():
-            try:
-                x16 = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
-            except torch.cuda.OutOfMemoryError:
-                x16 = None
-            if x16 is not None:
-                _check(lib().hipml_attn_output_chunk_q8_0(_stream(), _p(w), _p(x), 0, _p(y), m, k, tokens, _p(x16)))
-                return
+    y[tokens][m], f16 operands.  On the current stream with scratch for the rows as f16 where the library asks for it
+    (not for a stream that the allocator is not told of)."""
+    if stream is None and x is not None and x.data_ptr():
+        x16 = _scratch(lib().hipml_gemm_q8_0_f16_scratch(m, k, tokens))
+        if x16 is not None:
+            _check(lib().hipml_attn_output_chunk_q8_0(_stream(), _p(w), _p(x), 0, _p(y), m, k, tokens, _p(x16)))
+            return
     _check(lib().hipml_gemm_q8_0_f16(_stream(stream), _p(w), _p(x), _p(y), m, k, tokens))
 
 
 def output_chunk_q8_0(wo, attn_out, gate, y, m, k, tokens, x16, stream=None):
     """`AttnLayer::apply_output_chunk`: y = W_o (attn_out * sigmoid(gate)); gate may be None; x16 is
-    scratch of tokens*k f16.  attn_out None: x16 already holds the rows as f16."""
+    scratch of tokens*k f16.  attn_out None: x16 already holds the rows as f16 (and keeps them); scratch as above."""
+    if attn_out is None and gate is None and stream is None:
+        packed = _scratch(lib().hipml_gemm_q8_0_f16_rows_scratch(m, k, tokens))
+        if packed is not None:
+            _check(lib().hipml_gemm_q8_0_f16_rows(_stream(), _p(wo), _p(x16), _p(y), m, k, tokens, _p(packed)))
+            return
     _check(lib().hipml_attn_output_chunk_q8_0(_stream(stream), _p(wo), _p(attn_out),
                                               _p(gate) if gate is not None else None, _p(y), m, k,
                                               tokens, _p(x16)))

@@ -1326,14 +1326,36 @@ int hipml_gemm_q8_0_f16(hipml_stream_t stream, const void *w, const float *x, fl
     if (rc)
         return rc;
     return launch_gemm_q8_f16(as_stream(stream), static_cast<const uint8_t *>(w), x, nullptr, y, m, k,
-                              tokens, nullptr);
+                              tokens, nullptr, nullptr);
+}
+
+static size_t gemm_scratch(int m, int k, int tokens, bool f16_rows)
+{
+    if (m < 1 || k < 64 || k % 64 != 0 || tokens < 1)
+        return 0;
+    return gemm_wants_scratch(m, k, tokens, f16_rows) ? (size_t)tokens * (size_t)k * 2 : 0;
 }
 
 size_t hipml_gemm_q8_0_f16_scratch(int m, int k, int tokens)
 {
-    if (m < 1 || k < 64 || k % 64 != 0 || tokens < 1)
-        return 0;
-    return gemm_wants_scratch(m, k, tokens) ? (size_t)tokens * (size_t)k * 2 : 0;
+    return gemm_scratch(m, k, tokens, false);
+}
+
+size_t hipml_gemm_q8_0_f16_rows_scratch(int m, int k, int tokens)
+{
+    return gemm_scratch(m, k, tokens, true);
+}
+
+int hipml_gemm_q8_0_f16_rows(hipml_stream_t stream, const void *w, const void *x16, float *y, int m, int k,
+                             int tokens, void *scratch)
+{
+    clear_error();
+    REQUIRE_PTR(x16);
+    int rc = check_gemm(w, static_cast<const float *>(x16), y, m, k, tokens);
+    if (rc || (rc = check_aligned16(scratch, "scratch")))
+        return rc;
+    return launch_gemm_q8_f16(as_stream(stream), static_cast<const uint8_t *>(w), nullptr, nullptr, y, m, k,
+                              tokens, const_cast<void *>(x16), scratch);
 }
 
 int hipml_attn_output_chunk_q8_0(hipml_stream_t stream, const void *wo, const float *attn_out,
@@ -1350,7 +1372,7 @@ int hipml_attn_output_chunk_q8_0(hipml_stream_t stream, const void *wo, const fl
     if ((rc = check_aligned16(gate, "gate")) || (rc = check_aligned16(x16, "x16")))
         return rc;
     return launch_gemm_q8_f16(as_stream(stream), static_cast<const uint8_t *>(wo), attn_out, gate, y, m, k,
-                              tokens, x16);
+                              tokens, x16, nullptr);
 }
 
 // ---- measurement only --------------------------------------------------------------------------

@@ -157,11 +157,11 @@ int launch_gemv_q8_rows(hipStream_t st, const uint8_t *w, const float *x, float 
 // The same product for a prefill chunk: f16 operands on MFMA, fp32 accumulation (gemm.hip).
 // With a scratch of tokens*k f16 (x16) the activations are gated (gate may be null) and converted once
 // by a first kernel where that is faster or there is a gate; without it the GEMM converts the f32 activations itself
-// (gate must be null).
+// (gate must be null).  x null: x16 holds the rows, and `packed` may be another such scratch.
 int launch_gemm_q8_f16(hipStream_t st, const uint8_t *w, const float *x, const float *gate, float *y, int m,
-                       int k, int tokens, void *x16);
+                       int k, int tokens, void *x16, void *packed);
 // Whether a scratch makes the product without a gate faster.
-bool gemm_wants_scratch(int m, int k, int tokens);
+bool gemm_wants_scratch(int m, int k, int tokens, bool f16_rows);
 // Raise the projection kernels' dynamic LDS limit (once per process; called by hipml_attn_init).
 int proj_init();
 int gemm_init();

@@ -571,14 +571,17 @@ __global__ void __launch_bounds__(640) gemm_q8_few_kernel(const uint8_t *__restr
 // KB, P slices of 32 k ahead, and no other wave of the workgroup reads them; only the weights, which every consumer wave
 // needs, go through LDS, KU = 4 units a step, staged by NP producer waves (each half of a step's units of BT / (NP / 2) groups
 // of 16 rows, SETS steps ahead).  Consumers: 16 AT tokens x 16 BT weight rows each, NC of them side by side in tokens.
+// WB: slices of weight operands in registers, two, or one where the tile leaves no room for more (512 x 96).
 // Loaded from the row-major rows instead it is slower than the kernel above: 16 rows 10,240 bytes apart lie in two of
 // L2's channels.
 // What bounds it (12288 x 5120 over 672 tokens, 384 x 96 tiles, timing-only builds): MFMAs and LDS reads alone 72 us, all
-// of it 86, packing 5.  The kernel above with f32 rows before, this one with packing, us: 12288 x 5120 over 96 / 117 / 200 /
-// 382 / 672 / 1,500 / 2,048 tokens 37.1 / 39.6 / 58.3 / 85.3 / 115 / 227 / 290 -> 32.4 / 33.8 / 47.8 / 60.2 / 96.7 / 184 /
-// 252; after a gate 5120 x 6144 over 200 / 382 / 672 / 1,024 / 1,500 42.4 / 50.7 / 69.0 / 94.8 / 128 -> 33.5 / 43.3 / 62.3 /
-// 82.7 / 110.  Tried on it: weights by LDS DMA and dequantized by the consumers (behind the kernel above), weights loaded
-// non-temporally (20 % slower), three or four steps of weights on the way (no gain).
+// of it 86, packing 5.  The kernel above with f32 rows before, this one with packing, us: 12288 x 5120 over 117 / 200 / 382 /
+// 672 / 1,024 / 2,048 tokens 38.5 / 56.2 / 81.7 / 112 / 143 / 278 -> 32.8 / 44.6 / 58.2 / 94.0 / 121 / 233 (over 1,024 and
+// 2,048 without the 512 x 96 tile 137 and 252); after a gate 5120 x 6144 over 200 / 382 / 672 / 1,024 / 1,500 41.4 / 47.5 /
+// 66.8 / 91.9 / 123 -> 33.0 / 42.0 / 60.5 / 81.5 / 110; over f16 rows 5120 x 6144 over 200 / 382 / 512 / 1,024 / 1,500 37.2 /
+// 41.8 / 59.0 / 81.3 / 109 -> 32.7 / 38.4 / 50.1 / 77.0 / 99.9.  Tried on it: weights by LDS DMA and dequantized by the
+// consumers (behind the kernel above), weights loaded non-temporally (20 % slower), three or four steps of weights on the
+// way (no gain), one slice of weight operands in the smaller tiles too (1 % slower), 384 x 128 (60 % slower).
 // Layout of the packed activations: slice s (k from 32 s) starts at s * tokens * 64 bytes, its tokens from 16 t at t * 1024;
 // there value k = 32 s + 8 g + e of token 16 t + i at (g * n + i) * 16 + 2 e, with n = 16, or what is left of the tokens.
 // That is tokens * k * 2 bytes in all.
@@ -623,7 +626,28 @@ __global__ void __launch_bounds__(256) pack_f16_kernel(const float *__restrict__
         }
 }
 
-template <int NC, int AT, int BT, int NP, int P, int SETS>
+// The same of rows that are f16 already.
+__global__ void __launch_bounds__(256) pack_rows_f16_kernel(const uint8_t *__restrict__ rows, uint8_t *__restrict__ x16, int k,
+                                                            int tokens)
+{
+    const int lane = threadIdx.x & 63, i = lane & 15, g = lane >> 4;
+    const int t0 = blockIdx.x * 16, n = tokens - t0 < 16 ? tokens - t0 : 16;
+    const int s0 = (blockIdx.y * 4 + (threadIdx.x >> 6)) * 4;
+    if (i >= n)
+        return;
+    const uint8_t *const from = rows + (size_t)(t0 + i) * k * 2 + g * 16;
+    half8 v[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+        if (s0 + u < k / 32)
+            v[u] = *reinterpret_cast<const half8 *>(from + (s0 + u) * 64);
+#pragma unroll
+    for (int u = 0; u < 4; u++)
+        if (s0 + u < k / 32)
+            *reinterpret_cast<half8 *>(x16 + (size_t)(s0 + u) * tokens * 64 + (size_t)t0 * 64 + (g * n + i) * 16) = v[u];
+}
+
+template <int NC, int AT, int BT, int NP, int P, int SETS, int WB>
 __global__ void __launch_bounds__(64 * (NP + NC)) gemm_q8_direct_kernel(const uint8_t *__restrict__ w,
                                                                         const void *__restrict__ xv,
                                                                         float *__restrict__ y, int m, int k, int tokens)
@@ -697,7 +721,7 @@ __global__ void __launch_bounds__(64 * (NP + NC)) gemm_q8_direct_kernel(const ui
     const uint8_t *const xb = static_cast<const uint8_t *>(xv);
     const size_t xstep = (size_t)tokens * 64;
     const int nslice = k / 32;
-    half8 X[P][AT], W[2][BT];
+    half8 X[P][AT], W[WB][BT];
     auto load = [&](int v, int s) {
         const uint8_t *const xs = xb + (size_t)(s < nslice ? s : nslice - 1) * xstep;
 #pragma unroll
@@ -708,14 +732,14 @@ __global__ void __launch_bounds__(64 * (NP + NC)) gemm_q8_direct_kernel(const ui
     auto read = [&](int kk) {
 #pragma unroll
         for (int b = 0; b < BT; b++)
-            W[kk & 1][b] = *reinterpret_cast<const half8 *>(wl + b * 16 * kPitch + kk * 64);
+            W[kk % WB][b] = *reinterpret_cast<const half8 *>(wl + b * 16 * kPitch + kk * 64);
     };
     auto multiply = [&](int kk) { // (weights as the first operand: a lane's four sums are one token's)
 #pragma unroll
         for (int b = 0; b < BT; b++)
 #pragma unroll
             for (int a = 0; a < AT; a++)
-                acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(W[kk & 1][b], X[kk % P][a], acc[a][b], 0, 0, 0);
+                acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(W[kk % WB][b], X[kk % P][a], acc[a][b], 0, 0, 0);
     };
     constexpr int kSlices = 2 * KU;
     static_assert(kSlices % P == 0, "the records of a step are named at compile time");
@@ -723,23 +747,38 @@ __global__ void __launch_bounds__(64 * (NP + NC)) gemm_q8_direct_kernel(const ui
     for (int v = 0; v < P; v++)
         load(v, v);
     __syncthreads();
-    read(0);
-    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (WB == 2) {
+        read(0);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll 1
-    for (int s = 0; s < nsteps; s++) {
+        for (int s = 0; s < nsteps; s++) {
 #pragma unroll
-        for (int kk = 0; kk + 1 < kSlices; kk++) {
-            read(kk + 1);
-            multiply(kk);
-            load(kk % P, s * kSlices + kk + P);
+            for (int kk = 0; kk + 1 < kSlices; kk++) {
+                read(kk + 1);
+                multiply(kk);
+                load(kk % P, s * kSlices + kk + P);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            __syncthreads(); // (behind the step's last reads, in front of its last products)
+            wl += s & 1 ? -kBuf : kBuf;
+            read(0); // (behind the last step: whatever the other buffer holds, not used)
+            multiply(kSlices - 1);
+            load((kSlices - 1) % P, s * kSlices + kSlices - 1 + P);
             __builtin_amdgcn_sched_barrier(0);
         }
-        __syncthreads();
-        wl += s & 1 ? -kBuf : kBuf;
-        read(0); // (behind the last step: whatever the other buffer holds, not used)
-        multiply(kSlices - 1);
-        load((kSlices - 1) % P, s * kSlices + kSlices - 1 + P);
-        __builtin_amdgcn_sched_barrier(0);
+    } else {
+#pragma unroll 1
+        for (int s = 0; s < nsteps; s++) {
+#pragma unroll
+            for (int kk = 0; kk < kSlices; kk++) {
+                read(kk);
+                multiply(kk);
+                load(kk % P, s * kSlices + kk + P);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            __syncthreads();
+            wl += s & 1 ? -kBuf : kBuf;
+        }
     }
     // C tile: lane holds column lm (token), rows 4 lg + j (weight rows)
     const bool wide = (m & 3) == 0 && (reinterpret_cast<uintptr_t>(y) & 15) == 0;
@@ -935,30 +974,32 @@ struct DirectTile {
 constexpr DirectTile kDirectTiles[] = {
     {128, 32, 0.21f}, {128, 48, 0.248f}, {128, 64, 0.281f},  {128, 96, 0.366f},  {192, 48, 0.298f}, {192, 96, 0.522f},
     {192, 128, 0.691f}, {256, 64, 0.476f}, {256, 96, 0.668f}, {256, 128, 0.807f}, {384, 96, 0.825f},
+    {512, 96, 1.2f},
 };
 constexpr int kDirectNTiles = sizeof(kDirectTiles) / sizeof(kDirectTiles[0]);
 
 template <typename F>
 static bool with_direct_kernel(int i, F &&f)
 {
-#define HIPML_DIRECT(idx, NC, AT, BT, NP, P)                                                                           \
+#define HIPML_DIRECT(idx, NC, AT, BT, NP, P, WB)                                                                       \
     case idx: {                                                                                                       \
         constexpr int tt = 16 * AT * NC, tm = 16 * BT;                                                                \
         static_assert(kDirectTiles[idx].tt == tt && kDirectTiles[idx].tm == tm, "the table");                         \
-        return f(&gemm_q8_direct_kernel<NC, AT, BT, NP, P, 2>, 64 * (NP + NC), tt, tm, 2 * tm * gemm_pitch(4));       \
+        return f(&gemm_q8_direct_kernel<NC, AT, BT, NP, P, 2, WB>, 64 * (NP + NC), tt, tm, 2 * tm * gemm_pitch(4));       \
     }
     switch (i) {
-        HIPML_DIRECT(0, 4, 2, 2, 4, 8)
-        HIPML_DIRECT(1, 4, 2, 3, 6, 8)
-        HIPML_DIRECT(2, 4, 2, 4, 4, 4)
-        HIPML_DIRECT(3, 4, 2, 6, 4, 4)
-        HIPML_DIRECT(4, 4, 3, 3, 6, 4)
-        HIPML_DIRECT(5, 4, 3, 6, 4, 4)
-        HIPML_DIRECT(6, 4, 3, 8, 4, 4)
-        HIPML_DIRECT(7, 4, 4, 4, 4, 4)
-        HIPML_DIRECT(8, 4, 4, 6, 4, 4)
-        HIPML_DIRECT(9, 4, 4, 8, 4, 2)
-        HIPML_DIRECT(10, 8, 3, 6, 4, 4)
+        HIPML_DIRECT(0, 4, 2, 2, 4, 8, 2)
+        HIPML_DIRECT(1, 4, 2, 3, 6, 8, 2)
+        HIPML_DIRECT(2, 4, 2, 4, 4, 4, 2)
+        HIPML_DIRECT(3, 4, 2, 6, 4, 4, 2)
+        HIPML_DIRECT(4, 4, 3, 3, 6, 4, 2)
+        HIPML_DIRECT(5, 4, 3, 6, 4, 4, 2)
+        HIPML_DIRECT(6, 4, 3, 8, 4, 4, 2)
+        HIPML_DIRECT(7, 4, 4, 4, 4, 4, 2)
+        HIPML_DIRECT(8, 4, 4, 6, 4, 4, 2)
+        HIPML_DIRECT(9, 4, 4, 8, 4, 2, 2)
+        HIPML_DIRECT(10, 8, 3, 6, 4, 4, 2)
+        HIPML_DIRECT(11, 8, 4, 6, 4, 2, 1)
     default:
         return false;
     }
@@ -991,13 +1032,15 @@ int gemm_init()
 // the pass is not paid back (6000 x 1024 over 1,024 / 2,048 tokens: 24.3 / 39.3 us, with scratch 25.6 / 41.4).  The costs
 // are fitted like the table above at 253 shapes (1,024 to 16,384 weight rows, 32 to 2,048 tokens): 1 % behind the best of
 // all routes and tiles on average, 11 % at most; 12 % ahead of the tiles over the rows as they lie, at 3 shapes more than
-// 2 % behind them.
+// 2 % behind them (the 512 x 96 tile, added later, to its time at six shapes).
+// Rows that are f16 already are multiplied as they lie or packed, by a pass of half the bytes.
 enum class GemmRoute { kNone, kRows, kRowsF16, kPacked };
+enum class GemmRows { kF32, kGated, kF16 };
 struct GemmChoice {
     GemmRoute route;
     int tile;
 };
-static GemmChoice gemm_choice(int m, int k, int tokens, bool sectors, bool gated_rows)
+static GemmChoice gemm_choice(int m, int k, int tokens, bool sectors, GemmRows rows)
 {
     GemmChoice best = {GemmRoute::kNone, -1};
     float best_cost = 0.0f;
@@ -1007,16 +1050,19 @@ static GemmChoice gemm_choice(int m, int k, int tokens, bool sectors, bool gated
             best_cost = cost;
         }
     };
-    const float units = (float)(k / 64), pass = 3.0f + 0.75e-6f * (float)tokens * (float)k;
+    const float units = (float)(k / 64), values = (float)tokens * (float)k;
+    const float pass = 3.0f + (rows == GemmRows::kF16 ? 0.4e-6f : 0.75e-6f) * values;
     float cost = 0.0f;
-    if (!gated_rows) {
+    if (rows == GemmRows::kF32) {
         const int tile = gemm_tile(m, k, tokens, sectors, false, &cost);
         offer(GemmRoute::kRows, tile, units * cost);
-        if (k < 2048)
-            return best;
     }
+    if (rows != GemmRows::kGated && k < 2048 && best.tile >= 0)
+        return best;
     const int tile = gemm_tile(m, k, tokens, sectors, true, &cost);
-    offer(GemmRoute::kRowsF16, tile, units * cost + pass);
+    offer(GemmRoute::kRowsF16, tile, units * cost + (rows == GemmRows::kF16 ? 0.0f : pass));
+    if (rows == GemmRows::kF16 && k < 2048)
+        return best;
     // (32-bit offsets in a tile's weights and in a slice of the activations, and the passes' grids)
     if (sectors && tile >= 0 && k <= 1 << 23 && tokens <= 1 << 22)
         for (int i = 0; i < kDirectNTiles; i++) {
@@ -1026,51 +1072,58 @@ static GemmChoice gemm_choice(int m, int k, int tokens, bool sectors, bool gated
     return best;
 }
 
-// For tests and the benchmark: 100 x route (1 as they lie, 2 rounded, 3 packed) + tile of a call with scratch.
-extern "C" int hipml_dbg_gemm_choice(int m, int k, int tokens, int sectors, int gated_rows)
+// For tests and the benchmark: 100 x route (1 as they lie, 2 f16 row by row, 3 packed) + tile of a call with scratch, over
+// rows in f32 (0), in f32 with a gate (1), in f16 (2).
+extern "C" int hipml_dbg_gemm_choice(int m, int k, int tokens, int sectors, int rows)
 {
-    const GemmChoice c = gemm_choice(m, k, tokens, sectors != 0, gated_rows != 0);
+    const GemmChoice c = gemm_choice(m, k, tokens, sectors != 0, (GemmRows)rows);
     return c.tile < 0 ? -1 : 100 * (int)c.route + c.tile;
 }
 
-// Whether scratch for the rows as f16 makes hipml_gemm_q8_0_f16's product faster (W at a 64-byte boundary).
-bool gemm_wants_scratch(int m, int k, int tokens)
+// Whether scratch makes the product over rows without a gate faster (W at a 64-byte boundary): over f32 rows scratch for
+// them as f16, over f16 rows scratch to pack them into.
+bool gemm_wants_scratch(int m, int k, int tokens, bool f16_rows)
 {
-    const GemmChoice c = gemm_choice(m, k, tokens, k % 1024 == 0, false);
-    return c.tile >= 0 && c.route != GemmRoute::kRows;
+    const GemmChoice c = gemm_choice(m, k, tokens, k % 1024 == 0, f16_rows ? GemmRows::kF16 : GemmRows::kF32);
+    return c.tile >= 0 && c.route != (f16_rows ? GemmRoute::kRowsF16 : GemmRoute::kRows);
 }
 
-// x16 != nullptr: scratch for the rows as f16 (the gate, if any, applied first); x == nullptr: x16 already holds them, row
-// by row.
+// f32 rows x (with a gate or without): x16 != nullptr is scratch for them as f16.  x == nullptr: x16 holds the rows as
+// f16, row by row, and packed != nullptr is scratch to pack them into.
 int launch_gemm_q8_f16(hipStream_t st, const uint8_t *w, const float *x, const float *gate, float *y, int m,
-                       int k, int tokens, void *x16)
+                       int k, int tokens, void *x16, void *packed)
 {
     // (rows of weights in whole 64-byte sectors)
     const bool sectors = k % 1024 == 0 && (reinterpret_cast<uintptr_t>(w) & 63) == 0;
+    const bool f16_rows = x == nullptr;
     GemmChoice c;
-    if (x != nullptr && x16 != nullptr)
-        c = gemm_choice(m, k, tokens, sectors, gate != nullptr);
+    if (f16_rows ? packed != nullptr : x16 != nullptr)
+        c = gemm_choice(m, k, tokens, sectors, f16_rows ? GemmRows::kF16 : gate != nullptr ? GemmRows::kGated : GemmRows::kF32);
     else
-        c = {x != nullptr ? GemmRoute::kRows : GemmRoute::kRowsF16,
-             gemm_tile(m, k, tokens, sectors, x == nullptr, nullptr)};
+        c = {f16_rows ? GemmRoute::kRowsF16 : GemmRoute::kRows, gemm_tile(m, k, tokens, sectors, f16_rows, nullptr)};
     if (c.tile < 0)
         return fail(HIPML_ATTN_E_RANGE, "k %d: 32 rows of activations exceed 4 GB", k);
     const void *act = c.route == GemmRoute::kRows ? static_cast<const void *>(x) : x16;
+    int rc = 0;
     if (c.route == GemmRoute::kPacked) {
-        HIPML_LAUNCH(pack_f16_kernel, dim3((unsigned)((tokens + 15) / 16), (unsigned)((k / 32 + 15) / 16), 1),
-                     dim3(256, 1, 1), 0, st, x, gate, static_cast<uint8_t *>(x16), k, tokens);
-        int rc = launched("pack_f16");
-        if (rc)
-            return rc;
-    } else if (c.route == GemmRoute::kRowsF16 && x != nullptr) {
+        const dim3 grid((unsigned)((tokens + 15) / 16), (unsigned)((k / 32 + 15) / 16), 1);
+        if (f16_rows) {
+            act = packed;
+            HIPML_LAUNCH(pack_rows_f16_kernel, grid, dim3(256, 1, 1), 0, st, static_cast<const uint8_t *>(x16),
+                         static_cast<uint8_t *>(packed), k, tokens);
+        } else {
+            HIPML_LAUNCH(pack_f16_kernel, grid, dim3(256, 1, 1), 0, st, x, gate, static_cast<uint8_t *>(x16), k, tokens);
+        }
+        rc = launched("pack_f16");
+    } else if (c.route == GemmRoute::kRowsF16 && !f16_rows) {
         const size_t n8 = (size_t)tokens * k / 8;
         HIPML_LAUNCH(gate_f16_kernel, dim3((unsigned)((n8 + 255) / 256), 1, 1), dim3(256, 1, 1), 0, st,
                            reinterpret_cast<const float4v *>(x), reinterpret_cast<const float4v *>(gate),
                            static_cast<half8 *>(x16), n8);
-        int rc = launched("gate_f16");
-        if (rc)
-            return rc;
+        rc = launched("gate_f16");
     }
+    if (rc)
+        return rc;
     auto go = [&](auto kernel, int threads, int tt, int tm, int lds) {
         HIPML_LAUNCH(kernel, dim3((unsigned)((m + tm - 1) / tm), (unsigned)((tokens + tt - 1) / tt), 1),
                      dim3(threads, 1, 1), lds, st, w, act, y, m, k, tokens);

@@ -539,6 +539,14 @@ int hipml_gemm_q8_0_f16(hipml_stream_t stream, const void *w, const float *x, fl
  * scratch may gain nothing).  Launches nothing; for arguments the product refuses, 0. */
 size_t hipml_gemm_q8_0_f16_scratch(int m, int k, int tokens);
 
+/* The same product over rows that are f16 already (x16: [tokens][k], 16-byte aligned, left as it is):
+ * hipml_attn_output_chunk_q8_0 with attn_out == NULL, and its bits.  `scratch` may be NULL or, 16-byte aligned
+ * and in use until the product is done, as many bytes as hipml_gemm_q8_0_f16_rows_scratch names: it is faster
+ * with them where that is not 0 (the same conditions as hipml_gemm_q8_0_f16_scratch). */
+int hipml_gemm_q8_0_f16_rows(hipml_stream_t stream, const void *w, const void *x16, float *y, int m, int k,
+                             int tokens, void *scratch);
+size_t hipml_gemm_q8_0_f16_rows_scratch(int m, int k, int tokens);
+
 /* The output side of a chunk in one call: y = W_o (attn_out * sigmoid(gate)), gate may be NULL (the
  * rows are already gated, e.g. by hipml_attn_chunk_q8_split_gate).  x16 is caller scratch of
  * tokens*k f16 (2 bytes each, 16-byte aligned; the attention's split scratch is free by then): a

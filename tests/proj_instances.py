@@ -15,10 +15,10 @@ def gemm_tile(m, k, tokens, x16):
     return attn.lib().hipml_dbg_gemm_tile(m, k, tokens, sectors, x16), sectors
 
 
-def gemm_choice(m, k, tokens, gated):
-    """100 * route (1 the rows as they lie, 2 rounded to f16, 3 packed) + place in the route's table of tiles, for a call with
-    scratch, W at a 64-byte boundary."""
-    return attn.lib().hipml_dbg_gemm_choice(m, k, tokens, int(k % 1024 == 0), gated)
+def gemm_choice(m, k, tokens, rows):
+    """100 * route (1 the rows as they lie, 2 f16 row by row, 3 packed) + place in the route's table of tiles, for a call with
+    scratch over f32 rows (0), f32 rows with a gate (1) or f16 rows (2), W at a 64-byte boundary."""
+    return attn.lib().hipml_dbg_gemm_choice(m, k, tokens, int(k % 1024 == 0), rows)
 
 
 # (weight rows, k, activation rows): ragged in the rows of a workgroup, k of 19 chunks or 37 units (uneven shares of the
@@ -43,9 +43,9 @@ TILES = [
     (239, 1024, 51, 1), (2173, 3072, 97, 1), (7363, 3072, 97, 1), (10996, 3072, 258, 1), (10996, 3072, 396, 1),
     (12380, 3072, 396, 1), (7363, 3072, 985, 1), (10996, 3072, 143, 1), (1069, 3072, 210, 1), (7363, 3072, 210, 1),
 ]
-# (weight rows, k, tokens, gated rows): calls with scratch whose rows are packed, every tile of that kernel once
+# (weight rows, k, tokens, rows as above): calls with scratch whose rows are packed, every tile of that kernel once
 PACKED = [
     (5522, 1024, 69, 1), (8280, 3072, 69, 0), (12380, 2048, 69, 1), (16554, 1024, 69, 1), (8280, 1024, 137, 1),
-    (16554, 1024, 137, 1), (12380, 2048, 273, 0), (12380, 3072, 137, 1), (8280, 2048, 392, 1), (12380, 2048, 392, 0),
-    (16554, 2048, 273, 0),
+    (16554, 1024, 137, 1), (12380, 2048, 273, 0), (12380, 3072, 137, 1), (8280, 2048, 392, 1), (12380, 2048, 392, 2),
+    (16554, 2048, 273, 0), (10996, 2048, 789, 0),
 ]

@@ -67,20 +67,26 @@ def test_tile(m, k, tokens, x16):
     assert torch.equal(y[tokens // 2], one[0])
 
 
-@pytest.mark.parametrize("m,k,tokens,gated", inst.PACKED)
-def test_packed_tile(m, k, tokens, gated):
+@pytest.mark.parametrize("m,k,tokens,kind", inst.PACKED)
+def test_packed_tile(m, k, tokens, kind):
     w, _, _, x = inputs(m, k, tokens)
-    gate = torch.randn((tokens, k), device="cuda") if gated else None
+    gate = torch.randn((tokens, k), device="cuda") if kind == 1 else None
     rows = x
-    if gated:
+    if kind == 1:
         rows = torch.empty_like(x)
         attn.q_gate(x, gate, rows, tokens * k)
     y, want = padded(tokens, m), padded(tokens, m)
-    x16 = torch.full((tokens + 1, k), 3.0, dtype=torch.float16, device="cuda")
-    attn.output_chunk_q8_0(w, x, gate, y, m, k, tokens, x16)
-    attn.gemm_q8_0_f16(w, rows, want, m, k, tokens, stream=torch.cuda.current_stream())  # (no scratch: test_tile's kernels)
+    scratch = torch.full((tokens + 1, k), 3.0, dtype=torch.float16, device="cuda")
+    plain = torch.cuda.current_stream()  # (a stream by name: no scratch, test_tile's kernels)
+    attn.gemm_q8_0_f16(w, rows, want, m, k, tokens, stream=plain)
+    ready = rows.to(torch.float16)
+    if kind == 2:
+        assert attn.lib().hipml_gemm_q8_0_f16_rows(plain.cuda_stream, w.data_ptr(), ready.data_ptr(), y.data_ptr(), m, k, tokens,
+                                                   scratch.data_ptr()) == 0
+    else:
+        attn.output_chunk_q8_0(w, x, gate, y, m, k, tokens, scratch)
     assert torch.equal(y[:tokens], want[:tokens]) and bool(y[tokens].isnan().all())
-    assert bool((x16[tokens] == 3.0).all())
+    assert bool((scratch[tokens] == 3.0).all()) and torch.equal(ready, rows.to(torch.float16))
 
 
 def test_scratch_of_a_call_on_the_current_stream_and_under_capture():
@@ -91,11 +97,15 @@ def test_scratch_of_a_call_on_the_current_stream_and_under_capture():
     attn.gemm_q8_0_f16(w, x, want, m, k, tokens, stream=torch.cuda.current_stream())
     side = torch.cuda.Stream()
     side.wait_stream(torch.cuda.current_stream())
+    h, z = x.to(torch.float16), padded(tokens, m)
+    assert attn.lib().hipml_gemm_q8_0_f16_rows_scratch(m, k, tokens) == tokens * k * 2
+    torch.cuda.synchronize()
     with torch.cuda.stream(side):
         for _ in range(3):  # (the scratch of one call is the next one's)
             attn.gemm_q8_0_f16(w, x, y, m, k, tokens)
+            attn.output_chunk_q8_0(w, None, None, z, m, k, tokens, h)
     torch.cuda.current_stream().wait_stream(side)
-    assert torch.equal(y[:tokens], want[:tokens])
+    assert torch.equal(y[:tokens], want[:tokens]) and torch.equal(z[:tokens], want[:tokens])
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
         attn.gemm_q8_0_f16(w, x, y, m, k, tokens)

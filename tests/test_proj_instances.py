@@ -28,7 +28,7 @@ def test_every_packed_tile_has_a_shape():
     named = {inst.gemm_choice(*shape) for shape in inst.PACKED}
     assert len(named) == len(inst.PACKED) and min(named) >= 300
     tokens = [*range(1, 700, 17), *range(700, 4200, 83)]
-    taken = {inst.gemm_choice(m, k, t, g): (m, k, t, g) for m in M for t in tokens for k in (1024, 5120) for g in (0, 1)}
+    taken = {inst.gemm_choice(m, k, t, g): (m, k, t, g) for m in M for t in tokens for k in (1024, 5120) for g in (0, 1, 2)}
     assert not {c: s for c, s in taken.items() if c >= 300 and c not in named}
 
 
