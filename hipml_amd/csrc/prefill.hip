@@ -1339,6 +1339,8 @@ chunk_f16_t64_kernel(const ChunkArgs a)
 // (32 keys per step, dequantized by those two waves, single-buffered: 4 x 34 KB of LDS); the four
 // partial results of a head meet in LDS at the end, each wave finishing 64 of the 256 output
 // columns, gate included.  672 tokens x 24 heads are 252 such workgroups, one round of the chip.
+// SPLIT: few tokens behind a prefix are few such workgroups, so the keys are cut once more, across workgroups; these leave
+// their four slices' common sums, exponent and denominator to chunk_combine_kernel (chunk_wg_splits says when and how many).
 //
 // A step is a VALU slot (dequantize the next K tile and this step's V tile, softmax) and an MFMA slot (PV
 // of this step, scores of the next), each closed by a workgroup barrier; see the loop.
@@ -1362,7 +1364,7 @@ constexpr float kWgLazy = 8.0f;                // growth of a maximum (log2 unit
 // ROPE: the query rows are rotated (NeoX pairs (k, k + 32) of the first 64 columns, position pos0 + token)
 // between their load and their conversion to f16, with the expressions of the RoPE kernels and
 // without contraction, so the operands are the bits those kernels would have left in memory.
-template <bool Q4, bool ROPE>
+template <bool Q4, bool ROPE, bool SPLIT>
 __global__ void __launch_bounds__(kPfThreads, 1) chunk_wg_kernel(const ChunkArgs a)
 {
     typedef typename HalfOf<Q4>::type Half;
@@ -1379,21 +1381,37 @@ __global__ void __launch_bounds__(kPfThreads, 1) chunk_wg_kernel(const ChunkArgs
     const int sl = wave >> 1;                     // key slice
     const int hp = wave & 1;                      // head of the pair
 
-    // blockIdx.x -> (token tile, kv head, head pair), the token tiles with the most keys first
+    // blockIdx.x -> (token tile, kv head, head pair), the token tiles with the most keys first; SPLIT: (kv head, split, token
+    // tile, head pair), and XCD x takes the x-th eighth of them: the rows of a (kv head, split) pass through few L2s
     const int pairs = (a.group + 1) >> 1;
-    const int per_tt = a.n_kv * pairs;
     const int ntt = (a.tokens + kQTile - 1) / kQTile;
-    const int tt = ntt - 1 - (int)blockIdx.x / per_tt;
-    const int rem = (int)blockIdx.x % per_tt;
-    const int kvh = rem % a.n_kv;
-    const int hq = (rem / a.n_kv) * 2 + hp;
+    int tt, kvh, pair, split = 0;
+    if (SPLIT) {
+        const int total = ntt * pairs * a.n_kv * a.splits, eighth = (total + 7) >> 3;
+        const int item = ((int)blockIdx.x & 7) * eighth + ((int)blockIdx.x >> 3);
+        if (item >= total)
+            return; // (the whole workgroup)
+        const int combo = item / (ntt * pairs), r = item - combo * (ntt * pairs);
+        kvh = combo / a.splits;
+        split = combo - kvh * a.splits;
+        tt = ntt - 1 - r / pairs;
+        pair = r % pairs;
+    } else {
+        const int per_tt = a.n_kv * pairs;
+        tt = ntt - 1 - (int)blockIdx.x / per_tt;
+        const int rem = (int)blockIdx.x % per_tt;
+        kvh = rem % a.n_kv;
+        pair = rem / a.n_kv;
+    }
+    const int hq = pair * 2 + hp;
     const bool task_valid = hq < a.group;        // (an odd group leaves the last pair one head)
     const int head = kvh * a.group + (task_valid ? hq : a.group - 1);
     const int t0 = tt * kQTile;
     const int last_tok = ((tt + 1) * kQTile < a.tokens ? (tt + 1) * kQTile : a.tokens) - 1;
     const int khi = a.pos0 + last_tok + 1;                          // keys the tile's last token sees
-    const int nstep = ((khi + kWgStep - 1) / kWgStep + kWgSlices - 1) / kWgSlices; // per slice, same for all
-    const int kbeg = sl * nstep * kWgStep;                          // this slice's first key
+    const int nslice = SPLIT ? a.splits * kWgSlices : kWgSlices;
+    const int nstep = ((khi + kWgStep - 1) / kWgStep + nslice - 1) / nslice; // per slice, same for all
+    const int kbeg = (split * kWgSlices + sl) * nstep * kWgStep;    // this slice's first key
     const int tok = t0 + ln;
     const int my_last_key = a.pos0 + tok;
     const bool tok_valid = task_valid && tok < a.tokens;
@@ -1677,7 +1695,7 @@ __global__ void __launch_bounds__(kPfThreads, 1) chunk_wg_kernel(const ChunkArgs
     // gate values of the rows it will write are requested first.
     const int orow = lane >> 4, opiece = lane & 15; // output pass r2: token r2 * 4 + orow, 16-byte piece
     float4v gt[8];
-    if (a.gate) {
+    if (!SPLIT && a.gate) {
 #pragma unroll
         for (int r2 = 0; r2 < 8; r2++) {
             const int tr = t0 + r2 * 4 + orow;
@@ -1689,7 +1707,7 @@ __global__ void __launch_bounds__(kPfThreads, 1) chunk_wg_kernel(const ChunkArgs
     float2 *mlx = reinterpret_cast<float2 *>(lds); // [head 2][slice 4][token 32]
     if (lh == 0)
         mlx[(hp * kWgSlices + sl) * kQTile + ln] = make_float2(m_run, l_run);
-    float den = 0.0f, w_mine = 0.0f;
+    float den = 0.0f, w_mine = 0.0f, m_all = -INFINITY;
     float wj[kWgSlices]; // weight of each slice's sums for this lane's token
     auto weights = [&]() { // (after the first barrier below: the table travels with the first accumulators)
         float m = -INFINITY;
@@ -1700,6 +1718,7 @@ __global__ void __launch_bounds__(kPfThreads, 1) chunk_wg_kernel(const ChunkArgs
             if (v[j].y > 0.0f)
                 m = fmaxf(m, v[j].x);
         }
+        m_all = m;
 #pragma unroll
         for (int j = 0; j < kWgSlices; j++) {
             const bool on = v[j].y > 0.0f;
@@ -1758,7 +1777,13 @@ __global__ void __launch_bounds__(kPfThreads, 1) chunk_wg_kernel(const ChunkArgs
         }
         lds_barrier();
     }
-    const float inv = den > 0.0f ? 1.0f / den : 0.0f;
+    // (SPLIT: the sums as they are, with their exponent and denominator for chunk_combine_kernel)
+    const float inv = SPLIT ? 1.0f : den > 0.0f ? 1.0f / den : 0.0f;
+    if (SPLIT && sl == 0 && tok_valid && lh == 0) {
+        const size_t row = ((size_t)split * a.qslots + tok) * a.n_head + head;
+        a.part_ml[row * 2] = m_all;
+        a.part_ml[row * 2 + 1] = den;
+    }
     float16v R[2];
 #pragma unroll
     for (int qd = 0; qd < 4; qd++)
@@ -1783,6 +1808,11 @@ __global__ void __launch_bounds__(kPfThreads, 1) chunk_wg_kernel(const ChunkArgs
         const int r = r2 * 4 + orow;
         float4v x = *reinterpret_cast<const float4v *>(mine + r * kWgOutPitch + opiece * 16);
         if (task_valid && t0 + r < a.tokens) {
+            if (SPLIT) {
+                const size_t row = ((size_t)split * a.qslots + (t0 + r)) * a.n_head + head;
+                *reinterpret_cast<float4v *>(a.part_acc + row * kHeadDim + sl * 64 + opiece * 4) = x;
+                continue;
+            }
             const size_t o = ((size_t)(t0 + r) * a.n_head + head) * kHeadDim + sl * 64 + opiece * 4;
             if (a.gate)
                 x = (float4v){gated(x[0], gt[r2][0]), gated(x[1], gt[r2][1]), gated(x[2], gt[r2][2]),
@@ -2052,16 +2082,22 @@ int prefill_init()
         e = hipFuncSetAttribute(reinterpret_cast<const void *>(&kv_f16_tiles_kernel<true>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, kTilesLds);
     if (e == hipSuccess)
-        e = hipFuncSetAttribute(reinterpret_cast<const void *>(&chunk_wg_kernel<false, false>),
+        e = hipFuncSetAttribute(reinterpret_cast<const void *>(&chunk_wg_kernel<false, false, false>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, kWgLds);
     if (e == hipSuccess)
-        e = hipFuncSetAttribute(reinterpret_cast<const void *>(&chunk_wg_kernel<true, false>),
+        e = hipFuncSetAttribute(reinterpret_cast<const void *>(&chunk_wg_kernel<true, false, false>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, kWgLds);
     if (e == hipSuccess)
-        e = hipFuncSetAttribute(reinterpret_cast<const void *>(&chunk_wg_kernel<false, true>),
+        e = hipFuncSetAttribute(reinterpret_cast<const void *>(&chunk_wg_kernel<false, true, false>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, kWgLds);
     if (e == hipSuccess)
-        e = hipFuncSetAttribute(reinterpret_cast<const void *>(&chunk_wg_kernel<true, true>),
+        e = hipFuncSetAttribute(reinterpret_cast<const void *>(&chunk_wg_kernel<true, true, false>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, kWgLds);
+    if (e == hipSuccess)
+        e = hipFuncSetAttribute(reinterpret_cast<const void *>(&chunk_wg_kernel<false, false, true>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, kWgLds);
+    if (e == hipSuccess)
+        e = hipFuncSetAttribute(reinterpret_cast<const void *>(&chunk_wg_kernel<true, false, true>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, kWgLds);
     if (e != hipSuccess)
         return fail((int)e, "hipFuncSetAttribute(prefill LDS) failed: %d (%s)", (int)e,
@@ -2147,6 +2183,47 @@ int chunk_tile_slices(int pos0, int tokens, int n_head, int n_kv, int most)
     return best;
 }
 
+// Splits of the keys, of at most `splits`, with which chunk_wg_kernel runs a chunk over the cache; 0: chunk_q8_kernel does.
+// That kernel's workgroups hold 32 tokens x 8 heads and write the sums of every slice of the keys to memory: 117 tokens
+// behind 1,500 are 12 of them and take 10 slices, 28 MB written and read again.  This one's hold 32 tokens x 2 heads and
+// bring four slices together in LDS: 48 workgroups and 4 splits, 11 MB; but each dequantizes its K and V for two heads
+// alone, so it falls behind where the keys outweigh that.  By the costs of both, fitted at 102 shapes (4 to 256 tokens
+// behind 64 to 64,000; 5 % rms each): us, tiles of 64 keys and steps of 32 of a slice, rounds of 256 workgroups and how full
+// one is, 8 KB of sums per token and head.  us before / now over 4 @ 256 19.6 / 15.6, 16 @ 500 21.3 / 16.1, 32 @ 2,000 26.9 /
+// 20.7, 32 @ 8,000 42.6 / 31.3, 64 @ 2,000 31.4 / 25.4, 64 @ 32,000 114 / 104, 117 @ 1,500 33.5 / 28.6, 256 @ 1,000 34.7 /
+// 33.0; not taken at 128 @ 4,000 39.8 (here 41), 200 @ 4,000 49.7 (55), 256 @ 8,000 79 (120).
+static int chunk_wg_splits(int pos0, int tokens, int n_head, int n_kv, int splits)
+{
+    const int group = n_head / n_kv, keys = pos0 + tokens;
+    const long long ntt = (tokens + kQTile - 1) / kQTile, wgs = ntt * n_kv * ((group + 1) / 2);
+    if (wgs > 256 || splits < 2) // (without slices: the bits of the unsliced kernel over an f16 copy)
+        return 0;
+    const float sums = (float)tokens * (float)n_head / 24.0f;
+    int best = 0;
+    float best_cost = 0.0f;
+    for (int s = 1; s <= splits && s * wgs <= 256; s++) {
+        const int nslice = kWgSlices * s, steps = ((keys + kWgStep - 1) / kWgStep + nslice - 1) / nslice;
+        const float fill = (float)(s * wgs) / 256.0f;
+        const float cost = s == 1 ? 8.0f + 2.8f * (float)steps
+                                  : 8.6f + (float)steps * (2.94f + 0.22f * fill) + (float)s * (0.233f + 0.0137f * sums);
+        if (best == 0 || cost < best_cost) {
+            best = s;
+            best_cost = cost;
+        }
+    }
+    const int tiles = (keys + kKTile - 1) / kKTile, slice = (tiles + splits - 1) / splits;
+    const long long other = (long long)n_kv * splits * ((ntt * group + kTasks - 1) / kTasks), rounds = (other + 255) / 256;
+    const float fill = (float)other / (256.0f * (float)rounds);
+    const float cost = 12.6f + (float)rounds * (float)slice * (2.53f + fill) + (float)splits * (0.152f + 0.0067f * sums);
+    return best_cost < 0.95f * cost ? best : 0;
+}
+
+// For tests: the above, 0 for chunk_q8_kernel.
+extern "C" int hipml_dbg_chunk_wg_splits(int pos0, int tokens, int n_head, int n_kv, int splits)
+{
+    return chunk_wg_splits(pos0, tokens, n_head, n_kv, splits);
+}
+
 int launch_chunk_q8(hipStream_t st, const float *q, const uint8_t *kc, const uint8_t *vc,
                     float *out, int n_head, int n_kv, int pos0, int tokens, int stride,
                     float *part_acc, float *part_ml, int splits, const float *gate, int q4, void *out16,
@@ -2202,20 +2279,38 @@ int launch_chunk_q8(hipStream_t st, const float *q, const uint8_t *kc, const uin
     a.nblock = (a.ntask + kTasks - 1) / kTasks;
     a.scale_log2 = kLog2e / 16.0f; // 1/sqrt(256), as the reference's chunk launcher fixes it
     a.out16 = nullptr;
-    if (splits == 0 && kv_f16 == nullptr) {
+    const int wg_splits = kv_f16 == nullptr && rope_tab == nullptr && splits >= 2
+                              ? chunk_wg_splits(pos0, tokens, n_head, n_kv, splits) : 0;
+    if ((splits == 0 && kv_f16 == nullptr) || wg_splits == 1) {
         // the key slices stay inside the workgroup: no partial rows, gate and f16 rows in the same launch
         a.out16 = static_cast<_Float16 *>(out16);
         const unsigned wgs = (unsigned)((tokens + kQTile - 1) / kQTile * n_kv * ((a.group + 1) / 2));
         a.rope_tab = rope_tab;
         if (q4 && rope_tab)
-            HIPML_LAUNCH((chunk_wg_kernel<true, true>), dim3(wgs, 1, 1), dim3(kPfThreads, 1, 1), kWgLds, st, a);
+            HIPML_LAUNCH((chunk_wg_kernel<true, true, false>), dim3(wgs, 1, 1), dim3(kPfThreads, 1, 1), kWgLds, st, a);
         else if (q4)
-            HIPML_LAUNCH((chunk_wg_kernel<true, false>), dim3(wgs, 1, 1), dim3(kPfThreads, 1, 1), kWgLds, st, a);
+            HIPML_LAUNCH((chunk_wg_kernel<true, false, false>), dim3(wgs, 1, 1), dim3(kPfThreads, 1, 1), kWgLds, st, a);
         else if (rope_tab)
-            HIPML_LAUNCH((chunk_wg_kernel<false, true>), dim3(wgs, 1, 1), dim3(kPfThreads, 1, 1), kWgLds, st, a);
+            HIPML_LAUNCH((chunk_wg_kernel<false, true, false>), dim3(wgs, 1, 1), dim3(kPfThreads, 1, 1), kWgLds, st, a);
         else
-            HIPML_LAUNCH((chunk_wg_kernel<false, false>), dim3(wgs, 1, 1), dim3(kPfThreads, 1, 1), kWgLds, st, a);
+            HIPML_LAUNCH((chunk_wg_kernel<false, false, false>), dim3(wgs, 1, 1), dim3(kPfThreads, 1, 1), kWgLds, st, a);
         return launched(q4 ? "attn_chunk_q4_wg" : "attn_chunk_q8_wg");
+    }
+    if (wg_splits > 1) {
+        a.splits = wg_splits;
+        const unsigned total = (unsigned)((tokens + kQTile - 1) / kQTile * n_kv * ((a.group + 1) / 2) * a.splits);
+        const dim3 grid((total + 7) / 8 * 8, 1, 1);
+        if (q4)
+            HIPML_LAUNCH((chunk_wg_kernel<true, false, true>), grid, dim3(kPfThreads, 1, 1), kWgLds, st, a);
+        else
+            HIPML_LAUNCH((chunk_wg_kernel<false, false, true>), grid, dim3(kPfThreads, 1, 1), kWgLds, st, a);
+        int rc = launched(q4 ? "attn_chunk_q4_wg_split" : "attn_chunk_q8_wg_split");
+        if (rc)
+            return rc;
+        HIPML_LAUNCH(chunk_combine_kernel, dim3((unsigned)tokens, (unsigned)((n_head + 3) / 4), 1),
+                           dim3(256, 1, 1), 0, st, part_acc, part_ml, out, gate, n_head, a.qslots, a.splits, a.group,
+                           a.ntask, tokens, pos0, 0, 1, static_cast<_Float16 *>(out16));
+        return launched("attn_chunk_combine");
     }
     // slices per block: the last block (most keys) gets `splits`, a block with fewer key tiles gets
     // proportionally fewer, so a chunk near position 0 does not write and re-read `splits` partial

@@ -166,3 +166,39 @@ def test_fused_append_may_leave_the_query_rows_alone():
         res.append((host(kc), host(vc), host(kd)))
     for a, b in zip(*res):
         assert np.array_equal(a.view(np.uint8), b.view(np.uint8))
+
+
+@pytest.mark.parametrize("dtype", [0, 1])
+@pytest.mark.parametrize("tok,pos0,splits,n_head,n_kv", [
+    (1, 164, 2, 24, 4), (33, 227, 2, 24, 4), (4, 200, 8, 24, 4), (31, 500, 4, 24, 4), (64, 2000, 12, 24, 4),
+    (130, 1500, 10, 24, 4), (5, 3000, 16, 6, 2), (70, 900, 6, 14, 2), (17, 333, 3, 8, 1)])
+def test_few_tokens_behind_a_prefix(tok, pos0, splits, n_head, n_kv, dtype):
+    # calls with scratch for slices that the library gives to this kernel, with splits of the keys across workgroups and
+    # without: slices without a key, a last token tile and key step that are ragged, odd numbers of heads per KV head; plain,
+    # gated and as f16 rows, and nothing past the rows or the splits' share of the scratch
+    used = attn.lib().hipml_dbg_chunk_wg_splits(pos0, tok, n_head, n_kv, splits)
+    assert 1 <= used <= splits
+    r = orc.Rng(0xC4A1_0000 + tok * 131 + pos0)
+    stride = pos0 + tok + 3
+    kb = orc.quantize(dtype, r.normal_array((n_kv, stride, HD))).reshape(n_kv, stride, -1)
+    vb = orc.quantize(dtype, r.normal_array((n_kv, stride, HD))).reshape(n_kv, stride, -1)
+    q, gate = r.normal_array((tok, n_head, HD)), dev(r.normal_array((tok, n_head, HD)))
+    qd, kd, vd = dev(q), dev(kb), dev(vb)
+    acc, ml = attn.chunk_scratch(tok, n_head, splits)
+    acc.fill_(7.0), ml.fill_(7.0)
+    shape = (tok + 1, n_head, HD)
+    out, gated_rows, work = (torch.full(shape, float("nan"), device="cuda") for _ in range(3))
+    out16 = torch.full(shape, float("nan"), dtype=torch.float16, device="cuda")
+    args = (n_head, n_kv, HD, pos0, tok, dtype + 1, stride, acc, ml, splits)
+    attn.chunk_attention_q8_split(qd, kd, vd, out, *args)
+    attn.chunk_attention_q8_split_gate(qd, kd, vd, gate, gated_rows, *args)
+    attn.chunk_attention_q8_split_gate_f16(qd, kd, vd, gate, work, out16, *args)
+    two = torch.empty((tok, n_head, HD), device="cuda")
+    attn.q_gate(out[:tok].contiguous(), gate, two)
+    torch.cuda.synchronize()
+    want = orc.attn_chunk_kv(q, kb, vb, n_head, n_kv, HD, pos0, tok, stride, SCALE, n_threads=8, dtype=dtype)
+    assert report(f"chunk {tok}@{pos0}, {used} splits", want, host(out[:tok]), *GATE)[0]
+    assert torch.equal(two, gated_rows[:tok]) and torch.equal(out16[:tok], two.to(torch.float16))
+    assert bool(out[tok].isnan().all()) and bool(gated_rows[tok].isnan().all()) and bool(out16[tok].isnan().all())
+    first_unused = used if used > 1 else 0
+    assert bool((acc[first_unused:] == 7.0).all()) and bool((ml[first_unused:] == 7.0).all())
