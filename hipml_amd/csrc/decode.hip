@@ -436,6 +436,20 @@ __device__ __forceinline__ bool find_work(const DecodeArgs &a, const Front &f, i
         ncols = __builtin_amdgcn_readlane(l_cols, item);
         group = __builtin_amdgcn_readlane(l_nhead, item);
         head0 = __builtin_amdgcn_readlane(l_head0, item);
+        if (split == 0 && nsp < f.splits) {
+            // The splits of this item that no worker takes: empty partials, which the merge skips.  (Here, where a plain
+            // launch does not pass: behind this branch, or behind the worker's own work, the code cost a plain launch of
+            // one sequence 0.35 us at depth 673 and 1.4 at 32,768.)
+            const int empty = f.splits - nsp;
+            for (int e = threadIdx.x; e < ncols * group * empty; e += (int)blockDim.x) {
+                const int n = e / empty, sp = nsp + (e - n * empty);
+                const int col = n / group;
+                const int head = kvh * f.group + head0 + (n - col * group);
+                float *pm = a.part_ml + (size_t)(row0 + col) * a.ml_slot + ((size_t)head * f.splits + sp) * 2;
+                pm[0] = -INFINITY;
+                pm[1] = 0.0f;
+            }
+        }
     } else {
         kvh = blockIdx.x / f.splits;
         split = blockIdx.x - kvh * f.splits;
@@ -478,22 +492,6 @@ __device__ __forceinline__ bool find_work(const DecodeArgs &a, const Front &f, i
     return true;
 }
 
-// Worker launches: the splits of an item that no worker takes get empty partials, which the merge skips.
-__device__ __forceinline__ void leave_empty_splits(const DecodeArgs &a, const Front &f, const Work &wk)
-{
-    if (f.workers > 0 && wk.split == 0 && wk.nsp < f.splits) {
-        const int empty = f.splits - wk.nsp;
-        for (int e = threadIdx.x; e < wk.nvalid * empty; e += (int)blockDim.x) {
-            const int n = e / empty, sp = wk.nsp + (e - n * empty);
-            const int col = n / wk.group;
-            const int head = wk.hbase + (n - col * wk.group);
-            float *pm = a.part_ml + (size_t)(wk.row0 + col) * a.ml_slot + ((size_t)head * f.splits + sp) * 2;
-            pm[0] = -INFINITY;
-            pm[1] = 0.0f;
-        }
-    }
-}
-
 template <int NT, bool Q4, bool PLO>
 __device__ __forceinline__ void decode_body(const DecodeArgs &a)
 {
@@ -514,7 +512,6 @@ __device__ __forceinline__ void decode_body(const DecodeArgs &a)
     Work wk;
     if (!find_work(a, f, lane, wk))
         return;
-    leave_empty_splits(a, f, wk);
     const int kvh = wk.kvh, split = wk.split, nsp = wk.nsp, slot = wk.slot, row0 = wk.row0, ncols = wk.ncols,
               group = wk.group, hbase = wk.hbase, nvalid = wk.nvalid;
 
@@ -1900,13 +1897,11 @@ __global__ void __launch_bounds__(kThreads, 2)
     HIPML_STAMP(stamps_, 1); // work item found
     if (wk.nvalid > 8) { // uniform over the workgroup
         decode_body_dma<true>(a, f, wk HIPML_STAMPS_PASS);
-        leave_empty_splits(a, f, wk);
         HIPML_STAMP(stamps_, 7); // partial stored (not yet acknowledged)
         if (a.merge > 0)
             decode_merge_tail<true>(a, wk HIPML_STAMPS_PASS);
     } else {
         decode_body_dma<false>(a, f, wk HIPML_STAMPS_PASS);
-        leave_empty_splits(a, f, wk);
         HIPML_STAMP(stamps_, 7);
         if (a.merge > 0)
             decode_merge_tail<false>(a, wk HIPML_STAMPS_PASS);
@@ -1931,7 +1926,6 @@ __global__ void __launch_bounds__(kThreads, 2)
     if (!find_work(a, f, threadIdx.x & 63, wk))
         return;
     decode_body_dma<false, true>(a, f, wk HIPML_STAMPS_PASS);
-    leave_empty_splits(a, f, wk);
 }
 
 // Wave-wide reductions without LDS: DPP inside a row of 16 lanes, then the two row-swap
