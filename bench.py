@@ -802,7 +802,7 @@ def row_kernel_name(attn, m, k, rows):
 
 
 # W_o over 672 gated tokens: packed rows, 256 x 64 tiles (100 x route + place in the library's table of tiles)
-GEMM672_CHOICE, GEMM672_KERNEL = 307, "gemm_q8_direct_kernel<4, 4, 4, 4, 4, 2>"
+GEMM672_CHOICE, GEMM672_KERNEL = 307, "gemm_q8_direct_kernel<4, 4, 4, 4, 4, 2, 2>"
 
 
 def bench_gemv(torch, attn, rows, steps, layers, m=5120, k=6144):
