@@ -4,7 +4,7 @@
 // W is [m][k/32] blocks of 34 bytes (f16 scale d, 32 int8), row-major; y[r][row] = sum_k W[row][k] x[r][k]
 // (crates/hipml-core/src/quant.rs:653-675, crates/hipml-core/src/ops.rs:102-104,136-176).
 //
-// gemv_q8_rows_kernel: one or two activation rows over shapes the raw-row kernel does not take, bound by streaming W
+// gemv_q8_rows_kernel: one or two activation rows over shapes gemv_q8_digits_kernel does not take, bound by streaming W
 // once from HBM.
 //   All MFMAs are v_mfma_f32_16x16x32_f16 with A = x (activation rows), B = W (16 weight rows),
 //   one q8 block = one contraction, so the f16 block scale multiplies an exact integer dot product
