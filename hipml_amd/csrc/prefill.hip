@@ -66,7 +66,7 @@ constexpr int kVtRow = 144;
 constexpr int kKTileBytes = kKTile * kKRow;              // 33,792
 constexpr int kVtTileBytes = kHeadDim * kVtRow;          // 36,864
 constexpr int kBufBytesF = kKTileBytes + kVtTileBytes;   // 70,656
-constexpr int kTilesLds = kKTile * kVRow;                // 34,816: one staged tile of kv_f16_tiles_kernel (the V pitch is the larger)
+constexpr int kTilesLds = kVtTileBytes;                 // one tile of kv_f16_tiles_kernel (V^T as it leaves: the largest)
 constexpr int kPfLdsF = 2 * kBufBytesF;                  // 141,312: no Q steps parked, the staging registers are free
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kPfLazy = 8.0f; // growth of a maximum (log2 units) that moves the reference exponent of chunk_q8_kernel
@@ -1962,17 +1962,22 @@ __global__ void __launch_bounds__(256) rows_f16_kernel(const float4v *__restrict
 // The f16 copy of 64-key tiles of a cache: what a chunk workgroup would stage for itself, made once.
 // grid (tiles, n_kv, 2); tile = tile0 + blockIdx.x; rows at or past seq_end repeat row seq_end - 1 (the
 // attention kernels mask them; a later call that brings the rows overwrites the tile).
-// The K rows leave as they lie in LDS; the V tile leaves through the transposing reads of the PV
+// The K rows leave as they lie in LDS; the V tile goes through the transposing reads of the PV
 // product, so row d of the copy holds, for every 16 keys, the eight values of k-group 0 and the eight
-// of k-group 1 in operand order (key (j/4)*8 + g*4 + j%4 of the sixteen at position g*8 + j).
+// of k-group 1 in operand order (key (j/4)*8 + g*4 + j%4 of the sixteen at position g*8 + j), and back into LDS, from where
+// every wave stores its 64 rows in order.  Bound by its bytes: 264 MB for 40,000 rows of q8_0 on four KV heads at 5.5 TB/s.
+// Stored from the transposing reads (16 bytes a lane, 32 rows 144 bytes apart a request) the V tiles took longer than all
+// else: us before -> now over 1 / 672 / 1,536 / 4,096 / 9,216 / 40,000 rows 2.71 / 3.4 / 4.4 / 10.2 / 18.1 / 75.7 -> 2.70 / 3.3 /
+// 4.1 / 7.5 / 14.2 / 47.7, of q4_0 2.68 / 3.3 / 4.2 / 8.6 / 16.5 / 65.8 -> 2.68 / 3.1 / 3.9 / 6.6 / 11.9 / 40.3 (a barrier for the
+// stores of all four waves together: 0.05 more over 1 row).
 template <bool Q4>
 __global__ void __launch_bounds__(256) kv_f16_tiles_kernel(const uint8_t *__restrict__ kc,
                                                            const uint8_t *__restrict__ vc, uint8_t *__restrict__ k16,
                                                            uint8_t *__restrict__ vt, int stride, int tile0,
                                                            int seq_end, int tile_stride)
 {
-    // grid (tiles, n_kv, 2): blockIdx.z = 0 makes the K tile, 1 the V^T tile (35 KB of LDS either way: four
-    // workgroups per CU, which this pass needs more than anything else: it is all latency)
+    // grid (tiles, n_kv, 2): blockIdx.z = 0 makes the K tile, 1 the V^T tile (36 KB of LDS either way: four
+    // workgroups per CU)
     typedef typename HalfOf<Q4>::type Half;
     constexpr int kRowBytes = Q4 ? hipml::kRowBytesQ4 : hipml::kRowBytes;
     constexpr int kUnitBytes = Q4 ? 36 : 68;
@@ -2005,11 +2010,11 @@ __global__ void __launch_bounds__(256) kv_f16_tiles_kernel(const uint8_t *__rest
     } else {
         const int ln = lane & 31, lh = lane >> 5, gl = lane & 15;
         const int vtr_off = (gl >> 2) * kVRow + (((lane >> 4) & 1) * 16 + (gl & 3) * 4) * 2;
-        uint8_t *to = vt + at * kVtTileBytes;
+        uint4v pieces[8];
 #pragma unroll
         for (int o8 = 0; o8 < 8; o8++) {
-            const int o = wave * 8 + o8; // operand (half hk, step u, d tile dt) of the tile's 32
-            const int hk = o >> 4, u = (o >> 3) & 1, dt = o & 7;
+            // operand (half hk, step u, d tile dt) of the tile's 32: a wave's are 64 whole rows
+            const int hk = (o8 >> 1) & 1, u = o8 & 1, dt = wave * 2 + (o8 >> 2);
             const uint8_t *vp = lds + vtr_off + hk * 32 * kVRow + dt * 64;
             const short4v r0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
                 (short4v __attribute__((address_space(3))) *)(vp + ((2 * u) * 8 + lh * 4) * kVRow));
@@ -2017,8 +2022,22 @@ __global__ void __launch_bounds__(256) kv_f16_tiles_kernel(const uint8_t *__rest
                 (short4v __attribute__((address_space(3))) *)(vp + ((2 * u + 1) * 8 + lh * 4) * kVRow));
             const uint32_t *w0 = reinterpret_cast<const uint32_t *>(&r0), *w1 = reinterpret_cast<const uint32_t *>(&r1);
             const uint4v piece = {w0[0], w0[1], w1[0], w1[1]};
-            *reinterpret_cast<uint4v *>(to + (dt * 32 + ln) * kVtRow + (hk * 32 + u * 16 + lh * 8) * 2) = piece;
+            pieces[o8] = piece;
         }
+        __syncthreads(); // everybody has read the tile
+        uint8_t *mine = lds + wave * (64 * kVtRow); // this wave's rows
+#pragma unroll
+        for (int o8 = 0; o8 < 8; o8++)
+            *reinterpret_cast<uint4v *>(mine + ((o8 >> 2) * 32 + ln) * kVtRow + (((o8 >> 1) & 1) * 32 + (o8 & 1) * 16 + lh * 8) * 2) =
+                pieces[o8];
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // this wave's own writes
+        __builtin_amdgcn_wave_barrier();
+        const uint4v *from = reinterpret_cast<const uint4v *>(mine) + lane;
+        uint4v *to = reinterpret_cast<uint4v *>(vt + at * kVtTileBytes) + wave * (64 * kVtRow / 16) + lane;
+        static_assert(kVtTileBytes == 4 * 64 * kVtRow && kVtRow % 16 == 0, "four waves, whole pieces");
+#pragma unroll
+        for (int i = 0; i < kVtRow / 16; i++)
+            to[i * 64] = from[i * 64];
     }
 }
 
