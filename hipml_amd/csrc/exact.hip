@@ -556,6 +556,8 @@ struct FrontAppend {
 // them, 2 = the same to q4_0 -- the K wave keeps its row in registers (element lane + 64 j in slot
 // j, so a half-wave holds one block of 32, as the append kernels' 32-lane groups do) and n_kv more
 // waves per row take the V rows.  Same expressions on the same values: the bits of the two launches.
+typedef float float4a4 __attribute__((ext_vector_type(4), aligned(4))); // (rows at any 4-byte boundary)
+
 template <int ENC>
 __global__ void __launch_bounds__(256) front_kernel(
     const float *__restrict__ qg, float *__restrict__ q, float *__restrict__ gate, float *k,
@@ -565,8 +567,9 @@ __global__ void __launch_bounds__(256) front_kernel(
 {
     __shared__ float buf[4][kHeadDim];
     // (the wave's number as a scalar: row, head and addresses are scalar arithmetic then.  us over 1 / 16 / 672 / 1,024 / 2,048
-    // rows 3.26 / 3.58 / 15.9 / 23.4 / 40.8 -> 3.15 / 3.48 / 15.4 / 23.0 / 39.6.  Tried: 16 bytes a lane for the q rows, 17.3 us
-    // over 672: the tree's exchanges four times over)
+    // rows 3.26 / 3.58 / 15.9 / 23.4 / 40.8 -> 3.15 / 3.48 / 15.4 / 23.0 / 39.6; with the gate's half, which is copied as it is,
+    // 16 bytes a lane 3.07 / 3.34 / 14.8 / 22.6 / 39.2, 5.7 TB/s read and written.  Tried: 16 bytes a lane for the q rows,
+    // 17.3 us over 672: the tree's exchanges four times over)
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int per_row = n_heads + n_kv;
     const int idx = blockIdx.x * 4 + wave;
@@ -607,18 +610,16 @@ __global__ void __launch_bounds__(256) front_kernel(
 
     // everything this wave will need from memory is asked for here: the row, the gate half, the norm
     // weights and the rotation's cos/sin (the position does not depend on the data)
-    float x[4], wv[4], g[4];
+    float x[4], wv[4];
+    float4a4 g; // (copied as it is: 16 bytes a lane)
 #pragma unroll
     for (int j = 0; j < 4; j++)
         x[j] = src[lane + 64 * j];
 #pragma unroll
     for (int j = 0; j < 4; j++)
         wv[j] = w[lane + 64 * j];
-    if (is_q) {
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-            g[j] = src[kHeadDim + lane + 64 * j];
-    }
+    if (is_q)
+        g = *reinterpret_cast<const float4a4 *>(src + kHeadDim + 4 * lane);
     const int half = n_rot >> 1;
     const int sect = s0 + s1 + s2 + s3;
     float cs[4], sn[4];
@@ -644,12 +645,8 @@ __global__ void __launch_bounds__(256) front_kernel(
             rope_cs(tab, tab_rows, half, c, p, n_rot, theta, cs[j], sn[j]);
         }
     }
-    if (is_q) {
-        float *gd = gate + ((size_t)row * n_heads + h) * kHeadDim;
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-            gd[lane + 64 * j] = g[j];
-    }
+    if (is_q)
+        *reinterpret_cast<float4a4 *>(gate + ((size_t)row * n_heads + h) * kHeadDim + 4 * lane) = g;
     const float a0 = x[0] * x[0] + x[2] * x[2]; // off = 128
     const float a1 = x[1] * x[1] + x[3] * x[3];
     const float sum = tree_sum64(a0 + a1);      // off = 64, then 32 .. 1

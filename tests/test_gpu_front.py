@@ -75,6 +75,27 @@ def test_chunk_front_is_bit_exact(rows, pos0):
         assert np.array_equal(gk[t].ravel(), wk), f"k row {t}"
 
 
+@pytest.mark.parametrize("qg_off,gate_off", [(1, 0), (0, 1), (2, 3)])
+def test_rows_and_gate_at_any_float(qg_off, gate_off):
+    # the gate half is copied 16 bytes a lane: from and to any 4-byte boundary, and nothing beside it
+    rows = 3
+    qg, k, qw, kw = front_inputs(0xF20C, rows)
+    src = torch.zeros(qg.size + 8, device="cuda")
+    src[qg_off:qg_off + qg.size] = dev(qg).ravel()
+    n = rows * N_HEADS * HD
+    out = torch.full((n + 8,), 7.0, device="cuda")
+    q = torch.empty((rows, N_HEADS, HD), device="cuda")
+    want_q = torch.empty_like(q)
+    want = torch.empty_like(q)
+    attn.chunk_front(src[qg_off:], dev(k), q, out[gate_off:], dev(qw), dev(kw), N_HEADS, N_KV, HD, N_ROT, THETA, EPS, 29,
+                     rows)
+    attn.chunk_front(dev(qg), dev(k), want_q, want, dev(qw), dev(kw), N_HEADS, N_KV, HD, N_ROT, THETA, EPS, 29, rows)
+    torch.cuda.synchronize()
+    assert torch.equal(out[gate_off:gate_off + n], want.ravel()) and np.array_equal(host(want), qg[:, :, HD:])
+    assert torch.equal(q, want_q)
+    assert bool((out[:gate_off] == 7.0).all()) and bool((out[gate_off + n:] == 7.0).all())
+
+
 def test_front_then_existing_rope_free_path_agree():
     # with unit weights and a head already of unit RMS the norm is (nearly) the identity; the
     # rotation must be the stand-alone M-RoPE kernel's bits on the normalised values
