@@ -308,7 +308,9 @@ __global__ void __launch_bounds__(64 * WAVES, TILES == 1 ? 2 : 1) gemv_q8_rows_k
 // that this lane has read.  A lane's sum is thus one float for its weight row, its blocks and an activation row.
 // Three and four activation rows fill the operand without zeros: v_mfma_i32_16x16x32_i8 over one block, A row 4 r + i digit
 // i of row r, lane (lm, lg) holding 8 bytes of weight row lm and, in C, the digit sums of activation row lg; it adds the
-// blocks 0 .. 3 of a group of four apart, as the lanes lg above do, so that a row's bits are the same.
+// blocks 0 .. 3 of a group of four apart, as the lanes lg above do, so that a row's bits are the same.  Five to eight rows are
+// two such operands over the same weight registers, or two passes of four (gemv_digits_cut): a wave makes the second set's
+// digits in the place of the first's, whose operands it holds by then.
 //
 // A workgroup takes `ng` groups of GR weight rows (up to 16).  Wave v of V owns the runs v, v + V, ... of 512 values of k (544
 // bytes of each row: with runs of 272 a pass over 12288 x 5120 reads 1 us slower) for all of them, makes the digits of its
@@ -355,16 +357,14 @@ __device__ __forceinline__ void wait_vm()
     asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory");
 }
 
-
-
-// LDS of a wave: a group's rows of a run; the digits of its activations of the run, 2 KB a row, and their scales (four rows
-// beside groups of ten, which twelve waves have no room for, exchange those by ds_bpermute: 0.6 us), whose place takes the wave's sums when they are in
-// registers, unless a wave has several runs; behind the waves 64 zero bytes.
-constexpr bool gemv_digit_table(int r, int gr) { return r < 4 || gr != 10; }
-constexpr int gemv_digit_x(int r, int gr) { return (gemv_digit_table(r, gr) ? 2048 + 64 : 2048) * r; }
+// LDS of a wave: a group's rows of a run; the digits of its activations of the run, 2 KB a row of a set (eight rows are two
+// sets of four, one after the other in the same place), beside one and two rows their scales, whose place takes the wave's
+// sums when they are in registers, unless a wave has several runs; behind the waves 64 zero bytes.
+constexpr int gemv_digit_set(int r) { return r > 4 ? 4 : r; }
+constexpr int gemv_digit_x(int r) { return (r > 2 ? 2048 : 2048 + 64) * gemv_digit_set(r); }
 constexpr int gemv_digit_wave(int r, int gr, int ng, bool more)
 {
-    const int sums = ng * r * 64, x = gemv_digit_x(r, gr);
+    const int sums = ng * r * 64, x = gemv_digit_x(r);
     return gr * kRunBytes + (more ? x + sums : (x > sums ? x : sums));
 }
 static_assert(kDigitMaxWaves * gemv_digit_wave(4, 4, 11, true) + 64 <= kDigitLds, "groups of four rows always fit");
@@ -396,6 +396,7 @@ __global__ void __launch_bounds__(64 * kDigitMaxWaves) gemv_q8_digits_kernel(con
 {
     constexpr int kPerRow = kRunBytes / 16, kPieces = GR * kPerRow; // 16-byte pieces of a unit: a group's rows of a run
     constexpr int NI = (kPieces + 63) / 64;
+    constexpr int S = gemv_digit_set(R), kSets = R / S; // activation rows of a set, and sets
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int waves = (int)(blockDim.x >> 6);
@@ -409,22 +410,27 @@ __global__ void __launch_bounds__(64 * kDigitMaxWaves) gemv_q8_digits_kernel(con
     const bool more = nrun > waves;
     const int area = gemv_digit_wave(R, GR, ng, more);
     uint8_t *const place = lds + wave * area;
-    uint8_t *const xdig = place + kPieces * 16; // [chunk][row][block][digit][32], then the scales [chunk][row][block]
-    uint32_t *const scales = reinterpret_cast<uint32_t *>(xdig + 2048 * R);
-    auto sums_of = [&](int v) { return reinterpret_cast<float *>(lds + v * area + kPieces * 16 + (more ? gemv_digit_x(R, GR) : 0)); };
+    // one and two rows: [chunk][row][block][digit][32], then the scales [chunk][row][block]; more: [chunk][row][block][four
+    // values][digit][4], a lane's own 16 bytes (one write without bank conflicts for four that took four times as long: 0.4 us
+    // of a call over four rows), the scales by ds_bpermute
+    uint8_t *const xdig = place + kPieces * 16;
+    uint32_t *const scales = reinterpret_cast<uint32_t *>(xdig + 2048 * S);
+    auto sums_of = [&](int v) { return reinterpret_cast<float *>(lds + v * area + kPieces * 16 + (more ? gemv_digit_x(R) : 0)); };
     uint8_t *const zeros = lds + waves * area;
     const uint32_t place_at = proj_lds_address(place), xdig_at = proj_lds_address(xdig);
     const uint8_t *const xb = reinterpret_cast<const uint8_t *>(x + (size_t)r0 * k);
 
-    // ---- requests (a chunk past the end of k repeats the one before it, rows past the live ones the last: never used) ----
-    auto issue_x = [&](int run) {
+    // ---- requests (a chunk past the end of k repeats the one before it: never used; rows past the live ones are not asked
+    // for, and what is made of their places is not stored) ----
+    auto issue_x = [&](int run, int set) {
 #pragma unroll
         for (int cc = 0; cc < 2; cc++) {
             const int c = 2 * run + cc < nchunk ? 2 * run + cc : nchunk - 1;
 #pragma unroll
-            for (int r = 0; r < R; r++)
-                proj_dma16<false>(xdig_at + (cc * R + r) * 1024u, xb + (size_t)(r < nrows ? r : nrows - 1) * ((size_t)k * 4) + (size_t)c * 1024,
-                                  lane * 16u);
+            for (int r = 0; r < S; r++)
+                if (set * S + r < nrows)
+                    proj_dma16<false>(xdig_at + (cc * S + r) * 1024u, xb + (size_t)(set * S + r) * ((size_t)k * 4) + (size_t)c * 1024,
+                                      lane * 16u);
         }
     };
     // piece p = 64 j + lane of a unit: row p / kPerRow of the group, 16 bytes p % kPerRow of its run
@@ -447,13 +453,13 @@ __global__ void __launch_bounds__(64 * kDigitMaxWaves) gemv_q8_digits_kernel(con
                 proj_dma16<true>(place_at + j * 1024, src, woff[j] < most ? woff[j] : most);
     };
     if (wave < nrun) {
-        issue_x(wave);
+        issue_x(wave, 0);
         issue_w(wave, 0);
     }
     if (lane < 16) // (every wave writes the same zeros)
         reinterpret_cast<uint32_t *>(zeros)[lane] = 0;
 
-    constexpr bool kDense = R > 2, kTable = gemv_digit_table(R, GR);
+    constexpr bool kDense = R > 2;
     // (not dense) lanes lg = 0 .. 3 take the blocks 0, 2, 1, 3 of a group of four: their first dwords then start in different
     // banks; payload dwords start 2 bytes into the first dword, or at the next; A row lm is a digit of the block of lanes
     // lm / 4.  (Rows past a group's repeat its last: never stored.)
@@ -463,107 +469,126 @@ __global__ void __launch_bounds__(64 * kDigitMaxWaves) gemv_q8_digits_kernel(con
     const bool live = (lm >> 2) == lg;
     const uint8_t *const wrow = place + (lm < GR ? lm : GR - 1) * kRunBytes;
     const uint8_t *const wlane = kDense ? wrow + lg * 8 : wrow + blk * kQ8Block - 2 * (int)odd;
-    const uint8_t *const xlane = kDense  ? xdig + ((lm >> 2) < R ? lm >> 2 : R - 1) * 1024 + (lm & 3) * 32 + lg * 8
+    const uint8_t *const xlane = kDense  ? xdig + ((lm >> 2) < S ? lm >> 2 : S - 1) * 1024 + (lm & 3) * 4 + lg * 32
                                  : live ? xdig + blk * 128 + (lm & 3) * 32
                                         : zeros;
     const int xstep = kDense || live ? 1 : 0;
 
     for (int run = wave; run < nrun; run += waves) {
         const bool two = 2 * run + 1 < nchunk; // (the last run may be one chunk)
-        if (run == wave)
-            wait_vm<NI>(); // (the first weights are still travelling)
-        else
-            wait_vm<0>();
-        // ---- digits, in place: four values a lane, eight lanes a block ----------------------------------------------
-        float4v f[2 * R];
-#pragma unroll
-        for (int e = 0; e < 2 * R; e++)
-            f[e] = *reinterpret_cast<const float4v *>(xdig + e * 1024 + lane * 16);
-        asm volatile("" ::: "memory"); // (one wave: every lane has read before any writes)
-        __builtin_amdgcn_wave_barrier();
-        uint32_t sbits[kTable ? 1 : 2 * R]; // of block lane / 8
-#pragma unroll
-        for (int e = 0; e < 2 * R; e++) {
-            uint32_t b[4];
-            float v[4];
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                v[i] = f[e][i]; // (__builtin_bit_cast of a vector's element itself takes element 0)
-                b[i] = __builtin_bit_cast(uint32_t, v[i]) & 0x7fffffffu;
-            }
-            // the block's largest magnitude, as bits (infinities and NaN above all numbers)
-            uint32_t top = b[0] > b[1] ? b[0] : b[1];
-            top = top > b[2] ? top : b[2];
-            top = top > b[3] ? top : b[3];
-            uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)top, 0xB1, 0xf, 0xf, true); // lane ^ 1
-            top = o > top ? o : top;
-            o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)top, 0x4E, 0xf, 0xf, true); // lane ^ 2
-            top = o > top ? o : top;
-            o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)top, 0x141, 0xf, 0xf, true); // lane 7 - i of eight
-            top = o > top ? o : top;
-            const uint32_t most = 0x47ffe000u; // 131,008: beyond it activations count as that much
-            uint32_t bad = 0;
-            if (__builtin_amdgcn_ballot_w64(top > most) != 0) { // (in no block of the wave, as a rule)
-                bad = top >= 0x7f800000u ? 0x7fc00000u : 0u;
-                top = top < most ? top : most;
-#pragma unroll
-                for (int i = 0; i < 4; i++)
-                    v[i] = __builtin_amdgcn_fmed3f(v[i], -131008.0f, 131008.0f);
-            }
-            uint32_t ex = top & 0x7f800000u; // |x| < 2^(ex - 126)
-            ex = ex > (30u << 23) ? ex : 30u << 23;
-            const float up = __builtin_bit_cast(float, (283u << 23) - ex); // 2^(156 - ex)
-            uint32_t z[4];
-#pragma unroll
-            for (int i = 0; i < 4; i++) // X + 0x808080: the three low digits, each 128 up, and the fourth
-                z[i] = (uint32_t)(int)fmaf(v[i], up, 8421504.0f);
-            const uint32_t p0 = __builtin_amdgcn_perm(z[1], z[0], 0x05010400u), p1 = __builtin_amdgcn_perm(z[3], z[2], 0x05010400u);
-            const uint32_t p2 = __builtin_amdgcn_perm(z[1], z[0], 0x07030602u), p3 = __builtin_amdgcn_perm(z[3], z[2], 0x07030602u);
-            uint32_t *const dst = reinterpret_cast<uint32_t *>(xdig + e * 1024 + (lane >> 3) * 128 + (lane & 7) * 4);
-            dst[0] = __builtin_amdgcn_perm(p1, p0, 0x05040100u) ^ 0x80808080u;
-            dst[8] = __builtin_amdgcn_perm(p1, p0, 0x07060302u) ^ 0x80808080u;
-            dst[16] = __builtin_amdgcn_perm(p3, p2, 0x05040100u) ^ 0x80808080u;
-            dst[24] = __builtin_amdgcn_perm(p3, p2, 0x07060302u);
-            const uint32_t scale = (ex - (29u << 23)) | bad; // 2^(ex - 156), or NaN
-            if (!kTable)
-                sbits[kTable ? 0 : e] = scale;
-            else if ((lane & 7) == 0)
-                scales[e * 8 + (lane >> 3)] = scale;
-        }
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_wave_barrier();
         int4v a[kDense ? 1 : 2 * R][2][2];
-        uint2v ad[kDense ? 2 : 1][8];
+        uint2v ad[kDense ? kSets : 1][2][8];
         float sx[kDense ? 2 : 2 * R][kDense ? 8 : 2];
-        if constexpr (kDense) {
+        uint32_t pair[kSets][8]; // (dense) the scales of a block of either chunk, as the upper halves of their floats
+#pragma unroll
+        for (int set = 0; set < kSets; set++) {
+            if (set > 0) {
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); // (the set before is in registers)
+                issue_x(run, set);
+            }
+            if (run == wave && set == 0)
+                wait_vm<NI>(); // (the first weights are still travelling)
+            else
+                wait_vm<0>();
+            // ---- digits, in place: four values a lane, eight lanes a block ------------------------------------------
+            float4v f[2 * S];
+#pragma unroll
+            for (int e = 0; e < 2 * S; e++)
+                f[e] = *reinterpret_cast<const float4v *>(xdig + e * 1024 + lane * 16);
+            asm volatile("" ::: "memory"); // (one wave: every lane has read before any writes)
+            __builtin_amdgcn_wave_barrier();
+            uint32_t scale_of[2] = {0, 0}; // (dense) of block lane / 8 and row lane % 8
+#pragma unroll
+            for (int e = 0; e < 2 * S; e++) {
+                if (kDense && set * S + e % S >= nrows)
+                    continue;
+                uint32_t b[4];
+                float v[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    v[i] = f[e][i]; // (__builtin_bit_cast of a vector's element itself takes element 0)
+                    b[i] = __builtin_bit_cast(uint32_t, v[i]) & 0x7fffffffu;
+                }
+                // the block's largest magnitude, as bits (infinities and NaN above all numbers)
+                uint32_t top = b[0] > b[1] ? b[0] : b[1];
+                top = top > b[2] ? top : b[2];
+                top = top > b[3] ? top : b[3];
+                uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)top, 0xB1, 0xf, 0xf, true); // lane ^ 1
+                top = o > top ? o : top;
+                o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)top, 0x4E, 0xf, 0xf, true); // lane ^ 2
+                top = o > top ? o : top;
+                o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)top, 0x141, 0xf, 0xf, true); // lane 7 - i of eight
+                top = o > top ? o : top;
+                const uint32_t most = 0x47ffe000u; // 131,008: beyond it activations count as that much
+                uint32_t bad = 0;
+                if (__builtin_amdgcn_ballot_w64(top > most) != 0) { // (in no block of the wave, as a rule)
+                    bad = top >= 0x7f800000u ? 0x7fc00000u : 0u;
+                    top = top < most ? top : most;
+#pragma unroll
+                    for (int i = 0; i < 4; i++)
+                        v[i] = __builtin_amdgcn_fmed3f(v[i], -131008.0f, 131008.0f);
+                }
+                uint32_t ex = top & 0x7f800000u; // |x| < 2^(ex - 126)
+                ex = ex > (30u << 23) ? ex : 30u << 23;
+                const float up = __builtin_bit_cast(float, (283u << 23) - ex); // 2^(156 - ex)
+                uint32_t z[4];
+#pragma unroll
+                for (int i = 0; i < 4; i++) // X + 0x808080: the three low digits, each 128 up, and the fourth
+                    z[i] = (uint32_t)(int)fmaf(v[i], up, 8421504.0f);
+                const uint32_t p0 = __builtin_amdgcn_perm(z[1], z[0], 0x05010400u), p1 = __builtin_amdgcn_perm(z[3], z[2], 0x05010400u);
+                const uint32_t p2 = __builtin_amdgcn_perm(z[1], z[0], 0x07030602u), p3 = __builtin_amdgcn_perm(z[3], z[2], 0x07030602u);
+                const uint4v digit = {__builtin_amdgcn_perm(p1, p0, 0x05040100u) ^ 0x80808080u,
+                                      __builtin_amdgcn_perm(p1, p0, 0x07060302u) ^ 0x80808080u,
+                                      __builtin_amdgcn_perm(p3, p2, 0x05040100u) ^ 0x80808080u,
+                                      __builtin_amdgcn_perm(p3, p2, 0x07060302u)}; // each of four values
+                if (kDense) {
+                    *reinterpret_cast<uint4v *>(xdig + e * 1024 + lane * 16) = digit;
+                } else {
+                    uint32_t *const dst = reinterpret_cast<uint32_t *>(xdig + e * 1024 + (lane >> 3) * 128 + (lane & 7) * 4);
+#pragma unroll
+                    for (int i = 0; i < 4; i++)
+                        dst[8 * i] = digit[i];
+                }
+                const uint32_t scale = (ex - (29u << 23)) | bad; // 2^(ex - 156), or NaN
+                if (kDense)
+                    scale_of[e / S] = (lane & 7) == e % S ? scale : scale_of[e / S];
+                else if ((lane & 7) == 0)
+                    scales[e * 8 + (lane >> 3)] = scale;
+            }
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_wave_barrier();
+            if constexpr (kDense) {
+                const uint32_t both = __builtin_amdgcn_perm(scale_of[1], scale_of[0], 0x07060302u);
+#pragma unroll
+                for (int q = 0; q < 8; q++) {
+                    pair[set][q] = (uint32_t)__builtin_amdgcn_ds_bpermute(q * 32 + lg * 4, (int)both); // of row lg
+#pragma unroll
+                    for (int cc = 0; cc < 2; cc++) {
+                        const uint32_t *const src = reinterpret_cast<const uint32_t *>(xlane + cc * (S * 1024) + q * 128);
+                        ad[set][cc][q] = (uint2v){src[0], src[4]};
+                    }
+                }
+            } else {
+#pragma unroll
+                for (int e = 0; e < 2 * R; e++)
+#pragma unroll
+                    for (int h = 0; h < 2; h++) {
+#pragma unroll
+                        for (int j = 0; j < 2; j++)
+                            a[e][h][j] = *reinterpret_cast<const int4v *>(xlane + (e * 1024 + h * 512) * xstep + j * 16);
+                        sx[e][h] = __builtin_bit_cast(float, scales[e * 8 + h * 4 + blk]);
+                    }
+            }
+        }
+        auto scale_at = [&](int set, int cc, int q) {
+            return __builtin_bit_cast(float, cc == 0 ? pair[set][q] << 16 : pair[set][q] & 0xffff0000u);
+        };
+        if constexpr (kDense && kSets == 1) { // (two sets have no registers for them)
 #pragma unroll
             for (int cc = 0; cc < 2; cc++)
 #pragma unroll
-                for (int q = 0; q < 8; q++) {
-                    ad[cc][q] = *reinterpret_cast<const uint2v *>(xlane + cc * (R * 1024) + q * 128);
-                    uint32_t t; // of row lg
-                    if constexpr (kTable) {
-                        t = scales[(cc * R + (lg < R ? lg : R - 1)) * 8 + q];
-                    } else {
-                        t = (uint32_t)__builtin_amdgcn_ds_bpermute(q * 32, (int)sbits[cc * R]);
-#pragma unroll
-                        for (int r = 1; r < R; r++) {
-                            const uint32_t u = (uint32_t)__builtin_amdgcn_ds_bpermute(q * 32, (int)sbits[cc * R + r]);
-                            t = lg == r ? u : t;
-                        }
-                    }
-                    sx[cc][q] = __builtin_bit_cast(float, t);
-                }
-        } else {
-#pragma unroll
-            for (int e = 0; e < 2 * R; e++)
-#pragma unroll
-                for (int h = 0; h < 2; h++) {
-#pragma unroll
-                    for (int j = 0; j < 2; j++)
-                        a[e][h][j] = *reinterpret_cast<const int4v *>(xlane + (e * 1024 + h * 512) * xstep + j * 16);
-                    sx[e][h] = __builtin_bit_cast(float, scales[e * 8 + h * 4 + blk]);
-                }
+                for (int q = 0; q < 8; q++)
+                    sx[cc][q] = scale_at(0, cc, q);
         }
         // ---- the groups ---------------------------------------------------------------------------------------------
 #pragma unroll 1
@@ -574,12 +599,19 @@ __global__ void __launch_bounds__(64 * kDigitMaxWaves) gemv_q8_digits_kernel(con
                 if (g + 1 < ng) {
                     issue_w(run, g + 1);
                 } else if (run + waves < nrun) {
-                    issue_x(run + waves);
-                    issue_w(run + waves, 0);
+                    int next = run + waves;
+                    asm volatile("" : "+s"(next)); // (or its addresses are made ahead of the loop and held through it)
+                    issue_x(next, 0);
+                    issue_w(next, 0);
                 }
             };
             if constexpr (kDense) {
-                float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f}; // blocks 0 .. 3 of a group of four
+                float acc[kSets][4] = {}; // blocks 0 .. 3 of a group of four
+                if constexpr (kSets > 1) { // (or they are taken apart ahead of the loop, into 32 registers)
+#pragma unroll
+                    for (int e = 0; e < 8 * kSets; e++)
+                        asm volatile("" : "+v"(pair[e >> 3][e & 7]));
+                }
 #pragma unroll
                 for (int cc = 0; cc < 2; cc++) {
                     uint32_t q0[8], q1[8], q2[4];
@@ -604,22 +636,50 @@ __global__ void __launch_bounds__(64 * kDigitMaxWaves) gemv_q8_digits_kernel(con
                         if (!two)
                             break;
                     }
-#pragma unroll
-                    for (int q = 0; q < 8; q++) {
+                    int4v p[8][kSets];
+                    auto multiply = [&](int q) {
                         uint2v v = {q0[q], q1[q]};
                         if ((q & 1) == 0) {
                             v[0] = __builtin_amdgcn_alignbit(q1[q], q0[q], 16);
                             v[1] = __builtin_amdgcn_alignbit(q2[q >> 1], q1[q], 16);
                         }
-                        int4v p = {0, 0, 0, 0};
-                        p = __builtin_amdgcn_mfma_i32_16x16x32_i8(__builtin_bit_cast(long, ad[cc][q]), __builtin_bit_cast(long, v), p, 0, 0, 0);
-                        acc[q & 3] = add_digits(p, (float)dh[q] * sx[cc][q], acc[q & 3]);
+                        if (kSets > 1)
+                            asm volatile("" : "+v"(v));
+#pragma unroll
+                        for (int set = 0; set < kSets; set++) {
+                            p[q][set] = (int4v){0, 0, 0, 0};
+                            p[q][set] = __builtin_amdgcn_mfma_i32_16x16x32_i8(__builtin_bit_cast(long, ad[set][cc][q]),
+                                                                              __builtin_bit_cast(long, v), p[q][set], 0, 0, 0);
+                        }
+                    };
+                    auto add = [&](int q) {
+#pragma unroll
+                        for (int set = 0; set < kSets; set++) {
+                            const float of = kSets == 1 ? sx[cc][q] : scale_at(set, cc, q);
+                            float &to = acc[set][q & 3];
+                            to = add_digits(p[q][set], (float)dh[q] * of, to);
+                            if (kSets > 1)
+                                asm volatile("" : "+v"(to));
+                        }
+                    };
+                    // (two sets: the empty statements keep the products of three blocks in registers at a time; the compiler
+                    // puts all of a chunk's matrix instructions first)
+                    multiply(0);
+                    multiply(1);
+#pragma unroll
+                    for (int q = 0; q < 8; q++) {
+                        if (q + 2 < 8)
+                            multiply(q + 2);
+                        add(q);
                     }
                 }
-                const float s = (acc[0] + acc[2]) + (acc[1] + acc[3]);
-                float *const to = sums_of(wave) + (g * R + lg) * 16 + lm;
-                if (lg < R)
-                    *to = run == wave ? s : *to + s;
+#pragma unroll
+                for (int set = 0; set < kSets; set++) {
+                    const float s = (acc[set][0] + acc[set][2]) + (acc[set][1] + acc[set][3]);
+                    float *const to = sums_of(wave) + (g * R + set * S + lg) * 16 + lm;
+                    if (lg < S)
+                        *to = run == wave ? s : *to + s;
+                }
             } else {
                 float acc[R];
 #pragma unroll
@@ -1173,34 +1233,54 @@ static int launch_gemv_variant(hipStream_t st, const uint8_t *w, const float *x,
     return launch_gemv_xg<WAVES, TILES, CH, 8>(st, w, x, y, m, k, rows, rp);
 }
 
-// How a call of `rows` activation rows is cut: R rows a pass, waves, ng groups of gr weight rows per workgroup.
+// How a call of `rows` activation rows is cut: R rows a pass, waves, ng groups of gr weight rows per workgroup, and rounds of
+// the chip (ng = 0: no group fits the LDS).
 struct DigitsCut {
-    int r, waves, gr, ng, lds;
+    int r, waves, gr, ng, lds, rounds, n;
 };
 // One round of the chip's 256 CUs, every CU the same bytes, up to 48 weight rows per workgroup (44 where a wave has several
-// runs and keeps its sums apart) and several such rounds beyond; of the groups that fit the LDS the one that pads the rows
-// least.  A unit is what a wave has in flight: 10 and 8 weight rows keep the stream evener than 12 and 16 (12288 x 5120, one
-// row, 4 / 8 / 10 / 12 / 16 weight rows: 15.3 / 12.8 / 12.8 / 13.7 / 14.6 us), but with three and four rows a unit's fixed
-// work tells (three: 19.4 / 15.8 / 15.8 / 15.3 / 16.2).
-static const int kDigitGroups[] = {12, 10, 8, 4};
-static DigitsCut gemv_digits_cut(int m, int k, int rows)
+// runs and keeps its sums apart) and several such rounds beyond: n rows a workgroup.  A unit is what a wave has in flight
+// and has a fixed share of work: of the groups that fit the LDS the one for which the units cost least, as two rows more
+// than they have (over 60 matrices of 256 to 14,336 weight rows and k of 2,560 to 8,192 the mean call takes 0.1 to 0.6 %
+// longer than with its best group; the group that pads least, which this rule replaced, 4 to 7 %, 7168 x 5120 over three
+// rows 14.2 us with seven units of four rows, 12.1 with three of ten).  Four rows only for a workgroup that has no more, or
+// where nothing else fits.
+static const int kDigitGroups[] = {12, 8, 10, 4};
+static constexpr bool gemv_digit_group(int r, int gr) { return r <= 2 ? gr < 12 : r <= 4 || gr > 4; }
+static DigitsCut gemv_digits_cut_of(int m, int k, int rows, int r)
 {
-    DigitsCut c = {0, 0, 0, 0, 0};
+    DigitsCut c = {r, 0, 0, 0, 0, 0, 0};
     // (the waves follow from k alone: a row's bits depend on them)
     const int nrun = ((k >> 8) + 1) >> 1, passes = (nrun + kDigitMaxWaves - 1) / kDigitMaxWaves;
     c.waves = (nrun + passes - 1) / passes;
-    c.r = rows < 4 ? rows : 4;
-    const long long all = (long long)m * ((rows + c.r - 1) / c.r), most = 256 * (passes > 1 ? 44 : 48);
-    const long long round = 256 * ((all + most - 1) / most);
-    const int n = (int)((all + round - 1) / round);
+    const long long all = (long long)m * ((rows + r - 1) / r), most = 256 * (passes > 1 ? 44 : 48);
+    c.rounds = (int)((all + most - 1) / most);
+    c.n = (int)((all + 256LL * c.rounds - 1) / (256LL * c.rounds));
     for (int gr : kDigitGroups) {
-        const int ng = (n + gr - 1) / gr;
-        const int lds = c.waves * gemv_digit_wave(c.r, gr, ng, passes > 1) + 64;
-        if (lds <= kDigitLds && (c.r > 2 || gr < 12) && (c.ng == 0 || ng * gr < c.ng * c.gr)) {
+        const int ng = (c.n + gr - 1) / gr;
+        const int lds = c.waves * gemv_digit_wave(r, gr, ng, passes > 1) + 64;
+        if (lds > kDigitLds || !gemv_digit_group(r, gr))
+            continue;
+        if (c.ng == 0 || (gr == 4 ? c.n <= 4 : ng * (gr + 2) < c.ng * (c.gr + 2))) {
             c.gr = gr;
             c.ng = ng;
             c.lds = lds;
         }
+    }
+    return c;
+}
+// Five to eight rows: one pass over W with two sets of operands, or two passes of four rows.  One pass wherever two have more
+// rounds (12288 x 5120 over 5 / 8 rows: one 19.6 / 21.4 us, two 28.0 / 28.7; 7168 x 5120: one 16.2 / 17.5, two 22 / 24).
+// Within one round two passes read W twice but leave the second set's digits to other workgroups (1024 x 5120: one 9.6 /
+// 10.7, two 7.5 / 7.6); up to six rows and from about 4,600 weight rows on the bytes tell (5120 x 6144 over 5 / 6 / 8 rows:
+// one 14.7 / 15.3 / 16.2, two 15.5 / 15.5 / 15.6).
+static DigitsCut gemv_digits_cut(int m, int k, int rows)
+{
+    const DigitsCut c = gemv_digits_cut_of(m, k, rows, rows < 4 ? rows : 4);
+    if (rows > 4) {
+        const DigitsCut one = gemv_digits_cut_of(m, k, rows, 8);
+        if (one.ng > 0 && (c.rounds > one.rounds || (rows <= 6 && c.n > 36)))
+            return one;
     }
     return c;
 }
@@ -1209,14 +1289,16 @@ static DigitsCut gemv_digits_cut(int m, int k, int rows)
 template <int R, typename F>
 static void with_gemv_digits_kernel(int gr, F &&f)
 {
-    if (gr == 4)
-        return f(&gemv_q8_digits_kernel<R, 4>);
-    if (gr == 8)
-        return f(&gemv_q8_digits_kernel<R, 8>);
-    if (gr == 10)
-        return f(&gemv_q8_digits_kernel<R, 10>);
-    if constexpr (R > 2)
-        f(&gemv_q8_digits_kernel<R, 12>);
+    auto is = [&](auto g) {
+        constexpr int GR = decltype(g)::value;
+        if constexpr (gemv_digit_group(R, GR))
+            if (gr == GR)
+                f(&gemv_q8_digits_kernel<R, GR>);
+    };
+    is(std::integral_constant<int, 4>{});
+    is(std::integral_constant<int, 8>{});
+    is(std::integral_constant<int, 10>{});
+    is(std::integral_constant<int, 12>{});
 }
 
 // Which kernel a call takes, and its variant: kRows: -; kDigits: activation rows a pass, weight rows of a group, -; kBlocks
@@ -1309,7 +1391,7 @@ static void launch_gemv_digits(hipStream_t st, const uint8_t *w, const float *x,
 {
     const DigitsCut c = gemv_digits_cut(m, k, rows);
     const dim3 grid((unsigned)((m + c.ng * c.gr - 1) / (c.ng * c.gr)), (unsigned)((rows + R - 1) / R), 1);
-        with_gemv_digits_kernel<R>(c.gr, [&](auto kernel) {
+    with_gemv_digits_kernel<R>(c.gr, [&](auto kernel) {
         HIPML_LAUNCH(kernel, grid, dim3(64 * c.waves, 1, 1), (size_t)c.lds, st, w, x, y, m, k, rows, c.ng);
     });
 }
@@ -1335,7 +1417,8 @@ int launch_gemv_q8_rows(hipStream_t st, const uint8_t *w, const float *x, float 
         case 1: launch_gemv_digits<1>(st, w, x, y, m, k, rows); break;
         case 2: launch_gemv_digits<2>(st, w, x, y, m, k, rows); break;
         case 3: launch_gemv_digits<3>(st, w, x, y, m, k, rows); break;
-        default: launch_gemv_digits<4>(st, w, x, y, m, k, rows);
+        case 4: launch_gemv_digits<4>(st, w, x, y, m, k, rows); break;
+        default: launch_gemv_digits<8>(st, w, x, y, m, k, rows);
         }
         return launched("gemv_q8_0_rows");
     }
@@ -1388,6 +1471,7 @@ int proj_init()
     raise_digits(std::integral_constant<int, 2>{});
     raise_digits(std::integral_constant<int, 3>{});
     raise_digits(std::integral_constant<int, 4>{});
+    raise_digits(std::integral_constant<int, 8>{});
     for (int xt = 1; xt <= 4; xt++)
         for (bool half : {false, true}) {
             auto up = [&](auto kernel, int, int) { raise(reinterpret_cast<const void *>(kernel)); };

@@ -508,7 +508,7 @@ int hipml_kv_rows_copy(hipml_stream_t stream, int dtype, const void *k_src, cons
  * [rows][m]; k a multiple of 64 up to 32768, 1 <= rows <= 128.
  * fp32 accumulation of exact block products, so every row has the precision class of the reference's f32 GEMV kernels.
  * Finite activations are taken up to a magnitude of 131,008 and as that value beyond.  Up to 8 rows they enter as whole
- * numbers of 31 bits over each block's largest one, W streams from memory once per pass of 4 rows, and a row's result has
+ * numbers of 31 bits over each block's largest one, W streams from memory once per pass of 4 or 8 rows, and a row's result has
  * the same bits whatever `rows` is and whichever rows travel with it: the rows of a verify group match their plain decodes,
  * as the reference's batched GEMVs do (crates/hipml-kernels/src/attn_gpu.rs:930-932).  From 9 to 128 rows they enter as two
  * f16 halves (~22 bits up to 65,504, to the nearest 32 above), W streams once per pass of 16 to 64 rows, and a row's bits

@@ -24,9 +24,9 @@ def gemm_choice(m, k, tokens, rows):
 # (weight rows, k, activation rows): ragged in the rows of a workgroup, k of 19 chunks or 37 units (uneven shares of the
 # waves, several turns of every ring, a last run of one chunk), more runs than waves, one chunk in all
 ROWS = [
-    (3, 2368, 1), (3, 34560, 1), (1032, 32768, 1), (5117, 4864, 1), (6156, 256, 2), (5180, 4864, 2), (2069, 4864, 2),
+    (3, 2368, 1), (3, 34560, 1), (1032, 32768, 1), (5117, 4864, 1), (1003, 2560, 2), (5180, 4864, 2), (2069, 4864, 2),
     (3, 4864, 3), (1032, 4864, 3), (2069, 4864, 3), (12281, 4864, 3), (1003, 34560, 4), (597, 4864, 5), (5117, 6144, 4),
-    (12281, 4864, 5), (6156, 4864, 9), (8230, 4864, 9),
+    (12281, 4864, 4), (12281, 4864, 5), (8190, 8448, 7), (9973, 5120, 8), (6156, 4864, 9), (8230, 4864, 9),
     (6156, 4864, 25), (6156, 4864, 17), (8230, 4864, 25), (8230, 4864, 17), (6156, 4864, 41), (6156, 4864, 33),
     (8230, 4864, 41), (8230, 4864, 33), (6156, 4864, 57), (6156, 4864, 49), (8230, 4864, 57), (8230, 4864, 49),
     (3, 2368, 9), (3, 2368, 3), (2069, 2368, 17), (4143, 2368, 3), (2618, 2368, 17), (5180, 2368, 3),

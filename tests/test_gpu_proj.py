@@ -221,6 +221,32 @@ def test_activations_beyond_two_f16_halves_saturate(m, k, rows):
     assert not np.isfinite(inf[0]).any() and np.array_equal(inf[1:], got[1:])
 
 
+@pytest.mark.parametrize("m,k,rows", [(6150, 256, 5), (6150, 768, 8), (9973, 4864, 6), (8190, 8448, 7), (12_281, 5120, 8)])
+def test_five_to_eight_rows_in_one_pass(m, k, rows):
+    # two sets of four rows over one read of the weights: a last run of one chunk, one and several runs a wave, ragged last
+    # groups and workgroups, sets that are not full; every row has the bits it has alone, an infinite value reaches its own
+    # row only (which set it lies in does not matter), nothing is written behind the last row
+    assert attn.lib().hipml_dbg_rows_kernel(m, k, rows, 1) // 10_000 == 108
+    r = orc.Rng(0x0588 + m + rows)
+    w = dev(orc.random_q8_0_bytes(r, m * k // 32))
+    x = dev(r.normal_array((rows, k)))
+
+    def run(a):
+        y = torch.full((a.shape[0] + 1, m), float("nan"), device="cuda")
+        attn.gemv_q8_0_rows(w, a.contiguous(), y, m, k, a.shape[0])
+        assert bool(y[-1].isnan().all())
+        return y[:-1]
+    got = run(x)
+    alone = torch.cat([run(x[i:i + 1]) for i in range(rows)])
+    assert torch.equal(got, alone)
+    for at in (0, 3, 4, rows - 1):
+        bad = x.clone()
+        bad[at, k - 40] = float("inf")
+        inf = run(bad)
+        others = [i for i in range(rows) if i != at]
+        assert not bool(inf[at].isfinite().any()) and torch.equal(inf[others], got[others])
+
+
 def test_argument_errors():
     w = torch.zeros(34 * 4, dtype=torch.uint8, device="cuda")
     x = torch.zeros(64, device="cuda")

@@ -36,3 +36,11 @@ def test_every_packed_tile_has_a_shape():
 def test_the_models_projections_are_among_them(m, k):
     named = {inst.row_kernel(*shape) for shape in inst.ROWS}
     assert all(inst.row_kernel(m, k, rows) in named for rows in range(1, 129))
+
+
+@pytest.mark.parametrize("k", [256, 4864, 5120, 6144, 8192])
+@pytest.mark.parametrize("rows", [5, 6, 7, 8])
+def test_weights_that_fill_the_chip_are_read_once_for_five_to_eight_rows(k, rows):
+    # two passes of four rows over these take the chip twice: 1.3 to 1.6 times one pass of eight
+    for m in (6145, 7168, 8192, 10_240, 11_264, 12_288 if k <= 6144 else 11_200):
+        assert inst.row_kernel(m, k, rows) // 10_000 == 108, m
