@@ -530,13 +530,20 @@ def gemv_q8_0_rows(w, x, y, m, k, rows, stream=None):
 def _scratch(nbytes):
     """`nbytes` from torch's allocator for launches on the current stream, which the allocator then keeps them for; None where
     there is nothing to ask for, under capture (the memory would be free again before the graph is replayed) and
-    where the device has no more."""
+    where the device has no more.  The allocator may have to ask the driver, which HIP's default mode forbids while any
+    other stream is captured (and ends that capture): this thread asks in relaxed mode, two calls of about 0.3 us."""
     if not nbytes or torch.cuda.is_current_stream_capturing():
+        return None
+    mode = C.c_int(2)  # hipStreamCaptureModeRelaxed
+    exchange = lib().hipThreadExchangeStreamCaptureMode
+    if exchange(C.byref(mode)) != 0:
         return None
     try:
         return torch.empty(nbytes, dtype=torch.uint8, device="cuda")
     except torch.cuda.OutOfMemoryError:
         return None
+    finally:
+        exchange(C.byref(mode))  # (the thread's mode before)
 
 
 def gemm_q8_0_f16(w, x, y, m, k, tokens, stream=None):

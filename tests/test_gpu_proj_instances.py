@@ -1,5 +1,7 @@
 """Every variant of the projection kernels once, at the shapes of proj_instances.py: against the definition in 64 bits, with
 nothing written past the outputs, and a row's bits those it has in other company."""
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -115,3 +117,43 @@ def test_scratch_of_a_call_on_the_current_stream_and_under_capture():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(y[:tokens], want[:tokens]) and bool(junk.isfinite().all())
+
+
+@pytest.mark.parametrize("threaded", [False, True])
+def test_a_call_beside_another_streams_capture(threaded):
+    # the call's scratch may need new memory from the driver: the capture goes on, and so does the call (capture begins with
+    # the allocator's cache emptied, so that this one does)
+    m, k, tokens = 12380, 3072, 392
+    w, _, _, x = inputs(m, k, tokens)
+    h = x.to(torch.float16)
+    want, y, z = padded(tokens, m), padded(tokens, m), padded(tokens, m)
+    attn.gemm_q8_0_f16(w, x, want, m, k, tokens, stream=torch.cuda.current_stream())
+    count = torch.zeros(64, device="cuda")
+    side = torch.cuda.Stream()
+    raised = []
+
+    def body():
+        try:
+            with torch.cuda.stream(side):
+                attn.gemm_q8_0_f16(w, x, y, m, k, tokens)
+                attn.output_chunk_q8_0(w, None, None, z, m, k, tokens, h)
+        except Exception as e:
+            raised.append(e)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, capture_error_mode="global"):
+        count += 1
+        if threaded:
+            thread = threading.Thread(target=body)
+            thread.start()
+            thread.join()
+        else:
+            body()
+        count += 1
+    assert not raised
+    torch.cuda.synchronize()
+    assert torch.equal(y[:tokens], want[:tokens]) and torch.equal(z[:tokens], want[:tokens])
+    for i in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert count.eq(2 * i + 2).all()
