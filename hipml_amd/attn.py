@@ -546,25 +546,49 @@ def _scratch(nbytes):
         exchange(C.byref(mode))  # (the thread's mode before)
 
 
-def gemm_q8_0_f16(w, x, y, m, k, tokens, stream=None):
+def chunk_projection_scratch(m: int, k: int, tokens: int, f16_rows: bool = False) -> int:
+    """Bytes of scratch with which gemm_q8_0_f16 (or, with f16_rows, output_chunk_q8_0 without attn_out) is faster; 0
+    where it is not.  The same for every call of the shape."""
+    named = lib().hipml_gemm_q8_0_f16_rows_scratch if f16_rows else lib().hipml_gemm_q8_0_f16_scratch
+    return int(named(m, k, tokens))
+
+
+def _held(scratch, m, k, tokens, f16_rows):
+    """The caller's scratch if the call has a use for it."""
+    need = chunk_projection_scratch(m, k, tokens, f16_rows)
+    if need and scratch.numel() * scratch.element_size() < need:
+        raise ValueError(f"scratch of {scratch.numel() * scratch.element_size()} bytes, the call takes {need}")
+    return scratch if need else None
+
+
+def gemm_q8_0_f16(w, x, y, m, k, tokens, stream=None, scratch=None):
     """`AttnLayer::apply_output_chunk`'s tiled GEMM (after the gate) over a Q8_0 weight matrix:
     y[tokens][m], f16 operands.  On the current stream with scratch for the rows as f16 where the library asks for it
-    (not for a stream that the allocator is not told of)."""
-    if stream is None and x is not None and x.data_ptr():
-        x16 = _scratch(lib().hipml_gemm_q8_0_f16_scratch(m, k, tokens))
+    (not for a stream that the allocator is not told of, nor under capture).  `scratch`: a tensor of
+    chunk_projection_scratch bytes that the caller keeps until the product is done, or until no graph that the
+    call was captured into is replayed any more; with it the call allocates nothing."""
+    if x is not None and x.data_ptr():
+        if scratch is not None:
+            x16 = _held(scratch, m, k, tokens, False)
+        else:
+            x16 = _scratch(lib().hipml_gemm_q8_0_f16_scratch(m, k, tokens)) if stream is None else None
         if x16 is not None:
-            _check(lib().hipml_attn_output_chunk_q8_0(_stream(), _p(w), _p(x), 0, _p(y), m, k, tokens, _p(x16)))
+            _check(lib().hipml_attn_output_chunk_q8_0(_stream(stream), _p(w), _p(x), 0, _p(y), m, k, tokens, _p(x16)))
             return
     _check(lib().hipml_gemm_q8_0_f16(_stream(stream), _p(w), _p(x), _p(y), m, k, tokens))
 
 
-def output_chunk_q8_0(wo, attn_out, gate, y, m, k, tokens, x16, stream=None):
+def output_chunk_q8_0(wo, attn_out, gate, y, m, k, tokens, x16, stream=None, scratch=None):
     """`AttnLayer::apply_output_chunk`: y = W_o (attn_out * sigmoid(gate)); gate may be None; x16 is
-    scratch of tokens*k f16.  attn_out None: x16 already holds the rows as f16 (and keeps them); scratch as above."""
-    if attn_out is None and gate is None and stream is None:
-        packed = _scratch(lib().hipml_gemm_q8_0_f16_rows_scratch(m, k, tokens))
+    scratch of tokens*k f16.  attn_out None: x16 already holds the rows as f16 (and keeps them); scratch as above, of
+    chunk_projection_scratch(..., f16_rows=True) bytes where the caller brings it."""
+    if attn_out is None and gate is None:
+        if scratch is not None:
+            packed = _held(scratch, m, k, tokens, True)
+        else:
+            packed = _scratch(lib().hipml_gemm_q8_0_f16_rows_scratch(m, k, tokens)) if stream is None else None
         if packed is not None:
-            _check(lib().hipml_gemm_q8_0_f16_rows(_stream(), _p(wo), _p(x16), _p(y), m, k, tokens, _p(packed)))
+            _check(lib().hipml_gemm_q8_0_f16_rows(_stream(stream), _p(wo), _p(x16), _p(y), m, k, tokens, _p(packed)))
             return
     _check(lib().hipml_attn_output_chunk_q8_0(_stream(stream), _p(wo), _p(attn_out),
                                               _p(gate) if gate is not None else None, _p(y), m, k,

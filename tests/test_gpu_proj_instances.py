@@ -157,3 +157,51 @@ def test_a_call_beside_another_streams_capture(threaded):
         graph.replay()
         torch.cuda.synchronize()
         assert count.eq(2 * i + 2).all()
+
+
+def test_a_captured_call_with_the_callers_scratch():
+    # the packed route inside a graph: the scratch is used (nothing behind it is), every replay has the bits of the eager
+    # call, and scratch that is too short is refused
+    m, k, tokens = 12380, 3072, 392
+    w, _, _, x = inputs(m, k, tokens)
+    h = x.to(torch.float16)
+    want, y, z = padded(tokens, m), padded(tokens, m), padded(tokens, m)
+    attn.gemm_q8_0_f16(w, x, want, m, k, tokens, stream=torch.cuda.current_stream())
+    need = attn.chunk_projection_scratch(m, k, tokens)
+    assert need == attn.chunk_projection_scratch(m, k, tokens, f16_rows=True) == 2 * tokens * k
+    scratch = torch.full((need + 64,), 0x5A, dtype=torch.uint8, device="cuda")
+    rows = torch.full((need + 64,), 0x5A, dtype=torch.uint8, device="cuda")
+    with pytest.raises(ValueError):
+        attn.gemm_q8_0_f16(w, x, y, m, k, tokens, scratch=scratch[:need - 16])
+    with pytest.raises(ValueError):
+        attn.output_chunk_q8_0(w, None, None, z, m, k, tokens, h, scratch=scratch[:need - 16])
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        attn.gemm_q8_0_f16(w, x, y, m, k, tokens, scratch=scratch)
+        attn.output_chunk_q8_0(w, None, None, z, m, k, tokens, h, scratch=rows)
+    for _ in range(3):
+        for t in (y, z):
+            t.fill_(float("nan"))
+        for t in (scratch, rows):
+            t.fill_(0x5A)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y[:tokens], want[:tokens]) and torch.equal(z[:tokens], want[:tokens])
+        assert bool(y[tokens].isnan().all()) and bool(z[tokens].isnan().all())
+        assert torch.equal(scratch[:need], rows[:need]) and not bool((scratch[:need] == 0x5A).all())
+        assert bool((scratch[need:] == 0x5A).all()) and bool((rows[need:] == 0x5A).all())
+    # (a stream by name, with scratch: the packed route too)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    scratch.fill_(0x5A)
+    torch.cuda.synchronize()
+    attn.gemm_q8_0_f16(w, x, y, m, k, tokens, stream=side, scratch=scratch)
+    side.synchronize()
+    assert torch.equal(y[:tokens], want[:tokens]) and not bool((scratch[:need] == 0x5A).all())
+    # a shape that has no use for scratch leaves it alone
+    assert attn.chunk_projection_scratch(64, 320, 3) == 0
+    scratch.fill_(0x5A)
+    few = torch.empty((3, 64), device="cuda")
+    attn.gemm_q8_0_f16(w.flatten()[:64 * 340], x.flatten()[:960], few, 64, 320, 3, scratch=scratch)
+    assert bool((scratch == 0x5A).all())
