@@ -536,7 +536,9 @@ int hipml_gemm_q8_0_f16(hipml_stream_t stream, const void *w, const float *x, fl
 /* Bytes of scratch (tokens*k f16) with which the same product is faster, 0 where it is not: with it (16-byte
  * aligned, in use until the product is done) call hipml_attn_output_chunk_q8_0(stream, w, x, NULL, y, m, k,
  * tokens, scratch), which gives hipml_gemm_q8_0_f16's bits.  For W at a 64-byte aligned address (elsewhere the
- * scratch may gain nothing).  Launches nothing; for arguments the product refuses, 0. */
+ * scratch may gain nothing).  "Until the product is done" is, for a call under capture, until its graph is
+ * replayed no more: memory that an allocator takes back after the capture is written by every replay.  Launches
+ * nothing; for arguments the product refuses, 0. */
 size_t hipml_gemm_q8_0_f16_scratch(int m, int k, int tokens);
 
 /* The same product over rows that are f16 already (x16: [tokens][k], 16-byte aligned, left as it is):
@@ -551,8 +553,10 @@ size_t hipml_gemm_q8_0_f16_rows_scratch(int m, int k, int tokens);
  * rows are already gated, e.g. by hipml_attn_chunk_q8_split_gate).  x16 is caller scratch of
  * tokens*k f16 (2 bytes each, 16-byte aligned; the attention's split scratch is free by then): a
  * first kernel gates and rounds the rows to f16 once, the GEMM then reads half the bytes per
- * workgroup (what x16 holds afterwards is not specified, nor whether it was written).  Same bits as
- * hipml_q_gate_f32 followed by hipml_gemm_q8_0_f16, faster.
+ * workgroup.  x16 is scratch throughout: it may hold the rows in another order afterwards, or what it held before
+ * (a caller that wants the gated rows as f16 has them from hipml_attn_chunk_q8_split_gate_f16), and for a call under
+ * capture it has to stay the caller's until the graph is replayed no more.  Same bits as hipml_q_gate_f32 followed
+ * by hipml_gemm_q8_0_f16, faster.
  * attn_out == NULL (then gate must be NULL too): x16 already holds the rows as f16, as
  * hipml_attn_chunk_q8_split_gate_f16 writes them, and only the GEMM runs.
  * Replaces AttnLayer::apply_output_chunk (q_gate_f32 + the tiled GEMM),
