@@ -202,3 +202,32 @@ def test_few_tokens_behind_a_prefix(tok, pos0, splits, n_head, n_kv, dtype):
     assert bool(out[tok].isnan().all()) and bool(gated_rows[tok].isnan().all()) and bool(out16[tok].isnan().all())
     first_unused = used if used > 1 else 0
     assert bool((acc[first_unused:] == 7.0).all()) and bool((ml[first_unused:] == 7.0).all())
+
+
+@pytest.mark.parametrize("tok,pos0,splits,n_head,n_kv,dtype,used", [
+    (64, 32_000, 16, 24, 4, 0, 10), (32, 64_000, 21, 24, 4, 0, 21), (25, 60_001, 32, 16, 8, 1, 32), (1, 70_007, 16, 24, 4, 0, 16)])
+def test_few_tokens_behind_a_deep_prefix(tok, pos0, splits, n_head, n_kv, dtype, used):
+    # splits of many key steps each, up to the 256 workgroups of one round (32 splits of 8 KV heads), 252 and 240.  A softmax
+    # over that many keys averages small: beside the gate the relative error over all outputs, in the 2-norm, is held to the
+    # f16 operands' (2^-11 each in the queries, the keys and the probabilities: some 5e-4); a split that is missing, or has a
+    # wrong weight, moves it by a tenth
+    assert attn.lib().hipml_dbg_chunk_wg_splits(pos0, tok, n_head, n_kv, splits) == used
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(0xDEE9 + tok + pos0)
+    stride = pos0 + tok + 3
+    kd = torch.zeros((n_kv, stride, 272 if dtype == 0 else 144), dtype=torch.uint8, device="cuda")
+    vd = torch.zeros_like(kd)
+    kf, vf = (torch.randn((stride, n_kv, HD), device="cuda", generator=gen) for _ in range(2))
+    attn.kv_encode_bulk(dtype, kf, vf, kd, vd, n_kv, HD, stride, 0, 0, stride)
+    q = torch.randn((tok, n_head, HD), device="cuda", generator=gen)
+    acc, ml = attn.chunk_scratch(tok, n_head, splits)
+    acc.fill_(7.0), ml.fill_(7.0)
+    out = torch.full((tok + 1, n_head, HD), float("nan"), device="cuda")
+    attn.chunk_attention_q8_split(q, kd, vd, out, n_head, n_kv, HD, pos0, tok, dtype + 1, stride, acc, ml, splits)
+    torch.cuda.synchronize()
+    got = host(out[:tok])
+    want = orc.attn_chunk_kv(host(q), host(kd), host(vd), n_head, n_kv, HD, pos0, tok, stride, SCALE, n_threads=16,
+                             dtype=dtype).reshape(got.shape)
+    assert report(f"chunk {tok}@{pos0}, {used} splits", want, got, *GATE)[0]
+    assert np.linalg.norm(got - want) <= 2e-3 * np.linalg.norm(want)
+    assert bool(out[tok].isnan().all()) and bool((acc[used:] == 7.0).all()) and bool((ml[used:] == 7.0).all())
