@@ -38,7 +38,7 @@ def test_row_kernel(m, k, rows):
     assert bool(y[rows].isnan().all())
     exact = x.double() @ (d.double() * q.double()).reshape(m, k).T
     err = (y[:rows] - exact).abs().max().item()
-    # activations to ~22 bits, fp32 sums over eight chains; the raw-row kernel's 128 + q, whose 128 comes out in fp32
+    # activations to ~22 bits (24 of their block's largest up to eight rows), fp32 sums over eight chains or up to twelve waves
     assert err <= 2e-6 * exact.abs().max().item() * max(1.0, (k / 8192) ** 0.5) + 1e-5, err
     # the last row among others: the same bits where those take kernels of the same class
     kernel = inst.row_kernel(m, k, rows) // 1_000_000
