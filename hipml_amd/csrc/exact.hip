@@ -344,11 +344,12 @@ int launch_rope_chunk(hipStream_t st, float *q, float *k, int n_head, int n_kv, 
     return 0;
 }
 
+typedef float float4e __attribute__((ext_vector_type(4)));
+typedef float float4a4 __attribute__((ext_vector_type(4), aligned(4))); // (rows at any 4-byte boundary)
+
 // A block of 32 values held four per lane by 8 neighbouring lanes (value 4 l8 + j in component j):
 // the same quantizers as above (the maximum is exact whatever the order it is taken in; the q4_0
 // winner is the first of the largest, by index), with 16-bit stores of the packed bytes.
-typedef float float4e __attribute__((ext_vector_type(4)));
-
 __device__ __forceinline__ void q8_encode_store4(const float4e x, uint8_t *dst_block, int l8)
 {
     float m = fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3])));
@@ -556,8 +557,6 @@ struct FrontAppend {
 // them, 2 = the same to q4_0 -- the K wave keeps its row in registers (element lane + 64 j in slot
 // j, so a half-wave holds one block of 32, as the append kernels' 32-lane groups do) and n_kv more
 // waves per row take the V rows.  Same expressions on the same values: the bits of the two launches.
-typedef float float4a4 __attribute__((ext_vector_type(4), aligned(4))); // (rows at any 4-byte boundary)
-
 template <int ENC>
 __global__ void __launch_bounds__(256) front_kernel(
     const float *__restrict__ qg, float *__restrict__ q, float *__restrict__ gate, float *k,

@@ -1032,7 +1032,9 @@ int gemm_init()
 // the pass is not paid back (6000 x 1024 over 1,024 / 2,048 tokens: 24.3 / 39.3 us, with scratch 25.6 / 41.4).  The costs
 // are fitted like the table above at 253 shapes (1,024 to 16,384 weight rows, 32 to 2,048 tokens): 1 % behind the best of
 // all routes and tiles on average, 11 % at most; 12 % ahead of the tiles over the rows as they lie, at 3 shapes more than
-// 2 % behind them (the 512 x 96 tile, added later, to its time at six shapes).
+// 2 % behind them.  (The 512 x 96 tile came later and has its cost from six shapes: at 68 others the rule is 0.6 % behind the
+// best packed tile on average; it takes this tile at eight, where it is the best, and leaves it at two where it would be 4
+// and 11 % faster.)
 // Rows that are f16 already are multiplied as they lie or packed, by a pass of half the bytes.
 enum class GemmRoute { kNone, kRows, kRowsF16, kPacked };
 enum class GemmRows { kF32, kGated, kF16 };

@@ -48,9 +48,10 @@ constexpr int kQTile = 32;    // query tokens per task
 constexpr int kTasks = 8;     // tasks (= waves) per workgroup
 constexpr int kPfThreads = 64 * kTasks;
 constexpr int kKTile = 64;    // keys per LDS tile
-// f16 rows in LDS: 512 bytes + pad.  528 keeps the K operand's 128-bit reads (lane = row) and
-// the staging writes conflict free; 544 does the same for the V transpose reads (8 rows x 64
-// bytes per instruction) at the price of 2-way conflicts on V's staging writes.
+// f16 rows in LDS: 512 bytes + pad.  528 keeps the K operand's 128-bit reads (lane = row) free of bank
+// conflicts (counted: 4 cycles an instruction, as rows of 1,024 bytes in order take); V's transposing reads
+// (8 rows x 64 bytes) meet two ways at 544 (4 cycles for 2), and the staging writes, 4 rows x 2 units per 8
+// lanes, at both pitches (16 for 8 in order; with eight waves writing 8.0 clocks an instruction against 6.5).
 constexpr int kKRow = 528;
 constexpr int kVRow = 544;
 constexpr int kVOff = kKTile * kKRow;                  // V tile follows the K tile
@@ -1420,7 +1421,7 @@ __global__ void __launch_bounds__(kPfThreads, 1) chunk_wg_kernel(const ChunkArgs
     uint8_t *Vt = Kt + kWgK;
 
     // ---- staging role: lane -> one unit (two blocks) of the slice's K tile and one of its V tile ----
-    // (the (row, unit) pattern of chunk_q8_kernel over the slice's 128 lanes: conflict-free 128-bit writes)
+    // (the (row, unit) pattern of chunk_q8_kernel over the slice's 128 lanes)
     const int su = hp * 64 + lane;
     const int srow = (su >> 6) * 16 + ((su >> 1) & 7) + ((su >> 5) & 1) * 8;
     const int spr = (su & 1) | ((su >> 3) & 2);
@@ -1987,7 +1988,7 @@ __global__ void __launch_bounds__(256) kv_f16_tiles_kernel(const uint8_t *__rest
     const bool v_tile = blockIdx.z != 0;
     const int su = threadIdx.x;
     const int lane = su & 63, wave = su >> 6;
-    // thread -> (row, unit) as in the chunk kernel's staging: conflict-free 128-bit LDS writes
+    // thread -> (row, unit) as in the chunk kernel's staging
     const int srow = (su >> 6) * 16 + ((su >> 1) & 7) + ((su >> 5) & 1) * 8;
     const int spr = (su & 1) | ((su >> 3) & 2);
     int key = tile * kKTile + srow;
