@@ -334,20 +334,16 @@ __device__ __forceinline__ uint32_t proj_lds_address(const void *p)
     return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void *)p;
 }
 
-// 64 lanes x 16 bytes from base + voff (per lane) to LDS address lds_at + 16 * lane; ONCE: read once (weights)
-template <bool ONCE>
+// 64 lanes x 16 bytes from base + voff (per lane) to LDS address lds_at + 16 * lane.  Not non-temporal for the weights either,
+// though each byte is read once: a row's share of a request starts and ends inside a cache line, the rest of which the next
+// request wants, and a non-temporal line has left L2 by then and is fetched twice (12288 x 5120 over 16 / 24 / 32 / 48 rows
+// with the hint 22.9 / 26.3 / 27.2 / 33.3 us, without 21.4 / 23.5 / 24.7 / 31.8; over 1 and 2 rows 14.8 / 15.4 and 14.6 / 14.9).
 __device__ __forceinline__ void proj_dma16(uint32_t lds_at, const uint8_t *base, uint32_t voff)
 {
-    if (ONCE)
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt"
-                     :
-                     : "s"(lds_at), "v"(voff), "s"(base)
-                     : "memory");
-    else
-        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                     :
-                     : "s"(lds_at), "v"(voff), "s"(base)
-                     : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                 :
+                 : "s"(lds_at), "v"(voff), "s"(base)
+                 : "memory");
 }
 
 template <int N>
@@ -429,7 +425,7 @@ __global__ void __launch_bounds__(64 * kDigitMaxWaves) gemv_q8_digits_kernel(con
 #pragma unroll
             for (int r = 0; r < S; r++)
                 if (set * S + r < nrows)
-                    proj_dma16<false>(xdig_at + (cc * S + r) * 1024u, xb + (size_t)(set * S + r) * ((size_t)k * 4) + (size_t)c * 1024,
+                    proj_dma16(xdig_at + (cc * S + r) * 1024u, xb + (size_t)(set * S + r) * ((size_t)k * 4) + (size_t)c * 1024,
                                       lane * 16u);
         }
     };
@@ -450,7 +446,7 @@ __global__ void __launch_bounds__(64 * kDigitMaxWaves) gemv_q8_digits_kernel(con
 #pragma unroll
         for (int j = 0; j < NI; j++)
             if ((j + 1) * 64 <= kPieces || j * 64 + lane < kPieces)
-                proj_dma16<true>(place_at + j * 1024, src, woff[j] < most ? woff[j] : most);
+                proj_dma16(place_at + j * 1024, src, woff[j] < most ? woff[j] : most);
     };
     if (wave < nrun) {
         issue_x(wave, 0);
@@ -768,16 +764,18 @@ __global__ void __launch_bounds__(64 * kDigitMaxWaves) gemv_q8_digits_kernel(con
 // gemv_q8_units_kernel (m up to 6,144; any k of whole 64-value units, W at a 4-byte boundary): no barrier, a wave
 // streams units of its own.  gemv_q8_blocks_kernel (more rows, k of whole 256-value chunks, W at a 16-byte boundary):
 // the workgroup walks chunks together and shares 16-byte requests for the weights, where units take four times as many
-// dword requests, which tell where a workgroup has 48 weight rows.  The kernels before them had eight waves in step, a
-// block of each chunk per wave and two barriers per chunk.  us over 9 / 24 / 32 / 48 / 64 / 128 rows (k 5120, for 5,120
-// weight rows 6144; before / units / blocks):
-//    1,024 weight rows  11.2  8.9 14.7 | 14.5  9.1 14.7 | 15.7  9.2 15.1 | 20.7  9.3 15.1 | 24.5  9.6 15.4 | 24.8 12.7 15.7
-//    4,096              11.4  9.3 14.8 | 15.2 12.5 15.2 | 16.3 12.6 15.4 | 21.3 19.4 18.0 | 25.6 19.8 18.4 | 49.2 37.2 29.9
-//    5,120              14.8 13.3 17.1 | 23.5 18.4 22.3 | 22.3 20.5 23.1 | 29.7 29.1 27.3 | 34.2 29.7 28.6 | 68.4 55.3 40.7
-//    6,144              12.8 13.5 15.2 | 21.0 17.2 18.3 | 20.2 18.5 18.6 | 26.5 25.0 21.3 | 30.7 25.7 22.3 | 58.2 48.5 33.5
-//    7,168              14.7 15.4 15.4 | 19.1 19.2 17.6 | 22.0 22.4 18.9 | 26.6 33.4 28.0 | 30.1 38.7 30.9 | 57.6 70.6 61.3
-//    8,192              14.8 15.7 16.1 | 19.3 19.7 17.9 | 22.3 22.8 19.3 | 27.2 39.9 28.2 | 30.4 40.7 31.2 | 59.7 71.6 59.9
-//   12,288              26.9 20.7 20.7 | 36.8 25.8 22.6 | 41.2 29.7 26.0 | 50.6 51.4 32.8 | 57.6 52.2 35.5 | 88.0 97.8 69.6
+// dword requests, which tell where a workgroup has 48 weight rows.  us over 9 / 16 / 24 / 32 / 48 / 64 / 128 rows, units and
+// blocks (k 5120, for 5,120 weight rows 6144):
+//    1,024 weight rows   9.0 14.2 |  9.3 14.5 |  9.3 14.3 |  9.2 14.3 |  9.4 14.4 |  9.4 14.3 | 12.5 14.5
+//    4,096              10.5 14.6 | 12.0 15.1 | 14.4 15.0 | 15.3 15.2 | 19.8 17.6 | 20.6 17.8 | 37.7 28.9
+//    5,120              15.5 17.2 | 16.5 17.6 | 19.8 20.8 | 21.4 20.9 | 29.5 24.8 | 30.6 25.4 | 56.0 38.8
+//    6,144              15.2 15.7 | 16.0 16.2 | 18.6 18.0 | 19.8 18.4 | 25.7 21.3 | 26.8 22.0 | 49.1 34.0
+//    7,168              16.6 16.2 | 17.2 15.9 | 19.7 17.7 | 22.8 18.8 | 33.9 28.0 | 39.3 31.3 | 71.1 53.1
+//    8,192              17.2 16.8 | 17.7 16.1 | 20.6 18.3 | 23.2 19.2 | 40.3 28.1 | 40.6 31.6 | 71.5 56.9
+//   12,288              20.8 20.5 | 21.5 19.8 | 25.5 22.6 | 28.7 23.4 | 50.4 31.4 | 51.4 35.3 | 96.7 64.6
+// Requests for weights and activations add up, where one might expect the shorter to hide: 12288 x 5120 over 32 rows, weights
+// alone 14 us behind the launch, activations alone (every workgroup reads all of them, from L2) 7, both 23: a CU's requests
+// return in order, so those for L2 wait behind those for HBM.
 // The choice must not depend on the number of rows (their bits would), so the line lies where the row counts of verify
 // groups and batched decode, 9 to 32, change sides; over more rows the blocks would win from 4,096 weight rows on.
 
@@ -842,12 +840,12 @@ __global__ void __launch_bounds__(512, 2) gemv_q8_blocks_kernel(const uint8_t *_
         const uint8_t *xs = xb + (size_t)(8 * c + wave) * 128;
 #pragma unroll
         for (int j = 0; j < NX; j++)
-            proj_dma16<false>(at + S::kWBytes + wave * S::kXWave + j * 1024, xs, xoff[j]);
+            proj_dma16(at + S::kWBytes + wave * S::kXWave + j * 1024, xs, xoff[j]);
 #pragma unroll
         for (int j = 0; j < NWMost; j++) {
             const int q = wave + 8 * j;
             if (q < NW && (kPieces % 64 == 0 || q * 64 + lane < kPieces))
-                proj_dma16<true>(at + q * 1024, wb, woff[j] + (uint32_t)c * kChunkBytes);
+                proj_dma16(at + q * 1024, wb, woff[j] + (uint32_t)c * kChunkBytes);
         }
     };
     // chunk c has arrived: only the chunks asked for behind it, `most` of them, are outstanding
@@ -1056,7 +1054,7 @@ __global__ void __launch_bounds__((kUnitsThreads<XT, RW, HALF>), (UnitsShape<XT,
         const uint8_t *xs = xb + (size_t)u * 256, *ws = wb + (size_t)u * (2 * kQ8Block);
 #pragma unroll
         for (int j = 0; j < NX; j++)
-            proj_dma16<false>(at + j * 1024, xs, xoff[j]);
+            proj_dma16(at + j * 1024, xs, xoff[j]);
 #pragma unroll
         for (int j = 0; j < NW; j++) {
             if ((j + 1) * 64 <= RW * 17 || j * 64 + lane < RW * 17)
