@@ -334,16 +334,26 @@ __device__ __forceinline__ uint32_t proj_lds_address(const void *p)
     return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void *)p;
 }
 
-// 64 lanes x 16 bytes from base + voff (per lane) to LDS address lds_at + 16 * lane.  Not non-temporal for the weights either,
-// though each byte is read once: a row's share of a request starts and ends inside a cache line, the rest of which the next
-// request wants, and a non-temporal line has left L2 by then and is fetched twice (12288 x 5120 over 16 / 24 / 32 / 48 rows
-// with the hint 22.9 / 26.3 / 27.2 / 33.3 us, without 21.4 / 23.5 / 24.7 / 31.8; over 1 and 2 rows 14.8 / 15.4 and 14.6 / 14.9).
+// 64 lanes x 16 bytes from base + voff (per lane) to LDS address lds_at + 16 * lane.  ONCE: non-temporal, for bytes that are
+// read once.  gemv_q8_digits_kernel asks for its weights so (runs of 544 bytes of a row; from HBM 12288 x 5120 over 1 / 3 rows
+// 13.0 / 15.4 us with the hint, 13.8 / 15.7 without).  Where a request ends inside a cache line whose rest another one wants it
+// costs a second fetch: gemv_q8_units_kernel over 1024 x 5120 and 24 rows 8.8 and 7.6, gemv_q8_blocks_kernel over 12288 x 5120
+// and 9 / 16 rows 19.2 / 19.9 and 18.2 / 18.8.  gemv_q8_blocks_kernel over more rows asks with it all the same (over 24 / 32
+// rows 22.8 / 25.2 and 22.1 / 23.8): such a matrix, of 35 MB and more, otherwise pushes out of the last-level cache what is
+// there (a layer over 32 short sequences, whose W_o then comes from HBM, 86.2 and 89.6 us).
+template <bool ONCE>
 __device__ __forceinline__ void proj_dma16(uint32_t lds_at, const uint8_t *base, uint32_t voff)
 {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
-                 :
-                 : "s"(lds_at), "v"(voff), "s"(base)
-                 : "memory");
+    if (ONCE)
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt"
+                     :
+                     : "s"(lds_at), "v"(voff), "s"(base)
+                     : "memory");
+    else
+        asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                     :
+                     : "s"(lds_at), "v"(voff), "s"(base)
+                     : "memory");
 }
 
 template <int N>
@@ -425,7 +435,7 @@ __global__ void __launch_bounds__(64 * kDigitMaxWaves) gemv_q8_digits_kernel(con
 #pragma unroll
             for (int r = 0; r < S; r++)
                 if (set * S + r < nrows)
-                    proj_dma16(xdig_at + (cc * S + r) * 1024u, xb + (size_t)(set * S + r) * ((size_t)k * 4) + (size_t)c * 1024,
+                    proj_dma16<false>(xdig_at + (cc * S + r) * 1024u, xb + (size_t)(set * S + r) * ((size_t)k * 4) + (size_t)c * 1024,
                                       lane * 16u);
         }
     };
@@ -446,7 +456,7 @@ __global__ void __launch_bounds__(64 * kDigitMaxWaves) gemv_q8_digits_kernel(con
 #pragma unroll
         for (int j = 0; j < NI; j++)
             if ((j + 1) * 64 <= kPieces || j * 64 + lane < kPieces)
-                proj_dma16(place_at + j * 1024, src, woff[j] < most ? woff[j] : most);
+                proj_dma16<true>(place_at + j * 1024, src, woff[j] < most ? woff[j] : most);
     };
     if (wave < nrun) {
         issue_x(wave, 0);
@@ -763,21 +773,22 @@ __global__ void __launch_bounds__(64 * kDigitMaxWaves) gemv_q8_digits_kernel(con
 //
 // gemv_q8_units_kernel (m up to 6,144; any k of whole 64-value units, W at a 4-byte boundary): no barrier, a wave
 // streams units of its own.  gemv_q8_blocks_kernel (more rows, k of whole 256-value chunks, W at a 16-byte boundary):
-// the workgroup walks chunks together and shares 16-byte requests for the weights, where units take four times as many
-// dword requests, which tell where a workgroup has 48 weight rows.  us over 9 / 16 / 24 / 32 / 48 / 64 / 128 rows, units and
-// blocks (k 5120, for 5,120 weight rows 6144):
-//    1,024 weight rows   9.0 14.2 |  9.3 14.5 |  9.3 14.3 |  9.2 14.3 |  9.4 14.4 |  9.4 14.3 | 12.5 14.5
-//    4,096              10.5 14.6 | 12.0 15.1 | 14.4 15.0 | 15.3 15.2 | 19.8 17.6 | 20.6 17.8 | 37.7 28.9
-//    5,120              15.5 17.2 | 16.5 17.6 | 19.8 20.8 | 21.4 20.9 | 29.5 24.8 | 30.6 25.4 | 56.0 38.8
-//    6,144              15.2 15.7 | 16.0 16.2 | 18.6 18.0 | 19.8 18.4 | 25.7 21.3 | 26.8 22.0 | 49.1 34.0
-//    7,168              16.6 16.2 | 17.2 15.9 | 19.7 17.7 | 22.8 18.8 | 33.9 28.0 | 39.3 31.3 | 71.1 53.1
-//    8,192              17.2 16.8 | 17.7 16.1 | 20.6 18.3 | 23.2 19.2 | 40.3 28.1 | 40.6 31.6 | 71.5 56.9
-//   12,288              20.8 20.5 | 21.5 19.8 | 25.5 22.6 | 28.7 23.4 | 50.4 31.4 | 51.4 35.3 | 96.7 64.6
-// Requests for weights and activations add up, where one might expect the shorter to hide: 12288 x 5120 over 32 rows, weights
-// alone 14 us behind the launch, activations alone (every workgroup reads all of them, from L2) 7, both 23: a CU's requests
-// return in order, so those for L2 wait behind those for HBM.
+// the workgroup walks chunks together and shares its requests for the weights.  us over 9 / 16 / 24 / 32 / 40 / 48 / 64 / 128
+// rows, units (by 16-byte requests) and blocks, each with its best tile, the weights from HBM (k 5120, for 2,048 and 4,096
+// weight rows 4096, for 5,120 6144):
+//    1,024 weight rows   7.3 13.1 |  7.8 13.4 |  7.7 13.2 |  7.7 13.3 |  9.0 13.3 | 10.0 13.4 | 10.0 13.5 | 12.2 13.5
+//    2,048               6.6 11.3 |  7.0 11.3 |  7.8 11.4 |  8.8 11.4 | 10.0 11.4 | 10.8 11.5 | 10.8 11.8 | 14.7 15.0
+//    4,096               8.7 11.4 |  9.8 11.6 | 10.6 12.0 | 11.6 11.8 | 13.6 14.5 | 14.3 14.7 | 15.4 15.1 | 27.2 24.8
+//    5,120              13.7 15.8 | 15.0 16.2 | 18.6 19.5 | 20.1 19.0 | 23.2 22.3 | 23.7 22.8 | 26.1 24.9 | 46.8 38.5
+//    6,144              13.8 13.7 | 14.3 14.4 | 16.1 16.8 | 17.3 16.7 | 20.1 21.3 | 20.6 21.3 | 23.2 22.0 | 41.5 33.8
+//    7,168              15.3 14.0 | 15.8 15.0 | 18.4 17.5 | 20.8 18.7 | 29.2 23.2 | 29.8 27.5 | 34.2 31.1 | 59.5 52.1
+//    8,192              15.7 15.7 | 16.4 15.4 | 19.2 17.9 | 21.2 19.1 | 30.5 23.5 | 31.4 27.9 | 35.6 31.5 | 61.0 56.1
+//   12,288              20.9 19.7 | 21.1 19.4 | 24.3 22.2 | 27.4 24.7 | 39.6 28.2 | 40.9 32.1 | 46.0 36.0 | 83.8 64.8
+// What a workgroup asks for adds up, wherever it comes from: a CU takes 36 bytes a cycle out of L2 however many CUs ask and
+// whatever the pattern, and what comes from HBM waits in the same queue.  12288 x 5120 over 32 rows: weights alone 12 us,
+// activations (every workgroup reads all of them) 8 more.
 // The choice must not depend on the number of rows (their bits would), so the line lies where the row counts of verify
-// groups and batched decode, 9 to 32, change sides; over more rows the blocks would win from 4,096 weight rows on.
+// groups and batched decode, 9 to 40, change sides; over more rows the blocks would win from 5,120 weight rows on.
 
 template <int XT, int RW, bool HALF>
 struct BlocksShape {
@@ -787,7 +798,11 @@ struct BlocksShape {
     static constexpr int kXWave = kXRows * 128;             // one wave's block of them
     static constexpr int kSlot = kWBytes + 8 * kXWave;
     static constexpr int kFit = (160 << 10) / kSlot;
-    static constexpr int kDepth = kFit < 5 ? kFit : 5; // chunks in flight
+    // Chunks on the way, at most three: 12288 x 5120 over 9 / 16 rows with five / three / two 19.4 / 18.2 / 20.9 and 20.1 / 18.8 /
+    // 22.0 us, over 24 / 32 with three / two 22.1 / 24.2 and 23.8 / 27.8, from HBM; 8192 x 5120 over 16 with five / three 16.8 /
+    // 15.6 from the last-level cache.
+    static constexpr int kMost = 3;
+    static constexpr int kDepth = kFit < kMost ? kFit : kMost; // chunks on the way
     static constexpr int kSums = 8 * XT * kMT * 1024;
     static constexpr int kRead = HALF ? 1024 : 0; // (a HALF tile's dead rows are read past the wave's block)
     static constexpr int kLds = (kDepth * kSlot > kSums ? kDepth * kSlot : kSums) + kRead;
@@ -840,22 +855,20 @@ __global__ void __launch_bounds__(512, 2) gemv_q8_blocks_kernel(const uint8_t *_
         const uint8_t *xs = xb + (size_t)(8 * c + wave) * 128;
 #pragma unroll
         for (int j = 0; j < NX; j++)
-            proj_dma16(at + S::kWBytes + wave * S::kXWave + j * 1024, xs, xoff[j]);
+            proj_dma16<false>(at + S::kWBytes + wave * S::kXWave + j * 1024, xs, xoff[j]);
 #pragma unroll
         for (int j = 0; j < NWMost; j++) {
             const int q = wave + 8 * j;
             if (q < NW && (kPieces % 64 == 0 || q * 64 + lane < kPieces))
-                proj_dma16(at + q * 1024, wb, woff[j] + (uint32_t)c * kChunkBytes);
+                proj_dma16<(XT > 1)>(at + q * 1024, wb, woff[j] + (uint32_t)c * kChunkBytes);
         }
     };
     // chunk c has arrived: only the chunks asked for behind it, `most` of them, are outstanding
     auto wait_chunk = [&](int c, int most) {
         const int newer = nchunk - 1 - c < most ? nchunk - 1 - c : most;
         constexpr int a = NX + NWMost, b = NX + NWMost - 1; // requests of a chunk
-        static_assert(4 * a < 64, "vmcnt has six bits");
+        static_assert(2 * a < 64 && S::kMost <= 3, "vmcnt has six bits");
         switch (newer) {
-        case 4: return wreq == NWMost ? wait_vm<4 * a>() : wait_vm<4 * b>();
-        case 3: return wreq == NWMost ? wait_vm<3 * a>() : wait_vm<3 * b>();
         case 2: return wreq == NWMost ? wait_vm<2 * a>() : wait_vm<2 * b>();
         case 1: return wreq == NWMost ? wait_vm<a>() : wait_vm<b>();
         default: return wait_vm<0>();
@@ -985,23 +998,32 @@ __global__ void __launch_bounds__(512, 2) gemv_q8_blocks_kernel(const uint8_t *_
     }
 }
 
-template <int XT, int RW, bool HALF>
+// WIDE (k of whole 256-value chunks, W at a 16-byte boundary): weights by 16-byte requests, the five pieces that a row's 68
+// bytes of a unit lie in.  By dwords a row takes 17, and the requests cost a CU more than the activations': 1024 x 5120 over
+// 24 rows 10.1 -> 7.6 us, 5120 x 6144 over 9 / 24 rows 14.3 / 19.3 -> 12.8 / 18.5, with the depths and tiles below.  Tried on
+// it: a block of 34 bytes a turn instead of two (20 % slower: a turn costs 0.2 us beside its work), two blocks 256 values apart,
+// as gemv_q8_blocks_kernel sums them (10 %: twice the lines), the sums of a unit's second block taken a turn later (no gain),
+// weights asked for in front of the activations (2 % slower).
+template <int XT, int RW, bool HALF, bool WIDE>
 struct UnitsShape {
     static constexpr int kMT = (RW + 15) / 16;              // weight tiles
     static constexpr int kXRows = 16 * XT - (HALF ? 8 : 0); // activation rows that are fetched
     static constexpr int kXBytes = kXRows * 256;
-    static constexpr int kSlot = kXBytes + (RW * 68 + 15) / 16 * 16; // a unit
+    static constexpr int kWRow = WIDE ? 80 : 68;            // a weight row's bytes of a unit, as they are fetched
+    static constexpr int kSlot = kXBytes + (RW * kWRow + 15) / 16 * 16; // a unit
     static constexpr int kRead = HALF ? 2048 : 0;           // (a HALF tile's dead rows are read past the activations)
     static constexpr int kRoom = (160 << 10) - kRead;
     static constexpr int kWaves = kRoom / (8 * kSlot) >= 2 ? 8 : 4;
-    static constexpr int kFit = kRoom / (kWaves * kSlot);
-    static constexpr int kDepth = kFit < 4 ? kFit : 4; // units in flight per wave
+    // Units of a wave on the way.  More only lengthen the queue that everybody's first ones wait in: 1024 x 5120 over 24 rows
+    // with 4 / 3 / 2 of them 8.7 / 8.4 / 7.6 us from HBM and 7.4 / 7.3 / 6.7 from the last-level cache, 5120 x 6144 over 9 rows
+    // with 3 / 2 13.8 / 12.8 from HBM.
+    static constexpr int kDepth = 2;
     static constexpr int kLds = kWaves * kDepth * kSlot + kRead;
     static constexpr int kChains = 8 / kWaves; // of a wave
-    static_assert(kDepth >= 2 && kDepth * kSlot >= kChains * XT * kMT * 1024, "");
+    static_assert(kLds <= 160 << 10 && kDepth * kSlot >= kChains * XT * kMT * 1024, "");
 };
-template <int XT, int RW, bool HALF>
-constexpr int kUnitsThreads = 64 * UnitsShape<XT, RW, HALF>::kWaves;
+template <int XT, int RW, bool HALF, bool WIDE>
+constexpr int kUnitsThreads = 64 * UnitsShape<XT, RW, HALF, WIDE>::kWaves;
 
 __device__ __forceinline__ void proj_dma4(uint32_t lds_at, const uint8_t *base, uint32_t voff)
 {
@@ -1014,14 +1036,15 @@ __device__ __forceinline__ void proj_dma4(uint32_t lds_at, const uint8_t *base, 
 // Wave w of WV streams units (pairs of blocks, 64 values of k) w, w + WV, ... of its rows through a ring of its own; unit
 // u belongs to chain u % 8, so four waves keep two sets of sums each.  HALF: as above.
 // (One wave a SIMD may use all 512 registers: held to 256, two sets of 2 x 3 tiles spill, 200 us instead of 28.)
-template <int XT, int RW, bool HALF>
-__global__ void __launch_bounds__((kUnitsThreads<XT, RW, HALF>), (UnitsShape<XT, RW, HALF>::kWaves / 4))
+template <int XT, int RW, bool HALF, bool WIDE>
+__global__ void __launch_bounds__((kUnitsThreads<XT, RW, HALF, WIDE>), (UnitsShape<XT, RW, HALF, WIDE>::kWaves / 4))
     gemv_q8_units_kernel(const uint8_t *__restrict__ w, const float *__restrict__ x, float *__restrict__ y, int m, int k, int rows)
 {
-    typedef UnitsShape<XT, RW, HALF> S;
+    typedef UnitsShape<XT, RW, HALF, WIDE> S;
     constexpr int MT = S::kMT, D = S::kDepth, WV = S::kWaves;
     constexpr int NX = S::kXRows / 4;          // activation requests per unit: four rows of 256 bytes each
-    constexpr int NW = (RW * 17 + 63) / 64;    // weight requests: 64 dwords each
+    constexpr int kPer = WIDE ? 5 : 17;        // pieces of a weight row in a unit, of 16 or 4 bytes
+    constexpr int NW = (RW * kPer + 63) / 64;  // weight requests: 64 pieces each
     constexpr int REQ = NX + NW;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -1029,19 +1052,22 @@ __global__ void __launch_bounds__((kUnitsThreads<XT, RW, HALF>), (UnitsShape<XT,
     const int lm = lane & 15, lg = lane >> 4;
     const int nunits = k >> 6;
     const uint32_t row_bytes = (uint32_t)(k >> 5) * kQ8Block;
-    const int m0 = blockIdx.x * RW, r0 = blockIdx.y * (16 * XT);
-    const int nrows = rows - r0 < 16 * XT ? rows - r0 : 16 * XT;
+    const int m0 = blockIdx.x * RW, r0 = blockIdx.y * S::kXRows;
+    const int nrows = rows - r0 < S::kXRows ? rows - r0 : S::kXRows;
     const int mine = wave < nunits ? (nunits - wave + WV - 1) / WV : 0;
     uint8_t *ring = lds + wave * (D * S::kSlot);
     const uint32_t ring_at = proj_lds_address(ring);
     const uint8_t *wb = w + (size_t)m0 * row_bytes;
     const uint8_t *xb = reinterpret_cast<const uint8_t *>(x + (size_t)r0 * k);
+    // a unit begins 4 (u % 4) bytes into a piece, the same for all of a wave's
+    const uint32_t lead = WIDE ? 4u * (wave & 3) : 0u;
+    static_assert(!WIDE || WV % 4 == 0, "");
     uint32_t woff[NW], xoff[NX]; // rows past the matrix, and past the live activation rows, repeat the last
 #pragma unroll
     for (int j = 0; j < NW; j++) {
         const int p = j * 64 + lane;
-        const int pr = p / 17, pd = p - pr * 17;
-        woff[j] = (uint32_t)(m0 + pr < m ? pr : m - 1 - m0) * row_bytes + (uint32_t)pd * 4u;
+        const int pr = p / kPer, pd = p - pr * kPer;
+        woff[j] = (uint32_t)(m0 + pr < m ? pr : m - 1 - m0) * row_bytes + (uint32_t)pd * (WIDE ? 16u : 4u);
     }
 #pragma unroll
     for (int j = 0; j < NX; j++) {
@@ -1051,24 +1077,24 @@ __global__ void __launch_bounds__((kUnitsThreads<XT, RW, HALF>), (UnitsShape<XT,
     auto issue = [&](int i) {
         const uint32_t at = ring_at + (uint32_t)((i % D) * S::kSlot);
         const uint32_t u = (uint32_t)(wave + WV * i);
-        const uint8_t *xs = xb + (size_t)u * 256, *ws = wb + (size_t)u * (2 * kQ8Block);
+        const uint8_t *xs = xb + (size_t)u * 256, *ws = wb + (size_t)u * (2 * kQ8Block) - lead;
 #pragma unroll
         for (int j = 0; j < NX; j++)
-            proj_dma16(at + j * 1024, xs, xoff[j]);
+            proj_dma16<false>(at + j * 1024, xs, xoff[j]);
 #pragma unroll
         for (int j = 0; j < NW; j++) {
-            if ((j + 1) * 64 <= RW * 17 || j * 64 + lane < RW * 17)
-                proj_dma4(at + S::kXBytes + j * 256, ws, woff[j]);
+            if ((j + 1) * 64 <= RW * kPer || j * 64 + lane < RW * kPer) {
+                if (WIDE)
+                    proj_dma16<false>(at + S::kXBytes + j * 1024, ws, woff[j]);
+                else
+                    proj_dma4(at + S::kXBytes + j * 256, ws, woff[j]);
+            }
         }
     };
-    // unit i has arrived: only the units asked for behind it, `most` of them, are outstanding
-    auto wait_unit = [&](int i, int most) {
-        const int newer = mine - 1 - i < most ? mine - 1 - i : most;
-        if (newer >= 3 && D > 3)
-            wait_vm<(3 * REQ < 63 ? 3 * REQ : 63)>();
-        else if (newer >= 2 && D > 2)
-            wait_vm<(2 * REQ < 63 ? 2 * REQ : 63)>();
-        else if (newer >= 1)
+    // unit i has arrived: only the one asked for behind it is outstanding
+    static_assert(D == 2 && REQ < 64, "vmcnt has six bits");
+    auto wait_unit = [&](int i) {
+        if (i + 1 < mine)
             wait_vm<REQ>();
         else
             wait_vm<0>();
@@ -1081,7 +1107,7 @@ __global__ void __launch_bounds__((kUnitsThreads<XT, RW, HALF>), (UnitsShape<XT,
     int wrow[MT]; // (rows of the last tile past RW repeat the last: never stored)
 #pragma unroll
     for (int t = 0; t < MT; t++)
-        wrow[t] = (t * 16 + lm < RW ? t * 16 + lm : RW - 1) * (2 * kQ8Block);
+        wrow[t] = (t * 16 + lm < RW ? t * 16 + lm : RW - 1) * S::kWRow + (int)lead;
     auto load = [&](Regs &g, int i) {
         const uint8_t *buf = ring + (i % D) * S::kSlot;
 #pragma unroll
@@ -1154,7 +1180,7 @@ __global__ void __launch_bounds__((kUnitsThreads<XT, RW, HALF>), (UnitsShape<XT,
             issue(i);
     Regs even, odd;
     if (mine > 0) {
-        wait_unit(0, D - 1);
+        wait_unit(0);
         load(even, 0);
     }
     // unit i is in `now`
@@ -1164,7 +1190,7 @@ __global__ void __launch_bounds__((kUnitsThreads<XT, RW, HALF>), (UnitsShape<XT,
         if (i + D < mine)
             issue(i + D);
         if (i + 1 < mine) {
-            wait_unit(i + 1, D - 1);
+            wait_unit(i + 1);
             load(next, i + 1);
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -1325,13 +1351,30 @@ static void with_gemv_blocks_kernel(int xt, int rw, bool half, F &&f)
     HIPML_BLOCKS(4, 48);
 #undef HIPML_BLOCKS
 }
-template <typename F>
-static void with_gemv_units_kernel(int xt, int rw, bool half, F &&f)
+// The tiles that any call with 16-byte requests would take (the others lose to one of them at every shape).
+static constexpr bool wide_units_tile(int xt, int rw, bool half)
 {
+    return half ? xt == 2 || rw == 16 || rw == 32 : xt == 1 || (rw != 20 && rw != 24);
+}
+
+template <typename F>
+static void with_gemv_units_kernel(int xt, int rw, bool half, bool wide, F &&f)
+{
+    auto pick = [&](auto x, auto r, auto h, auto w16) {
+        constexpr int X = decltype(x)::value, R = decltype(r)::value;
+        constexpr bool H = decltype(h)::value, W = decltype(w16)::value;
+        if constexpr (!W || wide_units_tile(X, R, H))
+            f(&gemv_q8_units_kernel<X, R, H, W>, kUnitsThreads<X, R, H, W>, UnitsShape<X, R, H, W>::kLds);
+    };
+    const std::true_type yes;
+    const std::false_type no;
 #define HIPML_UNITS(X, R)                                                                                       \
-    if (xt == X && rw == R)                                                                                     \
-        return half ? f(&gemv_q8_units_kernel<X, R, true>, kUnitsThreads<X, R, true>, UnitsShape<X, R, true>::kLds) \
-                    : f(&gemv_q8_units_kernel<X, R, false>, kUnitsThreads<X, R, false>, UnitsShape<X, R, false>::kLds)
+    if (xt == X && rw == R) {                                                                                   \
+        const std::integral_constant<int, X> x;                                                                 \
+        const std::integral_constant<int, R> r;                                                                 \
+        return half ? (wide ? pick(x, r, yes, yes) : pick(x, r, yes, no))                                       \
+                    : (wide ? pick(x, r, no, yes) : pick(x, r, no, no));                                        \
+    }
     HIPML_UNITS(1, 16);
     HIPML_UNITS(1, 20);
     HIPML_UNITS(1, 24);
@@ -1349,29 +1392,42 @@ static const int kBlocksRw[2] = {32, 48}, kUnitsRw[5] = {16, 20, 24, 32, 48};
 static RowsPick pick_tiles(int m, int k, int rows, bool w16)
 {
     // by the shape of W alone: a row has the same bits however many travel with it
-    const bool blocks = m > 6144 && k % 256 == 0 && w16;
-    // the tile that costs least: rounds of 256 workgroups x the cycles of a unit in the eight waves of a CU, as the sum
-    // of its vector instructions (two waves a SIMD, 4 cycles each) and its requests (16 cycles).  At ten matrices of 1,024
-    // to 12,288 weight rows over 9 to 128 rows it picks the fastest tile or one within 5 %, but for 7 % at 3,072 weight
-    // rows over 64 (16.2 us, best 15.1) and 9 % at 7,168 over 100 (60.3, best 55.2)
-    int xt = 0, rw = 0;
-    long long best = 0;
-    for (int cx = 1; cx <= (blocks ? 4 : 2) && 16 * (cx - 1) < rows; cx++)
-        for (int cr : kUnitsRw) {
-            if (blocks && cr < 32)
-                continue;
-            const int mt = (cr + 15) / 16, ty = (rows + 16 * cx - 1) / (16 * cx);
-            const long long rounds = ((long long)((m + cr - 1) / cr) * ty + 255) / 256;
-            const int valu = 26 * mt + 28 * cx + 8 * mt * cx + 20;
-            const int requests = 4 * cx + (cr * 17 + 63) / 64 / (blocks ? 4 : 1);
-            const long long cost = rounds * (8 * valu + 8 * 16 * requests);
-            if (best == 0 || cost < best) {
-                best = cost;
-                xt = cx;
-                rw = cr;
+    const bool wide = k % 256 == 0 && w16, blocks = m > 6144 && wide;
+    // The tile that costs least, in rounds of 256 workgroups x the cost of a unit.
+    // Units by 16-byte requests, where a workgroup may also take 8 or 24 rows, whatever comes behind them: weight tiles, their
+    // products with activation tiles, and requests; fewer workgroups over the same weight rows where that is a tie.  Picks the
+    // fastest tile or one within 3 % at 63 shapes (512 to 6,144 weight rows, k 4096 to 6144, 9 to 128 rows), by the mean of
+    // its times with the weights in HBM and in the last-level cache.  A workgroup's own bytes are what it waits for: 1024 x
+    // 5120 over 16 / 24 / 32 rows by 16 rows 8.0 / 7.6 / 8.0 us (last-level cache), by 8 7.0 / 7.3 / 7.5; 6144 x 5120 over 40
+    // rows by 32 rows 22.1, by 24 18.2.
+    // The others: the cycles of a unit in the eight waves of a CU, as the sum of its vector instructions (two waves a SIMD,
+    // 4 cycles each) and its requests (16 cycles); blocks of 7,168 to 12,288 weight rows over 9 to 128 rows: the fastest
+    // tile or one within 6 %.
+    RowsPick best = {blocks ? RowsPick::kBlocks : RowsPick::kUnits, 0, 0, 0};
+    long long best_cost = 0;
+    for (int xt = 1; xt <= (blocks ? 4 : 2) && 16 * (xt - 1) < rows; xt++)
+        for (int rw : kUnitsRw)
+            for (int half = wide && !blocks ? 1 : 0; half >= 0; half--) {
+                if (blocks ? rw < 32 : wide && !wide_units_tile(xt, rw, half != 0))
+                    continue;
+                const int mt = (rw + 15) / 16, step = 16 * xt - 8 * half;
+                const long long rounds = ((long long)((m + rw - 1) / rw) * ((rows + step - 1) / step) + 255) / 256;
+                long long cost;
+                if (wide && !blocks) {
+                    cost = rounds * (mt + mt * xt + step / 4 + (rw * 5 + 63) / 64) * 128 + (rows + step - 1) / step;
+                } else {
+                    const int valu = 26 * mt + 28 * xt + 8 * mt * xt + 20;
+                    const int requests = 4 * xt + (rw * 17 + 63) / 64 / (blocks ? 4 : 1);
+                    cost = rounds * (8 * valu + 8 * 16 * requests);
+                }
+                if (best_cost == 0 || cost < best_cost) {
+                    best_cost = cost;
+                    best.a = xt;
+                    best.b = rw;
+                    best.c = wide && !blocks ? half : rows <= 16 * xt - 8 ? 1 : 0;
+                }
             }
-        }
-    return {blocks ? RowsPick::kBlocks : RowsPick::kUnits, xt, rw, rows <= 16 * xt - 8 ? 1 : 0};
+    return best;
 }
 
 static RowsPick pick_rows(int m, int k, int rows, bool w16)
@@ -1421,14 +1477,15 @@ int launch_gemv_q8_rows(hipStream_t st, const uint8_t *w, const float *x, float 
         return launched("gemv_q8_0_rows");
     }
     const int xt = p.a, rw = p.b;
-    const dim3 grid((unsigned)((m + rw - 1) / rw), (unsigned)((rows + 16 * xt - 1) / (16 * xt)), 1);
+    const int step = 16 * xt - 8 * p.c; // activation rows of a workgroup
+    const dim3 grid((unsigned)((m + rw - 1) / rw), (unsigned)((rows + step - 1) / step), 1);
     auto go = [&](auto kernel, int threads, int lds) {
         HIPML_LAUNCH(kernel, grid, dim3((unsigned)threads, 1, 1), (size_t)lds, st, w, x, y, m, k, rows);
     };
     if (p.kernel == RowsPick::kBlocks)
         with_gemv_blocks_kernel(xt, rw, p.c, go);
     else
-        with_gemv_units_kernel(xt, rw, p.c, go);
+        with_gemv_units_kernel(xt, rw, p.c, k % 256 == 0 && aligned16(w), go);
     return launched("gemv_q8_0_rows");
 }
 
@@ -1476,7 +1533,8 @@ int proj_init()
             for (int rw : kBlocksRw)
                 with_gemv_blocks_kernel(xt, rw, half, up);
             for (int rw : kUnitsRw)
-                with_gemv_units_kernel(xt, rw, half, up);
+                for (bool wide : {false, true})
+                    with_gemv_units_kernel(xt, rw, half, wide, up);
         }
     if (e != hipSuccess)
         return fail((int)e, "hipFuncSetAttribute(projection LDS) failed: %d (%s)", (int)e, hipGetErrorString(e));

@@ -30,7 +30,7 @@ ROWS = [
     (6156, 4864, 25), (6156, 4864, 17), (8230, 4864, 25), (8230, 4864, 17), (6156, 4864, 41), (6156, 4864, 33),
     (8230, 4864, 41), (8230, 4864, 33), (6156, 4864, 57), (6156, 4864, 49), (8230, 4864, 57), (8230, 4864, 49),
     (3, 2368, 9), (3, 2368, 3), (2069, 2368, 17), (4143, 2368, 3), (2618, 2368, 17), (5180, 2368, 3),
-    (3106, 2368, 17), (6156, 2368, 3), (8230, 2368, 9), (8230, 2368, 3), (2069, 2368, 49), (4143, 2368, 17),
+    (3106, 2368, 17), (6156, 2368, 3), (8230, 2368, 9), (8230, 2368, 3), (2069, 2368, 49), (773, 1280, 115), (4143, 2368, 17),
     (2740, 2368, 33), (5180, 2368, 17), (4082, 2368, 33), (6156, 2368, 17), (4143, 2368, 33), (8230, 2368, 17),
 ]
 # (weight rows, k, tokens, f16 activations)

@@ -50,6 +50,34 @@ def test_row_kernel(m, k, rows):
             assert torch.equal(z[more - 1], y[rows - 1]) and bool(z[more].isnan().all())
 
 
+# (weight rows, k, activation rows) of every tile of the kernel that streams units by 16-byte requests (k of whole 256-value
+# chunks, one among them): ragged in both directions, several workgroups of 8 and of 24 rows, waves with no unit or uneven shares
+@pytest.mark.parametrize("m,k,rows", [(3, 256, 9), (1003, 1280, 30), (2069, 1280, 31), (517, 1280, 125), (5180, 4864, 16),
+                                      (645, 1280, 115), (771, 1280, 127), (517, 1280, 115), (1029, 1280, 125), (1349, 1280, 81),
+                                      (773, 1280, 115), (1637, 1280, 65), (1029, 1280, 115), (1541, 1280, 125), (1541, 1280, 115),
+                                      (261, 1280, 125), (2053, 256, 125), (2053, 1280, 97), (5117, 4864, 24), (5117, 4864, 70)])
+def test_rows_by_wide_requests(m, k, rows):
+    assert inst.row_kernel(m, k, rows) // 1_000_000 == 3
+    w, d, q, x = inputs(m, k, rows)
+    y = padded(rows, m)
+    attn.gemv_q8_0_rows(w, x, y, m, k, rows)
+    assert bool(y[rows].isnan().all())
+    exact = x.double() @ (d.double() * q.double()).reshape(m, k).T
+    err = (y[:rows] - exact).abs().max().item()
+    assert err <= 2e-6 * exact.abs().max().item() + 1e-5, err  # as test_row_kernel, k below 8,192
+    for first, n in ((0, 9), (rows - 9, 9), (0, rows - 1)):    # a row's bits, whichever tile its company takes
+        if n > 8:
+            z = padded(n, m)
+            attn.gemv_q8_0_rows(w, x[first:first + n], z, m, k, n)
+            assert torch.equal(z[:n], y[first:first + n]) and bool(z[n].isnan().all())
+    bad = x.clone()                                            # infinite in one row: its own results only
+    bad[rows // 2, k - 3] = float("inf")
+    z = padded(rows, m)
+    attn.gemv_q8_0_rows(w, bad, z, m, k, rows)
+    others = [i for i in range(rows) if i != rows // 2]
+    assert torch.equal(z[others], y[others]) and not bool(z[rows // 2].isfinite().any())
+
+
 @pytest.mark.parametrize("m,k,tokens,x16", inst.TILES)
 def test_tile(m, k, tokens, x16):
     w, d, q, x = inputs(m, k, tokens)
