@@ -702,7 +702,7 @@ int hipml_attn_front_encode_f32(hipml_stream_t stream, const int32_t *step, int 
     shadow_rows_unknown(k_cache, 1);
     return launch_front(as_stream(stream), qg, q, gate, k, q_norm, k_norm, n_heads, n_kv, n_rot, s0, s1,
                         s2, s3, step + 4, 0, 1, theta_base, eps, g_rope, dtype, v,
-                        static_cast<uint8_t *>(k_cache), static_cast<uint8_t *>(v_cache), step, 0, stride);
+                        static_cast<uint8_t *>(k_cache), static_cast<uint8_t *>(v_cache), stride);
 }
 
 int hipml_attn_chunk_front_encode_f32(hipml_stream_t stream, int dtype, const float *qg, float *k,
@@ -729,8 +729,7 @@ int hipml_attn_chunk_front_encode_f32(hipml_stream_t stream, int dtype, const fl
         return 0;
     rc = launch_front(as_stream(stream), qg, q, gate, k, q_norm, k_norm, n_heads, n_kv, n_rot, 0, 0, 0,
                       0, nullptr, pos0, tokens, theta_base, eps, g_rope, dtype, v,
-                      static_cast<uint8_t *>(k_cache), static_cast<uint8_t *>(v_cache), nullptr, pos0,
-                      stride);
+                      static_cast<uint8_t *>(k_cache), static_cast<uint8_t *>(v_cache), stride);
     return rc ? rc : shadow_rows_written(as_stream(stream), k_cache, pos0, tokens);
 }
 
@@ -751,8 +750,7 @@ int hipml_attn_front_rows_f32(hipml_stream_t stream, const float *qg, float *k, 
     if (rows == 0)
         return 0;
     return launch_front(as_stream(stream), qg, q, gate, k, q_norm, k_norm, n_heads, n_kv, n_rot, 0, 0, 0,
-                        0, nullptr, 0, rows, theta_base, eps, g_rope, -1, nullptr, nullptr, nullptr, nullptr,
-                        0, 0, pos, 0);
+                        0, nullptr, 0, rows, theta_base, eps, g_rope, -1, nullptr, nullptr, nullptr, 0, pos, 0);
 }
 
 // The same with the append of every row's K and V into its sequence's cache (slot r starts
@@ -778,8 +776,7 @@ int hipml_attn_front_rows_encode_f32(hipml_stream_t stream, int dtype, const flo
     shadow_rows_unknown(k_cache, slot_bytes * (size_t)slots);
     return launch_front(as_stream(stream), qg, q, gate, k, q_norm, k_norm, n_heads, n_kv, n_rot, 0, 0, 0,
                         0, nullptr, 0, slots, theta_base, eps, g_rope, dtype, v,
-                        static_cast<uint8_t *>(k_cache), static_cast<uint8_t *>(v_cache), nullptr, 0, stride,
-                        pos, slot_bytes);
+                        static_cast<uint8_t *>(k_cache), static_cast<uint8_t *>(v_cache), stride, pos, slot_bytes);
 }
 
 int hipml_kv_encode(hipml_stream_t stream, const int32_t *step, int dtype, const float *k_in,

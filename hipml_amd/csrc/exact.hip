@@ -78,7 +78,7 @@ __device__ __forceinline__ float tree_sum64(float v)
 //
 // unit u reads source row (src0 + u) of a position-major f32 [.][n_kv*head_dim]
 // buffer and writes cache position pos[u*pos_stride] (or start + u when pos is
-// null) of the cache at base + u*slot_bytes.
+// null: the launcher puts src0 and start into the pointers) of the cache at base + u*slot_bytes.
 
 __device__ __forceinline__ float half_wave_amax(float x)
 {
@@ -99,25 +99,33 @@ __device__ __forceinline__ void q8_encode_store(float x, uint8_t *dst_block, int
     dst_block[2 + lane32] = (uint8_t)(int8_t)q;
 }
 
-__global__ void __launch_bounds__(256) kv_encode_q8_kernel(
-    const float *__restrict__ k, const float *__restrict__ v, uint8_t *__restrict__ kc,
-    uint8_t *__restrict__ vc, int n_kv, int head_dim, int stride, const int32_t *__restrict__ pos,
-    int pos_stride, size_t slot_bytes, int start, int src0)
+// The append kernels' common body.  Both rows and the position are asked for before any is used, and everything their
+// addresses need arrives in registers with the wave (the arguments up to `shape`, 14 dwords): one memory round trip and the
+// store, where position arguments, position, K row and V row were one behind the other.  us a launch of 3 / 12 rows, replayed: 1.92 /
+// 1.96 -> 1.90 / 1.94 (an empty launch 1.58).
+// shape: the head dim, and from bit 16 on the stride of the positions.
+template <typename F>
+__device__ __forceinline__ void encode_rows(const float *k, const float *v, uint8_t *kc, uint8_t *vc, const int32_t *pos,
+                                            size_t slot_bytes, int stride, uint32_t shape, int n_kv, int block_bytes, F &&encode)
 {
-    const int h = blockIdx.x;
-    const int u = blockIdx.y;
-    const int t = threadIdx.x;
+    const int head_dim = (int)(shape & 0xffffu), h = blockIdx.x, u = blockIdx.y, t = threadIdx.x;
     if (t >= head_dim)
         return;
-    const int chunk = t >> 5;
-    const int lane32 = t & 31;
+    const int p = pos ? pos[(size_t)u * (shape >> 16)] : u;
+    const size_t src = ((size_t)u * n_kv + h) * head_dim + t;
+    const float xk = k[src], xv = v[src];
     const int nchunk = head_dim >> 5;
-    const int p = pos ? pos[(size_t)u * pos_stride] : start + u;
-    const size_t src = ((size_t)(src0 + u) * n_kv + h) * head_dim + t;
-    const size_t off = (size_t)u * slot_bytes +
-                       (((size_t)h * stride + p) * nchunk + chunk) * kQ8BlockBytes;
-    q8_encode_store(k[src], kc + off, lane32);
-    q8_encode_store(v[src], vc + off, lane32);
+    const size_t off = (size_t)u * slot_bytes + (((size_t)h * stride + p) * nchunk + (t >> 5)) * block_bytes;
+    encode(xk, kc + off, t & 31);
+    encode(xv, vc + off, t & 31);
+}
+
+__global__ void __launch_bounds__(256) kv_encode_q8_kernel(
+    const float *__restrict__ k, const float *__restrict__ v, uint8_t *__restrict__ kc, uint8_t *__restrict__ vc,
+    const int32_t *__restrict__ pos, size_t slot_bytes, int stride, uint32_t shape, int n_kv)
+{
+    encode_rows(k, v, kc, vc, pos, slot_bytes, stride, shape, n_kv, kQ8BlockBytes,
+                [](float x, uint8_t *dst, int lane32) { q8_encode_store(x, dst, lane32); });
 }
 
 // ---- q4_0 quantize + append (crates/hipml-core/src/kv.rs:201-218) ---------------------------
@@ -156,24 +164,11 @@ __device__ __forceinline__ void q4_encode_store(float x, uint8_t *dst_block, int
 }
 
 __global__ void __launch_bounds__(256) kv_encode_q4_kernel(
-    const float *__restrict__ k, const float *__restrict__ v, uint8_t *__restrict__ kc,
-    uint8_t *__restrict__ vc, int n_kv, int head_dim, int stride, const int32_t *__restrict__ pos,
-    int pos_stride, size_t slot_bytes, int start, int src0)
+    const float *__restrict__ k, const float *__restrict__ v, uint8_t *__restrict__ kc, uint8_t *__restrict__ vc,
+    const int32_t *__restrict__ pos, size_t slot_bytes, int stride, uint32_t shape, int n_kv)
 {
-    const int h = blockIdx.x;
-    const int u = blockIdx.y;
-    const int t = threadIdx.x;
-    if (t >= head_dim)
-        return;
-    const int chunk = t >> 5;
-    const int lane32 = t & 31;
-    const int nchunk = head_dim >> 5;
-    const int p = pos ? pos[(size_t)u * pos_stride] : start + u;
-    const size_t src = ((size_t)(src0 + u) * n_kv + h) * head_dim + t;
-    const size_t off = (size_t)u * slot_bytes +
-                       (((size_t)h * stride + p) * nchunk + chunk) * kQ4BlockBytes;
-    q4_encode_store(k[src], kc + off, lane32);
-    q4_encode_store(v[src], vc + off, lane32);
+    encode_rows(k, v, kc, vc, pos, slot_bytes, stride, shape, n_kv, kQ4BlockBytes,
+                [](float x, uint8_t *dst, int lane32) { q4_encode_store(x, dst, lane32); });
 }
 
 int launch_kv_encode(hipStream_t st, int q4, const float *k, const float *v, uint8_t *kc, uint8_t *vc,
@@ -183,14 +178,15 @@ int launch_kv_encode(hipStream_t st, int q4, const float *k, const float *v, uin
     if (units == 0)
         return 0;
     const int block = head_dim < 64 ? 64 : head_dim;
+    const size_t row = (size_t)(head_dim / 32) * (q4 ? kQ4BlockBytes : kQ8BlockBytes); // bytes of a cache row
+    const uint32_t shape = (uint32_t)head_dim | (uint32_t)pos_stride << 16;
     // grid.y is limited to 65535: walk long chunks in slices.
     for (int u0 = 0; u0 < units; u0 += 32768) {
         const int n = units - u0 < 32768 ? units - u0 : 32768;
-        HIPML_LAUNCH(q4 ? kv_encode_q4_kernel : kv_encode_q8_kernel, dim3(n_kv, n, 1),
-                           dim3(block, 1, 1), 0, st, k, v, kc + (size_t)u0 * slot_bytes,
-                           vc + (size_t)u0 * slot_bytes, n_kv, head_dim, stride,
-                           pos ? pos + (size_t)u0 * pos_stride : nullptr, pos_stride, slot_bytes,
-                           start + u0, src0 + u0);
+        const size_t src = (size_t)(src0 + u0) * n_kv * head_dim;
+        const size_t at = (size_t)u0 * slot_bytes + (pos ? 0 : (size_t)(start + u0) * row); // (without positions: row start + u)
+        HIPML_LAUNCH(q4 ? kv_encode_q4_kernel : kv_encode_q8_kernel, dim3(n_kv, n, 1), dim3(block, 1, 1), 0, st, k + src,
+                     v + src, kc + at, vc + at, pos ? pos + (size_t)u0 * pos_stride : nullptr, slot_bytes, stride, shape, n_kv);
         int rc = launched(q4 ? "kv_encode_q4" : "kv_encode_q8");
         if (rc)
             return rc;
@@ -540,56 +536,71 @@ int launch_rope_encode_chunk(hipStream_t st, int q4, float *q, float *k, const f
 // exchanges; IEEE addition commutes, so every lane ends with red[0]); mean = sum / 256;
 // scale = 1 / sqrtf(mean + eps) with the correctly rounded divide and square root; the value is
 // (x * scale) * w; the rotation reads cos/sin as the other RoPE kernels here do.
-// grid: ceil((n_heads + n_kv) * rows / 4) workgroups of 4 waves.  `pos` (device int32[4]) gives
-// the four M-RoPE position ids of a single row; when it is null, row t rotates at pos0 + t.
-// Per-row positions of a batch of sequences, and what the append half of a fused launch needs.
-struct FrontAppend {
-    const int32_t *rowpos; // non-null: row r belongs to sequence r and sits at text position
-                           // rowpos[2 r] (device int32 [rows][2] = position, live length)
-    size_t slot_bytes;     // with rowpos: sequence r's cache starts r * slot_bytes into kc / vc
-    const float *v;        // [rows][n_kv][256]
-    uint8_t *kc, *vc;      // caches
-    const int32_t *step;   // row 0 goes to position step[0]; null: row r goes to start + r (or rowpos)
-    int start, stride;
+// grid: (ceil(heads of a row / 4), rows), workgroups of 4 waves.
+//
+// What a launch over few rows costs beside the launch itself is the chain of loads that wait for one another.  So the
+// pointers to the row, the weights, the table and the positions are leading arguments, which arrive in registers (14 dwords);
+// the other arguments and the position come in one round trip, in the shadow of the row, and the table's in the next; no
+// vector load lies in between, whose wait would be one for the rows as well.  (Arguments, the rest of them, the append's, the
+// position, the sections' positions as a vector load, the table and the append's position were seven, one behind the other: us
+// a launch, replayed, over 3 rows with append 2.93 -> 2.60, over 24 without 2.34 -> 2.20; an empty launch 1.58.)
+enum { kFrontIds, kFrontRows, kFrontChunk }; // where a row's position comes from
+struct FrontArgs {
+    float *q, *gate;
+    const float *v;      // [rows][n_kv][256]
+    uint8_t *kc, *vc;    // caches
+    size_t slot_bytes;   // kFrontRows: sequence r's cache starts r * slot_bytes into kc / vc
+    int n_rot, s0, s1, s2, s3, pos0, stride, tab_rows;
+    float theta, eps;
 };
 
 // ENC: 0 = front end only, 1 = also quantize the finished K row and the V row to q8_0 and append
 // them, 2 = the same to q4_0 -- the K wave keeps its row in registers (element lane + 64 j in slot
 // j, so a half-wave holds one block of 32, as the append kernels' 32-lane groups do) and n_kv more
 // waves per row take the V rows.  Same expressions on the same values: the bits of the two launches.
+// posp: kFrontIds (one row) the four M-RoPE ids, with ENC the append's position four before them (the step buffer);
+// kFrontRows [rows][2], a row's text position first; kFrontChunk unused, row r is at pos0 + r.
 template <int ENC>
-__global__ void __launch_bounds__(256) front_kernel(
-    const float *__restrict__ qg, float *__restrict__ q, float *__restrict__ gate, float *k,
-    const float *__restrict__ qw, const float *__restrict__ kw, int n_heads, int n_kv, int n_rot,
-    int s0, int s1, int s2, int s3, const int32_t *__restrict__ pos, int pos0, int rows, float theta,
-    float eps, const float *__restrict__ tab, int tab_rows, const FrontAppend ap)
+__global__ void __launch_bounds__(256) front_kernel(const float *__restrict__ qg, float *k, const float *__restrict__ qw,
+                                                    const float *__restrict__ kw, const float *__restrict__ tab,
+                                                    const int32_t *__restrict__ posp, uint32_t heads_mode, int n_kv,
+                                                    const FrontArgs a)
 {
     __shared__ float buf[4][kHeadDim];
-    // (the wave's number as a scalar: row, head and addresses are scalar arithmetic then.  us over 1 / 16 / 672 / 1,024 / 2,048
-    // rows 3.26 / 3.58 / 15.9 / 23.4 / 40.8 -> 3.15 / 3.48 / 15.4 / 23.0 / 39.6; with the gate's half, which is copied as it is,
-    // 16 bytes a lane 3.07 / 3.34 / 14.8 / 22.6 / 39.2, 5.7 TB/s read and written.  Tried: 16 bytes a lane for the q rows,
-    // 17.3 us over 672: the tree's exchanges four times over)
+    // (the wave's number as a scalar: row, head and addresses are scalar arithmetic then; the gate's half, which is copied as
+    // it is, 16 bytes a lane.  Tried: 16 bytes a lane for the q rows, 17.3 us over 672 rows where this takes 15: the tree's
+    // exchanges four times over)
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const int per_row = n_heads + n_kv;
-    const int idx = blockIdx.x * 4 + wave;
-    const int nfront = per_row * rows;
-    if (idx >= nfront + (ENC ? n_kv * rows : 0))
+    const int n_heads = (int)(heads_mode & 0x3fffffffu), mode = (int)(heads_mode >> 30);
+    const int row = blockIdx.y, hb = blockIdx.x * 4 + wave;
+    if (hb >= n_heads + n_kv + (ENC ? n_kv : 0))
         return; // no workgroup-wide barrier below: waves are independent
     const int lane32 = lane & 31;
-    if (ENC && idx >= nfront) {
+    // the position, and the append's
+    int id[4] = {0, 0, 0, 0}, at = 0;
+    if (mode == kFrontIds) {
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            id[j] = posp[j];
+        if (ENC)
+            at = posp[-4];
+    } else if (mode == kFrontRows) {
+        id[0] = at = posp[2 * (size_t)row];
+    } else {
+        id[0] = at = a.pos0 + row;
+    }
+    if (ENC && hb >= n_heads + n_kv) {
         // a V row: quantize and append
-        const int u = idx - nfront;
-        const int row = u / n_kv, h = u - row * n_kv;
-        const int p = ap.step ? ap.step[0] : ap.rowpos ? ap.rowpos[2 * row] : ap.start + row;
-        uint8_t *vc = ap.vc + (ap.rowpos ? (size_t)row * ap.slot_bytes : 0);
-        const float *src = ap.v + (size_t)u * kHeadDim;
+        const int h = hb - n_heads - n_kv;
+        const float *src = a.v + ((size_t)row * n_kv + h) * kHeadDim;
         float x[4];
 #pragma unroll
         for (int j = 0; j < 4; j++)
             x[j] = src[lane + 64 * j];
+        uint8_t *vc = a.vc + (mode == kFrontRows ? (size_t)row * a.slot_bytes : 0);
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            const size_t blk = ((size_t)h * ap.stride + p) * (kHeadDim / 32) + 2 * j + (lane >> 5);
+            const size_t blk = ((size_t)h * a.stride + at) * (kHeadDim / 32) + 2 * j + (lane >> 5);
             if (ENC == 2)
                 q4_encode_store(x[j], vc + blk * kQ4BlockBytes, lane32);
             else
@@ -597,14 +608,10 @@ __global__ void __launch_bounds__(256) front_kernel(
         }
         return;
     }
-    const int row = idx / per_row;
-    const int hb = idx - row * per_row;
     const bool is_q = hb < n_heads;
     const int h = is_q ? hb : hb - n_heads;
     const float *src = is_q ? qg + ((size_t)row * n_heads + h) * (2 * kHeadDim)
                             : k + ((size_t)row * n_kv + h) * kHeadDim;
-    float *dst = is_q ? q + ((size_t)row * n_heads + h) * kHeadDim
-                      : k + ((size_t)row * n_kv + h) * kHeadDim;
     const float *w = is_q ? qw : kw;
 
     // everything this wave will need from memory is asked for here: the row, the gate half, the norm
@@ -619,38 +626,32 @@ __global__ void __launch_bounds__(256) front_kernel(
         wv[j] = w[lane + 64 * j];
     if (is_q)
         g = *reinterpret_cast<const float4a4 *>(src + kHeadDim + 4 * lane);
-    const int half = n_rot >> 1;
-    const int sect = s0 + s1 + s2 + s3;
+    const int half = a.n_rot >> 1;
+    const int sect = mode == kFrontIds ? a.s0 + a.s1 + a.s2 + a.s3 : 0;
     float cs[4], sn[4];
 #pragma unroll
     for (int j = 0; j < 4; j++) {
-        const int e = lane + 64 * j;
         cs[j] = 1.0f;
         sn[j] = 0.0f;
-        if (e < n_rot) {
-            const int c = e < half ? e : e - half;
-            int p = pos ? pos[0] : ap.rowpos ? ap.rowpos[2 * row] : pos0 + row;
-            if (pos && sect > 0) {
-                const int sc = c % sect;
-                if (sc < s0)
-                    p = pos[0];
-                else if (sc < s0 + s1)
-                    p = pos[1];
-                else if (sc < s0 + s1 + s2)
-                    p = pos[2];
-                else
-                    p = pos[3];
-            }
-            rope_cs(tab, tab_rows, half, c, p, n_rot, theta, cs[j], sn[j]);
+        if (64 * j >= a.n_rot) // (the same for all lanes)
+            continue;
+        const int e = lane + 64 * j;
+        const int c = e < half ? e : e - half;
+        int p = id[0];
+        if (sect > 0) {
+            const int sc = sect >= half ? c : c % sect;
+            p = sc < a.s0 ? id[0] : sc < a.s0 + a.s1 ? id[1] : sc < a.s0 + a.s1 + a.s2 ? id[2] : id[3];
         }
+        if (e < a.n_rot)
+            rope_cs(tab, a.tab_rows, half, c, p, a.n_rot, a.theta, cs[j], sn[j]);
     }
     if (is_q)
-        *reinterpret_cast<float4a4 *>(gate + ((size_t)row * n_heads + h) * kHeadDim + 4 * lane) = g;
+        *reinterpret_cast<float4a4 *>(a.gate + ((size_t)row * n_heads + h) * kHeadDim + 4 * lane) = g;
     const float a0 = x[0] * x[0] + x[2] * x[2]; // off = 128
     const float a1 = x[1] * x[1] + x[3] * x[3];
     const float sum = tree_sum64(a0 + a1);      // off = 64, then 32 .. 1
     const float mean_sq = sum / (float)kHeadDim;
-    const float scale = 1.0f / sqrtf(mean_sq + eps);
+    const float scale = 1.0f / sqrtf(mean_sq + a.eps);
 #pragma unroll
     for (int j = 0; j < 4; j++)
         buf[wave][lane + 64 * j] = x[j] * scale * wv[j];
@@ -659,11 +660,13 @@ __global__ void __launch_bounds__(256) front_kernel(
 
     // element e = lane + 64 j: rotated with its partner when e < n_rot (the first half of the pairs
     // takes x1 c - x2 s, the second x1 s + x2 c), passed through otherwise
+    float *dst = is_q ? a.q + ((size_t)row * n_heads + h) * kHeadDim
+                      : k + ((size_t)row * n_kv + h) * kHeadDim;
 #pragma unroll
     for (int j = 0; j < 4; j++) {
         const int e = lane + 64 * j;
         float out = buf[wave][e];
-        if (e < n_rot) {
+        if (e < a.n_rot) {
             const bool first = e < half;
             const int c = first ? e : e - half;
             const float x1 = buf[wave][c];
@@ -674,11 +677,10 @@ __global__ void __launch_bounds__(256) front_kernel(
         x[j] = out;
     }
     if (ENC && !is_q) {
-        const int p = ap.step ? ap.step[0] : ap.rowpos ? ap.rowpos[2 * row] : ap.start + row;
-        uint8_t *kc = ap.kc + (ap.rowpos ? (size_t)row * ap.slot_bytes : 0);
+        uint8_t *kc = a.kc + (mode == kFrontRows ? (size_t)row * a.slot_bytes : 0);
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            const size_t blk = ((size_t)h * ap.stride + p) * (kHeadDim / 32) + 2 * j + (lane >> 5);
+            const size_t blk = ((size_t)h * a.stride + at) * (kHeadDim / 32) + 2 * j + (lane >> 5);
             if (ENC == 2)
                 q4_encode_store(x[j], kc + blk * kQ4BlockBytes, lane32);
             else
@@ -691,26 +693,40 @@ __global__ void __launch_bounds__(256) front_kernel(
 int launch_front(hipStream_t st, const float *qg, float *q, float *gate, float *k, const float *qw,
                  const float *kw, int n_heads, int n_kv, int n_rot, int s0, int s1, int s2, int s3,
                  const int32_t *pos, int pos0, int rows, float theta, float eps, const RopeTable &tab,
-                 int enc, const float *v, uint8_t *kc, uint8_t *vc, const int32_t *step, int start,
-                 int stride, const int32_t *rowpos, size_t slot_bytes)
+                 int enc, const float *v, uint8_t *kc, uint8_t *vc, int stride, const int32_t *rowpos,
+                 size_t slot_bytes)
 {
     int tab_rows = 0;
     const float *t = table_for(tab, theta, n_rot, &tab_rows);
     const int per_row = n_heads + n_kv + (enc >= 0 ? n_kv : 0);
-    const int max_rows = 1 << 22; // keeps (rows * per_row) far inside int
+    const int max_rows = 32768; // grid.y
     for (int r0 = 0; r0 < rows; r0 += max_rows) {
         const int n = rows - r0 < max_rows ? rows - r0 : max_rows;
-        const unsigned grid = (unsigned)(((long long)per_row * n + 3) / 4);
-        const FrontAppend ap = {rowpos ? rowpos + (size_t)r0 * 2 : nullptr, slot_bytes,
-                                v ? v + (size_t)r0 * n_kv * kHeadDim : nullptr,
-                                kc ? kc + (rowpos ? (size_t)r0 * slot_bytes : 0) : nullptr,
-                                vc ? vc + (rowpos ? (size_t)r0 * slot_bytes : 0) : nullptr, step, start + r0,
-                                stride};
+        const size_t slot_at = rowpos ? (size_t)r0 * slot_bytes : 0;
+        FrontArgs a;
+        a.q = q + (size_t)r0 * n_heads * kHeadDim;
+        a.gate = gate + (size_t)r0 * n_heads * kHeadDim;
+        a.v = v ? v + (size_t)r0 * n_kv * kHeadDim : nullptr;
+        a.kc = kc ? kc + slot_at : nullptr;
+        a.vc = vc ? vc + slot_at : nullptr;
+        a.slot_bytes = slot_bytes;
+        a.n_rot = n_rot;
+        a.s0 = s0;
+        a.s1 = s1;
+        a.s2 = s2;
+        a.s3 = s3;
+        a.pos0 = pos0 + r0;
+        a.stride = stride;
+        a.tab_rows = tab_rows;
+        a.theta = theta;
+        a.eps = eps;
+        // (the append's positions are the rotation's: the step buffer's own lies four in front of its ids, the others are the same)
+        const int32_t *posp = pos ? pos : rowpos ? rowpos + (size_t)r0 * 2 : nullptr;
+        const uint32_t mode = pos ? kFrontIds : rowpos ? kFrontRows : kFrontChunk;
         auto kern = enc < 0 ? front_kernel<0> : enc == 0 ? front_kernel<1> : front_kernel<2>;
-        HIPML_LAUNCH(kern, dim3(grid, 1, 1), dim3(256, 1, 1), 0, st,
-                           qg + (size_t)r0 * n_heads * 2 * kHeadDim, q + (size_t)r0 * n_heads * kHeadDim,
-                           gate + (size_t)r0 * n_heads * kHeadDim, k + (size_t)r0 * n_kv * kHeadDim, qw, kw,
-                           n_heads, n_kv, n_rot, s0, s1, s2, s3, pos, pos0 + r0, n, theta, eps, t, tab_rows, ap);
+        HIPML_LAUNCH(kern, dim3((unsigned)(per_row + 3) / 4, (unsigned)n, 1), dim3(256, 1, 1), 0, st,
+                     qg + (size_t)r0 * n_heads * 2 * kHeadDim, k + (size_t)r0 * n_kv * kHeadDim, qw, kw, t, posp,
+                     (uint32_t)n_heads | mode << 30, n_kv, a);
         int rc = launched(enc < 0 ? "attn_front_f32" : "attn_front_encode_f32");
         if (rc)
             return rc;
