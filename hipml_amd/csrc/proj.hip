@@ -1183,19 +1183,22 @@ __global__ void __launch_bounds__((kUnitsThreads<XT, RW, HALF, WIDE>), (UnitsSha
         wait_unit(0);
         load(even, 0);
     }
-    // unit i is in `now`
+    // Unit i is in `now`.  Its place is asked for anew at once and its products stand in front of the wait for unit i + 1: behind
+    // that wait they held up the next request as well.  us before / now over 1024 x 5120 and 9 / 24 / 32 rows 7.2 / 7.6 / 7.7 and
+    // 6.9 / 7.4 / 7.4, 4096 x 4096 and 24 rows 11.7 and 11.5, 5120 x 6144 and 16 / 24 / 40 rows 14.8 / 18.7 / 23.1 and 14.5 / 18.6
+    // / 22.8, from HBM.  (gemv_q8_blocks_kernel so: no gain.)
     auto turn = [&](Regs &now, Regs &next, float4v (&sum)[XT][MT], int i) {
         __builtin_amdgcn_s_waitcnt(0xc07f); // lgkmcnt(0), as above: unit i's place in the ring has been read
         asm volatile("" ::: "memory");
         if (i + D < mine)
             issue(i + D);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(now, sum);
+        __builtin_amdgcn_sched_barrier(0);
         if (i + 1 < mine) {
             wait_unit(i + 1);
             load(next, i + 1);
         }
-        __builtin_amdgcn_sched_barrier(0);
-        multiply(now, sum);
-        __builtin_amdgcn_sched_barrier(0);
     };
     for (int i = 0; i < mine; i += 2) {
         turn(even, odd, acc[0], i);
