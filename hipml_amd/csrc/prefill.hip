@@ -2203,6 +2203,49 @@ int chunk_tile_slices(int pos0, int tokens, int n_head, int n_kv, int most)
     return best;
 }
 
+// us of chunk_q8_kernel over the cache with `splits` slices and of the launch behind it: rounds of 256 workgroups, the key tiles
+// of a slice, how full a round is (workgroups share the chip's bandwidth and power), and the rows of sums that the slices write
+// and the second launch reads.  Fitted at 244 shapes (130 to 2,000 tokens behind 64 to 60,000, 2 to 32 slices, both formats;
+// 3.6 % rms).
+static float chunk_q8_us(int pos0, int tokens, int n_head, int n_kv, int splits)
+{
+    const int group = n_head / n_kv, ntask = (tokens + kQTile - 1) / kQTile * group, nblock = (ntask + kTasks - 1) / kTasks;
+    const int tiles = (pos0 + tokens + kKTile - 1) / kKTile, slice = (tiles + splits - 1) / splits;
+    int nslice = 0;
+    if (block_slices(0, ntask, group, tokens, pos0, splits, slice, nullptr) == splits)
+        nslice = nblock * splits;
+    else
+        for (int tb = 0; tb < nblock; tb++)
+            nslice += block_slices(tb, ntask, group, tokens, pos0, splits, slice, nullptr);
+    const int wgs = n_kv * nslice, rounds = (wgs + 255) / 256;
+    const float fill = (float)wgs / (256.0f * (float)rounds);
+    const float rows = (float)tokens * (float)n_head / 24.0f * (float)nslice / (float)nblock;
+    return 0.5f + (float)rounds * (12.3f + (float)slice * (1.99f + 1.69f * fill)) + 0.00615f * rows;
+}
+
+// Slices, of the `splits` that the scratch holds, with which chunk_q8_kernel runs a chunk over the cache.  A count that fills the
+// chip's rounds leaves out what a second round costs beside its keys and what the rows of sums cost; a chunk near position 0,
+// whose blocks see few key tiles, pays for slices most.  us with the count that fills / with this one: 350 tokens behind
+// 20,000 218 (14) / 200 (7), 420 behind 5,003 104 (12) / 85 (5), 512 behind 7,000 140 (10) / 118 (5) and behind 60,000 797 (16)
+// / 751 (5), 2,000 behind 300 199 (8) / 131 (3) and behind 1,700 269 (6) / 202 (3).  Within 3 % the given count stays: so close
+// the costs above do not tell which is faster.  With as many blocks as two rounds hold a chunk is not sliced to fill the chip.
+static int chunk_q8_slices(int pos0, int tokens, int n_head, int n_kv, int splits)
+{
+    const int nblock = ((tokens + kQTile - 1) / kQTile * (n_head / n_kv) + kTasks - 1) / kTasks;
+    if (n_kv * nblock >= 512)
+        return splits;
+    int best = splits;
+    float best_cost = 0.97f * chunk_q8_us(pos0, tokens, n_head, n_kv, splits);
+    for (int s = 2; s < splits; s++) {
+        const float cost = chunk_q8_us(pos0, tokens, n_head, n_kv, s);
+        if (cost < best_cost) {
+            best = s;
+            best_cost = cost;
+        }
+    }
+    return best;
+}
+
 // Splits of the keys, of at most `splits`, with which chunk_wg_kernel runs a chunk over the cache; 0: chunk_q8_kernel does.
 // That kernel's workgroups hold 32 tokens x 8 heads and write the sums of every slice of the keys to memory: 117 tokens
 // behind 1,500 are 12 of them and take 10 slices, 28 MB written and read again.  This one's hold 32 tokens x 2 heads and
@@ -2212,6 +2255,9 @@ int chunk_tile_slices(int pos0, int tokens, int n_head, int n_kv, int most)
 // one is, 8 KB of sums per token and head.  us before / now over 4 @ 256 19.6 / 15.6, 16 @ 500 21.3 / 16.1, 32 @ 2,000 26.9 /
 // 20.7, 32 @ 8,000 42.6 / 31.3, 64 @ 2,000 31.4 / 25.4, 64 @ 32,000 114 / 104, 117 @ 1,500 33.5 / 28.6, 256 @ 1,000 34.7 /
 // 33.0; not taken at 128 @ 4,000 39.8 (here 41), 200 @ 4,000 49.7 (55), 256 @ 8,000 79 (120).
+// And not where the other kernel's cost by chunk_q8_us, fitted at more tokens, is lower by a tenth, as with fewer slices than it
+// is given: 330 @ 1,862 54.9 here / 46.0 there, 464 @ 3,639 92.5 / 73.9, 226 @ 3,679 57.7 / 50.4; over
+// 33 shapes where the two estimates differ, those under a tenth take 19 % less to 1 % more here, those over it as long or more.
 static int chunk_wg_splits(int pos0, int tokens, int n_head, int n_kv, int splits)
 {
     const int group = n_head / n_kv, keys = pos0 + tokens;
@@ -2235,10 +2281,17 @@ static int chunk_wg_splits(int pos0, int tokens, int n_head, int n_kv, int split
     const long long other = (long long)n_kv * splits * ((ntt * group + kTasks - 1) / kTasks), rounds = (other + 255) / 256;
     const float fill = (float)other / (256.0f * (float)rounds);
     const float cost = 12.6f + (float)rounds * (float)slice * (2.53f + fill) + (float)splits * (0.152f + 0.0067f * sums);
-    return best_cost < 0.95f * cost ? best : 0;
+    if (best_cost >= 0.95f * cost)
+        return 0;
+    const int slices = chunk_q8_slices(pos0, tokens, n_head, n_kv, splits);
+    return best_cost < 1.1f * chunk_q8_us(pos0, tokens, n_head, n_kv, slices) ? best : 0;
 }
 
-// For tests: the above, 0 for chunk_q8_kernel.
+// For tests: the above two, 0 for chunk_q8_kernel in the second.
+extern "C" int hipml_dbg_chunk_q8_slices(int pos0, int tokens, int n_head, int n_kv, int splits)
+{
+    return chunk_q8_slices(pos0, tokens, n_head, n_kv, splits);
+}
 extern "C" int hipml_dbg_chunk_wg_splits(int pos0, int tokens, int n_head, int n_kv, int splits)
 {
     return chunk_wg_splits(pos0, tokens, n_head, n_kv, splits);
@@ -2294,6 +2347,8 @@ int launch_chunk_q8(hipStream_t st, const float *q, const uint8_t *kc, const uin
     a.tokens = tokens;
     a.stride = stride;
     a.splits = splits < 2 ? 1 : splits;
+    if (splits >= 2 && kv_f16 == nullptr)
+        a.splits = chunk_q8_slices(pos0, tokens, n_head, n_kv, splits);
     a.qslots = (tokens + 31) / 32 * 32;
     a.ntask = (tokens + kQTile - 1) / kQTile * a.group;
     a.nblock = (a.ntask + kTasks - 1) / kTasks;

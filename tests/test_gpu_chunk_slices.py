@@ -1,0 +1,71 @@
+"""Chunks over the cache for which fewer key slices run than the caller's scratch holds: the result is the oracle's (the gate of
+the chunk kernels) and that of a call which asks for those slices, and the rest of the scratch is left alone."""
+import numpy as np
+import pytest
+import torch
+
+from hipml_amd import attn
+
+N_HEAD, N_KV, HD = 24, 4, 256
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [0, 1])
+@pytest.mark.parametrize("tok,pos0,splits,n_head,n_kv", [
+    (450, 1800, 12, 24, 4),   # every block of tokens with all slices, a ragged last tile
+    (353, 5003, 14, 24, 4),   # twelve blocks, two rounds of workgroups in one
+    (900, 100, 8, 24, 4),     # blocks near position 0 with fewer slices than the last
+    (700, 0, 8, 24, 4), (600, 40, 8, 32, 8), (1501, 90, 12, 14, 2)])
+def test_fewer_slices_than_the_scratch_holds(tok, pos0, splits, n_head, n_kv, dtype):
+    from oracle import binding as orc
+    from gpu_util import SCALE, dev, host, report
+    from test_gpu_prefill import GATE
+    attn.init(0)
+    lib = attn.lib()
+    used = lib.hipml_dbg_chunk_q8_slices(pos0, tok, n_head, n_kv, splits)
+    assert 2 <= used < splits and lib.hipml_dbg_chunk_wg_splits(pos0, tok, n_head, n_kv, splits) == 0
+    assert lib.hipml_dbg_chunk_q8_slices(pos0, tok, n_head, n_kv, used) == used
+    r = orc.Rng(0x511C_0000 + tok * 131 + pos0)
+    stride = pos0 + tok + 3
+    kb = orc.quantize(dtype, r.normal_array((n_kv, stride, HD))).reshape(n_kv, stride, -1)
+    vb = orc.quantize(dtype, r.normal_array((n_kv, stride, HD))).reshape(n_kv, stride, -1)
+    q, gate = r.normal_array((tok, n_head, HD)), dev(r.normal_array((tok, n_head, HD)))
+    qd, kd, vd = dev(q), dev(kb), dev(vb)
+    acc, ml = attn.chunk_scratch(tok, n_head, splits)
+    acc.fill_(7.0), ml.fill_(7.0)
+    out, asked, gated_rows, work = (torch.full((tok + 1, n_head, HD), float("nan"), device="cuda") for _ in range(4))
+    out16 = torch.full((tok + 1, n_head, HD), float("nan"), dtype=torch.float16, device="cuda")
+    args = (n_head, n_kv, HD, pos0, tok, dtype + 1, stride, acc, ml)
+    attn.chunk_attention_q8_split(qd, kd, vd, out, *args, splits)
+    attn.chunk_attention_q8_split_gate(qd, kd, vd, gate, gated_rows, *args, splits)
+    attn.chunk_attention_q8_split_gate_f16(qd, kd, vd, gate, work, out16, *args, splits)
+    torch.cuda.synchronize()
+    assert bool((acc[used:] == 7.0).all()) and bool((ml[used:] == 7.0).all())
+    attn.chunk_attention_q8_split(qd, kd, vd, asked, *args, used)
+    two = torch.empty((tok, n_head, HD), device="cuda")
+    attn.q_gate(out[:tok].contiguous(), gate, two)
+    torch.cuda.synchronize()
+    want = orc.attn_chunk_kv(q, kb, vb, n_head, n_kv, HD, pos0, tok, stride, SCALE, n_threads=8, dtype=dtype)
+    assert report(f"chunk {tok}@{pos0}, {used} of {splits} slices", want, host(out[:tok]), *GATE)[0]
+    assert torch.equal(asked[:tok], out[:tok])
+    assert torch.equal(two, gated_rows[:tok]) and torch.equal(out16[:tok], two.to(torch.float16))
+    for x in (out, asked, gated_rows, out16):
+        assert bool(x[tok].isnan().all())
+
+
+def test_the_slices_that_run_fit_the_scratch():
+    # never more than asked for, never one alone (that is another kernel's sums), and no other count where the blocks fill the
+    # chip by themselves
+    lib = attn.lib()
+    rng = np.random.default_rng(7)
+    for _ in range(3000):
+        n_kv = int(rng.integers(1, 9))
+        n_head = n_kv * int(rng.integers(1, 9))
+        tok, pos0 = (int(np.exp(rng.uniform(0.0, np.log(top)))) for top in (6000, 200_000))
+        splits = int(rng.integers(2, 65))
+        used = lib.hipml_dbg_chunk_q8_slices(pos0, tok, n_head, n_kv, splits)
+        assert 2 <= used <= splits
+        blocks = ((tok + 31) // 32 * (n_head // n_kv) + 7) // 8
+        if n_kv * blocks >= 512:
+            assert used == splits
+        assert lib.hipml_dbg_chunk_wg_splits(pos0, tok, n_head, n_kv, splits) <= splits
