@@ -1100,9 +1100,10 @@ static int chunk_q8_common(hipml_stream_t stream, const float *q, const void *kc
                                part_acc, part_ml, splits, out16, want_f16);
     if (rc || tokens == 0)
         return rc;
-    // a cache with a registered f16 shadow: the sliced attention reads its tiles (as many slices as the policy
-    // gives a chunk over such a copy, within what the scratch was sized for)
-    if (splits >= 2 && kv_f16 == nullptr && rope_tab == nullptr) {
+    // a cache with a registered f16 shadow: the sliced attention reads its tiles (as many slices as pay, of
+    // those that the policy gives a chunk over such a copy and the scratch was sized for)
+    if (splits >= 2 && kv_f16 == nullptr && rope_tab == nullptr &&
+        !chunk_reads_cache(pos0, tokens, n_head, n_kv, splits)) {
         const void *copy = nullptr;
         if (shadow_for_chunk(as_stream(stream), kc, vc, n_kv, stride, dtype == 2 ? 1 : 0, pos0 + tokens, &copy, &rc)) {
             if (rc)
@@ -1110,6 +1111,8 @@ static int chunk_q8_common(hipml_stream_t stream, const float *q, const void *kc
             const int slices = hipml_attn_chunk_slices(pos0, tokens, n_kv);
             kv_f16 = copy;
             splits = slices < splits ? (slices < 1 ? 1 : slices) : splits;
+            if (splits >= 2)
+                splits = chunk_run_slices(pos0, tokens, n_head, n_kv, splits, true);
             dtype = 1; // (the tiles are f16 whatever the cache holds)
         }
     }

@@ -147,6 +147,9 @@ int chunk_tiles_splits(int pos0, int tokens, int n_head, int n_kv, int slices);
 // chunks over f16 tiles the one that costs least.
 int chunk_fill_slices(int pos0, int tokens, int n_kv);
 int chunk_tile_slices(int pos0, int tokens, int n_head, int n_kv, int most);
+// And the slices that a chunk over the cache runs, or over its registered copy (f16), of the `splits` that the scratch holds.
+int chunk_run_slices(int pos0, int tokens, int n_head, int n_kv, int splits, bool f16);
+bool chunk_reads_cache(int pos0, int tokens, int n_head, int n_kv, int splits); // also where a copy is registered
 bool chunk_tiles_pay(int pos0, int tokens); // the shapes for which hipml_attn_chunk_splits asks for that count
 int launch_kv_f16_rows(hipStream_t st, const uint8_t *kc, const uint8_t *vc, void *copy, int n_kv, int stride,
                        int start, int rows, int q4);

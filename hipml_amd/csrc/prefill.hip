@@ -2203,41 +2203,76 @@ int chunk_tile_slices(int pos0, int tokens, int n_head, int n_kv, int most)
     return best;
 }
 
-// us of chunk_q8_kernel over the cache with `splits` slices and of the launch behind it: rounds of 256 workgroups, the key tiles
-// of a slice, how full a round is (workgroups share the chip's bandwidth and power), and the rows of sums that the slices write
-// and the second launch reads.  Fitted at 244 shapes (130 to 2,000 tokens behind 64 to 60,000, 2 to 32 slices, both formats;
-// 3.6 % rms).
-static float chunk_q8_us(int pos0, int tokens, int n_head, int n_kv, int splits)
+// How a sliced chunk is cut: key tiles of a slice; slices of all blocks of 8 tasks of 32 tokens (the last block, which sees most
+// keys, gets `splits`, a block with fewer key tiles proportionally fewer, so that a chunk near position 0 does not write and read
+// again `splits` partial copies of rows that see only a few tiles); workgroups of chunk_q8_kernel; and whether
+// chunk_f16_t64_kernel takes the chunk, with its tasks, blocks and workgroups.  grid.x covers every (combo, task block): the
+// XCD-aware decode in the kernels may leave a few trailing workgroups without work when 8 is not a multiple of n_kv * splits.
+struct ChunkCut {
+    int slice, nslice, grid, ntask64, nblock64, grid64;
+    bool uniform, t64;
+};
+static ChunkCut chunk_cut(int pos0, int tokens, int n_head, int n_kv, int splits, bool f16)
 {
     const int group = n_head / n_kv, ntask = (tokens + kQTile - 1) / kQTile * group, nblock = (ntask + kTasks - 1) / kTasks;
-    const int tiles = (pos0 + tokens + kKTile - 1) / kKTile, slice = (tiles + splits - 1) / splits;
-    int nslice = 0;
-    if (block_slices(0, ntask, group, tokens, pos0, splits, slice, nullptr) == splits)
-        nslice = nblock * splits;
-    else
-        for (int tb = 0; tb < nblock; tb++)
-            nslice += block_slices(tb, ntask, group, tokens, pos0, splits, slice, nullptr);
-    const int wgs = n_kv * nslice, rounds = (wgs + 255) / 256;
-    const float fill = (float)wgs / (256.0f * (float)rounds);
-    const float rows = (float)tokens * (float)n_head / 24.0f * (float)nslice / (float)nblock;
-    return 0.5f + (float)rounds * (12.3f + (float)slice * (1.99f + 1.69f * fill)) + 0.00615f * rows;
+    const int tiles = (pos0 + tokens + kKTile - 1) / kKTile, combos = n_kv * splits;
+    auto workgroups = [&](int blocks) {
+        return combos % 8 != 0 && 8 % combos == 0 ? 8 * ((blocks + 8 / combos - 1) / (8 / combos)) : combos * blocks;
+    };
+    ChunkCut c;
+    c.slice = (tiles + splits - 1) / splits;
+    c.uniform = block_slices(0, ntask, group, tokens, pos0, splits, c.slice, nullptr) == splits; // (the first has the fewest)
+    c.nslice = c.uniform ? nblock * splits : 0;
+    for (int tb = 0; tb < nblock && !c.uniform; tb++)
+        c.nslice += block_slices(tb, ntask, group, tokens, pos0, splits, c.slice, nullptr);
+    c.grid = c.uniform ? workgroups(nblock) : n_kv * c.nslice;
+    // 64 tokens per wave: its own task blocks (4 tasks of 64 tokens, up to 32 left-over tokens as tasks of 32 tokens x 2 heads),
+    // every one with `splits` slices.  Both kernels run one workgroup per CU, so the hardware starts them in rounds of 256; where
+    // the other cut of the tokens needs a round more, the kernel of 32 tokens per wave keeps the chunk.
+    const int rem = tokens % kT64Tile;
+    c.ntask64 = (tokens / kT64Tile + (rem > 32 ? 1 : 0)) * group + (rem > 0 && rem <= 32 ? (group + 1) / 2 : 0);
+    c.nblock64 = (c.ntask64 + kT64Tasks - 1) / kT64Tasks;
+    c.grid64 = workgroups(c.nblock64);
+    c.t64 = f16 && splits >= 2 && c.uniform && (c.grid64 + 255) / 256 <= (c.grid + 255) / 256;
+    return c;
 }
 
-// Slices, of the `splits` that the scratch holds, with which chunk_q8_kernel runs a chunk over the cache.  A count that fills the
-// chip's rounds leaves out what a second round costs beside its keys and what the rows of sums cost; a chunk near position 0,
-// whose blocks see few key tiles, pays for slices most.  us with the count that fills / with this one: 350 tokens behind
-// 20,000 218 (14) / 200 (7), 420 behind 5,003 104 (12) / 85 (5), 512 behind 7,000 140 (10) / 118 (5) and behind 60,000 797 (16)
-// / 751 (5), 2,000 behind 300 199 (8) / 131 (3) and behind 1,700 269 (6) / 202 (3).  Within 3 % the given count stays: so close
-// the costs above do not tell which is faster.  With as many blocks as two rounds hold a chunk is not sliced to fill the chip.
-static int chunk_q8_slices(int pos0, int tokens, int n_head, int n_kv, int splits)
+// us of a sliced chunk with `splits` slices: rounds of 256 workgroups, the key tiles of a slice, how full a round is (workgroups
+// share the chip's bandwidth and power), and the rows of sums that the slices write and the second launch reads.  Fitted over the
+// cache (chunk_q8_kernel) at 244 shapes, 130 to 2,000 tokens behind 64 to 60,000, 2 to 32 slices, both formats, 3.6 % rms, and
+// over f16 tiles at 253 shapes from 8 tokens on: chunk_f16_t64_kernel 2.9 % rms, chunk_q8_kernel 4.1 %.
+static float chunk_us(int pos0, int tokens, int n_head, int n_kv, int splits, bool f16)
+{
+    const ChunkCut c = chunk_cut(pos0, tokens, n_head, n_kv, splits, f16);
+    const int nblock = ((tokens + kQTile - 1) / kQTile * (n_head / n_kv) + kTasks - 1) / kTasks;
+    const int wgs = c.t64 ? c.grid64 : n_kv * c.nslice, rounds = (wgs + 255) / 256;
+    const float fill = (float)wgs / (256.0f * (float)rounds), slice = (float)c.slice;
+    const float rows = (float)tokens * (float)n_head / 24.0f * (float)c.nslice / (float)nblock;
+    if (c.t64)
+        return 6.5f + (float)rounds * (13.7f + slice * (2.03f + 0.887f * fill)) + 0.00638f * rows;
+    if (f16)
+        return 3.5f + (float)rounds * (11.1f + slice * (2.18f + 0.888f * fill)) + 0.00583f * rows;
+    return 0.5f + (float)rounds * (12.3f + slice * (1.99f + 1.69f * fill)) + 0.00615f * rows;
+}
+
+// Slices, of the `splits` that the scratch holds, with which a chunk runs.  A count that fills the chip's rounds leaves out what
+// a second round costs beside its keys and what the rows of sums cost; a chunk near position 0, whose blocks see few key tiles,
+// pays for slices most; and few tokens over f16 tiles run faster with a count that leaves the first block a slice short, in
+// chunk_q8_kernel.  us with the count that fills / with this one, over the cache: 350 tokens behind 20,000 218 (14) / 200 (7), 420
+// behind 5,003 104 (12) / 85 (5), 512 behind 7,000 140 (10) / 118 (5) and behind 60,000 797 (16) / 751 (5), 2,000 behind 300 199
+// (8) / 131 (3) and behind 1,700 269 (6) / 202 (3); over f16 tiles: 64 behind 2,500 35.5 (14) / 28.6 (12), 420 behind 5,003 95
+// (12) / 83 (5), 512 behind 7,000 132 (10) / 109 (5), 2,000 behind 300 188 (8) / 123 (3).  Within 3 % the given count stays: so
+// close the costs above do not tell which is faster.  With as many blocks as two rounds hold a chunk is not sliced to fill the
+// chip.
+int chunk_run_slices(int pos0, int tokens, int n_head, int n_kv, int splits, bool f16)
 {
     const int nblock = ((tokens + kQTile - 1) / kQTile * (n_head / n_kv) + kTasks - 1) / kTasks;
     if (n_kv * nblock >= 512)
         return splits;
     int best = splits;
-    float best_cost = 0.97f * chunk_q8_us(pos0, tokens, n_head, n_kv, splits);
+    float best_cost = 0.97f * chunk_us(pos0, tokens, n_head, n_kv, splits, f16);
     for (int s = 2; s < splits; s++) {
-        const float cost = chunk_q8_us(pos0, tokens, n_head, n_kv, s);
+        const float cost = chunk_us(pos0, tokens, n_head, n_kv, s, f16);
         if (cost < best_cost) {
             best = s;
             best_cost = cost;
@@ -2255,7 +2290,7 @@ static int chunk_q8_slices(int pos0, int tokens, int n_head, int n_kv, int split
 // one is, 8 KB of sums per token and head.  us before / now over 4 @ 256 19.6 / 15.6, 16 @ 500 21.3 / 16.1, 32 @ 2,000 26.9 /
 // 20.7, 32 @ 8,000 42.6 / 31.3, 64 @ 2,000 31.4 / 25.4, 64 @ 32,000 114 / 104, 117 @ 1,500 33.5 / 28.6, 256 @ 1,000 34.7 /
 // 33.0; not taken at 128 @ 4,000 39.8 (here 41), 200 @ 4,000 49.7 (55), 256 @ 8,000 79 (120).
-// And not where the other kernel's cost by chunk_q8_us, fitted at more tokens, is lower by a tenth, as with fewer slices than it
+// And not where the other kernel's cost by chunk_us, fitted at more tokens, is lower by a tenth, as with fewer slices than it
 // is given: 330 @ 1,862 54.9 here / 46.0 there, 464 @ 3,639 92.5 / 73.9, 226 @ 3,679 57.7 / 50.4; over
 // 33 shapes where the two estimates differ, those under a tenth take 19 % less to 1 % more here, those over it as long or more.
 static int chunk_wg_splits(int pos0, int tokens, int n_head, int n_kv, int splits)
@@ -2283,14 +2318,31 @@ static int chunk_wg_splits(int pos0, int tokens, int n_head, int n_kv, int split
     const float cost = 12.6f + (float)rounds * (float)slice * (2.53f + fill) + (float)splits * (0.152f + 0.0067f * sums);
     if (best_cost >= 0.95f * cost)
         return 0;
-    const int slices = chunk_q8_slices(pos0, tokens, n_head, n_kv, splits);
-    return best_cost < 1.1f * chunk_q8_us(pos0, tokens, n_head, n_kv, slices) ? best : 0;
+    const int slices = chunk_run_slices(pos0, tokens, n_head, n_kv, splits, false);
+    return best_cost < 1.1f * chunk_us(pos0, tokens, n_head, n_kv, slices, false) ? best : 0;
 }
 
-// For tests: the above two, 0 for chunk_q8_kernel in the second.
+// A chunk of few tokens behind a prefix reads the cache although its f16 copy is registered: one to two tiles of 32 tokens are
+// latency, which chunk_wg_kernel's workgroups of four slices share and the kernels over tiles pay slice by slice, and the rows
+// are half the bytes.  us over q8_0 / q4_0 rows and over the copy (with the slices above): 16 tokens behind 2,048 17.9 / 17.2 and
+// 21.9, behind 90,000 136 / 124 and 221, 32 behind 7,000 28.7 / 27.2 and 36.3, 64 behind 4,500 30.5 / 28.8 and 31.8, behind
+// 90,000 226 / 197 and 240; 80 behind 4,500 33.7 / 32.0 and 33.0 are the first for which it is no loss.  Behind less than 2,048 a
+// registered copy is read as before: there a call's bits are those of hipml_attn_chunk_kv_f16.
+bool chunk_reads_cache(int pos0, int tokens, int n_head, int n_kv, int splits)
+{
+    return tokens <= 64 && pos0 >= 2048 && chunk_wg_splits(pos0, tokens, n_head, n_kv, splits) > 0;
+}
+
+// For tests: the above, 0 for chunk_q8_kernel in the last; *t64: chunk_f16_t64_kernel runs.
 extern "C" int hipml_dbg_chunk_q8_slices(int pos0, int tokens, int n_head, int n_kv, int splits)
 {
-    return chunk_q8_slices(pos0, tokens, n_head, n_kv, splits);
+    return chunk_run_slices(pos0, tokens, n_head, n_kv, splits, false);
+}
+extern "C" int hipml_dbg_chunk_f16_slices(int pos0, int tokens, int n_head, int n_kv, int splits, int *t64)
+{
+    const int s = chunk_run_slices(pos0, tokens, n_head, n_kv, splits, true);
+    *t64 = chunk_cut(pos0, tokens, n_head, n_kv, s, true).t64;
+    return s;
 }
 extern "C" int hipml_dbg_chunk_wg_splits(int pos0, int tokens, int n_head, int n_kv, int splits)
 {
@@ -2347,8 +2399,8 @@ int launch_chunk_q8(hipStream_t st, const float *q, const uint8_t *kc, const uin
     a.tokens = tokens;
     a.stride = stride;
     a.splits = splits < 2 ? 1 : splits;
-    if (splits >= 2 && kv_f16 == nullptr)
-        a.splits = chunk_q8_slices(pos0, tokens, n_head, n_kv, splits);
+    if (splits >= 2 && kv_f16 == nullptr) // (over f16 tiles the caller has chosen)
+        a.splits = chunk_run_slices(pos0, tokens, n_head, n_kv, splits, false);
     a.qslots = (tokens + 31) / 32 * 32;
     a.ntask = (tokens + kQTile - 1) / kQTile * a.group;
     a.nblock = (a.ntask + kTasks - 1) / kTasks;
@@ -2387,30 +2439,12 @@ int launch_chunk_q8(hipStream_t st, const float *q, const uint8_t *kc, const uin
                            a.ntask, tokens, pos0, 0, 1, static_cast<_Float16 *>(out16));
         return launched("attn_chunk_combine");
     }
-    // slices per block: the last block (most keys) gets `splits`, a block with fewer key tiles gets
-    // proportionally fewer, so a chunk near position 0 does not write and re-read `splits` partial
-    // copies of rows that see only a few tiles
-    const int tiles_last = (pos0 + tokens + kKTile - 1) / kKTile;
-    a.slice_tiles = (tiles_last + a.splits - 1) / a.splits;
-    a.nslice = 0;
-    for (int tb = 0; tb < a.nblock; tb++)
-        a.nslice += block_slices(tb, a.ntask, a.group, tokens, pos0, a.splits, a.slice_tiles, nullptr);
-    a.uniform = a.nslice == a.nblock * a.splits;
+    const ChunkCut cut = chunk_cut(pos0, tokens, n_head, n_kv, a.splits, kv_f16 != nullptr);
+    a.slice_tiles = cut.slice;
+    a.nslice = cut.nslice;
+    a.uniform = cut.uniform;
     const dim3 block(kPfThreads, 1, 1);
-    unsigned grid;
-    if (a.splits > 1 && !a.uniform) {
-        grid = (unsigned)(n_kv * a.nslice);
-    } else {
-        // grid.x covers every (combo, task block); the XCD-aware decode in the kernel may leave a
-        // few trailing workgroups without work when 8 is not a multiple of `combos`.
-        const int combos = n_kv * a.splits;
-        if (combos % 8 == 0)
-            grid = (unsigned)(combos * a.nblock);
-        else if (8 % combos == 0)
-            grid = (unsigned)(8 * ((a.nblock + 8 / combos - 1) / (8 / combos)));
-        else
-            grid = (unsigned)(combos * a.nblock);
-    }
+    const unsigned grid = (unsigned)cut.grid;
     if (splits < 2) {
         if (kv_f16)
             HIPML_LAUNCH((chunk_q8_kernel<false, false, true>), dim3(grid, 1, 1), block, kPfLdsF, st, a);
@@ -2426,20 +2460,11 @@ int launch_chunk_q8(hipStream_t st, const float *q, const uint8_t *kc, const uin
                            reinterpret_cast<const float4v *>(out), static_cast<half4 *>(out16), n4);
         return launched("attn_chunk_rows_f16");
     }
-    // 64 tokens per wave: its own task blocks (4 tasks of 64 tokens), every one with `splits` slices.  Both
-    // kernels run one workgroup per CU, so the hardware starts them in rounds of 256; where the other cut of
-    // the tokens needs a round more, the kernel of 32 tokens per wave keeps the chunk.
-    ChunkArgs b = a;
-    {
-        const int rem = tokens % kT64Tile; // (up to 32 left-over tokens: tasks of 32 tokens x 2 heads, see the kernel)
-        b.ntask = (tokens / kT64Tile + (rem > 32 ? 1 : 0)) * a.group + (rem > 0 && rem <= 32 ? (a.group + 1) / 2 : 0);
-    }
-    b.nblock = (b.ntask + kT64Tasks - 1) / kT64Tasks;
-    unsigned g64 = (unsigned)(n_kv * a.splits * b.nblock);
-    if ((n_kv * a.splits) % 8 != 0 && 8 % (n_kv * a.splits) == 0)
-        g64 = (unsigned)(8 * ((b.nblock + 8 / (n_kv * a.splits) - 1) / (8 / (n_kv * a.splits))));
-    if (kv_f16 && a.uniform && (g64 + 255) / 256 <= (grid + 255) / 256) {
-        HIPML_LAUNCH(chunk_f16_t64_kernel, dim3(g64, 1, 1), dim3(kT64Threads, 1, 1), kT64Lds, st, b);
+    if (cut.t64) {
+        ChunkArgs b = a;
+        b.ntask = cut.ntask64;
+        b.nblock = cut.nblock64;
+        HIPML_LAUNCH(chunk_f16_t64_kernel, dim3((unsigned)cut.grid64, 1, 1), dim3(kT64Threads, 1, 1), kT64Lds, st, b);
     } else if (kv_f16)
         HIPML_LAUNCH((chunk_q8_kernel<true, false, true>), dim3(grid, 1, 1), block, kPfLdsF, st, a);
     else if (q4)

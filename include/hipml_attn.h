@@ -471,11 +471,11 @@ int hipml_attn_chunk_kv_f16(hipml_stream_t stream, const float *q, const void *k
  *     hipml_kv_encode_rows, hipml_attn_front_rows_encode_f32) mark the shadow stale, and the next chunk
  *     attention over the cache converts every live row once (0.13 ms per 100,000 rows);
  *   - hipml_attn_chunk_q8_split, _gate and _gate_f16 over (k_cache, v_cache) with the registered stride,
- *     n_kv and format and splits >= 2 read the tiles: min(splits, hipml_attn_chunk_slices) slices, no
- *     tiles made per call in the scratch (2,048 tokens at depth 100,000: 4.06 against 4.19 ms).  Chunks of about 64
- *     tokens and fewer are slower so (us with the copy / without, 32 tokens at depth 8,000: 41 / 30, at 32,000: 96 / 63;
- *     64 at 8,000: 45 / 38; 117 at 5,003: 42 / 41.5, at 32,000: 118 / 133; 400 at 32,000: 319 / 363), and an append of
- *     such a chunk costs 3 to 4 us more: attach it to caches that long chunks extend.
+ *     n_kv and format and splits >= 2 read the tiles: at most min(splits, hipml_attn_chunk_slices) slices, no
+ *     tiles made per call in the scratch (2,048 tokens at depth 100,000: 4.06 against 4.19 ms).  Up to 64 tokens
+ *     behind 2,048 rows and more read the cache itself, which is faster for so few (32 tokens at depth 7,000: 29 us,
+ *     over the copy 36), and an append of such a chunk costs 3 to 4 us more than without a copy: attach it to caches
+ *     that long chunks extend (us with the copy / without: 117 tokens at depth 20,000 81 / 87, 400 at 20,000 194 / 220).
  * The bookkeeping is host state that changes when a call is issued or captured, not when a captured
  * graph is replayed.  Rows written into the cache by any other means (a device copy, another library)
  * must be followed by hipml_kv_f16_rows for those rows.  hipml_kv_f16_detach must be called before

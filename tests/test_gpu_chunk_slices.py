@@ -1,5 +1,7 @@
-"""Chunks over the cache for which fewer key slices run than the caller's scratch holds: the result is the oracle's (the gate of
+"""Chunks over the cache, and over its registered f16 copy, for which fewer key slices run than the caller's scratch holds: the result is the oracle's (the gate of
 the chunk kernels) and that of a call which asks for those slices, and the rest of the scratch is left alone."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -53,11 +55,66 @@ def test_fewer_slices_than_the_scratch_holds(tok, pos0, splits, n_head, n_kv, dt
         assert bool(x[tok].isnan().all())
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [0, 1])
+@pytest.mark.parametrize("tok,pos0,splits,t64", [
+    (96, 1700, 10, 0),    # a count that leaves the first block a slice short: the kernel of 32 tokens per wave
+    (420, 5003, 12, 1), (1079, 492, 8, 0)])
+def test_fewer_slices_over_a_registered_copy(tok, pos0, splits, t64, dtype):
+    from test_gpu_kv_f16 import run_chunk_f16
+    from test_gpu_kv_shadow import Attached, attend
+    from oracle import binding as orc
+    attn.init(0)
+    took = ctypes.c_int()
+    used = attn.lib().hipml_dbg_chunk_f16_slices(pos0, tok, N_HEAD, N_KV, splits, ctypes.byref(took))
+    assert splits == attn.chunk_slices(pos0, tok, N_KV) and 2 <= used < splits and took.value == t64
+    r = orc.Rng(0x511C_1000 + tok)
+    stride = pos0 + tok + 5
+    kb = orc.quantize(dtype, r.normal_array((N_KV, stride, HD))).reshape(N_KV, stride, -1)
+    vb = orc.quantize(dtype, r.normal_array((N_KV, stride, HD))).reshape(N_KV, stride, -1)
+    q = r.normal_array((tok, N_HEAD, HD))
+    with Attached(kb, vb, stride, pos0 + tok, dtype=dtype) as c:
+        got = attend(q, c.k, c.v, pos0, tok, stride, splits, dtype=dtype + 1)
+    by_hand = run_chunk_f16(q, kb, vb, pos0, tok, stride, used, dtype=dtype)
+    assert np.array_equal(got.view(np.uint32), by_hand.view(np.uint32))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [0, 1])
+@pytest.mark.parametrize("tok,pos0,splits,cache", [
+    (64, 2048, 12, True), (1, 2048, 12, True), (33, 5000, 16, True), (64, 2047, 12, False), (65, 2048, 12, False)])
+def test_few_tokens_read_the_cache_beside_a_registered_copy(tok, pos0, splits, cache, dtype):
+    # both sides of the rule's two lines; the registered copy is made NaN after its conversion, so a call that reads it shows
+    from test_gpu_kv_f16 import run_chunk_f16
+    from test_gpu_kv_shadow import Attached, attend
+    from gpu_util import dev
+    from oracle import binding as orc
+    attn.init(0)
+    r = orc.Rng(0x511C_2000 + tok)
+    stride = pos0 + tok + 5
+    kb = orc.quantize(dtype, r.normal_array((N_KV, stride, HD))).reshape(N_KV, stride, -1)
+    vb = orc.quantize(dtype, r.normal_array((N_KV, stride, HD))).reshape(N_KV, stride, -1)
+    q = r.normal_array((tok, N_HEAD, HD))
+    plain = attend(q, dev(kb), dev(vb), pos0, tok, stride, splits, dtype=dtype + 1)
+    with Attached(kb, vb, stride, pos0 + tok, dtype=dtype) as c:
+        if cache:
+            c.copy.fill_(0xFF)
+        got = attend(q, c.k, c.v, pos0, tok, stride, splits, dtype=dtype + 1)
+    if cache:
+        assert np.array_equal(got.view(np.uint32), plain.view(np.uint32))
+    else:
+        took = ctypes.c_int()
+        most = min(splits, attn.chunk_slices(pos0, tok, N_KV))
+        used = attn.lib().hipml_dbg_chunk_f16_slices(pos0, tok, N_HEAD, N_KV, most, ctypes.byref(took))
+        assert np.array_equal(got.view(np.uint32), run_chunk_f16(q, kb, vb, pos0, tok, stride, used, dtype=dtype).view(np.uint32))
+
+
 def test_the_slices_that_run_fit_the_scratch():
     # never more than asked for, never one alone (that is another kernel's sums), and no other count where the blocks fill the
     # chip by themselves
     lib = attn.lib()
     rng = np.random.default_rng(7)
+    took = ctypes.c_int()
     for _ in range(3000):
         n_kv = int(rng.integers(1, 9))
         n_head = n_kv * int(rng.integers(1, 9))
@@ -65,7 +122,9 @@ def test_the_slices_that_run_fit_the_scratch():
         splits = int(rng.integers(2, 65))
         used = lib.hipml_dbg_chunk_q8_slices(pos0, tok, n_head, n_kv, splits)
         assert 2 <= used <= splits
+        over_tiles = lib.hipml_dbg_chunk_f16_slices(pos0, tok, n_head, n_kv, splits, ctypes.byref(took))
+        assert 2 <= over_tiles <= splits
         blocks = ((tok + 31) // 32 * (n_head // n_kv) + 7) // 8
         if n_kv * blocks >= 512:
-            assert used == splits
+            assert used == over_tiles == splits
         assert lib.hipml_dbg_chunk_wg_splits(pos0, tok, n_head, n_kv, splits) <= splits
