@@ -2142,22 +2142,6 @@ bool chunk_tiles_pay(int pos0, int tokens)
     return (tokens >= 768 && pos0 >= tokens) || (tokens >= 640 && pos0 >= 8 * tokens);
 }
 
-bool chunk_tiles_plan(int pos0, int tokens, int n_head, int n_kv, int splits, int *use, size_t *tiles_at)
-{
-    if (!chunk_tiles_pay(pos0, tokens) || splits < 3)
-        return false;
-    const int s = hipml_attn_chunk_slices(pos0, tokens, n_kv);
-    if (s < 2)
-        return false;
-    const size_t per_slice = (size_t)((tokens + 31) / 32 * 32) * n_head * kHeadDim * sizeof(float);
-    const size_t tiles = (size_t)n_kv * ((pos0 + tokens + kKTile - 1) / kKTile) * kBufBytesF;
-    if ((size_t)splits * per_slice < (size_t)s * per_slice + tiles)
-        return false;
-    *use = s;
-    *tiles_at = (size_t)s * per_slice;
-    return true;
-}
-
 int chunk_tiles_splits(int pos0, int tokens, int n_head, int n_kv, int slices)
 {
     const size_t per_slice = (size_t)((tokens + 31) / 32 * 32) * n_head * kHeadDim * sizeof(float);
@@ -2240,7 +2224,8 @@ static ChunkCut chunk_cut(int pos0, int tokens, int n_head, int n_kv, int splits
 // us of a sliced chunk with `splits` slices: rounds of 256 workgroups, the key tiles of a slice, how full a round is (workgroups
 // share the chip's bandwidth and power), and the rows of sums that the slices write and the second launch reads.  Fitted over the
 // cache (chunk_q8_kernel) at 244 shapes, 130 to 2,000 tokens behind 64 to 60,000, 2 to 32 slices, both formats, 3.6 % rms, and
-// over f16 tiles at 253 shapes from 8 tokens on: chunk_f16_t64_kernel 2.9 % rms, chunk_q8_kernel 4.1 %.
+// over f16 tiles at 253 shapes from 8 tokens on: chunk_f16_t64_kernel 2.9 % rms, chunk_q8_kernel 4.1 %.  (The first takes whole
+// slices of every block, and the ones behind a block's own tokens end early, which shows from the second round on.)
 static float chunk_us(int pos0, int tokens, int n_head, int n_kv, int splits, bool f16)
 {
     const ChunkCut c = chunk_cut(pos0, tokens, n_head, n_kv, splits, f16);
@@ -2248,8 +2233,9 @@ static float chunk_us(int pos0, int tokens, int n_head, int n_kv, int splits, bo
     const int wgs = c.t64 ? c.grid64 : n_kv * c.nslice, rounds = (wgs + 255) / 256;
     const float fill = (float)wgs / (256.0f * (float)rounds), slice = (float)c.slice;
     const float rows = (float)tokens * (float)n_head / 24.0f * (float)c.nslice / (float)nblock;
+    const float early = rounds > 1 ? 1.0f - 0.31f * (float)tokens / (float)(pos0 + tokens) : 1.0f;
     if (c.t64)
-        return 6.5f + (float)rounds * (13.7f + slice * (2.03f + 0.887f * fill)) + 0.00638f * rows;
+        return 1.3f + (float)rounds * (19.0f + slice * (2.01f + 0.93f * fill) * early) + 0.00628f * rows;
     if (f16)
         return 3.5f + (float)rounds * (11.1f + slice * (2.18f + 0.888f * fill)) + 0.00583f * rows;
     return 0.5f + (float)rounds * (12.3f + slice * (1.99f + 1.69f * fill)) + 0.00615f * rows;
@@ -2279,6 +2265,33 @@ int chunk_run_slices(int pos0, int tokens, int n_head, int n_kv, int splits, boo
         }
     }
     return best;
+}
+
+// Whether a chunk over the cache makes f16 tiles in its scratch first (above).  Behind a prefix little longer than itself it does
+// not where the count of slices for the tiles, all of which every block has to get, leaves a second round of workgroups nearly
+// empty, or where three shorter slices of the kernel over the cache fit one: us over tiles / over the cache, 768 tokens behind
+// 1,300 78 (2 slices) / 65 (3), 900 behind 900 78 (2) / 65 (3), 1,400 behind 1,700 172 (2) / 151 (3), 1,500 behind 3,000 236 (2) /
+// 199 (3), 1,800 behind 2,500 227 (2) / 216 (3); over 88 shapes (both formats) for which the two costs differ by 4 % so, the
+// cache is 4 to 23 % faster (by 3 %: 2 % slower to 23 % faster); 1,024 behind 8,192 and 672 behind 8,192 keep their tiles.
+bool chunk_tiles_plan(int pos0, int tokens, int n_head, int n_kv, int splits, int *use, size_t *tiles_at)
+{
+    if (!chunk_tiles_pay(pos0, tokens) || splits < 3)
+        return false;
+    const int s = hipml_attn_chunk_slices(pos0, tokens, n_kv);
+    if (s < 2)
+        return false;
+    const size_t per_slice = (size_t)((tokens + 31) / 32 * 32) * n_head * kHeadDim * sizeof(float);
+    const size_t tiles = (size_t)n_kv * ((pos0 + tokens + kKTile - 1) / kKTile) * kBufBytesF;
+    if ((size_t)splits * per_slice < (size_t)s * per_slice + tiles)
+        return false;
+    // What the tiles cost, and the kernel over them, against the kernel over the cache with the same scratch.
+    const float tiles_us = 0.23f + 1.86e-3f * (float)(pos0 + tokens) * (float)n_kv / 4.0f;
+    const int slices = chunk_run_slices(pos0, tokens, n_head, n_kv, splits, false);
+    if (tiles_us + chunk_us(pos0, tokens, n_head, n_kv, s, true) > 1.04f * chunk_us(pos0, tokens, n_head, n_kv, slices, false))
+        return false;
+    *use = s;
+    *tiles_at = (size_t)s * per_slice;
+    return true;
 }
 
 // Splits of the keys, of at most `splits`, with which chunk_wg_kernel runs a chunk over the cache; 0: chunk_q8_kernel does.
@@ -2337,6 +2350,12 @@ bool chunk_reads_cache(int pos0, int tokens, int n_head, int n_kv, int splits)
 extern "C" int hipml_dbg_chunk_q8_slices(int pos0, int tokens, int n_head, int n_kv, int splits)
 {
     return chunk_run_slices(pos0, tokens, n_head, n_kv, splits, false);
+}
+extern "C" int hipml_dbg_chunk_makes_tiles(int pos0, int tokens, int n_head, int n_kv, int splits)
+{
+    int use;
+    size_t tiles_at;
+    return chunk_tiles_plan(pos0, tokens, n_head, n_kv, splits, &use, &tiles_at) ? use : 0;
 }
 extern "C" int hipml_dbg_chunk_f16_slices(int pos0, int tokens, int n_head, int n_kv, int splits, int *t64)
 {

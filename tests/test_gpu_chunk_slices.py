@@ -109,6 +109,38 @@ def test_few_tokens_read_the_cache_beside_a_registered_copy(tok, pos0, splits, c
         assert np.array_equal(got.view(np.uint32), run_chunk_f16(q, kb, vb, pos0, tok, stride, used, dtype=dtype).view(np.uint32))
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [0, 1])
+@pytest.mark.parametrize("tok,pos0", [(768, 1300), (900, 900), (1400, 1700)])
+def test_a_scratch_with_room_for_tiles_that_would_not_pay(tok, pos0, dtype):
+    from oracle import binding as orc
+    from gpu_util import SCALE, dev, report
+    from test_gpu_prefill import GATE
+    from test_gpu_kv_shadow import attend
+    attn.init(0)
+    splits = attn.chunk_splits(pos0, tok, N_KV)
+    assert splits > attn.chunk_slices(pos0, tok, N_KV) >= 2
+    assert attn.lib().hipml_dbg_chunk_makes_tiles(pos0, tok, N_HEAD, N_KV, splits) == 0
+    r = orc.Rng(0x511C_3000 + tok)
+    stride = pos0 + tok + 5
+    kb = orc.quantize(dtype, r.normal_array((N_KV, stride, HD))).reshape(N_KV, stride, -1)
+    vb = orc.quantize(dtype, r.normal_array((N_KV, stride, HD))).reshape(N_KV, stride, -1)
+    q = r.normal_array((tok, N_HEAD, HD))
+    got = attend(q, dev(kb), dev(vb), pos0, tok, stride, splits, dtype=dtype + 1)
+    rows = np.array([0, 31, 32, 400, tok - 33, tok - 1], dtype=np.int32)
+    want = orc.attn_chunk_kv(q, kb, vb, N_HEAD, N_KV, HD, pos0, tok, stride, SCALE, rows=rows, n_threads=8, dtype=dtype)
+    assert report(f"chunk {tok}@{pos0} without tiles", want, got[rows], *GATE)[0]
+    assert np.isfinite(got).all()
+
+
+@pytest.mark.parametrize("tok,pos0,use", [(1024, 8192, 2), (672, 8192, 4), (2048, 100_000, 4), (800, 6500, 3), (800, 1000, 0)])
+def test_where_a_chunk_makes_tiles(tok, pos0, use):
+    # and never in a scratch of a slice less than hipml_attn_chunk_splits says
+    lib, splits = attn.lib(), attn.chunk_splits(pos0, tok, N_KV)
+    assert lib.hipml_dbg_chunk_makes_tiles(pos0, tok, N_HEAD, N_KV, splits) == use
+    assert lib.hipml_dbg_chunk_makes_tiles(pos0, tok, N_HEAD, N_KV, splits - 1) == 0
+
+
 def test_the_slices_that_run_fit_the_scratch():
     # never more than asked for, never one alone (that is another kernel's sums), and no other count where the blocks fill the
     # chip by themselves
