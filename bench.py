@@ -798,7 +798,10 @@ def row_kernel_name(attn, m, k, rows):
         return "gemv_q8_rows_kernel"
     if kernel == 1:
         return f"gemv_q8_digits_kernel<{a}, {b}>"
-    return f"gemv_q8_{'blocks' if kernel == 2 else 'units'}_kernel<{a}, {b}, {'true' if c else 'false'}>"
+    half = "true" if c else "false"
+    if kernel == 2:
+        return f"gemv_q8_blocks_kernel<{a}, {b}, {half}>"
+    return f"gemv_q8_units_kernel<{a}, {b}, {half}, {'true' if k % 256 == 0 else 'false'}>"  # (weights at a 16-byte boundary)
 
 
 # W_o over 672 gated tokens: packed rows, 256 x 64 tiles (100 x route + place in the library's table of tiles)
