@@ -776,11 +776,11 @@ __global__ void __launch_bounds__(64 * kDigitMaxWaves) gemv_q8_digits_kernel(con
 // the workgroup walks chunks together and shares its requests for the weights.  us over 9 / 16 / 24 / 32 / 40 / 48 / 64 / 128
 // rows, units (by 16-byte requests) and blocks, each with its best tile, the weights from HBM (k 5120, for 2,048 and 4,096
 // weight rows 4096, for 5,120 6144):
-//    1,024 weight rows 6.8 13.1 |  7.5 13.4 |  7.4 13.2 |  7.3 13.3 |  8.8 13.3 |  9.6 13.4 |  9.5 13.5 | 11.9 13.5
-//    2,048             6.2 11.3 |  6.6 11.3 |  7.6 11.4 |  8.4 11.4 |  9.9 11.4 | 10.7 11.5 | 10.5 11.8 | 13.8 15.0
-//    4,096             7.9 11.4 |  9.2 11.6 | 11.4 12.0 | 11.2 11.8 | 13.2 14.5 | 13.6 14.7 | 14.7 15.1 | 26.4 24.8
-//    5,120             12.9 15.8 | 14.3 16.2 | 18.0 19.5 | 19.6 19.0 | 22.6 22.3 | 23.2 22.8 | 25.7 24.9 | 45.8 38.5
-//    6,144             12.3 13.7 | 13.6 14.4 | 16.8 16.8 | 16.9 16.7 | 19.8 21.3 | 20.4 21.3 | 22.9 22.0 | 41.2 33.8
+//    1,024 weight rows  6.8 13.1 |  7.5 13.4 |  7.4 13.2 |  7.3 13.3 |  8.8 13.3 |  9.6 13.4 |  9.5 13.5 | 11.9 13.5
+//    2,048              6.2 11.3 |  6.6 11.3 |  7.6 11.4 |  8.4 11.4 |  9.9 11.4 | 10.7 11.5 | 10.5 11.8 | 13.8 15.0
+//    4,096              7.9 11.4 |  9.2 11.6 | 11.4 12.0 | 11.2 11.8 | 13.2 14.5 | 13.6 14.7 | 14.7 15.1 | 26.4 24.8
+//    5,120              12.9 15.8 | 14.3 16.2 | 18.0 19.5 | 19.6 19.0 | 22.6 22.3 | 23.2 22.8 | 25.7 24.9 | 45.8 38.5
+//    6,144              12.3 13.7 | 13.6 14.4 | 16.8 16.8 | 16.9 16.7 | 19.8 21.3 | 20.4 21.3 | 22.9 22.0 | 41.2 33.8
 //    7,168              15.3 14.0 | 15.8 15.0 | 18.4 17.5 | 20.8 18.7 | 29.2 23.2 | 29.8 27.5 | 34.2 31.1 | 59.5 52.1
 //    8,192              15.7 15.7 | 16.4 15.4 | 19.2 17.9 | 21.2 19.1 | 30.5 23.5 | 31.4 27.9 | 35.6 31.5 | 61.0 56.1
 //   12,288              20.9 19.7 | 21.1 19.4 | 24.3 22.2 | 27.4 24.7 | 39.6 28.2 | 40.9 32.1 | 46.0 36.0 | 83.8 64.8
