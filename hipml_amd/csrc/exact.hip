@@ -536,12 +536,13 @@ int launch_rope_encode_chunk(hipStream_t st, int q4, float *q, float *k, const f
 // exchanges; IEEE addition commutes, so every lane ends with red[0]); mean = sum / 256;
 // scale = 1 / sqrtf(mean + eps) with the correctly rounded divide and square root; the value is
 // (x * scale) * w; the rotation reads cos/sin as the other RoPE kernels here do.
-// grid: (ceil(heads of a row / 4), rows), workgroups of 4 waves.
+// Workgroups of 4 waves; grid (ceil(heads of a row / 4), rows), or flat: all q and K rows one behind the other and the V rows
+// to append behind them (front_flat has the reasons).
 //
 // What a launch over few rows costs beside the launch itself is the chain of loads that wait for one another.  So the
-// pointers to the row, the weights, the table and the positions are leading arguments, which arrive in registers (14 dwords);
-// the other arguments and the position come in one round trip, in the shadow of the row, and the table's in the next; no
-// vector load lies in between, whose wait would be one for the rows as well.  (Arguments, the rest of them, the append's, the
+// pointers to the row, the weights and the positions are leading arguments, which arrive in registers (14 dwords); the other
+// arguments and the position come in one round trip, in the shadow of the row, and the table's in the next; no vector load
+// lies in between, whose wait would be one for the rows as well.  (Arguments, the rest of them, the append's, the
 // position, the sections' positions as a vector load, the table and the append's position were seven, one behind the other: us
 // a launch, replayed, over 3 rows with append 2.93 -> 2.60, over 24 without 2.34 -> 2.20; an empty launch 1.58.)
 enum { kFrontIds, kFrontRows, kFrontChunk }; // where a row's position comes from
@@ -550,8 +551,10 @@ struct FrontArgs {
     const float *v;      // [rows][n_kv][256]
     uint8_t *kc, *vc;    // caches
     size_t slot_bytes;   // kFrontRows: sequence r's cache starts r * slot_bytes into kc / vc
+    const float *tab;
     int n_rot, s0, s1, s2, s3, pos0, stride, tab_rows;
     float theta, eps;
+    uint32_t kv_inverse; // as head_inverse, of n_kv (unused where that is 1)
 };
 
 // ENC: 0 = front end only, 1 = also quantize the finished K row and the V row to q8_0 and append
@@ -560,10 +563,12 @@ struct FrontArgs {
 // waves per row take the V rows.  Same expressions on the same values: the bits of the two launches.
 // posp: kFrontIds (one row) the four M-RoPE ids, with ENC the append's position four before them (the step buffer);
 // kFrontRows [rows][2], a row's text position first; kFrontChunk unused, row r is at pos0 + r.
-template <int ENC>
+// FLAT: one grid dimension; head_inverse is 2^32 / (n_heads + n_kv), rounded up: the high half of its product with a wave's
+// number is the wave's row (exact while wave x heads is below 2^32).
+template <int ENC, bool FLAT>
 __global__ void __launch_bounds__(256) front_kernel(const float *__restrict__ qg, float *k, const float *__restrict__ qw,
-                                                    const float *__restrict__ kw, const float *__restrict__ tab,
-                                                    const int32_t *__restrict__ posp, uint32_t heads_mode, int n_kv,
+                                                    const float *__restrict__ kw, const int32_t *__restrict__ posp,
+                                                    uint32_t heads_mode, int n_kv, int rows, uint32_t head_inverse,
                                                     const FrontArgs a)
 {
     __shared__ float buf[4][kHeadDim];
@@ -572,9 +577,21 @@ __global__ void __launch_bounds__(256) front_kernel(const float *__restrict__ qg
     // exchanges four times over)
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int n_heads = (int)(heads_mode & 0x3fffffffu), mode = (int)(heads_mode >> 30);
-    const int row = blockIdx.y, hb = blockIdx.x * 4 + wave;
-    if (hb >= n_heads + n_kv + (ENC ? n_kv : 0))
+    int row = blockIdx.y, hb = blockIdx.x * 4 + wave; // hb: q head, behind those K head, behind those V head
+    if (FLAT) {
+        const uint32_t heads = (uint32_t)(n_heads + n_kv), front = heads * (uint32_t)rows, i = (uint32_t)hb;
+        if (i < front) {
+            row = (int)__umulhi(i, head_inverse);
+            hb = (int)(i - (uint32_t)row * heads);
+        } else {
+            if (!ENC || i - front >= (uint32_t)(n_kv * rows))
+                return;
+            row = (int)(n_kv == 1 ? i - front : __umulhi(i - front, a.kv_inverse));
+            hb = (int)(heads + i - front - (uint32_t)(row * n_kv));
+        }
+    } else if (hb >= n_heads + n_kv + (ENC ? n_kv : 0)) {
         return; // no workgroup-wide barrier below: waves are independent
+    }
     const int lane32 = lane & 31;
     // the position, and the append's
     int id[4] = {0, 0, 0, 0}, at = 0;
@@ -643,7 +660,7 @@ __global__ void __launch_bounds__(256) front_kernel(const float *__restrict__ qg
             p = sc < a.s0 ? id[0] : sc < a.s0 + a.s1 ? id[1] : sc < a.s0 + a.s1 + a.s2 ? id[2] : id[3];
         }
         if (e < a.n_rot)
-            rope_cs(tab, a.tab_rows, half, c, p, a.n_rot, a.theta, cs[j], sn[j]);
+            rope_cs(a.tab, a.tab_rows, half, c, p, a.n_rot, a.theta, cs[j], sn[j]);
     }
     if (is_q)
         *reinterpret_cast<float4a4 *>(a.gate + ((size_t)row * n_heads + h) * kHeadDim + 4 * lane) = g;
@@ -689,6 +706,32 @@ __global__ void __launch_bounds__(256) front_kernel(const float *__restrict__ qg
     }
 }
 
+// Rows of a launch (grid.y).
+static constexpr int kFrontMaxRows = 32768;
+
+// Whether a launch is flat (above).  Its waves find their row by a product, and a V row's first needs an argument from memory:
+// up to 7 % over few rows (24 + 4 heads with append, 8 rows: 3.5 us by rows, 3.7 flat).  It is flat all the same
+//   - where the workgroups of a row are a multiple of eight, with whole ones for K and for V: workgroups go to the XCDs in turn,
+//     so by rows one XCD gets all the K rows, another all the V rows and the others all the q rows.  That tells while a launch is
+//     about one round of workgroups (2,048 are resident), above the latency and below the bandwidth of the whole chip: 24 + 4
+//     heads with append over 96 / 128 / 160 / 257 / 320 / 416 / 512 / 600 rows 4.5 / 5.1 / 5.6 / 7.6 / 8.5 / 10.1 / 11.6 / 13.0 us by
+//     rows and 4.5 / 4.9 / 5.2 / 6.2 / 7.1 / 9.3 / 11.5 / 13.1 flat; 48 + 8 heads over 64 / 128 / 192 / 256 rows 5.3 / 7.4 / 9.5 /
+//     11.6 and 4.9 / 6.1 / 8.5 / 11.1.  (Flat with other counts of workgroups, or with fewer KV heads, is 5 % faster to 20 % slower.)
+//   - where a quarter of the waves by rows would have no row: 5 + 1 heads without append over 257 / 1,024 / 2,048 rows 3.5 / 5.3 /
+//     9.7 us by rows and 3.5 / 5.1 / 8.3 flat, 3 + 1 with append 4.0 / 6.0 / 9.5 and 3.9 / 5.0 / 7.2.
+// The product needs wave x heads below 2^32: 17,600 waves at most in the first case, 9 heads x 32,768 rows in the second.
+static bool front_flat(int n_heads, int n_kv, int rows, bool append)
+{
+    const long long waves = (long long)n_heads + n_kv + (append ? n_kv : 0), row_wgs = (waves + 3) / 4, wgs = row_wgs * rows;
+    return (append && n_kv >= 4 && row_wgs % 8 == 0 && wgs >= 800 && wgs <= 4400) || (wgs >= 500 && 3 * row_wgs >= waves);
+}
+
+// For tests.
+extern "C" int hipml_dbg_front_flat(int n_heads, int n_kv, int rows, int append)
+{
+    return front_flat(n_heads, n_kv, rows, append != 0);
+}
+
 // enc: -1 = front end only (v, kc, vc unused), 0 = q8_0, 1 = q4_0 append of the K and V rows.
 int launch_front(hipStream_t st, const float *qg, float *q, float *gate, float *k, const float *qw,
                  const float *kw, int n_heads, int n_kv, int n_rot, int s0, int s1, int s2, int s3,
@@ -698,10 +741,11 @@ int launch_front(hipStream_t st, const float *qg, float *q, float *gate, float *
 {
     int tab_rows = 0;
     const float *t = table_for(tab, theta, n_rot, &tab_rows);
-    const int per_row = n_heads + n_kv + (enc >= 0 ? n_kv : 0);
-    const int max_rows = 32768; // grid.y
-    for (int r0 = 0; r0 < rows; r0 += max_rows) {
-        const int n = rows - r0 < max_rows ? rows - r0 : max_rows;
+    const int heads = n_heads + n_kv, waves = heads + (enc >= 0 ? n_kv : 0); // of a row
+    auto inverse = [](int d) { return (uint32_t)((0xffffffffull + (uint64_t)d) / (uint64_t)d); };
+    for (int r0 = 0; r0 < rows; r0 += kFrontMaxRows) {
+        const int n = rows - r0 < kFrontMaxRows ? rows - r0 : kFrontMaxRows;
+        const bool flat = front_flat(n_heads, n_kv, n, enc >= 0);
         const size_t slot_at = rowpos ? (size_t)r0 * slot_bytes : 0;
         FrontArgs a;
         a.q = q + (size_t)r0 * n_heads * kHeadDim;
@@ -720,13 +764,17 @@ int launch_front(hipStream_t st, const float *qg, float *q, float *gate, float *
         a.tab_rows = tab_rows;
         a.theta = theta;
         a.eps = eps;
+        a.tab = t;
+        a.kv_inverse = inverse(n_kv);
         // (the append's positions are the rotation's: the step buffer's own lies four in front of its ids, the others are the same)
         const int32_t *posp = pos ? pos : rowpos ? rowpos + (size_t)r0 * 2 : nullptr;
         const uint32_t mode = pos ? kFrontIds : rowpos ? kFrontRows : kFrontChunk;
-        auto kern = enc < 0 ? front_kernel<0> : enc == 0 ? front_kernel<1> : front_kernel<2>;
-        HIPML_LAUNCH(kern, dim3((unsigned)(per_row + 3) / 4, (unsigned)n, 1), dim3(256, 1, 1), 0, st,
-                     qg + (size_t)r0 * n_heads * 2 * kHeadDim, k + (size_t)r0 * n_kv * kHeadDim, qw, kw, t, posp,
-                     (uint32_t)n_heads | mode << 30, n_kv, a);
+        auto kern = flat ? enc < 0 ? front_kernel<0, true> : enc == 0 ? front_kernel<1, true> : front_kernel<2, true>
+                         : enc < 0 ? front_kernel<0, false> : enc == 0 ? front_kernel<1, false> : front_kernel<2, false>;
+        const dim3 grid = flat ? dim3((unsigned)(waves * n + 3) / 4, 1, 1)
+                               : dim3((unsigned)(waves + 3) / 4, (unsigned)n, 1);
+        HIPML_LAUNCH(kern, grid, dim3(256, 1, 1), 0, st, qg + (size_t)r0 * n_heads * 2 * kHeadDim,
+                     k + (size_t)r0 * n_kv * kHeadDim, qw, kw, posp, (uint32_t)n_heads | mode << 30, n_kv, n, inverse(heads), a);
         int rc = launched(enc < 0 ? "attn_front_f32" : "attn_front_encode_f32");
         if (rc)
             return rc;

@@ -1,0 +1,107 @@
+"""How the front end's launches are laid out (by rows, or flat with the V rows behind): the same bits as calls of few rows, and
+nothing beside the rows."""
+import numpy as np
+import pytest
+import torch
+
+from hipml_amd import attn
+
+HD, N_ROT, THETA, EPS = 256, 64, 1e7, 1e-6
+
+
+def flat(n_heads, n_kv, rows, append):
+    return attn.lib().hipml_dbg_front_flat(n_heads, n_kv, rows, int(append)) != 0
+
+
+def test_which_launches_are_flat():
+    assert [flat(24, 4, rows, True) for rows in (1, 99, 100, 257, 550, 551, 672)] == [False, False, True, True, True, False, False]
+    assert not any(flat(24, 4, rows, False) for rows in (1, 257, 2048))
+    assert not any(flat(h, kv, 257, True) for h, kv in ((28, 2), (32, 8), (16, 2), (14, 2), (40, 8)))
+    assert [flat(5, 1, rows, False) for rows in (249, 250, 2048)] == [False, True, True]
+    assert [flat(3, 1, rows, True) for rows in (249, 250, 2048)] == [False, True, True]
+    assert not any(flat(5, 1, rows, True) for rows in (250, 2048))
+
+
+@pytest.mark.parametrize("n_heads,n_kv,append", [(24, 4, True), (48, 8, True), (1000, 4, True), (4, 1, False), (5, 1, False),
+                                                 (1, 1, True), (3, 3, True), (6, 1, True), (7, 1, True), (1, 1, False)])
+def test_rows_found_by_a_product(n_heads, n_kv, append):
+    # every wave of the largest flat launch of these heads: its row is the quotient
+    rows = max((r for r in range(1, 32_769) if flat(n_heads, n_kv, r, append)), default=0)
+    for d, n in ((n_heads + n_kv, rows), (n_kv, rows)):
+        if rows and d > 1:
+            waves = np.arange(d * n, dtype=np.uint64)
+            inverse = np.uint64((0xFFFFFFFF + d) // d)
+            assert int(inverse) < 1 << 32
+            assert np.array_equal(waves * inverse >> np.uint64(32), waves // np.uint64(d))
+
+
+def run(dtype, qg, k, v, qw, kw, n_heads, n_kv, pos0, stride, cuts, caches, pos=None):
+    """The chunk's front end (with append where dtype is not None) as one call per piece between two cuts; with `pos` the rows of
+    a batch of sequences, a cache slot each."""
+    rows = qg.shape[0]
+    q, gate = (torch.full((rows + 1, n_heads, HD), 7.0, device="cuda") for _ in range(2))
+    kd = torch.cat((k, torch.full_like(k[:1], 7.0)))
+    kc, vc = (c.clone() for c in caches)
+    shape = (n_heads, n_kv, HD, N_ROT, THETA, EPS)
+    for a, b in zip(cuts, cuts[1:]):
+        if pos is not None:
+            slot = kc[0].numel()
+            attn.front_rows_encode(dtype, qg[a:], kd[a:], v[a:], q[a:], gate[a:], qw, kw, kc[a:], vc[a:], *shape, stride, pos[a:],
+                                   slot, b - a)
+        elif dtype is None:
+            attn.chunk_front(qg[a:], kd[a:], q[a:], gate[a:], qw, kw, *shape, pos0 + a, b - a)
+        else:
+            attn.chunk_front_encode(dtype, qg[a:], kd[a:], v[a:], q[a:], gate[a:], qw, kw, kc, vc, *shape, pos0 + a, b - a, stride)
+    torch.cuda.synchronize()
+    assert all(bool((t[rows] == 7.0).all()) for t in (q, gate, kd))
+    return q, gate, kd, kc, vc
+
+
+def same(one, many):
+    for name, a, b in zip(("q", "gate", "k", "k cache", "v cache"), one, many):
+        assert torch.equal(a, b), name
+
+
+def inputs(n_heads, n_kv, rows, seed):
+    attn.init(0)
+    attn.rope_table(THETA, N_ROT, 131_072)
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(seed)
+    made = [torch.randn(s, device="cuda", generator=gen) for s in ((rows, n_heads, 2 * HD), (rows, n_kv, HD), (rows, n_kv, HD))]
+    return made + [1.0 + 0.1 * torch.randn(HD, device="cuda", generator=gen) for _ in range(2)]
+
+
+# both sides of the rule's lines, ragged last workgroups, one and several KV heads
+@pytest.mark.gpu
+@pytest.mark.parametrize("n_heads,n_kv,rows,dtype,is_flat", [
+    (24, 4, 99, 0, False), (24, 4, 100, 0, True), (24, 4, 257, 1, True), (24, 4, 550, 0, True), (24, 4, 551, 0, False),
+    (48, 8, 67, 0, True), (26, 6, 101, 1, False), (27, 5, 101, 0, False), (20, 5, 131, 0, True), (5, 1, 251, None, True),
+    (5, 1, 251, 0, False), (3, 1, 337, 0, True), (3, 1, 337, 1, True), (1, 1, 513, 0, True), (2, 2, 513, 1, True)])
+def test_one_launch_has_the_bits_of_small_ones(n_heads, n_kv, rows, dtype, is_flat):
+    assert flat(n_heads, n_kv, rows, dtype is not None) == is_flat and not flat(n_heads, n_kv, 47, dtype is not None)
+    made = inputs(n_heads, n_kv, rows, rows * 100 + n_heads)
+    pos0, stride = 1000, 1000 + rows + 5
+    caches = [torch.full((n_kv, stride, 144 if dtype == 1 else 272), 0x5A, dtype=torch.uint8, device="cuda") for _ in range(2)]
+    args = (n_heads, n_kv, pos0, stride)
+    one = run(dtype, *made, *args, [0, rows], caches)
+    same(one, run(dtype, *made, *args, [*range(0, rows, 47), rows], caches))
+    if dtype is not None:
+        for c in one[3:]:
+            assert bool((c[:, :pos0] == 0x5A).all()) and bool((c[:, pos0 + rows:] == 0x5A).all())
+            assert not bool((c[:, pos0:pos0 + rows] == 0x5A).all(dim=2).any())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n_heads,n_kv,dtype", [(24, 4, 0), (24, 4, 1), (3, 1, 0)])
+def test_a_flat_launch_over_a_batch(n_heads, n_kv, dtype):
+    rows, stride = 260, 96
+    assert flat(n_heads, n_kv, rows, True)
+    made = inputs(n_heads, n_kv, rows, 77 + n_heads)
+    at = torch.randint(0, stride, (rows, 1), dtype=torch.int32, device="cuda")
+    caches = [torch.full((rows, n_kv, stride, 144 if dtype == 1 else 272), 0x5A, dtype=torch.uint8, device="cuda") for _ in range(2)]
+    pos = torch.cat((at, at + 1), dim=1).contiguous()
+    args = (n_heads, n_kv, 0, stride)
+    one = run(dtype, *made, *args, [0, rows], caches, pos)
+    same(one, run(dtype, *made, *args, [*range(0, rows, 47), rows], caches, pos))
+    touched = (one[3] != 0x5A).any(dim=3).any(dim=1).sum(dim=1)
+    assert bool((touched == 1).all())
