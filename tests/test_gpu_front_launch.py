@@ -1,5 +1,5 @@
-"""How the front end's launches are laid out (by rows, or flat with the V rows behind): the same bits as calls of few rows, and
-nothing beside the rows."""
+"""How the front end's launches are laid out (by rows, or flat with the V rows behind) and where long calls are cut into several
+launches: the same bits as calls of few rows, and nothing beside the rows."""
 import numpy as np
 import pytest
 import torch
@@ -105,3 +105,31 @@ def test_a_flat_launch_over_a_batch(n_heads, n_kv, dtype):
     same(one, run(dtype, *made, *args, [*range(0, rows, 47), rows], caches, pos))
     touched = (one[3] != 0x5A).any(dim=3).any(dim=1).sum(dim=1)
     assert bool((touched == 1).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n_heads,n_kv,dtype", [(2, 1, 0), (2, 1, None), (1, 1, 1)])
+def test_a_chunk_longer_than_a_launch(n_heads, n_kv, dtype):
+    rows = 32_770  # a launch holds 32,768: by rows, and flat (one head)
+    made = inputs(n_heads, n_kv, rows, 5)
+    pos0, stride = 9, 9 + rows + 2
+    caches = [torch.full((n_kv, stride, 144 if dtype == 1 else 272), 0x5A, dtype=torch.uint8, device="cuda") for _ in range(2)]
+    args = (n_heads, n_kv, pos0, stride)
+    same(run(dtype, *made, *args, [0, rows], caches), run(dtype, *made, *args, [0, 20_000, 32_767, rows], caches))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [0, 1])
+def test_a_bulk_append_longer_than_a_launch(dtype):
+    attn.init(0)
+    n_kv, rows, start, src0 = 2, 32_771, 11, 3
+    stride, row_bytes = start + rows + 2, 144 if dtype else 272
+    k, v = (torch.randn((src0 + rows, n_kv, HD), device="cuda") for _ in range(2))
+    whole, pieces = ([torch.full((n_kv, stride, row_bytes), 0x5A, dtype=torch.uint8, device="cuda") for _ in range(2)] for _ in range(2))
+    attn.kv_encode_bulk(dtype, k, v, *whole, n_kv, HD, stride, start, src0, rows)
+    for a, b in ((0, 16_000), (16_000, 32_767), (32_767, rows)):
+        attn.kv_encode_bulk(dtype, k[src0 + a:], v[src0 + a:], *pieces, n_kv, HD, stride, start + a, 0, b - a)
+    torch.cuda.synchronize()
+    for a, b in zip(whole, pieces):
+        assert torch.equal(a, b) and bool((a[:, :start] == 0x5A).all()) and bool((a[:, start + rows:] == 0x5A).all())
+        assert not bool((a[:, start:start + rows] == 0x5A).all(dim=2).any())
