@@ -2196,6 +2196,22 @@ struct ChunkCut {
     int slice, nslice, grid, ntask64, nblock64, grid64;
     bool uniform, t64;
 };
+// block_slices of all blocks, added up slice by slice instead of block by block: slice j + 1 runs for the blocks whose last token
+// sees more than j x slice_tiles tiles, which are the last ones.  (Block by block, 62 times over the 500 blocks of 16,000 tokens,
+// the choice of a count took 165 us of the host's time, now 4.)
+static int chunk_slices_of_all(int ntask, int group, int tokens, int pos0, int splits, int slice_tiles)
+{
+    const int nblock = (ntask + kTasks - 1) / kTasks;
+    int n = nblock;
+    for (int j = 1; j < splits; j++) {
+        const long long behind = (long long)j * slice_tiles * kKTile - pos0; // tokens that do not see as many
+        if (behind >= tokens)
+            break;
+        n += nblock - (behind < 0 ? 0 : (int)behind / kQTile * group / kTasks);
+    }
+    return n;
+}
+
 static ChunkCut chunk_cut(int pos0, int tokens, int n_head, int n_kv, int splits, bool f16)
 {
     const int group = n_head / n_kv, ntask = (tokens + kQTile - 1) / kQTile * group, nblock = (ntask + kTasks - 1) / kTasks;
@@ -2206,9 +2222,7 @@ static ChunkCut chunk_cut(int pos0, int tokens, int n_head, int n_kv, int splits
     ChunkCut c;
     c.slice = (tiles + splits - 1) / splits;
     c.uniform = block_slices(0, ntask, group, tokens, pos0, splits, c.slice, nullptr) == splits; // (the first has the fewest)
-    c.nslice = c.uniform ? nblock * splits : 0;
-    for (int tb = 0; tb < nblock && !c.uniform; tb++)
-        c.nslice += block_slices(tb, ntask, group, tokens, pos0, splits, c.slice, nullptr);
+    c.nslice = c.uniform ? nblock * splits : chunk_slices_of_all(ntask, group, tokens, pos0, splits, c.slice);
     c.grid = c.uniform ? workgroups(nblock) : n_kv * c.nslice;
     // 64 tokens per wave: its own task blocks (4 tasks of 64 tokens, up to 32 left-over tokens as tasks of 32 tokens x 2 heads),
     // every one with `splits` slices.  Both kernels run one workgroup per CU, so the hardware starts them in rounds of 256; where
@@ -2273,7 +2287,8 @@ int chunk_run_slices(int pos0, int tokens, int n_head, int n_kv, int splits, boo
 // 1,300 78 (2 slices) / 65 (3), 900 behind 900 78 (2) / 65 (3), 1,400 behind 1,700 172 (2) / 151 (3), 1,500 behind 3,000 236 (2) /
 // 199 (3), 1,800 behind 2,500 227 (2) / 216 (3); over 88 shapes (both formats) for which the two costs differ by 4 % so, the
 // cache is 4 to 23 % faster (by 3 %: 2 % slower to 23 % faster); 1,024 behind 8,192 and 672 behind 8,192 keep their tiles.
-bool chunk_tiles_plan(int pos0, int tokens, int n_head, int n_kv, int splits, int *use, size_t *tiles_at)
+// (slices: what chunk_run_slices gives for this scratch.)
+bool chunk_tiles_plan(int pos0, int tokens, int n_head, int n_kv, int splits, int slices, int *use, size_t *tiles_at)
 {
     if (!chunk_tiles_pay(pos0, tokens) || splits < 3)
         return false;
@@ -2286,7 +2301,6 @@ bool chunk_tiles_plan(int pos0, int tokens, int n_head, int n_kv, int splits, in
         return false;
     // What the tiles cost, and the kernel over them, against the kernel over the cache with the same scratch.
     const float tiles_us = 0.23f + 1.86e-3f * (float)(pos0 + tokens) * (float)n_kv / 4.0f;
-    const int slices = chunk_run_slices(pos0, tokens, n_head, n_kv, splits, false);
     if (tiles_us + chunk_us(pos0, tokens, n_head, n_kv, s, true) > 1.04f * chunk_us(pos0, tokens, n_head, n_kv, slices, false))
         return false;
     *use = s;
@@ -2306,7 +2320,8 @@ bool chunk_tiles_plan(int pos0, int tokens, int n_head, int n_kv, int splits, in
 // And not where the other kernel's cost by chunk_us, fitted at more tokens, is lower by a tenth, as with fewer slices than it
 // is given: 330 @ 1,862 54.9 here / 46.0 there, 464 @ 3,639 92.5 / 73.9, 226 @ 3,679 57.7 / 50.4; over
 // 33 shapes where the two estimates differ, those under a tenth take 19 % less to 1 % more here, those over it as long or more.
-static int chunk_wg_splits(int pos0, int tokens, int n_head, int n_kv, int splits)
+// (slices: of the other kernel, what chunk_run_slices gives for this scratch; 0: not known yet.)
+static int chunk_wg_splits(int pos0, int tokens, int n_head, int n_kv, int splits, int slices = 0)
 {
     const int group = n_head / n_kv, keys = pos0 + tokens;
     const long long ntt = (tokens + kQTile - 1) / kQTile, wgs = ntt * n_kv * ((group + 1) / 2);
@@ -2331,7 +2346,8 @@ static int chunk_wg_splits(int pos0, int tokens, int n_head, int n_kv, int split
     const float cost = 12.6f + (float)rounds * (float)slice * (2.53f + fill) + (float)splits * (0.152f + 0.0067f * sums);
     if (best_cost >= 0.95f * cost)
         return 0;
-    const int slices = chunk_run_slices(pos0, tokens, n_head, n_kv, splits, false);
+    if (slices == 0)
+        slices = chunk_run_slices(pos0, tokens, n_head, n_kv, splits, false);
     return best_cost < 1.1f * chunk_us(pos0, tokens, n_head, n_kv, slices, false) ? best : 0;
 }
 
@@ -2355,7 +2371,13 @@ extern "C" int hipml_dbg_chunk_makes_tiles(int pos0, int tokens, int n_head, int
 {
     int use;
     size_t tiles_at;
-    return chunk_tiles_plan(pos0, tokens, n_head, n_kv, splits, &use, &tiles_at) ? use : 0;
+    const int slices = splits < 2 ? 1 : chunk_run_slices(pos0, tokens, n_head, n_kv, splits, false);
+    return chunk_tiles_plan(pos0, tokens, n_head, n_kv, splits, slices, &use, &tiles_at) ? use : 0;
+}
+// The slices of all blocks together (chunk_q8_kernel's workgroups of a KV head).
+extern "C" int hipml_dbg_chunk_slices_of_all(int pos0, int tokens, int n_head, int n_kv, int splits)
+{
+    return chunk_cut(pos0, tokens, n_head, n_kv, splits, false).nslice;
 }
 extern "C" int hipml_dbg_chunk_f16_slices(int pos0, int tokens, int n_head, int n_kv, int splits, int *t64)
 {
@@ -2373,11 +2395,14 @@ int launch_chunk_q8(hipStream_t st, const float *q, const uint8_t *kc, const uin
                     float *part_acc, float *part_ml, int splits, const float *gate, int q4, void *out16,
                     const void *kv_f16, const float *rope_tab)
 {
+    // over the cache: the slices that run of those that the scratch holds (over f16 tiles the caller has chosen)
+    int slices = splits >= 2 && kv_f16 == nullptr ? chunk_run_slices(pos0, tokens, n_head, n_kv, splits, false)
+                                                  : splits < 2 ? 1 : splits;
     {
         int use;
         size_t tiles_at;
         if (kv_f16 == nullptr && rope_tab == nullptr &&
-            chunk_tiles_plan(pos0, tokens, n_head, n_kv, splits, &use, &tiles_at)) {
+            chunk_tiles_plan(pos0, tokens, n_head, n_kv, splits, slices, &use, &tiles_at)) {
             const int live_tiles = (pos0 + tokens + kKTile - 1) / kKTile;
             uint8_t *tiles = reinterpret_cast<uint8_t *>(part_acc) + tiles_at;
             if (int rc = launch_kv_f16_tiles(st, kc, vc, tiles, n_kv, stride, live_tiles, 0, pos0 + tokens, q4))
@@ -2395,6 +2420,7 @@ int launch_chunk_q8(hipStream_t st, const float *q, const uint8_t *kc, const uin
             if (s >= 2 && s < splits && splits == chunk_tiles_splits(pos0, tokens, 6 * n_kv, n_kv, s)) {
                 const int fill = chunk_fill_slices(pos0, tokens, n_kv);
                 splits = fill < splits ? fill : splits;
+                slices = splits < 2 ? 1 : chunk_run_slices(pos0, tokens, n_head, n_kv, splits, false);
             }
         }
     }
@@ -2417,16 +2443,14 @@ int launch_chunk_q8(hipStream_t st, const float *q, const uint8_t *kc, const uin
     a.pos0 = pos0;
     a.tokens = tokens;
     a.stride = stride;
-    a.splits = splits < 2 ? 1 : splits;
-    if (splits >= 2 && kv_f16 == nullptr) // (over f16 tiles the caller has chosen)
-        a.splits = chunk_run_slices(pos0, tokens, n_head, n_kv, splits, false);
+    a.splits = slices;
     a.qslots = (tokens + 31) / 32 * 32;
     a.ntask = (tokens + kQTile - 1) / kQTile * a.group;
     a.nblock = (a.ntask + kTasks - 1) / kTasks;
     a.scale_log2 = kLog2e / 16.0f; // 1/sqrt(256), as the reference's chunk launcher fixes it
     a.out16 = nullptr;
     const int wg_splits = kv_f16 == nullptr && rope_tab == nullptr && splits >= 2
-                              ? chunk_wg_splits(pos0, tokens, n_head, n_kv, splits) : 0;
+                              ? chunk_wg_splits(pos0, tokens, n_head, n_kv, splits, slices) : 0;
     if ((splits == 0 && kv_f16 == nullptr) || wg_splits == 1) {
         // the key slices stay inside the workgroup: no partial rows, gate and f16 rows in the same launch
         a.out16 = static_cast<_Float16 *>(out16);
