@@ -9,6 +9,13 @@ def row_kernel(m, k, rows):
     return attn.lib().hipml_dbg_rows_kernel(m, k, rows, 1)
 
 
+def row_variant(m, k, rows):
+    """The same with what the code leaves out: the kernel that streams units takes its weights by 16-byte requests where k is of
+    whole 256-value chunks, by dwords elsewhere."""
+    kernel = row_kernel(m, k, rows)
+    return kernel, kernel // 1_000_000 == 3 and k % 256 == 0
+
+
 def gemm_tile(m, k, tokens, x16):
     """(place in the table of tiles, whole sectors of weights), W at a 64-byte boundary."""
     sectors = int(k % 1024 == 0)
@@ -30,8 +37,15 @@ ROWS = [
     (6156, 4864, 25), (6156, 4864, 17), (8230, 4864, 25), (8230, 4864, 17), (6156, 4864, 41), (6156, 4864, 33),
     (8230, 4864, 41), (8230, 4864, 33), (6156, 4864, 57), (6156, 4864, 49), (8230, 4864, 57), (8230, 4864, 49),
     (3, 2368, 9), (3, 2368, 3), (2069, 2368, 17), (4143, 2368, 3), (2618, 2368, 17), (5180, 2368, 3),
-    (3106, 2368, 17), (6156, 2368, 3), (8230, 2368, 9), (8230, 2368, 3), (2069, 2368, 49), (773, 1280, 115), (4143, 2368, 17),
+    (3106, 2368, 17), (6156, 2368, 3), (8230, 2368, 9), (8230, 2368, 3), (2069, 2368, 49), (1345, 2368, 81), (773, 1280, 115), (4143, 2368, 17),
     (2740, 2368, 33), (5180, 2368, 17), (4082, 2368, 33), (6156, 2368, 17), (4143, 2368, 33), (8230, 2368, 17),
+]
+# And of every tile of the kernel that streams units by 16-byte requests (k of whole 256-value chunks, one among them): ragged in
+# both directions, several workgroups of 8 and of 24 rows, waves with no unit or uneven shares
+WIDE = [
+    (3, 256, 9), (1003, 1280, 30), (2069, 1280, 31), (517, 1280, 125), (5180, 4864, 16), (645, 1280, 115), (771, 1280, 127),
+    (517, 1280, 115), (1029, 1280, 125), (1349, 1280, 81), (773, 1280, 115), (1637, 1280, 65), (1029, 1280, 115),
+    (1541, 1280, 125), (1541, 1280, 115), (261, 1280, 125), (2053, 256, 125), (2053, 1280, 97), (5117, 4864, 24), (5117, 4864, 70),
 ]
 # (weight rows, k, tokens, f16 activations)
 TILES = [

@@ -50,14 +50,9 @@ def test_row_kernel(m, k, rows):
             assert torch.equal(z[more - 1], y[rows - 1]) and bool(z[more].isnan().all())
 
 
-# (weight rows, k, activation rows) of every tile of the kernel that streams units by 16-byte requests (k of whole 256-value
-# chunks, one among them): ragged in both directions, several workgroups of 8 and of 24 rows, waves with no unit or uneven shares
-@pytest.mark.parametrize("m,k,rows", [(3, 256, 9), (1003, 1280, 30), (2069, 1280, 31), (517, 1280, 125), (5180, 4864, 16),
-                                      (645, 1280, 115), (771, 1280, 127), (517, 1280, 115), (1029, 1280, 125), (1349, 1280, 81),
-                                      (773, 1280, 115), (1637, 1280, 65), (1029, 1280, 115), (1541, 1280, 125), (1541, 1280, 115),
-                                      (261, 1280, 125), (2053, 256, 125), (2053, 1280, 97), (5117, 4864, 24), (5117, 4864, 70)])
+@pytest.mark.parametrize("m,k,rows", inst.WIDE)
 def test_rows_by_wide_requests(m, k, rows):
-    assert inst.row_kernel(m, k, rows) // 1_000_000 == 3
+    assert inst.row_variant(m, k, rows)[1]
     w, d, q, x = inputs(m, k, rows)
     y = padded(rows, m)
     attn.gemv_q8_0_rows(w, x, y, m, k, rows)

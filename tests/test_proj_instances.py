@@ -3,14 +3,15 @@ import pytest
 
 import proj_instances as inst
 
-M = sorted({*range(1, 400, 13), *range(400, 20_000, 197), *range(20_000, 130_000, 7_777), 1024, 2048, 5120, 6144, 12_288})
+M = sorted({*range(1, 400, 13), *range(400, 20_000, 197), *range(20_000, 130_000, 7_777), 1024, 1345, 2048, 5120, 6144, 12_288})
 
 
-@pytest.mark.parametrize("k", [64, 256, 1088, 5120, 32_768, 34_560, 36_096])
+@pytest.mark.parametrize("k", [64, 256, 1088, 1280, 5120, 32_768, 34_560, 36_096])
 def test_every_row_kernel_has_a_shape(k):
-    named = {inst.row_kernel(*shape) for shape in inst.ROWS}
+    named = {inst.row_variant(*shape) for shape in inst.ROWS}
     assert len(named) == len(inst.ROWS)
-    taken = {inst.row_kernel(m, k, rows): (m, rows) for m in M for rows in range(1, 129)}
+    named |= {inst.row_variant(*shape) for shape in inst.WIDE}
+    taken = {inst.row_variant(m, k, rows): (m, rows) for m in M for rows in range(1, 129)}
     assert not {c: s for c, s in taken.items() if c not in named}
 
 
@@ -34,8 +35,8 @@ def test_every_packed_tile_has_a_shape():
 
 @pytest.mark.parametrize("m,k", [(12_288, 5120), (1024, 5120), (5120, 6144)])
 def test_the_models_projections_are_among_them(m, k):
-    named = {inst.row_kernel(*shape) for shape in inst.ROWS}
-    assert all(inst.row_kernel(m, k, rows) in named for rows in range(1, 129))
+    named = {inst.row_variant(*shape) for shape in inst.ROWS + inst.WIDE}
+    assert all(inst.row_variant(m, k, rows) in named for rows in range(1, 129))
 
 
 @pytest.mark.parametrize("k", [256, 4864, 5120, 6144, 8192])
