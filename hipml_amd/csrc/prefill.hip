@@ -2355,8 +2355,11 @@ static int chunk_wg_splits(int pos0, int tokens, int n_head, int n_kv, int split
 // latency, which chunk_wg_kernel's workgroups of four slices share and the kernels over tiles pay slice by slice, and the rows
 // are half the bytes.  us over q8_0 / q4_0 rows and over the copy (with the slices above): 16 tokens behind 2,048 17.9 / 17.2 and
 // 21.9, behind 90,000 136 / 124 and 221, 32 behind 7,000 28.7 / 27.2 and 36.3, 64 behind 4,500 30.5 / 28.8 and 31.8, behind
-// 90,000 226 / 197 and 240; 80 behind 4,500 33.7 / 32.0 and 33.0 are the first for which it is no loss.  Behind less than 2,048 a
-// registered copy is read as before: there a call's bits are those of hipml_attn_chunk_kv_f16.
+// 90,000 226 / 197 and 240; 80 behind 4,500 33.7 / 32.0 and 33.0 are the first for which it is no loss.
+// Behind less than 2,048 rows the cache would be the faster one too (16 tokens behind 512 / 1,024 / 2,047 15.9 / 16.7 / 18.1 us over
+// q8_0 rows and 19.3 / 24.7 / 21.9 over the copy, 64 behind 512 / 1,800 19.2 / 23.7 and 22.2 / 29.2): that line is no crossover.
+// Short prefixes keep what a registered copy promised before this rule: the bits of hipml_attn_chunk_kv_f16 over it, with the
+// slices that run (chunk_run_slices: 9 for 64 tokens behind 1,819 and a scratch of 10).
 bool chunk_reads_cache(int pos0, int tokens, int n_head, int n_kv, int splits)
 {
     return tokens <= 64 && pos0 >= 2048 && chunk_wg_splits(pos0, tokens, n_head, n_kv, splits) > 0;

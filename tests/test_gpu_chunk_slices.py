@@ -59,7 +59,8 @@ def test_fewer_slices_than_the_scratch_holds(tok, pos0, splits, n_head, n_kv, dt
 @pytest.mark.parametrize("dtype", [0, 1])
 @pytest.mark.parametrize("tok,pos0,splits,t64", [
     (96, 1700, 10, 0),    # a count that leaves the first block a slice short: the kernel of 32 tokens per wave
-    (420, 5003, 12, 1), (1079, 492, 8, 0)])
+    (420, 5003, 12, 1), (1079, 492, 8, 0),
+    (64, 1819, 10, 0), (33, 1400, 8, 0)])  # few tokens behind less than 2,048 rows, which read the copy
 def test_fewer_slices_over_a_registered_copy(tok, pos0, splits, t64, dtype):
     from test_gpu_kv_f16 import run_chunk_f16
     from test_gpu_kv_shadow import Attached, attend
