@@ -334,13 +334,20 @@ __device__ __forceinline__ uint32_t proj_lds_address(const void *p)
     return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void *)p;
 }
 
-// 64 lanes x 16 bytes from base + voff (per lane) to LDS address lds_at + 16 * lane.  ONCE: non-temporal, for bytes that are
-// read once.  gemv_q8_digits_kernel asks for its weights so (runs of 544 bytes of a row; from HBM 12288 x 5120 over 1 / 3 rows
+// 64 lanes x 16 bytes from base + voff (per lane) to LDS address lds_at + 16 * lane.  ONCE: non-temporal.
+// gemv_q8_digits_kernel asks for its weights so (runs of 544 bytes of a row, read once; from HBM 12288 x 5120 over 1 / 3 rows
 // 13.0 / 15.4 us with the hint, 13.8 / 15.7 without).  Where a request ends inside a cache line whose rest another one wants it
 // costs a second fetch: gemv_q8_units_kernel over 1024 x 5120 and 24 rows 8.8 and 7.6, gemv_q8_blocks_kernel over 12288 x 5120
-// and 9 / 16 rows 19.2 / 19.9 and 18.2 / 18.8.  gemv_q8_blocks_kernel over more rows asks with it all the same (over 24 / 32
-// rows 22.8 / 25.2 and 22.1 / 23.8): such a matrix, of 35 MB and more, otherwise pushes out of the last-level cache what is
-// there (a layer over 32 short sequences, whose W_o then comes from HBM, 86.2 and 89.6 us).
+// and 9 / 16 rows 19.2 / 19.9 and 18.2 / 18.8.
+// gemv_q8_blocks_kernel asks with it from 17 rows on, whatever the size of the matrix, and also where the workgroups of further
+// activation rows, from 65 on, read the weights again.  To the call by itself it is a loss: us with / without over 12288 x 5120
+// from HBM and 24 / 32 / 48 / 64 / 65 / 128 rows 22.2 / 24.5 / 31.6 / 34.4 / 57.0 / 67.8 and 21.7 / 23.6 / 31.5 / 35.4 / 53.2 / 65.0,
+// with all weights in the last-level cache 24.1 / 26.5 / 33.7 / 36.6 / 59.3 / 70.7 and 22.9 / 23.8 / 28.1 / 34.6 / 49.8 / 64.5;
+// 6400 x 1024 over 32 / 128 rows 6.7 / 17.3 and 6.7 / 15.5.  What it buys is that the weights do not push out of that cache what the
+// next calls find there, which shows only while a few layers are all that runs: a layer over 32 short / 20 short / 24 deeper
+// sequences, three layers in turn (333 MB of weights) 86.6 / 75.1 / 90.5 with and 89.5 / 77.9 / 94.8 without, sixteen, whose W_o
+// comes from HBM either way, 90.7 / 78.9 / 93.4 and 89.2 / 77.8 / 93.0, one layer again and again 90.6 / 79.9 / 94.3 and 84.4 /
+// 75.9 / 91.7.
 template <bool ONCE>
 __device__ __forceinline__ void proj_dma16(uint32_t lds_at, const uint8_t *base, uint32_t voff)
 {
@@ -1016,7 +1023,10 @@ struct UnitsShape {
     static constexpr int kWaves = kRoom / (8 * kSlot) >= 2 ? 8 : 4;
     // Units of a wave on the way.  More only lengthen the queue that everybody's first ones wait in: 1024 x 5120 over 24 rows
     // with 4 / 3 / 2 of them 8.7 / 8.4 / 7.6 us from HBM and 7.4 / 7.3 / 6.7 from the last-level cache, 5120 x 6144 over 9 rows
-    // with 3 / 2 13.8 / 12.8 from HBM.
+    // with 3 / 2 13.8 / 12.8 from HBM.  By dwords as well, where it was up to four: over k 5184 from HBM and 3 / 9 / 24 / 64 / 128
+    // rows 1,024 weight rows 8.5 / 9.9 / 10.2 / 10.8 / 14.4 -> 7.5 / 9.3 / 9.6 / 10.0 / 13.3, 5,120 11.3 / 12.4 / 16.9 / 26.9 / 49.3 ->
+    // 10.0 / 11.6 / 16.7 / 25.5 / 45.3, 12,288 19.0 / 19.8 / 24.9 / 52.7 / 98.1 -> 18.2 / 19.8 / 24.8 / 49.8 / 91.7 (the order of a
+    // turn, below, is in both); 216 shapes from 512 to 12,288 weight rows 12 % less to 1 % more.
     static constexpr int kDepth = 2;
     static constexpr int kLds = kWaves * kDepth * kSlot + kRead;
     static constexpr int kChains = 8 / kWaves; // of a wave
