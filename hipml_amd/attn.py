@@ -192,7 +192,8 @@ def batch_splits(stride: int, n_kv: int, slots: int) -> int:
 
 
 def chunk_splits(pos0: int, tokens: int, n_kv: int = 4) -> int:
-    """0 = keys cut inside the workgroups (no scratch), 1 = single pass, n >= 2 = n key slices with scratch."""
+    """0 = keys cut inside the workgroups (no scratch), 1 = single pass, n >= 2 = key slices with a scratch for n of them
+    (a call runs as many of those as cost least)."""
     return lib().hipml_attn_chunk_splits(pos0, tokens, n_kv)
 
 

@@ -2130,11 +2130,12 @@ int prefill_init()
 // the attention then runs over those with the 64-token kernel and fewer slices.  That needs a scratch sized for
 // more slices than the attention uses: `splits` (the count the scratch was sized for) must cover `*use` slices
 // of partial rows plus the tiles, which start at byte *tiles_at of part_acc.  hipml_attn_chunk_splits returns
-// such a count where the detour pays (the pass over the cache costs 1.3 us per 1,000 rows, the kernel of 32
+// such a count where the detour may pay (the pass over the cache costs 1.3 us per 1,000 rows, the kernel of 32
 // tokens per wave with its own dequantization 15 % of the attention; measured gain, 2,048 tokens at depth
 // 2,048 / 8,192 / 16,384 / 100,000: 13 / 10 / 11 / 13 %, 1,024 tokens at 2,048 / 8,192: 3 / 4 %, 768 tokens at
-// 3,072 / 6,144: 0.5 / 3 %); with any smaller count the chunk runs as before.
-// Where the detour pays: chunks of 768 tokens or more behind a prefix at least as long, and chunks of 640 or
+// 3,072 / 6,144: 0.5 / 3 %); with any smaller count the chunk runs as before, and so it does where the costs of both say that
+// the kernel over the cache is the faster one (chunk_tiles_plan).
+// Where the detour may pay: chunks of 768 tokens or more behind a prefix at least as long, and chunks of 640 or
 // more (the 672 tokens of the usual prefill chunk) behind a prefix of eight times their length (672 tokens at
 // depth 672 / 2,048 / 8,192 / 32,768 / 100,000: -3 / -3 / +5 / +7 / +6 %).
 bool chunk_tiles_pay(int pos0, int tokens)

@@ -85,15 +85,18 @@ int hipml_attn_batch_splits(int stride, int n_kv, int slots);
 /* Key splits for a prefill chunk starting at pos0.  Same role as split_count,
  * crates/hipml-model/src/gpu/attn_tile.rs:138-151.  0 (chunks near position 0: pos0 + tokens <=
  * 1,792 and pos0 <= 2 * tokens) selects the kernel that cuts the keys inside its workgroups and
- * needs no scratch; 1 the single-pass kernel; n >= 2 that kernel over n key slices with scratch
- * and a merge launch.  For long chunks behind a prefix at least as long (tokens >= 768 and pos0 >= tokens, or tokens >= 640
+ * needs no scratch; 1 the single-pass kernel; n >= 2 that kernel over key slices with a scratch for n of
+ * them and a merge launch.  n is what the scratch has to hold, not what runs: a call takes the count, of 2 to n, that
+ * costs least at its shape, and for few tokens a kernel that slices inside its workgroups as well (2,000 tokens at
+ * depth 300: 8, of which 3 run; 350 at 20,000: 14 and 7).  For long chunks behind a prefix at least as long (tokens >= 768 and pos0 >= tokens, or tokens >= 640
  * and pos0 >= 8 * tokens) n is larger
  * than the number of slices that run (hipml_attn_chunk_slices): the chunk entry points then write the
  * live rows of the cache as f16 tiles (70,656 bytes per KV head and 64 rows) into the tail of part_acc
  * and run the attention over those, which is faster than dequantizing inside the attention (2,048 tokens
  * at depth 100,000: n = 13 for 4 slices, 654 MB of scratch, 4.1 against 4.7 ms).  A caller that passes fewer
- * than that (the reference's own policy gives 8) gets so many slices of the kernel that dequantizes for itself:
- * the scratch is never written beyond the n slices it was sized for.
+ * than that (the reference's own policy gives 8) gets the kernel that dequantizes for itself, and so does one whose chunk
+ * is faster so (768 tokens at depth 1,300, 1,500 at 3,000): the scratch is never written beyond the n slices it was
+ * sized for.
  * How that count grows: the partial rows are ceil32(tokens) * n_heads * 1,024 bytes per slice (50.3 MB at
  * 2,048 tokens and 24 heads), the tiles n_kv * ceil((pos0 + tokens) / 64) * 70,656 bytes (4.4 MB per 1,000
  * rows of depth at 4 KV heads), so n = slices + ceil(tiles / partial rows of one slice): 2,048-token chunks
@@ -107,10 +110,11 @@ int hipml_attn_batch_splits(int stride, int n_kv, int slots);
  * 4 at these shapes), and 8 is always enough.
  * NOTE: unlike the reference's split_count, which is at least 1, this returns 0 near position 0. */
 int hipml_attn_chunk_splits(int pos0, int tokens, int n_kv);
-/* The slice count (>= 1) for callers that want the sliced kernel whatever the shape, and for
- * hipml_attn_chunk_kv_f16, which has no in-workgroup variant: the count that fills the chip's last round
- * of workgroups, and for the long chunks named above the count that runs fastest over f16 tiles, often
- * fewer (1,024 tokens at depth 8,192: 2, 1,500 at 20,000: 3, 2,048 at 100,000: 4). */
+/* The slice count (>= 1) for callers that want the sliced kernel whatever the shape (an upper bound, as above),
+ * and for hipml_attn_chunk_kv_f16, which has no in-workgroup variant and runs exactly the count it is given: the
+ * count that fills the chip's last round of workgroups, and for the long chunks named above the count that runs
+ * fastest over f16 tiles, often fewer (1,024 tokens at depth 8,192: 2, 1,500 at 20,000: 3, 2,048 at 100,000: 4).  Elsewhere fewer slices than these can be
+ * faster over the copy too (420 tokens at depth 5,003: 95 us with the 12, 83 with the 5 that a registered copy runs). */
 int hipml_attn_chunk_slices(int pos0, int tokens, int n_kv);
 
 /* ---- RoPE ----------------------------------------------------------------
@@ -375,10 +379,11 @@ int hipml_attn_decode_one_launch(int on);
  * and splits == 0 the kernel that cuts the keys into four slices inside each workgroup (one
  * workgroup per 32 tokens x 2 heads; made for chunks near position 0, correct at any depth);
  * both ignore the scratch.  Otherwise part_acc is f32
- * [splits][ceil32(tokens)][n_head][head_dim] and part_ml [..][2]; how that memory is used is the
- * library's business (with a count from hipml_attn_chunk_splits for a long chunk behind a prefix,
- * fewer slices run and the rest of part_acc holds the cache rows as f16 tiles for the length of the
- * call), and nothing beyond those sizes is touched.
+ * [splits][ceil32(tokens)][n_head][head_dim] and part_ml [..][2], and `splits` is an upper bound: at most so many slices
+ * of the keys run, the count that costs least at this shape.  How that memory is used is the library's business (with a
+ * count from hipml_attn_chunk_splits for a long chunk behind a prefix, and where that costs less, the rest of part_acc
+ * holds the cache rows as f16 tiles for the length of the call), and nothing beyond those sizes is touched.  The bits of a
+ * result depend on the slices that run: the same arguments give the same bits.
  * Replaces AttnLayer::chunk_attention_q8_split -> attn_chunk_wmma_f16 /
  * attn_chunk_full_f16 + attn_chunk_combine_f32,
  * crates/hipml-kernels/src/attn_gpu/imp/attn_chunk_kv.rs:72-107,129-305. */
@@ -471,9 +476,9 @@ int hipml_attn_chunk_kv_f16(hipml_stream_t stream, const float *q, const void *k
  *     hipml_kv_encode_rows, hipml_attn_front_rows_encode_f32) mark the shadow stale, and the next chunk
  *     attention over the cache converts every live row once (0.13 ms per 100,000 rows);
  *   - hipml_attn_chunk_q8_split, _gate and _gate_f16 over (k_cache, v_cache) with the registered stride,
- *     n_kv and format and splits >= 2 read the tiles: at most min(splits, hipml_attn_chunk_slices) slices, no
- *     tiles made per call in the scratch (2,048 tokens at depth 100,000: 4.06 against 4.19 ms).  Up to 64 tokens
- *     behind 2,048 rows and more read the cache itself, which is faster for so few (32 tokens at depth 7,000: 29 us,
+ *     n_kv and format and splits >= 2 read the tiles: at most min(splits, hipml_attn_chunk_slices) slices, with
+ *     the bits of hipml_attn_chunk_kv_f16 over the count that runs, and no tiles made per call in the scratch
+ *     (2,048 tokens at depth 100,000: 4.06 against 4.19 ms).  Up to 64 tokens behind 2,048 rows and more read the cache itself, which is faster for so few (32 tokens at depth 7,000: 29 us,
  *     over the copy 36), and an append of such a chunk costs 3 to 4 us more than without a copy: attach it to caches
  *     that long chunks extend (us with the copy / without: 117 tokens at depth 20,000 81 / 87, 400 at 20,000 194 / 220).
  * The bookkeeping is host state that changes when a call is issued or captured, not when a captured
@@ -514,7 +519,7 @@ int hipml_kv_rows_copy(hipml_stream_t stream, int dtype, const void *k_src, cons
  * numbers of 31 bits over each block's largest one, W streams from memory once per pass of 4 or 8 rows, and a row's result has
  * the same bits whatever `rows` is and whichever rows travel with it: the rows of a verify group match their plain decodes,
  * as the reference's batched GEMVs do (crates/hipml-kernels/src/attn_gpu.rs:930-932).  From 9 to 128 rows they enter as two
- * f16 halves (~22 bits up to 65,504, to the nearest 32 above), W streams once per pass of 16 to 64 rows, and a row's bits
+ * f16 halves (~22 bits up to 65,504, to the nearest 32 above), W streams once per pass of 8 to 64 rows, and a row's bits
  * are the same for every such `rows`.  The two classes differ from each other in the last bits.  (W at a 16-byte
  * aligned address and k a multiple of 256 take these roads; where they do not, 1 and 2 rows are a class of their own, as
  * two f16 halves, and 3 to 8 belong to the second.)
