@@ -540,9 +540,9 @@ int launch_rope_encode_chunk(hipStream_t st, int q4, float *q, float *k, const f
 // to append behind them (front_flat has the reasons).
 //
 // What a launch over few rows costs beside the launch itself is the chain of loads that wait for one another.  So the
-// pointers to the row, the weights and the positions are leading arguments, which arrive in registers (14 dwords); the other
-// arguments and the position come in one round trip, in the shadow of the row, and the table's in the next; no vector load
-// lies in between, whose wait would be one for the rows as well.  (Arguments, the rest of them, the append's, the
+// pointers to the row, the weights, the table and the positions are leading arguments, which arrive in registers (14 dwords);
+// the other arguments and the position come in one round trip, in the shadow of the row, and the table's in the next; no
+// vector load lies in between, whose wait would be one for the rows as well.  (Arguments, the rest of them, the append's, the
 // position, the sections' positions as a vector load, the table and the append's position were seven, one behind the other: us
 // a launch, replayed, over 3 rows with append 2.93 -> 2.60, over 24 without 2.34 -> 2.20; an empty launch 1.58.)
 enum { kFrontIds, kFrontRows, kFrontChunk }; // where a row's position comes from
@@ -551,10 +551,10 @@ struct FrontArgs {
     const float *v;      // [rows][n_kv][256]
     uint8_t *kc, *vc;    // caches
     size_t slot_bytes;   // kFrontRows: sequence r's cache starts r * slot_bytes into kc / vc
-    const float *tab;
+    const float *tab;    // (of a flat launch)
     int n_rot, s0, s1, s2, s3, pos0, stride, tab_rows;
     float theta, eps;
-    uint32_t kv_inverse; // as head_inverse, of n_kv (unused where that is 1)
+    uint32_t kv_inverse; // (of a flat launch) as head_inverse, of n_kv; unused where that is 1
 };
 
 // ENC: 0 = front end only, 1 = also quantize the finished K row and the V row to q8_0 and append
@@ -563,35 +563,14 @@ struct FrontArgs {
 // waves per row take the V rows.  Same expressions on the same values: the bits of the two launches.
 // posp: kFrontIds (one row) the four M-RoPE ids, with ENC the append's position four before them (the step buffer);
 // kFrontRows [rows][2], a row's text position first; kFrontChunk unused, row r is at pos0 + r.
-// FLAT: one grid dimension; head_inverse is 2^32 / (n_heads + n_kv), rounded up: the high half of its product with a wave's
-// number is the wave's row (exact while wave x heads is below 2^32).
-template <int ENC, bool FLAT>
-__global__ void __launch_bounds__(256) front_kernel(const float *__restrict__ qg, float *k, const float *__restrict__ qw,
-                                                    const float *__restrict__ kw, const int32_t *__restrict__ posp,
-                                                    uint32_t heads_mode, int n_kv, int rows, uint32_t head_inverse,
-                                                    const FrontArgs a)
+template <int ENC>
+__device__ __forceinline__ void front_head(const float *__restrict__ qg, float *k, const float *__restrict__ qw,
+                                           const float *__restrict__ kw, const float *__restrict__ tab,
+                                           const int32_t *__restrict__ posp, uint32_t heads_mode, int n_kv, const FrontArgs &a,
+                                           int row, int hb, int wave, int lane, float (&buf)[4][kHeadDim])
 {
-    __shared__ float buf[4][kHeadDim];
-    // (the wave's number as a scalar: row, head and addresses are scalar arithmetic then; the gate's half, which is copied as
-    // it is, 16 bytes a lane.  Tried: 16 bytes a lane for the q rows, 17.3 us over 672 rows where this takes 15: the tree's
-    // exchanges four times over)
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    // hb: a q head of the row, behind those a K head, behind those a V head
     const int n_heads = (int)(heads_mode & 0x3fffffffu), mode = (int)(heads_mode >> 30);
-    int row = blockIdx.y, hb = blockIdx.x * 4 + wave; // hb: q head, behind those K head, behind those V head
-    if (FLAT) {
-        const uint32_t heads = (uint32_t)(n_heads + n_kv), front = heads * (uint32_t)rows, i = (uint32_t)hb;
-        if (i < front) {
-            row = (int)__umulhi(i, head_inverse);
-            hb = (int)(i - (uint32_t)row * heads);
-        } else {
-            if (!ENC || i - front >= (uint32_t)(n_kv * rows))
-                return;
-            row = (int)(n_kv == 1 ? i - front : __umulhi(i - front, a.kv_inverse));
-            hb = (int)(heads + i - front - (uint32_t)(row * n_kv));
-        }
-    } else if (hb >= n_heads + n_kv + (ENC ? n_kv : 0)) {
-        return; // no workgroup-wide barrier below: waves are independent
-    }
     const int lane32 = lane & 31;
     // the position, and the append's
     int id[4] = {0, 0, 0, 0}, at = 0;
@@ -660,7 +639,7 @@ __global__ void __launch_bounds__(256) front_kernel(const float *__restrict__ qg
             p = sc < a.s0 ? id[0] : sc < a.s0 + a.s1 ? id[1] : sc < a.s0 + a.s1 + a.s2 ? id[2] : id[3];
         }
         if (e < a.n_rot)
-            rope_cs(a.tab, a.tab_rows, half, c, p, a.n_rot, a.theta, cs[j], sn[j]);
+            rope_cs(tab, a.tab_rows, half, c, p, a.n_rot, a.theta, cs[j], sn[j]);
     }
     if (is_q)
         *reinterpret_cast<float4a4 *>(a.gate + ((size_t)row * n_heads + h) * kHeadDim + 4 * lane) = g;
@@ -704,6 +683,47 @@ __global__ void __launch_bounds__(256) front_kernel(const float *__restrict__ qg
                 q8_encode_store(x[j], kc + blk * kQ8BlockBytes, lane32);
         }
     }
+}
+
+// (The wave's number as a scalar: row, head and addresses are scalar arithmetic then; the gate's half, which is copied as
+// it is, 16 bytes a lane.  Tried: 16 bytes a lane for the q rows, 17.3 us over 672 rows where this takes 15: the tree's
+// exchanges four times over.)  No workgroup-wide barrier: waves are independent.
+template <int ENC>
+__global__ void __launch_bounds__(256) front_kernel(const float *__restrict__ qg, float *k, const float *__restrict__ qw,
+                                                    const float *__restrict__ kw, const float *__restrict__ tab,
+                                                    const int32_t *__restrict__ posp, uint32_t heads_mode, int n_kv,
+                                                    const FrontArgs a)
+{
+    __shared__ float buf[4][kHeadDim];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int hb = blockIdx.x * 4 + wave;
+    if (hb >= (int)(heads_mode & 0x3fffffffu) + n_kv + (ENC ? n_kv : 0))
+        return;
+    front_head<ENC>(qg, k, qw, kw, tab, posp, heads_mode, n_kv, a, blockIdx.y, hb, wave, lane, buf);
+}
+
+// head_inverse: 2^32 / (n_heads + n_kv), rounded up.  The high half of its product with a wave's number is the wave's row: exact
+// while wave x heads is below 2^32.
+template <int ENC>
+__global__ void __launch_bounds__(256) front_flat_kernel(const float *__restrict__ qg, float *k, const float *__restrict__ qw,
+                                                         const float *__restrict__ kw, const int32_t *__restrict__ posp,
+                                                         uint32_t heads_mode, int n_kv, int rows, uint32_t head_inverse,
+                                                         const FrontArgs a)
+{
+    __shared__ float buf[4][kHeadDim];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const uint32_t i = blockIdx.x * 4 + wave, heads = (heads_mode & 0x3fffffffu) + (uint32_t)n_kv, front = heads * (uint32_t)rows;
+    int row, hb;
+    if (i < front) {
+        row = (int)__umulhi(i, head_inverse);
+        hb = (int)(i - (uint32_t)row * heads);
+    } else {
+        if (!ENC || i - front >= (uint32_t)(n_kv * rows))
+            return;
+        row = (int)(n_kv == 1 ? i - front : __umulhi(i - front, a.kv_inverse));
+        hb = (int)(heads + i - front - (uint32_t)(row * n_kv));
+    }
+    front_head<ENC>(qg, k, qw, kw, a.tab, posp, heads_mode, n_kv, a, row, hb, wave, lane, buf);
 }
 
 // Rows of a launch (grid.y).
@@ -769,12 +789,17 @@ int launch_front(hipStream_t st, const float *qg, float *q, float *gate, float *
         // (the append's positions are the rotation's: the step buffer's own lies four in front of its ids, the others are the same)
         const int32_t *posp = pos ? pos : rowpos ? rowpos + (size_t)r0 * 2 : nullptr;
         const uint32_t mode = pos ? kFrontIds : rowpos ? kFrontRows : kFrontChunk;
-        auto kern = flat ? enc < 0 ? front_kernel<0, true> : enc == 0 ? front_kernel<1, true> : front_kernel<2, true>
-                         : enc < 0 ? front_kernel<0, false> : enc == 0 ? front_kernel<1, false> : front_kernel<2, false>;
-        const dim3 grid = flat ? dim3((unsigned)(waves * n + 3) / 4, 1, 1)
-                               : dim3((unsigned)(waves + 3) / 4, (unsigned)n, 1);
-        HIPML_LAUNCH(kern, grid, dim3(256, 1, 1), 0, st, qg + (size_t)r0 * n_heads * 2 * kHeadDim,
-                     k + (size_t)r0 * n_kv * kHeadDim, qw, kw, posp, (uint32_t)n_heads | mode << 30, n_kv, n, inverse(heads), a);
+        const float *qg0 = qg + (size_t)r0 * n_heads * 2 * kHeadDim;
+        float *k0 = k + (size_t)r0 * n_kv * kHeadDim;
+        const uint32_t heads_mode = (uint32_t)n_heads | mode << 30;
+        if (flat)
+            HIPML_LAUNCH(enc < 0 ? front_flat_kernel<0> : enc == 0 ? front_flat_kernel<1> : front_flat_kernel<2>,
+                         dim3((unsigned)(waves * n + 3) / 4, 1, 1), dim3(256, 1, 1), 0, st, qg0, k0, qw, kw, posp, heads_mode, n_kv, n,
+                         inverse(heads), a);
+        else
+            HIPML_LAUNCH(enc < 0 ? front_kernel<0> : enc == 0 ? front_kernel<1> : front_kernel<2>,
+                         dim3((unsigned)(waves + 3) / 4, (unsigned)n, 1), dim3(256, 1, 1), 0, st, qg0, k0, qw, kw, t, posp, heads_mode,
+                         n_kv, a);
         int rc = launched(enc < 0 ? "attn_front_f32" : "attn_front_encode_f32");
         if (rc)
             return rc;
