@@ -732,18 +732,22 @@ static constexpr int kFrontMaxRows = 32768;
 // Whether a launch is flat (above).  Its waves find their row by a product, and a V row's first needs an argument from memory:
 // up to 7 % over few rows (24 + 4 heads with append, 8 rows: 3.5 us by rows, 3.7 flat).  It is flat all the same
 //   - where the workgroups of a row are a multiple of eight, with whole ones for K and for V: workgroups go to the XCDs in turn,
-//     so by rows one XCD gets all the K rows, another all the V rows and the others all the q rows.  That tells while a launch is
-//     about one round of workgroups (2,048 are resident), above the latency and below the bandwidth of the whole chip: 24 + 4
-//     heads with append over 96 / 128 / 160 / 257 / 320 / 416 / 512 / 600 rows 4.5 / 5.1 / 5.6 / 7.6 / 8.5 / 10.1 / 11.6 / 13.0 us by
-//     rows and 4.5 / 4.9 / 5.2 / 6.2 / 7.1 / 9.3 / 11.5 / 13.1 flat; 48 + 8 heads over 64 / 128 / 192 / 256 rows 5.3 / 7.4 / 9.5 /
-//     11.6 and 4.9 / 6.1 / 8.5 / 11.1.  (Flat with other counts of workgroups, or with fewer KV heads, is 5 % faster to 20 % slower.)
-//   - where a quarter of the waves by rows would have no row: 5 + 1 heads without append over 257 / 1,024 / 2,048 rows 3.5 / 5.3 /
-//     9.7 us by rows and 3.5 / 5.1 / 8.3 flat, 3 + 1 with append 4.0 / 6.0 / 9.5 and 3.9 / 5.0 / 7.2.
-// The product needs wave x heads below 2^32: 17,600 waves at most in the first case, 9 heads x 32,768 rows in the second.
+//     so by rows one XCD gets all the K rows, another all the V rows and the others all the q rows, seven eighths of the bytes.
+//     It tells from a round of workgroups on (2,048 are resident) and where the rows are in the caches, as the projections leave
+//     them: 24 + 4 heads with append, in a layer, over 257 / 420 / 672 / 1,024 / 1,400 / 2,048 rows 8.9 / 11.8 / 16.8 / 23.6 / 30.9 /
+//     43.4 us by rows and 8.4 / 11.2 / 15.5 / 22.5 / 29.7 / 40.0 flat (the layer 0 to 2 us less); over 130 to 224 rows neither is
+//     ahead, over 16,000 flat is 4 % behind.  The same rows again and again 7.6 / 10.1 over 257 / 416 and 6.2 / 9.3; from HBM by
+//     rows is the faster one, 8.8 / 17.3 over 257 / 672 and 9.2 / 18.2.  (Flat with other counts of workgroups, or with fewer KV
+//     heads, is 5 % faster to 20 % slower, the same rows again and again);
+//   - where a quarter of the waves by rows would have no row, wherever the rows are: 5 + 1 heads without append over 300 / 1,024 /
+//     2,048 rows 3.9 / 7.8 / 12.8 us by rows and 3.8 / 6.8 / 11.8 flat, 3 + 1 with append 4.5 / 7.2 / 11.7 and 4.4 / 6.6 / 10.4, from
+//     HBM; over 257 / 2,048 rows again and again 3.5 / 9.7 and 3.5 / 8.3, 4.0 / 9.5 and 3.9 / 7.2.
 static bool front_flat(int n_heads, int n_kv, int rows, bool append)
 {
     const long long waves = (long long)n_heads + n_kv + (append ? n_kv : 0), row_wgs = (waves + 3) / 4, wgs = row_wgs * rows;
-    return (append && n_kv >= 4 && row_wgs % 8 == 0 && wgs >= 800 && wgs <= 4400) || (wgs >= 500 && 3 * row_wgs >= waves);
+    if (waves * waves * rows >> 32 != 0) // (more than the product is exact for)
+        return false;
+    return (append && n_kv >= 4 && row_wgs % 8 == 0 && wgs >= 2048 && wgs <= 40000) || (wgs >= 500 && 3 * row_wgs >= waves);
 }
 
 // For tests.

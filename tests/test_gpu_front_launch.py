@@ -14,7 +14,7 @@ def flat(n_heads, n_kv, rows, append):
 
 
 def test_which_launches_are_flat():
-    assert [flat(24, 4, rows, True) for rows in (1, 99, 100, 257, 550, 551, 672)] == [False, False, True, True, True, False, False]
+    assert [flat(24, 4, rows, True) for rows in (1, 255, 256, 672, 5000, 5001)] == [False, False, True, True, True, False]
     assert not any(flat(24, 4, rows, False) for rows in (1, 257, 2048))
     assert not any(flat(h, kv, 257, True) for h, kv in ((28, 2), (32, 8), (16, 2), (14, 2), (40, 8)))
     assert [flat(5, 1, rows, False) for rows in (249, 250, 2048)] == [False, True, True]
@@ -74,8 +74,8 @@ def inputs(n_heads, n_kv, rows, seed):
 # both sides of the rule's lines, ragged last workgroups, one and several KV heads
 @pytest.mark.gpu
 @pytest.mark.parametrize("n_heads,n_kv,rows,dtype,is_flat", [
-    (24, 4, 99, 0, False), (24, 4, 100, 0, True), (24, 4, 257, 1, True), (24, 4, 550, 0, True), (24, 4, 551, 0, False),
-    (48, 8, 67, 0, True), (26, 6, 101, 1, False), (27, 5, 101, 0, False), (20, 5, 131, 0, True), (5, 1, 251, None, True),
+    (24, 4, 255, 0, False), (24, 4, 256, 0, True), (24, 4, 257, 1, True), (24, 4, 673, 0, True),
+    (48, 8, 129, 0, True), (26, 6, 261, 1, False), (27, 5, 261, 0, False), (20, 5, 257, 0, True), (5, 1, 251, None, True),
     (5, 1, 251, 0, False), (3, 1, 337, 0, True), (3, 1, 337, 1, True), (1, 1, 513, 0, True), (2, 2, 513, 1, True)])
 def test_one_launch_has_the_bits_of_small_ones(n_heads, n_kv, rows, dtype, is_flat):
     assert flat(n_heads, n_kv, rows, dtype is not None) == is_flat and not flat(n_heads, n_kv, 47, dtype is not None)
