@@ -551,10 +551,11 @@ struct FrontArgs {
     const float *v;      // [rows][n_kv][256]
     uint8_t *kc, *vc;    // caches
     size_t slot_bytes;   // kFrontRows: sequence r's cache starts r * slot_bytes into kc / vc
-    const float *tab;    // (of a flat launch)
     int n_rot, s0, s1, s2, s3, pos0, stride, tab_rows;
     float theta, eps;
-    uint32_t kv_inverse; // (of a flat launch) as head_inverse, of n_kv; unused where that is 1
+    // of a flat launch: the table, and as head_inverse, of n_kv (unused where that is 1)
+    const float *tab;
+    uint32_t kv_inverse;
 };
 
 // ENC: 0 = front end only, 1 = also quantize the finished K row and the V row to q8_0 and append
@@ -796,14 +797,14 @@ int launch_front(hipStream_t st, const float *qg, float *q, float *gate, float *
         const float *qg0 = qg + (size_t)r0 * n_heads * 2 * kHeadDim;
         float *k0 = k + (size_t)r0 * n_kv * kHeadDim;
         const uint32_t heads_mode = (uint32_t)n_heads | mode << 30;
-        if (flat)
-            HIPML_LAUNCH(enc < 0 ? front_flat_kernel<0> : enc == 0 ? front_flat_kernel<1> : front_flat_kernel<2>,
-                         dim3((unsigned)(waves * n + 3) / 4, 1, 1), dim3(256, 1, 1), 0, st, qg0, k0, qw, kw, posp, heads_mode, n_kv, n,
-                         inverse(heads), a);
-        else
+        if (!flat)
             HIPML_LAUNCH(enc < 0 ? front_kernel<0> : enc == 0 ? front_kernel<1> : front_kernel<2>,
                          dim3((unsigned)(waves + 3) / 4, (unsigned)n, 1), dim3(256, 1, 1), 0, st, qg0, k0, qw, kw, t, posp, heads_mode,
                          n_kv, a);
+        else
+            HIPML_LAUNCH(enc < 0 ? front_flat_kernel<0> : enc == 0 ? front_flat_kernel<1> : front_flat_kernel<2>,
+                         dim3((unsigned)(waves * n + 3) / 4, 1, 1), dim3(256, 1, 1), 0, st, qg0, k0, qw, kw, posp, heads_mode, n_kv, n,
+                         inverse(heads), a);
         int rc = launched(enc < 0 ? "attn_front_f32" : "attn_front_encode_f32");
         if (rc)
             return rc;
