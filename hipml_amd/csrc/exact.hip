@@ -204,12 +204,14 @@ int launch_kv_encode(hipStream_t st, int q4, const float *k, const float *v, uin
 // one f32 ulp of the table but not bit-identical to it.  The kernels take the table's row count with
 // a sign: tab_rows >= 0 allows the device angles, -(rows) - 1 does not.
 
-__device__ __forceinline__ int rope_rows(int tab_rows) { return tab_rows >= 0 ? tab_rows : -(tab_rows + 1); }
+__host__ __device__ __forceinline__ int rope_rows(int tab_rows) { return tab_rows >= 0 ? tab_rows : -(tab_rows + 1); }
 
 __device__ __forceinline__ void rope_cs(const float *__restrict__ tab, int tab_rows, int half,
                                         int k, int p, int n_rot, float theta, float &cs, float &sn)
 {
-    if (tab != nullptr && p >= 0 && p < rope_rows(tab_rows)) {
+    // (expected, so that the device's own angles, 4 KB of code at every place, lie behind a kernel's path and not in it: amidst it a
+    // layer over 32 sequences took up to 1 us more by where front_kernel happened to be loaded)
+    if (__builtin_expect(tab != nullptr && p >= 0 && p < rope_rows(tab_rows), 1)) {
         const float2 e = reinterpret_cast<const float2 *>(tab)[(size_t)p * half + k];
         cs = e.x;
         sn = e.y;
@@ -564,14 +566,15 @@ struct FrontArgs {
 // waves per row take the V rows.  Same expressions on the same values: the bits of the two launches.
 // posp: kFrontIds (one row) the four M-RoPE ids, with ENC the append's position four before them (the step buffer);
 // kFrontRows [rows][2], a row's text position first; kFrontChunk unused, row r is at pos0 + r.
-template <int ENC>
+// CHUNK: kFrontChunk with every position inside the table, so that the angles computed on the device, most of the code, are not in.
+template <int ENC, bool CHUNK>
 __device__ __forceinline__ void front_head(const float *__restrict__ qg, float *k, const float *__restrict__ qw,
                                            const float *__restrict__ kw, const float *__restrict__ tab,
                                            const int32_t *__restrict__ posp, uint32_t heads_mode, int n_kv, const FrontArgs &a,
                                            int row, int hb, int wave, int lane, float (&buf)[4][kHeadDim])
 {
     // hb: a q head of the row, behind those a K head, behind those a V head
-    const int n_heads = (int)(heads_mode & 0x3fffffffu), mode = (int)(heads_mode >> 30);
+    const int n_heads = (int)(heads_mode & 0x3fffffffu), mode = CHUNK ? kFrontChunk : (int)(heads_mode >> 30);
     const int lane32 = lane & 31;
     // the position, and the append's
     int id[4] = {0, 0, 0, 0}, at = 0;
@@ -639,8 +642,13 @@ __device__ __forceinline__ void front_head(const float *__restrict__ qg, float *
             const int sc = sect >= half ? c : c % sect;
             p = sc < a.s0 ? id[0] : sc < a.s0 + a.s1 ? id[1] : sc < a.s0 + a.s1 + a.s2 ? id[2] : id[3];
         }
-        if (e < a.n_rot)
+        if (CHUNK && e < a.n_rot) {
+            const float2 at_p = reinterpret_cast<const float2 *>(tab)[(size_t)p * half + c];
+            cs[j] = at_p.x;
+            sn[j] = at_p.y;
+        } else if (e < a.n_rot) {
             rope_cs(tab, a.tab_rows, half, c, p, a.n_rot, a.theta, cs[j], sn[j]);
+        }
     }
     if (is_q)
         *reinterpret_cast<float4a4 *>(a.gate + ((size_t)row * n_heads + h) * kHeadDim + 4 * lane) = g;
@@ -700,20 +708,19 @@ __global__ void __launch_bounds__(256) front_kernel(const float *__restrict__ qg
     const int hb = blockIdx.x * 4 + wave;
     if (hb >= (int)(heads_mode & 0x3fffffffu) + n_kv + (ENC ? n_kv : 0))
         return;
-    front_head<ENC>(qg, k, qw, kw, tab, posp, heads_mode, n_kv, a, blockIdx.y, hb, wave, lane, buf);
+    front_head<ENC, false>(qg, k, qw, kw, tab, posp, heads_mode, n_kv, a, blockIdx.y, hb, wave, lane, buf);
 }
 
-// head_inverse: 2^32 / (n_heads + n_kv), rounded up.  The high half of its product with a wave's number is the wave's row: exact
+// Chunks whose positions lie inside the table.  head_inverse: 2^32 / (n_heads + n_kv), rounded up.  The high half of its product with a wave's number is the wave's row: exact
 // while wave x heads is below 2^32.
 template <int ENC>
 __global__ void __launch_bounds__(256) front_flat_kernel(const float *__restrict__ qg, float *k, const float *__restrict__ qw,
-                                                         const float *__restrict__ kw, const int32_t *__restrict__ posp,
-                                                         uint32_t heads_mode, int n_kv, int rows, uint32_t head_inverse,
-                                                         const FrontArgs a)
+                                                         const float *__restrict__ kw, int n_heads, int n_kv, int rows,
+                                                         uint32_t head_inverse, const FrontArgs a)
 {
     __shared__ float buf[4][kHeadDim];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-    const uint32_t i = blockIdx.x * 4 + wave, heads = (heads_mode & 0x3fffffffu) + (uint32_t)n_kv, front = heads * (uint32_t)rows;
+    const uint32_t i = blockIdx.x * 4 + wave, heads = (uint32_t)(n_heads + n_kv), front = heads * (uint32_t)rows;
     int row, hb;
     if (i < front) {
         row = (int)__umulhi(i, head_inverse);
@@ -724,13 +731,13 @@ __global__ void __launch_bounds__(256) front_flat_kernel(const float *__restrict
         row = (int)(n_kv == 1 ? i - front : __umulhi(i - front, a.kv_inverse));
         hb = (int)(heads + i - front - (uint32_t)(row * n_kv));
     }
-    front_head<ENC>(qg, k, qw, kw, a.tab, posp, heads_mode, n_kv, a, row, hb, wave, lane, buf);
+    front_head<ENC, true>(qg, k, qw, kw, a.tab, nullptr, (uint32_t)n_heads, n_kv, a, row, hb, wave, lane, buf);
 }
 
 // Rows of a launch (grid.y).
 static constexpr int kFrontMaxRows = 32768;
 
-// Whether a launch is flat (above).  Its waves find their row by a product, and a V row's first needs an argument from memory:
+// Whether a chunk's launch is flat (above).  Its waves find their row by a product, and a V row's first needs an argument from memory:
 // up to 7 % over few rows (24 + 4 heads with append, 8 rows: 3.5 us by rows, 3.7 flat).  It is flat all the same
 //   - where the workgroups of a row are a multiple of eight, with whole ones for K and for V: workgroups go to the XCDs in turn,
 //     so by rows one XCD gets all the K rows, another all the V rows and the others all the q rows, seven eighths of the bytes.
@@ -770,7 +777,8 @@ int launch_front(hipStream_t st, const float *qg, float *q, float *gate, float *
     auto inverse = [](int d) { return (uint32_t)((0xffffffffull + (uint64_t)d) / (uint64_t)d); };
     for (int r0 = 0; r0 < rows; r0 += kFrontMaxRows) {
         const int n = rows - r0 < kFrontMaxRows ? rows - r0 : kFrontMaxRows;
-        const bool flat = front_flat(n_heads, n_kv, n, enc >= 0);
+        const bool flat = !pos && !rowpos && t && pos0 >= 0 && (long long)pos0 + r0 + n <= rope_rows(tab_rows) &&
+                          front_flat(n_heads, n_kv, n, enc >= 0);
         const size_t slot_at = rowpos ? (size_t)r0 * slot_bytes : 0;
         FrontArgs a;
         a.q = q + (size_t)r0 * n_heads * kHeadDim;
@@ -803,8 +811,8 @@ int launch_front(hipStream_t st, const float *qg, float *q, float *gate, float *
                          n_kv, a);
         else
             HIPML_LAUNCH(enc < 0 ? front_flat_kernel<0> : enc == 0 ? front_flat_kernel<1> : front_flat_kernel<2>,
-                         dim3((unsigned)(waves * n + 3) / 4, 1, 1), dim3(256, 1, 1), 0, st, qg0, k0, qw, kw, posp, heads_mode, n_kv, n,
-                         inverse(heads), a);
+                         dim3((unsigned)(waves * n + 3) / 4, 1, 1), dim3(256, 1, 1), 0, st, qg0, k0, qw, kw, n_heads, n_kv, n, inverse(heads),
+                         a);
         int rc = launched(enc < 0 ? "attn_front_f32" : "attn_front_encode_f32");
         if (rc)
             return rc;

@@ -35,20 +35,15 @@ def test_rows_found_by_a_product(n_heads, n_kv, append):
             assert np.array_equal(waves * inverse >> np.uint64(32), waves // np.uint64(d))
 
 
-def run(dtype, qg, k, v, qw, kw, n_heads, n_kv, pos0, stride, cuts, caches, pos=None):
-    """The chunk's front end (with append where dtype is not None) as one call per piece between two cuts; with `pos` the rows of
-    a batch of sequences, a cache slot each."""
+def run(dtype, qg, k, v, qw, kw, n_heads, n_kv, pos0, stride, cuts, caches):
+    """The chunk's front end (with append where dtype is not None) as one call per piece between two cuts."""
     rows = qg.shape[0]
     q, gate = (torch.full((rows + 1, n_heads, HD), 7.0, device="cuda") for _ in range(2))
     kd = torch.cat((k, torch.full_like(k[:1], 7.0)))
     kc, vc = (c.clone() for c in caches)
     shape = (n_heads, n_kv, HD, N_ROT, THETA, EPS)
     for a, b in zip(cuts, cuts[1:]):
-        if pos is not None:
-            slot = kc[0].numel()
-            attn.front_rows_encode(dtype, qg[a:], kd[a:], v[a:], q[a:], gate[a:], qw, kw, kc[a:], vc[a:], *shape, stride, pos[a:],
-                                   slot, b - a)
-        elif dtype is None:
+        if dtype is None:
             attn.chunk_front(qg[a:], kd[a:], q[a:], gate[a:], qw, kw, *shape, pos0 + a, b - a)
         else:
             attn.chunk_front_encode(dtype, qg[a:], kd[a:], v[a:], q[a:], gate[a:], qw, kw, kc, vc, *shape, pos0 + a, b - a, stride)
@@ -92,19 +87,25 @@ def test_one_launch_has_the_bits_of_small_ones(n_heads, n_kv, rows, dtype, is_fl
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("n_heads,n_kv,dtype", [(24, 4, 0), (24, 4, 1), (3, 1, 0)])
-def test_a_flat_launch_over_a_batch(n_heads, n_kv, dtype):
-    rows, stride = 260, 96
+@pytest.mark.parametrize("append", [False, True])
+def test_a_chunk_that_leaves_the_table(append):
+    # angles of positions past the table are computed on the device, where that is allowed: by rows, whatever the shape
+    rows, n_heads, n_kv = 300, 24, 4
+    made = inputs(n_heads, n_kv, rows, 11)
     assert flat(n_heads, n_kv, rows, True)
-    made = inputs(n_heads, n_kv, rows, 77 + n_heads)
-    at = torch.randint(0, stride, (rows, 1), dtype=torch.int32, device="cuda")
-    caches = [torch.full((rows, n_kv, stride, 144 if dtype == 1 else 272), 0x5A, dtype=torch.uint8, device="cuda") for _ in range(2)]
-    pos = torch.cat((at, at + 1), dim=1).contiguous()
-    args = (n_heads, n_kv, 0, stride)
-    one = run(dtype, *made, *args, [0, rows], caches, pos)
-    same(one, run(dtype, *made, *args, [*range(0, rows, 47), rows], caches, pos))
-    touched = (one[3] != 0x5A).any(dim=3).any(dim=1).sum(dim=1)
-    assert bool((touched == 1).all())
+    pos0, stride = 131_072 - rows + 1, 131_080
+    caches = [torch.full((n_kv, stride, 272), 0x5A, dtype=torch.uint8, device="cuda") for _ in range(2)]
+    args = (n_heads, n_kv, pos0, stride)
+    dtype = 0 if append else None
+    with pytest.raises(attn.HipmlError):
+        run(dtype, *made, *args, [0, rows], caches)
+    attn.rope_allow_device_angles(1)
+    try:
+        one, many = (run(dtype, *made, *args, cuts, caches) for cuts in ([0, rows], [*range(0, rows, 47), rows]))
+    finally:
+        attn.rope_allow_device_angles(0)
+    same(one, many)
+    assert bool(one[0][:rows].isfinite().all())
 
 
 @pytest.mark.gpu
