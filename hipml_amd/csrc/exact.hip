@@ -538,8 +538,8 @@ int launch_rope_encode_chunk(hipStream_t st, int q4, float *q, float *k, const f
 // exchanges; IEEE addition commutes, so every lane ends with red[0]); mean = sum / 256;
 // scale = 1 / sqrtf(mean + eps) with the correctly rounded divide and square root; the value is
 // (x * scale) * w; the rotation reads cos/sin as the other RoPE kernels here do.
-// Workgroups of 4 waves; grid (ceil(heads of a row / 4), rows), or flat: all q and K rows one behind the other and the V rows
-// to append behind them (front_flat has the reasons).
+// Workgroups of 4 waves; grid (ceil(heads of a row / 4), rows), or, where that leaves many waves without a row (front_flat), flat:
+// all q and K rows one behind the other and the V rows to append behind them.
 //
 // What a launch over few rows costs beside the launch itself is the chain of loads that wait for one another.  So the
 // pointers to the row, the weights, the table and the positions are leading arguments, which arrive in registers (14 dwords);
@@ -737,25 +737,18 @@ __global__ void __launch_bounds__(256) front_flat_kernel(const float *__restrict
 // Rows of a launch (grid.y).
 static constexpr int kFrontMaxRows = 32768;
 
-// Whether a chunk's launch is flat (above).  Its waves find their row by a product, and a V row's first needs an argument from memory:
-// up to 7 % over few rows (24 + 4 heads with append, 8 rows: 3.5 us by rows, 3.7 flat).  It is flat all the same
-//   - where the workgroups of a row are a multiple of eight, with whole ones for K and for V: workgroups go to the XCDs in turn,
-//     so by rows one XCD gets all the K rows, another all the V rows and the others all the q rows, seven eighths of the bytes.
-//     It tells from a round of workgroups on (2,048 are resident) and where the rows are in the caches, as the projections leave
-//     them: 24 + 4 heads with append, in a layer, over 257 / 420 / 672 / 1,024 / 1,400 / 2,048 rows 8.9 / 11.8 / 16.8 / 23.6 / 30.9 /
-//     43.4 us by rows and 8.4 / 11.2 / 15.5 / 22.5 / 29.7 / 40.0 flat (the layer 0 to 2 us less); over 130 to 224 rows neither is
-//     ahead, over 16,000 flat is 4 % behind.  The same rows again and again 7.6 / 10.1 over 257 / 416 and 6.2 / 9.3; from HBM by
-//     rows is the faster one, 8.8 / 17.3 over 257 / 672 and 9.2 / 18.2.  (Flat with other counts of workgroups, or with fewer KV
-//     heads, is 5 % faster to 20 % slower, the same rows again and again);
-//   - where a quarter of the waves by rows would have no row, wherever the rows are: 5 + 1 heads without append over 300 / 1,024 /
-//     2,048 rows 3.9 / 7.8 / 12.8 us by rows and 3.8 / 6.8 / 11.8 flat, 3 + 1 with append 4.5 / 7.2 / 11.7 and 4.4 / 6.6 / 10.4, from
-//     HBM; over 257 / 2,048 rows again and again 3.5 / 9.7 and 3.5 / 8.3, 4.0 / 9.5 and 3.9 / 7.2.
+// Whether a chunk's launch is flat (above): where a quarter of the waves by rows would have no row.  5 + 1 heads without append over
+// 300 / 1,024 / 2,048 rows 3.9 / 7.8 / 12.7 us by rows and 3.6 / 6.8 / 11.6 flat, 3 + 1 with append 4.5 / 7.2 / 11.6 and 4.3 / 6.7 /
+// 10.4, from HBM; over 257 / 2,048 rows again and again 3.5 / 9.8 and 3.5 / 8.4, 4.0 / 9.5 and 3.7 / 7.3.  Under 500 workgroups
+// neither is ahead.
+// Nowhere else: 24 + 4 heads with append, whose eight workgroups a row always go to the same XCDs (one gets all K rows, one all V
+// rows, the others all q rows), over 257 / 420 rows again and again 7.6 / 10.1 by rows and 6.2 / 9.3 flat, but 8.8 / 12.1 and 9.2 /
+// 12.9 from HBM, and layers of 257 to 4,096 tokens the same within 0.6 us.
 static bool front_flat(int n_heads, int n_kv, int rows, bool append)
 {
-    const long long waves = (long long)n_heads + n_kv + (append ? n_kv : 0), row_wgs = (waves + 3) / 4, wgs = row_wgs * rows;
-    if (waves * waves * rows >> 32 != 0) // (more than the product is exact for)
-        return false;
-    return (append && n_kv >= 4 && row_wgs % 8 == 0 && wgs >= 2048 && wgs <= 40000) || (wgs >= 500 && 3 * row_wgs >= waves);
+    const long long waves = (long long)n_heads + n_kv + (append ? n_kv : 0), row_wgs = (waves + 3) / 4;
+    // (that is 9 waves a row at most: far below what the product is exact for)
+    return row_wgs * rows >= 500 && 3 * row_wgs >= waves;
 }
 
 // For tests.
