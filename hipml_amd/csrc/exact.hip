@@ -711,8 +711,8 @@ __global__ void __launch_bounds__(256) front_kernel(const float *__restrict__ qg
     front_head<ENC, false>(qg, k, qw, kw, tab, posp, heads_mode, n_kv, a, blockIdx.y, hb, wave, lane, buf);
 }
 
-// Chunks whose positions lie inside the table.  head_inverse: 2^32 / (n_heads + n_kv), rounded up.  The high half of its product with a wave's number is the wave's row: exact
-// while wave x heads is below 2^32.
+// Chunks whose positions lie inside the table.  head_inverse: 2^32 / (n_heads + n_kv), rounded up.  The high half of its product
+// with a wave's number is the wave's row: exact while wave x heads is below 2^32.
 template <int ENC>
 __global__ void __launch_bounds__(256) front_flat_kernel(const float *__restrict__ qg, float *k, const float *__restrict__ qw,
                                                          const float *__restrict__ kw, int n_heads, int n_kv, int rows,
@@ -804,8 +804,8 @@ int launch_front(hipStream_t st, const float *qg, float *q, float *gate, float *
                          n_kv, a);
         else
             HIPML_LAUNCH(enc < 0 ? front_flat_kernel<0> : enc == 0 ? front_flat_kernel<1> : front_flat_kernel<2>,
-                         dim3((unsigned)(waves * n + 3) / 4, 1, 1), dim3(256, 1, 1), 0, st, qg0, k0, qw, kw, n_heads, n_kv, n, inverse(heads),
-                         a);
+                         dim3((unsigned)(waves * n + 3) / 4, 1, 1), dim3(256, 1, 1), 0, st, qg0, k0, qw, kw, n_heads, n_kv, n,
+                         inverse(heads), a);
         int rc = launched(enc < 0 ? "attn_front_f32" : "attn_front_encode_f32");
         if (rc)
             return rc;

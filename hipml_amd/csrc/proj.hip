@@ -1025,8 +1025,8 @@ struct UnitsShape {
     // with 4 / 3 / 2 of them 8.7 / 8.4 / 7.6 us from HBM and 7.4 / 7.3 / 6.7 from the last-level cache, 5120 x 6144 over 9 rows
     // with 3 / 2 13.8 / 12.8 from HBM.  By dwords as well, where it was up to four: over k 5184 from HBM and 3 / 9 / 24 / 64 / 128
     // rows 1,024 weight rows 8.5 / 9.9 / 10.2 / 10.8 / 14.4 -> 7.5 / 9.3 / 9.6 / 10.0 / 13.3, 5,120 11.3 / 12.4 / 16.9 / 26.9 / 49.3 ->
-    // 10.0 / 11.6 / 16.7 / 25.5 / 45.3, 12,288 19.0 / 19.8 / 24.9 / 52.7 / 98.1 -> 18.2 / 19.8 / 24.8 / 49.8 / 91.7 (the order of a
-    // turn, below, is in both); 216 shapes from 512 to 12,288 weight rows 12 % less to 1 % more.
+    // 10.0 / 11.6 / 16.7 / 25.5 / 45.3, 12,288 19.0 / 19.8 / 24.9 / 52.7 / 98.1 -> 18.2 / 19.8 / 24.8 / 49.8 / 91.7 (with
+    // the order of a turn below); 216 shapes from 512 to 12,288 weight rows 12 % less to 1 % more.
     static constexpr int kDepth = 2;
     static constexpr int kLds = kWaves * kDepth * kSlot + kRead;
     static constexpr int kChains = 8 / kWaves; // of a wave

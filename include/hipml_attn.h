@@ -88,9 +88,9 @@ int hipml_attn_batch_splits(int stride, int n_kv, int slots);
  * needs no scratch; 1 the single-pass kernel; n >= 2 that kernel over key slices with a scratch for n of
  * them and a merge launch.  n is what the scratch has to hold, not what runs: a call takes the count, of 2 to n, that
  * costs least at its shape, and for few tokens a kernel that slices inside its workgroups as well (2,000 tokens at
- * depth 300: 8, of which 3 run; 350 at 20,000: 14 and 7).  For long chunks behind a prefix at least as long (tokens >= 768 and pos0 >= tokens, or tokens >= 640
- * and pos0 >= 8 * tokens) n is larger
- * than the number of slices that run (hipml_attn_chunk_slices): the chunk entry points then write the
+ * depth 300: 8, of which 3 run; 350 at 20,000: 14 and 7).  For long chunks behind a prefix at least as long
+ * (tokens >= 768 and pos0 >= tokens, or tokens >= 640 and pos0 >= 8 * tokens) n is larger than the number of slices
+ * that run (hipml_attn_chunk_slices): the chunk entry points then write the
  * live rows of the cache as f16 tiles (70,656 bytes per KV head and 64 rows) into the tail of part_acc
  * and run the attention over those, which is faster than dequantizing inside the attention (2,048 tokens
  * at depth 100,000: n = 13 for 4 slices, 654 MB of scratch, 4.1 against 4.7 ms).  A caller that passes fewer
@@ -113,8 +113,8 @@ int hipml_attn_chunk_splits(int pos0, int tokens, int n_kv);
 /* The slice count (>= 1) for callers that want the sliced kernel whatever the shape (an upper bound, as above),
  * and for hipml_attn_chunk_kv_f16, which has no in-workgroup variant and runs exactly the count it is given: the
  * count that fills the chip's last round of workgroups, and for the long chunks named above the count that runs
- * fastest over f16 tiles, often fewer (1,024 tokens at depth 8,192: 2, 1,500 at 20,000: 3, 2,048 at 100,000: 4).  Elsewhere fewer slices than these can be
- * faster over the copy too (420 tokens at depth 5,003: 95 us with the 12, 83 with the 5 that a registered copy runs). */
+ * fastest over f16 tiles, often fewer (1,024 tokens at depth 8,192: 2, 1,500 at 20,000: 3, 2,048 at 100,000: 4).
+ * Elsewhere fewer slices than these can be faster over the copy too (420 tokens at depth 5,003: 95 us with the 12, 83 with the 5 that a registered copy runs). */
 int hipml_attn_chunk_slices(int pos0, int tokens, int n_kv);
 
 /* ---- RoPE ----------------------------------------------------------------
@@ -383,7 +383,8 @@ int hipml_attn_decode_one_launch(int on);
  * of the keys run, the count that costs least at this shape.  How that memory is used is the library's business (with a
  * count from hipml_attn_chunk_splits for a long chunk behind a prefix, and where that costs less, the rest of part_acc
  * holds the cache rows as f16 tiles for the length of the call), and nothing beyond those sizes is touched.  The bits of a
- * result depend on the slices that run: the same arguments give the same bits.
+ * result depend on the slices that run: the same arguments give the same bits while the
+ * cache has a registered copy (below), and while it has none.
  * Replaces AttnLayer::chunk_attention_q8_split -> attn_chunk_wmma_f16 /
  * attn_chunk_full_f16 + attn_chunk_combine_f32,
  * crates/hipml-kernels/src/attn_gpu/imp/attn_chunk_kv.rs:72-107,129-305. */
@@ -478,8 +479,8 @@ int hipml_attn_chunk_kv_f16(hipml_stream_t stream, const float *q, const void *k
  *   - hipml_attn_chunk_q8_split, _gate and _gate_f16 over (k_cache, v_cache) with the registered stride,
  *     n_kv and format and splits >= 2 read the tiles: at most min(splits, hipml_attn_chunk_slices) slices, with
  *     the bits of hipml_attn_chunk_kv_f16 over the count that runs, and no tiles made per call in the scratch
- *     (2,048 tokens at depth 100,000: 4.06 against 4.19 ms).  Up to 64 tokens behind 2,048 rows and more read the cache itself, which is faster for so few (32 tokens at depth 7,000: 29 us,
- *     over the copy 36), and an append of such a chunk costs 3 to 4 us more than without a copy: attach it to caches
+ *     (2,048 tokens at depth 100,000: 4.06 against 4.19 ms).  Up to 64 tokens behind 2,048 rows and more read the
+ *     cache itself, which is faster for so few (32 tokens at depth 7,000: 29 us, over the copy 36), and an append of such a chunk costs 3 to 4 us more than without a copy: attach it to caches
  *     that long chunks extend (us with the copy / without: 117 tokens at depth 20,000 81 / 87, 400 at 20,000 194 / 220).
  * The bookkeeping is host state that changes when a call is issued or captured, not when a captured
  * graph is replayed.  Rows written into the cache by any other means (a device copy, another library)
